@@ -90,7 +90,9 @@ int residentWorkgroups(int tile) {
       if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ti->kernel[v], (int)ti->threads, ti->lds))) return 0;
       perCU = std::min(perCU, n);
     }
-    const void* others[2] = { reinterpret_cast<const void*>(ti->chainKernel), reinterpret_cast<const void*>(ti->kernelNoChunkWaits) };
+    const void* others[5] = { reinterpret_cast<const void*>(ti->chainKernel), reinterpret_cast<const void*>(ti->kernelNoChunkWaits),
+                              reinterpret_cast<const void*>(ti->kernelOnce), reinterpret_cast<const void*>(ti->kernelOnceNoChunkWaits),
+                              reinterpret_cast<const void*>(ti->chainKernelOnce) };
     for (const void* k : others) {
       if (!k) continue;
       int n = 0;
@@ -327,8 +329,10 @@ cusync_error cusync_gemm_run(const cusync_gemm_args* a, void* stream) {
 
   const GemmParams p = gemmParams(a, ti, launched);
   void (*kernel)(GemmParams) = ti->kernel[a->a_mode == CUSYNC_A_SWIGLU ? 1 : 0];
-  // the few-row tiles come with a kernel compiled without the per-chunk waits, for stages that never make them
-  if (a->a_mode != CUSYNC_A_SWIGLU && ti->kernelNoChunkWaits && !waitsPerChunk(s)) kernel = ti->kernelNoChunkWaits;
+  // the few-row tiles come with a kernel compiled without the per-chunk waits, for stages that never make them, and
+  // both again for a grid of one row, which reads B once
+  if (ti->kernelOnce && s.grid.y == 1) kernel = waitsPerChunk(s) ? ti->kernelOnce : ti->kernelOnceNoChunkWaits;
+  else if (a->a_mode != CUSYNC_A_SWIGLU && ti->kernelNoChunkWaits && !waitsPerChunk(s)) kernel = ti->kernelNoChunkWaits;
   // A consumer's workgroups are dispatched while the producer's hold their CUs, and where two of them fit a CU the
   // dispatcher packs them in pairs onto the CUs the producer left free: when the producer is done, half the device
   // runs the consumer two to a CU and the other half nothing (LLaMA MLP, 640 to 1024 rows under RowSync: 144-175 us
@@ -381,8 +385,12 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
   launched = std::min<uint32_t>(launched, mostTiles);
   GemmChainParams cp = {};
   cp.count = (uint32_t)count;
-  for (int i = 0; i < count; i++) cp.gemm[i] = gemmParams(&args[i], ti, launched);
-  hipLaunchKernelGGL(ti->chainKernel, dim3(launched), dim3(ti->threads), ti->lds, (hipStream_t)stream, cp);
+  bool once = ti->chainKernelOnce != nullptr;
+  for (int i = 0; i < count; i++) {
+    cp.gemm[i] = gemmParams(&args[i], ti, launched);
+    once = once && args[i].stage.grid.y == 1;
+  }
+  hipLaunchKernelGGL(once ? ti->chainKernelOnce : ti->chainKernel, dim3(launched), dim3(ti->threads), ti->lds, (hipStream_t)stream, cp);
   if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
   return CUSYNC_SUCCESS;
 }

@@ -51,8 +51,16 @@
 namespace cusync {
 namespace gemm {
 
-template<int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_, int WAVES_PER_SIMD_ = 1, bool BT_ = false, bool PIPE_ = false, bool PINGPONG_ = false>
+template<int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_, int WAVES_PER_SIMD_ = 1, bool BT_ = false, bool PIPE_ = false, bool PINGPONG_ = false,
+         bool ONCE_ = false>
 struct DmaCfg {
+  // B is read by one row tile only (a grid of one row): its loads carry the non-temporal hint.  A launch of few rows
+  // is bound by streaming the weights, and a probe that only reads 151 MB takes 26.2 us with the hint and 29.0 without
+  // (5.8 against 5.2 TB/s, 1.9 GB at a time 6.9 against 6.1).  The MLPs at 1 / 64 rows, RowSync: GPT-3 69.3 / 81.9 ->
+  // 66.0 / 77.6 us, LLaMA 41.0 / 50.1 -> 40.6 / 48.9.  Where several row tiles read the same weights the hint costs the
+  // L2 lines the neighbours were about to ask for: 96 rows on 64-row tiles 96.9 -> 106.2 us, LLaMA at 512 rows
+  // 103.3 -> 119.8.
+  static constexpr bool ONCE = ONCE_;
   static constexpr bool PIPE = PIPE_;                      // barrier in the middle of a chunk, fragments prefetched across chunks
   static constexpr bool PINGPONG = PINGPONG_;              // K loop in assembly, operands in whole cache lines (see above)
   static constexpr bool BT = BT_;                          // B given as [N][K] (k contiguous), e.g. KRSC filters
@@ -94,10 +102,19 @@ struct DmaCfg {
   static_assert(!PINGPONG || (WAVES == 8 && !PIPE && !BT && BM == 256 && ((BN == 384 && BK == 32) || (BN == 192 && BK == 64))), "the assembly K loops are written for two tiles");
 };
 
+template<int BM, int BN, int BK, int WM, int WN, int STAGES, int WAVES_PER_SIMD>
+using DmaCfgOnce = DmaCfg<BM, BN, BK, WM, WN, STAGES, WAVES_PER_SIMD, false, false, false, true>;
+
 // One direct load: 64 lanes x 16 bytes from buffer `rsrc` at per-lane byte offset
 // `voff` into LDS at ldsAddr + 16*lane.  ldsAddr must be wave-uniform.
 __device__ __forceinline__ void loadToLds(uint4v rsrc, uint32_t ldsAddr, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(ldsAddr), "v"(voff), "s"(rsrc) : "memory");
+}
+
+// The same with the non-temporal hint.
+__device__ __forceinline__ void loadToLdsOnce(uint4v rsrc, uint32_t ldsAddr, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
                :: "s"(ldsAddr), "v"(voff), "s"(rsrc) : "memory");
 }
 
@@ -338,7 +355,8 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p) {
         uint32_t off;
         if constexpr (C::BT) off = (bVoff0[Q] != kOutOfRange && k0 + bLoadChunk[Q] * 8 < kEnd) ? bVoff0[Q] + k0 * 2 : kOutOfRange;
         else off = (bVoff0[Q] != kOutOfRange && k0 < kEnd) ? bVoff0[Q] + k0 * p.ldb * 2 : kOutOfRange;
-        loadToLds(rB, __builtin_amdgcn_readfirstlane(lds), off);
+        if constexpr (C::ONCE) loadToLdsOnce(rB, __builtin_amdgcn_readfirstlane(lds), off);
+        else loadToLds(rB, __builtin_amdgcn_readfirstlane(lds), off);
       } else {
         constexpr int QA = Q - C::B_LOADS;
         const bool aInRange = k0 + aLoadChunk * 8 < kEnd;   // never touch columns the slice has not waited for

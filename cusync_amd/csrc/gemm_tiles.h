@@ -23,6 +23,10 @@ struct TileInfo {
   // kernel[0] compiled without the per-chunk waits of the tile policies, for stages that wait for whole rows or
   // for nothing (the few-row direct-to-LDS tiles only, see CUSYNC_TILE_DMA_FEW)
   void (*kernelNoChunkWaits)(GemmParams);
+  // the few-row tiles for a grid of one row (DmaCfg::ONCE): with and without chunk waits, and several GEMMs
+  void (*kernelOnce)(GemmParams);
+  void (*kernelOnceNoChunkWaits)(GemmParams);
+  void (*chainKernelOnce)(GemmChainParams);
 };
 
 void fillStagedTiles(TileInfo* tiles);     // register-staged tiles (the only ones with a SwiGLU A operand)
@@ -34,12 +38,13 @@ void fillDmaTilesXWide(TileInfo* tiles);   // direct-to-LDS, 256x384, eight wave
 // Entry of a register-staged tile.
 #define CUSYNC_TILE(BM, BN, BK, WM, WN) \
   TileInfo{ BM, BN, BK, kThreads, (size_t)TileCfg<BM, BN, BK, WM, WN>::LDS_BYTES, \
-    { gemmKernel<TileCfg<BM, BN, BK, WM, WN>, false>, gemmKernel<TileCfg<BM, BN, BK, WM, WN>, true> }, -1, nullptr, nullptr }
+    { gemmKernel<TileCfg<BM, BN, BK, WM, WN>, false>, gemmKernel<TileCfg<BM, BN, BK, WM, WN>, true> }, -1, nullptr, nullptr, nullptr, nullptr, nullptr }
 
 // Entry of a direct-to-LDS tile: no SwiGLU variant (that operand needs arithmetic on its way into LDS).
 #define CUSYNC_TILE_DMA(...) \
   TileInfo{ DmaCfg<__VA_ARGS__>::BM, DmaCfg<__VA_ARGS__>::BN, DmaCfg<__VA_ARGS__>::BK, DmaCfg<__VA_ARGS__>::THREADS, \
-    (size_t)DmaCfg<__VA_ARGS__>::LDS_BYTES, { gemmDmaKernel<DmaCfg<__VA_ARGS__>>, nullptr }, -1, gemmDmaChainKernel<DmaCfg<__VA_ARGS__>>, nullptr }
+    (size_t)DmaCfg<__VA_ARGS__>::LDS_BYTES, { gemmDmaKernel<DmaCfg<__VA_ARGS__>>, nullptr }, -1, gemmDmaChainKernel<DmaCfg<__VA_ARGS__>>, \
+    nullptr, nullptr, nullptr, nullptr }
 
 // Entry of a few-row direct-to-LDS tile: also the kernel compiled without the per-chunk waits.  A launch of these
 // tiles is short (40 us), and the wait code a kernel carries without running it (stream order, RowSync) costs it
@@ -48,7 +53,8 @@ void fillDmaTilesXWide(TileInfo* tiles);   // direct-to-LDS, 256x384, eight wave
 #define CUSYNC_TILE_DMA_FEW(...) \
   TileInfo{ DmaCfg<__VA_ARGS__>::BM, DmaCfg<__VA_ARGS__>::BN, DmaCfg<__VA_ARGS__>::BK, DmaCfg<__VA_ARGS__>::THREADS, \
     (size_t)DmaCfg<__VA_ARGS__>::LDS_BYTES, { gemmDmaKernel<DmaCfg<__VA_ARGS__>>, nullptr }, -1, gemmDmaChainKernel<DmaCfg<__VA_ARGS__>>, \
-    gemmDmaKernel<DmaCfg<__VA_ARGS__>, kAPlain, false> }
+    gemmDmaKernel<DmaCfg<__VA_ARGS__>, kAPlain, false>, gemmDmaKernel<DmaCfgOnce<__VA_ARGS__>>, \
+    gemmDmaKernel<DmaCfgOnce<__VA_ARGS__>, kAPlain, false>, gemmDmaChainKernel<DmaCfgOnce<__VA_ARGS__>> }
 
 }  // namespace gemm
 }  // namespace cusync
