@@ -16,6 +16,7 @@
 #include "../../include/cusync_amd.h"
 #include "rt_internal.h"
 #include "attention_kernel.h"
+#include "attention_few_kernel.h"
 #include "split_choice.h"
 
 namespace {
@@ -24,15 +25,18 @@ using cusync::rt::setError;
 using namespace cusync::attn;
 
 std::mutex g_attnMutex;
-int g_attnResidentPerCU[2] = {-1, -1};      // [0] two stages, [1] four
+int g_attnResidentPerCU[3] = {-1, -1, -1};
 int g_attnNumCUs = 0;
 int g_attnLdsPerCU = 0;
 
 typedef void (*AttnKernel)(AttnParams);
-AttnKernel attnKernel(bool deep) { return deep ? attentionKernel<4> : attentionKernel<2>; }
-int attnLds(bool deep) { return cusync::attn::ldsBytes(deep ? 4 : 2); }
+// two or four blocks in LDS; up to 32 query rows and split key ranges: the keys over the wavefronts (16 rows behind 2048
+// in six blocks per split, 12 heads: the stage 25.8 -> 19.6 us, behind 8192 in twelve: 39 -> 25.8)
+enum Form { kShallow = 0, kDeep = 1, kFew = 2 };
+AttnKernel attnKernel(Form f) { return f == kFew ? attentionFewKernel : f == kDeep ? attentionKernel<4> : attentionKernel<2>; }
+int attnLds(Form f) { return f == kFew ? kFewLdsBytes : cusync::attn::ldsBytes(f == kDeep ? 4 : 2); }
 
-int residentAttention(bool deep);
+int residentAttention(Form form);
 
 // Four stages where the kernel has the device to itself anyway: as a stage of its own between stream-ordered
 // launches, and from 2048 key rows on, where the projections around it run 256-row tiles that take a whole CU's
@@ -45,23 +49,23 @@ int residentAttention(bool deep);
 bool deepPipeline(const cusync_attention_args* a) {
   const bool alone = a->stage.in.kind == CUSYNC_POLICY_NOSYNC && a->stage.out.kind == CUSYNC_POLICY_NOSYNC;
   if (alone || a->seq + a->cached_rows >= 2048) return true;
-  if (g_attnNumCUs == 0) residentAttention(false);      // reads the device's CU count
+  if (g_attnNumCUs == 0) residentAttention(kShallow);      // reads the device's CU count
   return g_attnNumCUs > 0 && a->stage.grid.x * a->stage.grid.y * a->stage.grid.z > (uint32_t)g_attnNumCUs;
 }
 
-int residentAttention(bool deep) {
+int residentAttention(Form form) {
   std::lock_guard<std::mutex> lock(g_attnMutex);
-  int& perCU = g_attnResidentPerCU[deep ? 1 : 0];
+  int& perCU = g_attnResidentPerCU[form];
   if (perCU < 0) {
     int dev = 0;
     hipDeviceProp_t prop;
     if (CUSYNC_HIP(hipGetDevice(&dev)) || CUSYNC_HIP(hipGetDeviceProperties(&prop, dev))) return 0;
     g_attnNumCUs = prop.multiProcessorCount;
     g_attnLdsPerCU = (int)prop.maxSharedMemoryPerMultiProcessor;
-    if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(attnKernel(deep)),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, std::max(attnLds(deep), g_attnLdsPerCU / 2)))) return 0;
+    if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(attnKernel(form)),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, std::max(attnLds(form), g_attnLdsPerCU / 2)))) return 0;
     int n = 0;
-    if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attnKernel(deep), kThreads, attnLds(deep)))) return 0;
+    if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attnKernel(form), kThreads, attnLds(form)))) return 0;
     perCU = n;
   }
   return perCU * g_attnNumCUs;
@@ -172,13 +176,13 @@ cusync_error cusync_attention_can_implement(const cusync_attention_args* a) {
   return CUSYNC_SUCCESS;
 }
 
-int cusync_attention_max_resident(void) { return residentAttention(false); }
+int cusync_attention_max_resident(void) { return residentAttention(kShallow); }
 
 cusync_error cusync_attention_run(const cusync_attention_args* a, void* stream) {
   cusync_error e = cusync_attention_can_implement(a);
   if (e != CUSYNC_SUCCESS) return e;
-  const bool deep = deepPipeline(a);
-  const int resident = residentAttention(deep);
+  const Form form = a->seq <= (uint32_t)kFewRows && a->stage.grid.z > 1 ? kFew : deepPipeline(a) ? kDeep : kShallow;
+  const int resident = residentAttention(form);
   if (resident <= 0) { setError("attention: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
   const cusync_stage_desc& s = a->stage;
   uint32_t launched = std::min<uint32_t>(s.grid.x * s.grid.y * s.grid.z, (uint32_t)resident);
@@ -212,11 +216,11 @@ cusync_error cusync_attention_run(const cusync_attention_args* a, void* stream) 
   // workgroups, 264 -> 244 us for the chain under every policy.  Not a launch of up to half as many workgroups as
   // CUs: packed, those are all resident beside the producer early and leave whole CUs to the output projection's
   // workgroups (512 rows, 96 workgroups: 124 us packed, 129 spread).
-  int lds = attnLds(deep);
+  int lds = attnLds(form);
   if (s.in.kind != CUSYNC_POLICY_NOSYNC && !(s.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL) && launched <= (uint32_t)g_attnNumCUs &&
       launched > (uint32_t)g_attnNumCUs / 2 && resident > g_attnNumCUs)
     lds = std::max(lds, g_attnLdsPerCU / 2);
-  hipLaunchKernelGGL(attnKernel(deep), dim3(launched), dim3(kThreads), lds, (hipStream_t)stream, p);
+  hipLaunchKernelGGL(attnKernel(form), dim3(launched), dim3(kThreads), lds, (hipStream_t)stream, p);
   if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
   cusync::rt::noteLaunch(s, launched >= (uint32_t)resident);
   return CUSYNC_SUCCESS;
@@ -267,8 +271,21 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   // 26.7 -> 25.3 us, 1024 rows 37.8 -> 30.8 us, 2048 rows 61 -> 50 us; finer cuts lose again (2048 rows in four:
   // 62 us, in eight: 89 us): every cut adds a tile's fixed cost (first blocks, Q fragments, a pass over the
   // partial results) and tickets without work.
+  // With a cache in front of the rows there are few row tiles and their key ranges are all long: the stage takes about
+  // (blocks per split) x the time of a block + (splits) x the time a split's share takes to be read back, and the two
+  // times are alike, so the blocks are cut into about as many splits as a split has blocks, within one workgroup per
+  // CU.  With several row tiles not below eight blocks (the chain under RowSync in us, half the range -> this: 16 rows
+  // behind 2048 66.5 -> 60.6, behind 8192 94.9 -> 67.5; 64 behind 2048 85.8 -> 75.4; 128 behind 8192 164.5 -> 107.2;
+  // 256 behind 4096 132 -> 109; 512 behind 2048 143 -> 135; 1 behind 512 57.1 -> 56.4).
   const uint32_t kvBlocks = (cfg->cached_rows + cfg->seq + kBKV - 1) / kBKV;
-  L->kvSplit = cfg->kv_split_blocks >= 0 ? (uint32_t)cfg->kv_split_blocks : kvBlocks >= 8 ? (kvBlocks + 1) / 2 : 0u;
+  uint32_t perSplit = kvBlocks >= 8 ? (kvBlocks + 1) / 2 : 0u;
+  if (cfg->cached_rows) {
+    if (residentAttention(kShallow) <= 0) { discardLayer(L); return nullptr; }      // reads the device's CU count
+    const uint32_t rowTiles = (cfg->seq + kBQ - 1) / kBQ, most = std::max(1u, (uint32_t)g_attnNumCUs / (cfg->heads * rowTiles));
+    perSplit = std::max((kvBlocks + most - 1) / most, rowTiles > 1 ? 8u : 1u);
+    while (perSplit * perSplit < kvBlocks) perSplit++;
+  }
+  L->kvSplit = cfg->kv_split_blocks >= 0 ? (uint32_t)cfg->kv_split_blocks : perSplit < kvBlocks ? perSplit : 0u;
   uint32_t tm1 = 0, tn1 = 0;
   if (cusync_gemm_tile_shape(L->tile1, &tm1, &tn1, nullptr) || cusync_gemm_tile_shape(L->tile3, nullptr, nullptr, nullptr)) {
     setError("attn layer: unknown tile id");
