@@ -180,7 +180,7 @@ def main():
             self.tiles = self.m.tiles()
 
         def step(self, split=False):
-            """One pass; elapsed microseconds by HIP events on the chain's own streams (a wait that gave up raises)."""
+            """One pass; microseconds from the first kernel's start to the last one's end by the device's clock (a wait that gave up raises)."""
             out = self.m.run(self.x.data_ptr(), self.h.data_ptr(), self.y.data_ptr(), runs=1, split=split)
             return (out[0][0], out[1][0], out[2][0]) if split else out[0]
 
@@ -236,7 +236,7 @@ def main():
         c.close()
 
     def roofline_leg(B, warm, timed):
-        """Durations of the two GEMM launches, HIP events on the stream they run on."""
+        """Durations of the two GEMM launches by the device's clock: first workgroup's start to last workgroup's end, and from there to the second's."""
         c = Chain(B, api.SYNC.STREAM)
         # The settling steps run on this very chain, with nothing between them and the timed ones: after an idle gap of
         # tens of milliseconds (a handle being created is one) the device runs these launches at boost for 2 ms, then
@@ -440,7 +440,8 @@ def main():
                 "default_launches": {k: 1 if v else 2 for k, v in default_one.items()},
                 "rowsync_default_us": round(m["rowsync_one_launch" if default_one["rowsync"] and "rowsync_one_launch" in m else "rowsync"][0], 2),
                 "tilesync_default_us": round(m["tilesync_one_launch" if default_one["tilesync"] and "tilesync_one_launch" in m else "tilesync"][0], 2),
-                # medians of 60 steps in the driver's process: the launcher objects' loop, and the handle beside it there
+                # medians of 60 steps in the driver's process: the launcher objects' loop by its events, and the handle beside
+                # it by the device's clock, which leaves out the 4 to 6 us that lie between the events and the kernels
                 "launcher_rowsync_us": launcher[(b, "rowsync")]["launcher_us"], "launcher_tilesync_us": launcher[(b, "tilesync")]["launcher_us"],
                 "launcher_vs_handle_pct": {k: round(launcher[(b, k)]["launcher_us"] / launcher[(b, k)]["handle_us"] * 100 - 100, 2)
                                            for k in ("rowsync", "tilesync")},
@@ -558,7 +559,8 @@ def main():
     # ---- the timed step: B = args.batch, CuSync against stream-ordered, interleaved ----------
     # Both policies and the stream-ordered pair are alive together and take turns, one step each per round: the
     # settling preamble (fixed, whatever --warmup says), then --warmup untimed rounds, then --steps timed rounds.
-    # `value` is the better policy's mean; the gain is computed from steps that ran next to each other.
+    # `value` is the better policy's mean, by the host's clock: launch, kernels and the return to the caller.  The gain is
+    # computed from steps that ran next to each other.
     settle(B)
     names = ["stream", "rowsync", "tilesync"]
     chains = [Chain(B, api.SYNC.STREAM), Chain(B, api.SYNC.ROW), Chain(B, api.SYNC.TILE)]
@@ -582,8 +584,9 @@ def main():
     for _ in range(args.steps):
         for n, c in zip(names, chains):
             t0 = time.perf_counter()
-            step_times[n].append(c.step())        # returns after the step's last kernel has finished
-            wall[n] += time.perf_counter() - t0
+            c.step()                              # returns when the step's last workgroup has its outputs in memory
+            step_times[n].append((time.perf_counter() - t0) * 1e6)
+            wall[n] += step_times[n][-1] / 1e6
     for c in chains:
         c.close()
     policy = min((n for n in names if n != "stream"), key=lambda k: statistics.fmean(step_times[k]))
@@ -596,7 +599,7 @@ def main():
     stream_mean = statistics.fmean(step_times["stream"])
     value = statistics.fmean(step_times[policy])
 
-    # the kernels' own durations (stream-ordered, HIP events on the launching stream) for the roofline
+    # the kernels' own durations (stream-ordered, device clock) for the roofline
     roof, _, _ = roofline_leg(B, 5, max(10, args.steps))
     # what the matrix pipes alone sustain on this machine (register operands, no LDS, no memory): the clock
     # drops under a device-wide MFMA load, further with random operands than with zeros

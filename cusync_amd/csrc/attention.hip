@@ -94,7 +94,7 @@ struct cusync_attn_layer {
   void* ws2;                       // workspace of the split attention
   cusync_stage_desc st[3];         // QKV projection, attention, output projection
   hipStream_t stream[3];
-  hipEvent_t eStart, eMid1, eMid2, eEnd;
+  hipEvent_t done[3];              // behind the run's last launch on each stream (see rt::waitEnd)
   uint32_t timeoutsSeen;           // sum of the stages' give-up counters when the last run returned
 };
 
@@ -376,8 +376,10 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   }
   for (int i = 0; i < 3; i++)
     if (CUSYNC_HIP(hipStreamCreateWithFlags(&L->stream[i], hipStreamNonBlocking))) { discardLayer(L); return nullptr; }
-  if (CUSYNC_HIP(hipEventCreate(&L->eStart)) || CUSYNC_HIP(hipEventCreate(&L->eMid1)) ||
-      CUSYNC_HIP(hipEventCreate(&L->eMid2)) || CUSYNC_HIP(hipEventCreate(&L->eEnd))) { discardLayer(L); return nullptr; }
+  for (auto& e : L->done)
+    if (CUSYNC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming))) { discardLayer(L); return nullptr; }
+  L->st[0].flags |= CUSYNC_STAGE_STAMPS_START;
+  for (int i = 0; i < 3; i++) L->st[i].flags |= CUSYNC_STAGE_STAMPS_END;
   return L;
 }
 
@@ -387,7 +389,7 @@ void cusync_attn_layer_destroy(cusync_attn_layer* L) {
   if (!L) return;
   for (int i = 0; i < 3; i++) if (L->stream[i]) (void)hipStreamSynchronize(L->stream[i]);
   for (int i = 0; i < 3; i++) cusync_stage_free(&L->st[i]);
-  for (hipEvent_t e : {L->eStart, L->eMid1, L->eMid2, L->eEnd}) if (e) (void)hipEventDestroy(e);
+  for (auto e : L->done) if (e) (void)hipEventDestroy(e);
   for (int i = 0; i < 3; i++) if (L->stream[i]) (void)hipStreamDestroy(L->stream[i]);
   if (L->ws1) (void)hipFree(L->ws1);
   if (L->ws3) (void)hipFree(L->ws3);
@@ -419,32 +421,21 @@ cusync_error cusync_attn_layer_run(cusync_attn_layer* L, const void* x, void* qk
 
     hipStream_t s0 = L->stream[0], s1 = overlapped ? L->stream[1] : s0, s2 = overlapped ? L->stream[2] : s0;
     cusync_error e;
-    if (CUSYNC_HIP(hipEventRecord(L->eStart, s0))) return CUSYNC_ERROR_DEVICE;
     if ((e = cusync_gemm_run(&a1, s0)) != CUSYNC_SUCCESS) return e;
     // overlapped: each consumer's stream is held back until every workgroup of its producer has started: from the
     // host when the producer's launch took every workgroup slot of the device (a wait kernel's wave would keep its
-    // last workgroup off the device), by the wait kernel otherwise.  eMid1 / eMid2 only serve the stage timing.
+    // last workgroup off the device), by the wait kernel otherwise.
     if (overlapped && (e = cusync_hold_back(&L->st[0], s1)) != CUSYNC_SUCCESS) return e;
-    if (CUSYNC_HIP(hipEventRecord(L->eMid1, s1))) return CUSYNC_ERROR_DEVICE;
     if ((e = cusync_attention_run(&a2, s1)) != CUSYNC_SUCCESS) return e;
-    if (overlapped) { if ((e = cusync_hold_back(&L->st[1], s2)) != CUSYNC_SUCCESS) return e; }
-    else if (CUSYNC_HIP(hipEventRecord(L->eMid2, s0))) return CUSYNC_ERROR_DEVICE;
+    if (overlapped && (e = cusync_hold_back(&L->st[1], s2)) != CUSYNC_SUCCESS) return e;
     if ((e = cusync_gemm_run(&a3, s2)) != CUSYNC_SUCCESS) return e;
-    if (CUSYNC_HIP(hipEventRecord(L->eEnd, s2))) return CUSYNC_ERROR_DEVICE;
-    if (CUSYNC_HIP(hipEventSynchronize(L->eEnd))) return CUSYNC_ERROR_DEVICE;
-    if (overlapped && (CUSYNC_HIP(hipStreamSynchronize(s0)) || CUSYNC_HIP(hipStreamSynchronize(s1)))) return CUSYNC_ERROR_DEVICE;
-    float ms = 0;
-    if (times_us) {
-      if (CUSYNC_HIP(hipEventElapsedTime(&ms, L->eStart, L->eEnd))) return CUSYNC_ERROR_DEVICE;
-      times_us[r] = (double)ms * 1000.0;
-    }
-    if (!overlapped && stage_us) {
-      hipEvent_t ev[4] = {L->eStart, L->eMid1, L->eMid2, L->eEnd};
-      for (int i = 0; i < 3; i++) {
-        if (CUSYNC_HIP(hipEventElapsedTime(&ms, ev[i], ev[i + 1]))) return CUSYNC_ERROR_DEVICE;
-        stage_us[3 * r + i] = (double)ms * 1000.0;
-      }
-    }
+    hipStream_t on[3] = {s0, s1, s2};
+    for (int i = overlapped ? 0 : 2; i < 3; i++) if (CUSYNC_HIP(hipEventRecord(L->done[i], on[i]))) return CUSYNC_ERROR_DEVICE;
+    for (int i = 2; i >= (overlapped ? 0 : 2); i--)
+      if ((e = cusync::rt::waitEnd(L->st[i], on[i], "attn layer")) != CUSYNC_SUCCESS) return e;
+    if (times_us) times_us[r] = cusync::rt::stampsUs(L->st[0], false, L->st[2]);
+    if (!overlapped && stage_us)
+      for (int i = 0; i < 3; i++) stage_us[3 * r + i] = cusync::rt::stampsUs(L->st[i ? i - 1 : 0], i > 0, L->st[i]);
     for (int i = 0; i < 3; i++) L->st[i].iter += 1;
   }
   // every run above was synchronised with; a wait that gave up let its kernel go on with unposted data

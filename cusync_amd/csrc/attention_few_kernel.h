@@ -70,6 +70,7 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
 
   uint32_t dryXcds = 0, nextRaw = 0;
   const unsigned long long tlEntry = p.timeline ? wall_clock64() : 0;
+  if (tid == 0) stage.enter();
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   const bool noDraws = stage.noDraws;
   for (uint32_t round = 0;; round++) {
@@ -303,6 +304,7 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
     else __syncthreads();
     if (tid == 0) recordTileAt(p.timeline, p.timelineCap, stage, p.launched, t, round, tlEntry, tl0, tl1, tl2, p.timeline ? wall_clock64() : 0);
   }
+  stage.leave(p.launched);
 }
 
 }  // namespace attn

@@ -280,7 +280,7 @@ struct cusync_conv_chain {
   std::vector<const void*> w;
   std::vector<cusync_stage_desc> st;
   std::vector<hipStream_t> stream;
-  std::vector<hipEvent_t> ev;        // layers + 1 events: start, after each layer
+  std::vector<hipEvent_t> done;      // behind the run's last launch on each stream (see rt::waitEnd)
   std::vector<void*> ws;             // per layer: partial sums and counters of the runs a tile's steps are cut into
   int splitK = 1;
   uint32_t timeoutsSeen = 0;         // sum of the stages' give-up counters when the last run returned
@@ -307,7 +307,7 @@ void freeChain(cusync_conv_chain* c) {
   for (auto s : c->stream) (void)hipStreamSynchronize(s);
   for (auto& d : c->st) cusync_stage_free(&d);
   for (auto w : c->ws) (void)hipFree(w);
-  for (auto e : c->ev) (void)hipEventDestroy(e);
+  for (auto e : c->done) (void)hipEventDestroy(e);
   for (auto s : c->stream) (void)hipStreamDestroy(s);
   delete c;
 }
@@ -410,12 +410,15 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
     hipStream_t s;
     if (CUSYNC_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking))) { freeChain(c); return nullptr; }
     c->stream.push_back(s);
-  }
-  for (uint32_t i = 0; i <= cfg->layers; i++) {
     hipEvent_t e;
-    if (CUSYNC_HIP(hipEventCreate(&e))) { freeChain(c); return nullptr; }
-    c->ev.push_back(e);
+    if (CUSYNC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming))) { freeChain(c); return nullptr; }
+    c->done.push_back(e);
   }
+  // all layers in one launch: the last one's end is the launch's
+  const bool oneLaunch = c->cfg.fused && cfg->sync != CUSYNC_SYNC_STREAM;
+  c->st[0].flags |= CUSYNC_STAGE_STAMPS_START;
+  for (uint32_t i = 0; i < cfg->layers; i++)
+    if (!oneLaunch || i + 1 == cfg->layers) c->st[i].flags |= CUSYNC_STAGE_STAMPS_END;
   if (c->splitK > 1) {
     cusync_conv2d_args a;
     memset(&a, 0, sizeof a);
@@ -472,21 +475,16 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
         if (e != CUSYNC_SUCCESS) return e;
         cp.layer[i] = convParams(&a, ti, launched);
       }
-      if (CUSYNC_HIP(hipEventRecord(c->ev[0], c->stream[0]))) return CUSYNC_ERROR_DEVICE;
       hipLaunchKernelGGL(ti->chainKernel, dim3(launched), dim3(kThreads), lds, c->stream[0], cp);
-      if (CUSYNC_HIP(hipGetLastError()) || CUSYNC_HIP(hipEventRecord(c->ev[n], c->stream[0])) ||
-          CUSYNC_HIP(hipEventSynchronize(c->ev[n]))) return CUSYNC_ERROR_DEVICE;
-      float ms = 0;
-      if (times_us) {
-        if (CUSYNC_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[n]))) return CUSYNC_ERROR_DEVICE;
-        times_us[r] = (double)ms * 1000.0;
-      }
+      if (CUSYNC_HIP(hipGetLastError()) || CUSYNC_HIP(hipEventRecord(c->done[0], c->stream[0]))) return CUSYNC_ERROR_DEVICE;
+      const cusync_error e = cusync::rt::waitEnd(c->st[n - 1], c->stream[0], "conv chain");
+      if (e != CUSYNC_SUCCESS) return e;
+      if (times_us) times_us[r] = cusync::rt::stampsUs(c->st[0], false, c->st[n - 1]);
       for (uint32_t i = 0; i < n; i++) c->st[i].iter += 1;
     }
     return chainTimeouts(c);
   }
   for (int r = 0; r < runs; r++) {
-    if (CUSYNC_HIP(hipEventRecord(c->ev[0], c->stream[0]))) return CUSYNC_ERROR_DEVICE;
     for (uint32_t i = 0; i < n; i++) {
       hipStream_t s = c->stream[overlapped ? i : 0];
       const cusync_conv2d_args a = layerArgs(i);
@@ -496,22 +494,15 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
       // that the wait kernel's wave takes nothing from the producer; from this thread where the launch took them all.
       if (overlapped && i > 0 && (e = cusync_hold_back(&c->st[i - 1], s)) != CUSYNC_SUCCESS) return e;
       if ((e = cusync_conv2d_run(&a, s)) != CUSYNC_SUCCESS) return e;
-      if ((!overlapped || i + 1 == n) && CUSYNC_HIP(hipEventRecord(c->ev[i + 1], s))) return CUSYNC_ERROR_DEVICE;
     }
-    if (CUSYNC_HIP(hipEventSynchronize(c->ev[n]))) return CUSYNC_ERROR_DEVICE;
-    if (overlapped)
-      for (uint32_t i = 0; i + 1 < n; i++)
-        if (CUSYNC_HIP(hipStreamSynchronize(c->stream[i]))) return CUSYNC_ERROR_DEVICE;
-    float ms = 0;
-    if (times_us) {
-      if (CUSYNC_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[n]))) return CUSYNC_ERROR_DEVICE;
-      times_us[r] = (double)ms * 1000.0;
+    for (uint32_t i = 0; i < (overlapped ? n : 1); i++) if (CUSYNC_HIP(hipEventRecord(c->done[i], c->stream[i]))) return CUSYNC_ERROR_DEVICE;
+    for (uint32_t i = n; i-- > (overlapped ? 0 : n - 1);) {
+      const cusync_error e = cusync::rt::waitEnd(c->st[i], c->stream[overlapped ? i : 0], "conv chain");
+      if (e != CUSYNC_SUCCESS) return e;
     }
+    if (times_us) times_us[r] = cusync::rt::stampsUs(c->st[0], false, c->st[n - 1]);
     if (!overlapped && layer_us)
-      for (uint32_t i = 0; i < n; i++) {
-        if (CUSYNC_HIP(hipEventElapsedTime(&ms, c->ev[i], c->ev[i + 1]))) return CUSYNC_ERROR_DEVICE;
-        layer_us[(size_t)r * n + i] = (double)ms * 1000.0;
-      }
+      for (uint32_t i = 0; i < n; i++) layer_us[(size_t)r * n + i] = cusync::rt::stampsUs(c->st[i ? i - 1 : 0], i > 0, c->st[i]);
     for (uint32_t i = 0; i < n; i++) c->st[i].iter += 1;
   }
   return chainTimeouts(c);

@@ -103,6 +103,7 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
 
   uint32_t dryXcds = 0, nextRaw = 0;
   const unsigned long long tlEntry = p.timeline ? wall_clock64() : 0;
+  if (tid == 0) stage.enter();
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   const bool noDraws = stage.noDraws;     // every tile is some workgroup's static first tile
   for (uint32_t round = 0;; round++) {
@@ -233,6 +234,7 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
     else __syncthreads();
     if (tid == 0) recordTile(p, t, round, tlEntry, tl0, tl1, tl2, p.timeline ? wall_clock64() : 0);
   }
+  stage.leave(p.launched);
 }
 
 template<class C, bool SPLIT = false>

@@ -76,6 +76,7 @@ __global__ __launch_bounds__(kThreads) void gemmKernel(GemmParams p) {
   // first tile's loads are under way; the draw of the next ticket is issued while a tile is
   // being computed and settled when the tile is done.
   uint32_t dryXcds = 0, nextRaw = 0;
+  if (tid == 0) stage.enter();
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   const bool noDraws = stage.noDraws;     // every tile is some workgroup's static first tile
   for (uint32_t round = 0;; round++) {
@@ -273,6 +274,7 @@ __global__ __launch_bounds__(kThreads) void gemmKernel(GemmParams p) {
     if (completed && stage.isProducer()) stage.post(done, postsPerTile(p), stage.storesThrough());
     else __syncthreads();
   }
+  stage.leave(p.launched);
 }
 
 }  // namespace gemm

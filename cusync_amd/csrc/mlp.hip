@@ -31,7 +31,7 @@ struct cusync_mlp {
   int epilogue1, aMode2;
   cusync_stage_desc prod, cons;
   hipStream_t sProd, sCons;
-  hipEvent_t eStart, eMid, eEnd;
+  hipEvent_t done[3];                // behind the run's last launch on sProd, sCons, sMid (see rt::waitEnd)
   // LLaMA with silu(gate) * up as GEMM1's epilogue: w1p holds W1 with the gate and up columns interleaved in
   // groups of eight, the intermediate is [batch][inner]
   bool fused;
@@ -129,6 +129,7 @@ __global__ __launch_bounds__(kActThreads) void swigluStageKernel(ActParams p) {
     if (stage.isProducer()) stage.post(done);
     else __syncthreads();
   }
+  stage.leave(p.launched);      // (its output is read by GEMM2 only, behind a post or a kernel boundary)
 }
 
 // Workgroups of the activation kernel that stay resident on the device; 0 if the runtime would not say.
@@ -511,13 +512,17 @@ cusync_mlp* cusync_mlp_create(const cusync_mlp_config* cfg, const void* w1, cons
     if (CUSYNC_HIP(hipMalloc(&ws, bytes)) || CUSYNC_HIP(hipMemset(ws, 0, bytes))) { discard(m); return nullptr; }
     (which == 0 ? m->ws1 : m->ws2) = ws;
   }
+  // in one launch the second GEMM's end is the launch's
+  m->prod.flags |= CUSYNC_STAGE_STAMPS_START | (m->cfg.one_launch ? 0 : CUSYNC_STAGE_STAMPS_END);
+  m->cons.flags |= CUSYNC_STAGE_STAMPS_END;
+  m->mid.flags |= CUSYNC_STAGE_STAMPS_END;
   if (CUSYNC_HIP(hipStreamCreateWithFlags(&m->sProd, hipStreamNonBlocking)) ||
-      CUSYNC_HIP(hipStreamCreateWithFlags(&m->sCons, hipStreamNonBlocking)) ||
-      CUSYNC_HIP(hipEventCreate(&m->eStart)) || CUSYNC_HIP(hipEventCreate(&m->eMid)) ||
-      CUSYNC_HIP(hipEventCreate(&m->eEnd))) {
+      CUSYNC_HIP(hipStreamCreateWithFlags(&m->sCons, hipStreamNonBlocking))) {
     discard(m);
     return nullptr;
   }
+  for (auto& e : m->done)
+    if (CUSYNC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming))) { discard(m); return nullptr; }
   return m;
 }
 
@@ -558,9 +563,7 @@ void cusync_mlp_destroy(cusync_mlp* m) {
   if (m->ws2) (void)hipFree(m->ws2);
   if (m->w1p) (void)hipFree(m->w1p);
   if (m->w2p) (void)hipFree(m->w2p);
-  if (m->eStart) (void)hipEventDestroy(m->eStart);
-  if (m->eMid) (void)hipEventDestroy(m->eMid);
-  if (m->eEnd) (void)hipEventDestroy(m->eEnd);
+  for (auto e : m->done) if (e) (void)hipEventDestroy(e);
   if (m->sProd) (void)hipStreamDestroy(m->sProd);
   if (m->sCons) (void)hipStreamDestroy(m->sCons);
   if (m->sMid) (void)hipStreamDestroy(m->sMid);
@@ -575,12 +578,10 @@ cusync_error cusync_mlp_run_split(cusync_mlp* m, const void* x, void* h, void* y
     cusync_gemm_args a1 = gemmArgs(m, 0, x, h, y);
     cusync_gemm_args a2 = gemmArgs(m, 1, x, h, y);
     cusync_error e;
-    if (CUSYNC_HIP(hipEventRecord(m->eStart, m->sProd))) return CUSYNC_ERROR_DEVICE;
     if (overlapped && m->cfg.one_launch) {
       // both GEMMs in one launch: same stages and semaphores, no wait kernel, no second launch
       const cusync_gemm_args both[2] = {a1, a2};
       if ((e = cusync_gemm_chain_run(both, 2, m->sProd)) != CUSYNC_SUCCESS) return e;
-      if (CUSYNC_HIP(hipEventRecord(m->eEnd, m->sProd))) return CUSYNC_ERROR_DEVICE;
     } else if ((e = cusync_gemm_run(&a1, m->sProd)) != CUSYNC_SUCCESS) {
       return e;
     } else if (overlapped) {
@@ -596,31 +597,22 @@ cusync_error cusync_mlp_run_split(cusync_mlp* m, const void* x, void* h, void* y
         return e;
       }
       if ((e = cusync_gemm_run(&a2, m->sCons)) != CUSYNC_SUCCESS) return e;
-      if (CUSYNC_HIP(hipEventRecord(m->eEnd, m->sCons))) return CUSYNC_ERROR_DEVICE;
     } else {
-      if (CUSYNC_HIP(hipEventRecord(m->eMid, m->sProd))) return CUSYNC_ERROR_DEVICE;
       if (m->actStage && (e = runActStage(m, h, m->sProd)) != CUSYNC_SUCCESS) return e;     // counted with GEMM2
       if ((e = cusync_gemm_run(&a2, m->sProd)) != CUSYNC_SUCCESS) return e;
-      if (CUSYNC_HIP(hipEventRecord(m->eEnd, m->sProd))) return CUSYNC_ERROR_DEVICE;
     }
-    if (CUSYNC_HIP(hipEventSynchronize(m->eEnd))) return CUSYNC_ERROR_DEVICE;
-    // The consumer finishing implies every producer tile was posted, but the
-    // producer kernel itself must have retired before its stage is reused.
-    if (overlapped && CUSYNC_HIP(hipStreamSynchronize(m->sProd))) return CUSYNC_ERROR_DEVICE;
-    if (overlapped && m->actStage && CUSYNC_HIP(hipStreamSynchronize(m->sMid))) return CUSYNC_ERROR_DEVICE;
-    float ms = 0;
-    if (times_us) {
-      if (CUSYNC_HIP(hipEventElapsedTime(&ms, m->eStart, m->eEnd))) return CUSYNC_ERROR_DEVICE;
-      times_us[r] = (double)ms * 1000.0;
+    // Every launch of the run reports its end, the consumer's last: the stages are then free for the next run.
+    const bool ownStreams = overlapped && !m->cfg.one_launch;
+    if (CUSYNC_HIP(hipEventRecord(m->done[0], m->sProd)) || (ownStreams && CUSYNC_HIP(hipEventRecord(m->done[1], m->sCons))) ||
+        (ownStreams && m->actStage && CUSYNC_HIP(hipEventRecord(m->done[2], m->sMid)))) return CUSYNC_ERROR_DEVICE;
+    if ((e = cusync::rt::waitEnd(m->cons, ownStreams ? m->sCons : m->sProd, "mlp")) != CUSYNC_SUCCESS) return e;
+    if (ownStreams) {
+      if ((e = cusync::rt::waitEnd(m->prod, m->sProd, "mlp")) != CUSYNC_SUCCESS) return e;
+      if (m->actStage && (e = cusync::rt::waitEnd(m->mid, m->sMid, "mlp")) != CUSYNC_SUCCESS) return e;
     }
-    if (!overlapped && gemm1_us) {
-      if (CUSYNC_HIP(hipEventElapsedTime(&ms, m->eStart, m->eMid))) return CUSYNC_ERROR_DEVICE;
-      gemm1_us[r] = (double)ms * 1000.0;
-    }
-    if (!overlapped && gemm2_us) {
-      if (CUSYNC_HIP(hipEventElapsedTime(&ms, m->eMid, m->eEnd))) return CUSYNC_ERROR_DEVICE;
-      gemm2_us[r] = (double)ms * 1000.0;
-    }
+    if (times_us) times_us[r] = cusync::rt::stampsUs(m->prod, false, m->cons);
+    if (!overlapped && gemm1_us) gemm1_us[r] = cusync::rt::stampsUs(m->prod, false, m->prod);
+    if (!overlapped && gemm2_us) gemm2_us[r] = cusync::rt::stampsUs(m->prod, true, m->cons);
     m->prod.iter += 1;     // incrementIter on both stages, mlp.cu:709-712
     m->cons.iter += 1;
     m->mid.iter += 1;

@@ -82,6 +82,34 @@ cusync_error checkSpinTimeouts(const cusync_stage_desc* const* stages, int count
   return CUSYNC_ERROR_DEVICE;
 }
 
+static unsigned long long stampOf(const cusync_stage_desc& s, int which) {
+  return __atomic_load_n(reinterpret_cast<const unsigned long long*>(s.spinTimeouts + CUSYNC_HOST_STAMP_OFFSET) + which, __ATOMIC_ACQUIRE);
+}
+
+cusync_error waitEnd(const cusync_stage_desc& s, hipStream_t stream, const char* what) {
+  const unsigned long long want = (uint32_t)s.iter & 0xffffu;
+  auto looked = std::chrono::steady_clock::now();
+  for (uint32_t spins = 1;; spins++) {
+    if ((stampOf(s, 1) & 0xffffu) == want) return CUSYNC_SUCCESS;
+    __builtin_ia32_pause();      // the stamp arrives over the bus
+    if (spins % 1024 == 0 && std::chrono::steady_clock::now() - looked > std::chrono::milliseconds(2)) {
+      // A launch that failed on the device leaves no stamp: what does its stream say?
+      const hipError_t e = hipStreamQuery(stream);
+      if (e != hipErrorNotReady) {
+        if ((stampOf(s, 1) & 0xffffu) == want) return CUSYNC_SUCCESS;
+        if (check(e, "hipStreamQuery", __FILE__, __LINE__) == 0) setError(std::string(what) + ": a stage's launch ended without reporting its end");
+        return CUSYNC_ERROR_DEVICE;
+      }
+      looked = std::chrono::steady_clock::now();
+    }
+  }
+}
+
+double stampsUs(const cusync_stage_desc& from, bool fromEnd, const cusync_stage_desc& to) {
+  const unsigned long long ticks = ((stampOf(to, 1) >> 16) - (stampOf(from, fromEnd ? 1 : 0) >> 16)) & 0xffffffffffffull;
+  return (double)ticks * 0.01;
+}
+
 }  // namespace rt
 }  // namespace cusync
 
@@ -159,11 +187,11 @@ cusync_error cusync_stage_alloc(cusync_stage_desc* d, const cusync_dim3* host_ti
   if (n == 0) { cusync::rt::setError("cusync_stage_alloc: empty grid"); return CUSYNC_ERROR_NOT_INITIALIZED; }
   d->tileOrder = nullptr; d->tileCounter = nullptr; d->startCounter = nullptr; d->xcdTickets = nullptr;
   d->kernelExecuted = nullptr; d->spinTimeouts = nullptr; d->tileStatusWrite = nullptr;
-  // The small device counters share one allocation: [tileCounter, startCounter, -, kernelExecuted, xcdTickets[9]], each on its
+  // The small device counters share one allocation: [tileCounter, startCounter, -, kernelExecuted, xcdTickets[9], workgroups that left], each on its
   // own 128-byte line so that polling one does not disturb the others.
   const size_t line = 128;
   char* counters = nullptr;
-  if (RT(hipMalloc((void**)&counters, 13 * line))) return CUSYNC_ERROR_DEVICE;
+  if (RT(hipMalloc((void**)&counters, 14 * line))) return CUSYNC_ERROR_DEVICE;
   d->tileCounter = (uint32_t*)(counters);         // base of the block: what cusync_stage_free releases
   // a failure from here on gives back what was allocated so far; the text of the failed call is kept
   auto fail = [&]() {
@@ -172,16 +200,17 @@ cusync_error cusync_stage_alloc(cusync_stage_desc* d, const cusync_dim3* host_ti
     cusync::rt::setError(why);
     return CUSYNC_ERROR_DEVICE;
   };
-  if (RT(hipMemset(counters, 0, 13 * line))) return fail();
+  if (RT(hipMemset(counters, 0, 14 * line))) return fail();
   d->startCounter = (uint32_t*)(counters + line);
   d->xcdTickets = (uint32_t*)(counters + 4 * line);
   // The two words the host wants to look at while kernels run, or without a copy after them, live in pinned host
   // memory the device reaches over the bus: the count of waits that gave up (first line: the base of the block)
-  // and a mirror of the wait-kernel flag (second line, CUSYNC_HOST_FLAG_OFFSET words on).  Each is written at most
-  // once per kernel; the flag the wait kernel polls stays in device memory.
+  // and a mirror of the wait-kernel flag (second line, CUSYNC_HOST_FLAG_OFFSET words on), and behind them the stamps of
+  // the stage's start and end (CUSYNC_HOST_STAMP_OFFSET).  Each is written at most once per kernel; the flag the wait
+  // kernel polls stays in device memory.
   char* shared = nullptr;
-  if (RT(hipHostMalloc((void**)&shared, 2 * line, hipHostMallocDefault))) return fail();
-  memset(shared, 0, 2 * line);
+  if (RT(hipHostMalloc((void**)&shared, 3 * line, hipHostMallocDefault))) return fail();
+  memset(shared, 0, 3 * line);
   d->spinTimeouts = (uint32_t*)shared;
   const bool producer = d->out.kind != CUSYNC_POLICY_NOSYNC;
   if (producer && !(d->opts & CUSYNC_OPT_AVOID_WAIT_KERNEL)) d->kernelExecuted = (uint32_t*)(counters + 3 * line);

@@ -29,6 +29,14 @@ bool forceWaitKernel();
 // whether that launch took every workgroup slot of the device.  cusync_hold_back reads it.  No-op for a stage that
 // posts nothing.
 void noteLaunch(const cusync_stage_desc& stage, bool fillsDevice);
+// For the chain handles, whose stages carry CUSYNC_STAGE_STAMPS_*: waits on the host until the run s.iter of the stage
+// has stamped its end (its launch is on `stream`), and the time between two stamps of a finished run, the start or the
+// end of one stage and the end of another, by the device's 100 MHz clock.
+// Before it waits, a handle records an event nobody waits for behind the last launch of each stream: with it the runtime
+// learns by itself that the stream is idle, and a caller's hipDeviceSynchronize() after the run takes 5.5 us instead of
+// 8.3 (6.1 instead of 17.3 for a chain on two streams); the record costs the run nothing, the kernels are under way.
+cusync_error waitEnd(const cusync_stage_desc& s, hipStream_t stream, const char* what);
+double stampsUs(const cusync_stage_desc& from, bool fromEnd, const cusync_stage_desc& to);
 // Adds up the counters of waits that gave up (cusync_stage_desc::spinTimeouts) of the stages given; null
 // entries and stages without a counter are skipped.  Returns false if a copy from the device failed.
 bool spinTimeoutsOf(const cusync_stage_desc* const* stages, int count, uint32_t* sum);

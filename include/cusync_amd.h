@@ -74,13 +74,22 @@ typedef struct cusync_policy_desc {
  * by value.  Device pointers are owned by whoever called cusync_stage_alloc. */
 /* tileOrder[i] == (i % gx, (i / gx) % gy, i / (gx*gy)) for every i: true of both tile orders the reference
  * ships (CS/tile-orders.h:52-75).  The prebuilt kernels then compute a ticket's tile instead of loading it. */
-enum { CUSYNC_STAGE_IDENTITY_ORDER = 1 };
+enum {
+  CUSYNC_STAGE_IDENTITY_ORDER = 1,
+  /* Set by the chain handles on the stages of a run, for the prebuilt kernels: the launch's first workgroup stamps the
+   * stage's start, the workgroup that leaves last, with all outputs written through to memory, its end (64-bit words in
+   * the stage's block of host memory, CUSYNC_HOST_STAMP_OFFSET).  The host then waits for the end stamps, and takes a
+   * run's times from them, instead of recording and waiting for events. */
+  CUSYNC_STAGE_STAMPS_START = 2,
+  CUSYNC_STAGE_STAMPS_END = 4
+};
 
 /* Semaphore i of a stage lives at tileStatus[i * CUSYNC_SEM_STRIDE]: each on its own 128-byte line, so that the
  * waves polling one semaphore do not queue up behind those polling its neighbours (the reference packs them,
  * CS/cusync.h:186-190).  cusync_stage_read_state returns them packed. */
 #define CUSYNC_SEM_STRIDE 32
 #define CUSYNC_HOST_FLAG_OFFSET 32
+#define CUSYNC_HOST_STAMP_OFFSET 64
 
 typedef struct cusync_stage_desc {
   cusync_dim3 grid;           /* grid_     : logical tile grid of this stage */
@@ -102,7 +111,9 @@ typedef struct cusync_stage_desc {
                                  that the device writes to, so that the host reads it without a copy; the word
                                  CUSYNC_HOST_FLAG_OFFSET words behind it mirrors the wait-kernel flag for
                                  cusync_wait_producer_started (written right after the flag itself), and the word after
-                                 that is the launchers' note for cusync_hold_back (host-written only) */
+                                 that is the launchers' note for cusync_hold_back (host-written only).  CUSYNC_HOST_STAMP_OFFSET words
+                                 behind it two 64-bit stamps (CUSYNC_STAGE_STAMPS_*): 100 MHz device clock << 16 | low 16
+                                 bits of iter */
   uint32_t *tileStatusWrite;  /* semaphores this stage posts, CUSYNC_SEM_STRIDE apart */
   uint32_t *tileStatusRead;   /* semaphores this stage waits on (its producer's) */
 } cusync_stage_desc;
@@ -406,7 +417,7 @@ typedef struct cusync_conv_chain cusync_conv_chain;
 cusync_conv_chain *cusync_conv_chain_create(const cusync_conv_chain_config *cfg, const void *const *weights);
 void cusync_conv_chain_destroy(cusync_conv_chain *chain);
 /* x: [N][H][W][C]; ys[i]: output of layer i, same shape.  Synchronises after each of the `runs` runs;
- * times_us[r] = start of the first kernel to end of the last; in the stream-ordered mode
+ * times_us[r] = start of the first kernel to end of the last (as cusync_mlp_run); in the stream-ordered mode
  * layer_us[r*layers + i] receives the time of layer i. */
 cusync_error cusync_conv_chain_run(cusync_conv_chain *chain, const void *x, void *const *ys, int runs,
                                    double *times_us, double *layer_us);
@@ -474,7 +485,7 @@ typedef struct cusync_attn_layer cusync_attn_layer;
 cusync_attn_layer *cusync_attn_layer_create(const cusync_attn_layer_config *cfg, const void *wqkv, const void *wo);
 void cusync_attn_layer_destroy(cusync_attn_layer *layer);
 /* x: [seq][hidden]; qkv: [cached_rows + seq][3*heads*head_dim] (the cache rows filled by the caller); o: [seq][heads*head_dim]; y: [seq][hidden].  Runs `runs`
- * times, synchronising after each; times_us[r] = start of the first kernel to end of the last.  For the
+ * times, synchronising after each; times_us[r] = start of the first kernel to end of the last (as cusync_mlp_run).  For the
  * stream-ordered mode stage_us[3*r + i] receives the time of stage i. */
 cusync_error cusync_attn_layer_run(cusync_attn_layer *layer, const void *x, void *qkv, void *o, void *y, int runs,
                                    double *times_us, double *stage_us);
@@ -541,8 +552,9 @@ cusync_error cusync_mlp_reload_weights(cusync_mlp *mlp);
  * passes x -> h -> y.  h is the intermediate [batch, inner] (GPT-3) or a buffer of
  * [batch, 2*inner] (LLaMA: gate|up, or silu(gate)*up in its first batch*inner elements
  * when the activation is GEMM1's epilogue, see cusync_mlp_config::swiglu_in_gemm2).  If times_us != NULL it receives one elapsed time
- * per run, measured with events start (producer stream) -> end (consumer stream)
- * exactly as TB/mlp.cu:691-708; each run is then followed by an event wait. */
+ * per run (TB/mlp.cu:691-708 measures it with events): from the moment the first kernel's first workgroup starts to the
+ * moment the last kernel's last workgroup has its outputs in memory, by the device's 100 MHz clock.  The call returns
+ * when that has happened for the last run; the outputs may be read, and every operand changed or freed, at once. */
 /* Returns CUSYNC_ERROR_DEVICE (text in cusync_rt_last_error) when a wait of one of the chain's stages, the wait
  * kernel's included, gave up after CUSYNC_SPIN_LIMIT polls during the call: the kernel went on with data that
  * had not been posted, so the outputs of the call are not valid.  The same holds for cusync_conv_chain_run and

@@ -1,0 +1,76 @@
+"""The chain handles return when their outputs are in memory, on the word of the device's own stamps."""
+import time
+
+import numpy as np
+import pytest
+
+from cusync_amd import api
+from util import empty_dev, normal_f16, to_dev, uniform_f16
+
+pytestmark = pytest.mark.gpu
+
+
+def chain(kind, sync):
+    """(handle, one pass as a call that returns its times, the buffers a pass fills)"""
+    if kind == "conv":
+        N, H, C = 8, 28, 128
+        x = to_dev(uniform_f16((N, H, H, C), 1))
+        ws = [to_dev(normal_f16((C, 3, 3, C), k, std=0.03)) for k in (2, 3, 4)]
+        ys = [empty_dev((N, H, H, C)) for _ in ws]
+        h = api.ConvChain(N, H, H, C, [w.data_ptr() for w in ws], sync)
+        return h, lambda: h.run(x.data_ptr(), [y.data_ptr() for y in ys]), ys + [x] + ws, len(ys)
+    if kind == "attention":
+        S, cached, hidden, heads = 40, 300, 1024, 3
+        E = heads * 128
+        x, wqkv, wo = to_dev(uniform_f16((S, hidden), 1)), to_dev(normal_f16((hidden, 3 * E), 2)), to_dev(normal_f16((E, hidden), 3))
+        qkv, o, y = to_dev(normal_f16((cached + S, 3 * E), 4, std=1.0)), empty_dev((S, E)), empty_dev((S, hidden))
+        h = api.AttnLayer(S, hidden, heads, sync, wqkv.data_ptr(), wo.data_ptr(), cached_rows=cached)
+        return h, lambda: h.run(x.data_ptr(), qkv.data_ptr(), o.data_ptr(), y.data_ptr()), [o, y, qkv, x, wqkv, wo], 2
+    model, rows, one, where = kind
+    hidden, inner = 4096, 2816
+    n1 = inner * (2 if model == api.MODEL.LLAMA else 1)
+    x, w1, w2 = to_dev(uniform_f16((rows, hidden), 1)), to_dev(normal_f16((hidden, n1), 2)), to_dev(normal_f16((inner, hidden), 3))
+    hb, y = empty_dev((rows, inner if where == 0 else n1)), empty_dev((rows, hidden))
+    h = api.Mlp(model, rows, hidden, inner, sync, w1.data_ptr(), w2.data_ptr(), one_launch=one, swiglu_in_gemm2=where)
+    return h, lambda: h.run(x.data_ptr(), hb.data_ptr(), y.data_ptr()), [hb, y, x, w1, w2], 2
+
+
+@pytest.mark.parametrize("sync", [api.SYNC.STREAM, api.SYNC.ROW, api.SYNC.TILE])
+@pytest.mark.parametrize("kind", [(api.MODEL.GPT3, 1, -1, 0), (api.MODEL.GPT3, 40, 0, 0), (api.MODEL.GPT3, 700, -1, 0), (api.MODEL.LLAMA, 300, -1, 0),
+                                  (api.MODEL.LLAMA, 300, -1, -1), (api.MODEL.LLAMA, 300, -1, 1), "conv", "attention"])
+def test_outputs_are_there_when_a_run_returns(kind, sync):
+    import torch
+    print("run returns", kind, sync, flush=True)
+    torch.cuda.synchronize()
+    handle, run, buffers, outputs = chain(kind, sync)
+    copies = [torch.empty_like(b) for b in buffers[:outputs]]
+    other = torch.cuda.Stream()
+    for _ in range(20):
+        for b in buffers[:outputs]:
+            b.fill_(float("nan"))
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        (us,) = run()
+        wall = (time.perf_counter() - t0) * 1e6
+        with torch.cuda.stream(other):            # a stream that knows nothing of the chain's
+            for c, b in zip(copies, buffers):
+                c.copy_(b, non_blocking=True)
+        torch.cuda.synchronize()
+        assert 0 < us < wall
+        for c, b in zip(copies, buffers):
+            assert torch.equal(c.view(torch.int16), b.view(torch.int16))
+            assert not torch.isnan(b).any()
+    handle.destroy()
+
+
+def test_split_times_add_up():
+    import torch
+    torch.cuda.synchronize()
+    rows, hidden, inner = 64, 4096, 2816
+    x, w1, w2 = to_dev(uniform_f16((rows, hidden), 1)), to_dev(normal_f16((hidden, inner), 2)), to_dev(normal_f16((inner, hidden), 3))
+    h, y = empty_dev((rows, inner)), empty_dev((rows, hidden))
+    torch.cuda.synchronize()
+    m = api.Mlp(api.MODEL.GPT3, rows, hidden, inner, api.SYNC.STREAM, w1.data_ptr(), w2.data_ptr())
+    total, g1, g2 = m.run(x.data_ptr(), h.data_ptr(), y.data_ptr(), runs=5, split=True)
+    m.destroy()
+    assert np.allclose(np.array(g1) + np.array(g2), total, atol=0.02) and min(g1) > 0 and min(g2) > 0
