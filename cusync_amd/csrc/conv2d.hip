@@ -31,6 +31,7 @@ using namespace cusync::gemm;
 
 struct ConvTile {
   uint32_t bm, bn, bk;
+  uint32_t threads;
   size_t lds;
   void (*kernel)(GemmParams);
   int residentPerCU;
@@ -39,21 +40,21 @@ struct ConvTile {
 };
 
 #define CUSYNC_CONV_TILE(BM, BN, BK, WM, WN, ST, OCC) \
-  { BM, BN, BK, (size_t)DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>::LDS_BYTES, \
+  { BM, BN, BK, kThreads, (size_t)DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>::LDS_BYTES, \
     gemmDmaKernel<DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>, kAConv>, -1, nullptr, nullptr }
 
 using HaloA = Halo3x3Cfg<256, 64, 4, 1, 4, 2>;     // 64 output channels per tile: four waves of 64 x 64 stacked
-using HaloB = Halo3x3Cfg<128, 128, 2, 2, 3, 1>;    // 128 output channels per tile
-using HaloC = Halo3x3Cfg<64, 128, 2, 2, 3, 1>;     // 64 pixels: what fits beside the halo of 512-channel pixels (7 x 7 images)
+using HaloB = Halo3x3Cfg<128, 128, 2, 2, 3, 2, 2>;    // 128 output channels per tile
+using HaloC = Halo3x3Cfg<64, 128, 2, 2, 3, 2, 2>;     // 64 pixels: what fits beside the halo of 512-channel pixels (7 x 7 images)
 
 ConvTile g_convTiles[CUSYNC_CONV_TILE_COUNT] = {
   CUSYNC_CONV_TILE(128, 64, 32, 2, 2, 4, 3),    // CUSYNC_CONV_TILE_128x64x32
   CUSYNC_CONV_TILE(128, 128, 32, 2, 2, 4, 2),   // CUSYNC_CONV_TILE_128x128x32
   CUSYNC_CONV_TILE(256, 64, 32, 4, 1, 3, 2),    // CUSYNC_CONV_TILE_256x64x32
   // the halo tiles: 3x3 / pad 1 / stride 1 only; LDS size depends on the image width and channels
-  { HaloA::BM, HaloA::BN, HaloA::BK, 0, convHalo3x3Kernel<HaloA>, -1, convHalo3x3ChainKernel<HaloA>, convHalo3x3Kernel<HaloA, true> },   // CUSYNC_CONV_TILE_HALO_256x64x64
-  { HaloB::BM, HaloB::BN, HaloB::BK, 0, convHalo3x3Kernel<HaloB>, -1, convHalo3x3ChainKernel<HaloB>, convHalo3x3Kernel<HaloB, true> },   // CUSYNC_CONV_TILE_HALO_128x128x64
-  { HaloC::BM, HaloC::BN, HaloC::BK, 0, convHalo3x3Kernel<HaloC>, -1, convHalo3x3ChainKernel<HaloC>, convHalo3x3Kernel<HaloC, true> },   // CUSYNC_CONV_TILE_HALO_64x128x64
+  { HaloA::BM, HaloA::BN, HaloA::BK, HaloA::THREADS, 0, convHalo3x3Kernel<HaloA>, -1, convHalo3x3ChainKernel<HaloA>, convHalo3x3Kernel<HaloA, true> },   // CUSYNC_CONV_TILE_HALO_256x64x64
+  { HaloB::BM, HaloB::BN, HaloB::BK, HaloB::THREADS, 0, convHalo3x3Kernel<HaloB>, -1, convHalo3x3ChainKernel<HaloB>, convHalo3x3Kernel<HaloB, true> },   // CUSYNC_CONV_TILE_HALO_128x128x64
+  { HaloC::BM, HaloC::BN, HaloC::BK, HaloC::THREADS, 0, convHalo3x3Kernel<HaloC>, -1, convHalo3x3ChainKernel<HaloC>, convHalo3x3Kernel<HaloC, true> },   // CUSYNC_CONV_TILE_HALO_64x128x64
 };
 
 bool isHalo(int tile) { return tile >= CUSYNC_CONV_TILE_HALO_256x64x64 && tile <= CUSYNC_CONV_TILE_HALO_64x128x64; }
@@ -90,20 +91,20 @@ int residentConv(ConvTile* ti, size_t lds) {
     if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ti->kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, halo ? (int)kMaxLds : (int)lds))) return 0;
     int n = 0;
-    if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ti->kernel, kThreads, lds))) return 0;
+    if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ti->kernel, (int)ti->threads, lds))) return 0;
     if (ti->chainKernel) {
       // the chain kernel is the same code in a loop: it gets the same LDS allowance and must fit as often
       int m = 0;
       if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ti->chainKernel),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds)) ||
-          CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, ti->chainKernel, kThreads, lds))) return 0;
+          CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, ti->chainKernel, (int)ti->threads, lds))) return 0;
       n = std::min(n, m);
     }
     if (ti->splitKernel) {
       int m = 0;
       if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ti->splitKernel),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds)) ||
-          CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, ti->splitKernel, kThreads, lds))) return 0;
+          CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, ti->splitKernel, (int)ti->threads, lds))) return 0;
       n = std::min(n, m);
     }
     ti->residentPerCU = n;
@@ -265,7 +266,7 @@ cusync_error cusync_conv2d_run(const cusync_conv2d_args* a, void* stream) {
   if (a->max_workgroups > 0) launched = std::min<uint32_t>(launched, (uint32_t)a->max_workgroups);
 
   GemmParams p = convParams(a, ti, launched);
-  hipLaunchKernelGGL(a->split_k > 1 ? ti->splitKernel : ti->kernel, dim3(launched), dim3(kThreads), lds, (hipStream_t)stream, p);
+  hipLaunchKernelGGL(a->split_k > 1 ? ti->splitKernel : ti->kernel, dim3(launched), dim3(ti->threads), lds, (hipStream_t)stream, p);
   if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
   cusync::rt::noteLaunch(a->stage, launched >= (uint32_t)resident);
   return CUSYNC_SUCCESS;
@@ -475,7 +476,7 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
         if (e != CUSYNC_SUCCESS) return e;
         cp.layer[i] = convParams(&a, ti, launched);
       }
-      hipLaunchKernelGGL(ti->chainKernel, dim3(launched), dim3(kThreads), lds, c->stream[0], cp);
+      hipLaunchKernelGGL(ti->chainKernel, dim3(launched), dim3(ti->threads), lds, c->stream[0], cp);
       if (CUSYNC_HIP(hipGetLastError()) || CUSYNC_HIP(hipEventRecord(c->done[0], c->stream[0]))) return CUSYNC_ERROR_DEVICE;
       const cusync_error e = cusync::rt::waitEnd(c->st[n - 1], c->stream[0], "conv chain");
       if (e != CUSYNC_SUCCESS) return e;

@@ -16,10 +16,14 @@
 // measured the same: four and five stages against three on 28x28x128).
 //
 // LDS: [filter stages of BN x 64 halfs][halo: (BM + 2W + 2) pixels x C halfs][one pixel of zeros].
-// A pixel's 16-byte channel chunks are stored at chunk ^ (pixel & (C/8 - 1)),
-// so the 32 consecutive pixels an MFMA fragment reads fall on distinct banks.
+// An LDS read of 16 bytes per lane is served sixteen lanes at a time over all 64 banks, so the sixteen consecutive
+// pixels (or filter rows) of such a group must fall into sixteen different places of 16 bytes.  A pixel's chunks are
+// stored at chunk ^ (pixel & (C/8 - 1)); where a pixel is 128 bytes (C = 64), and in the filter's 128-byte rows, two
+// neighbours cover all banks once and take one position: chunk ^ (pixel/2 & 7).  (With neighbours in different
+// positions, rows r and r + 8 share their banks: pairs under RowSync 38.7 -> 37.6 us at 32x28x28x128, 51.5 -> 49.8 at
+// 32x7x7x512, level at the other stages.)
 //
-// Every wavefront owns a 64 x 64 piece of the tile (two by two MFMA tiles): with
+// Every wavefront (of a group) owns a 64 x 64 piece of the tile (two by two MFMA tiles), 32 x 64 of the 64-pixel tile: with
 // 64 x 32 the kernel spent its time on LDS reads, three 16-byte reads per two
 // MFMAs (measured: 0.54 us per 64-channel step against 0.1 us of MFMA work).
 #pragma once
@@ -34,20 +38,45 @@ namespace gemm {
 // 39.9 / 48.6 / 63.8; two 39.7 / 49.4 / 65.2; the whole step up front 39.9 / 52.3 / 71.6.
 constexpr int kFragsAhead = 1;
 
-template<int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_>
+// How the accumulators leave a tile: as the kernel's wavefronts hold them, or (two groups, see KG) as they hold them
+// once the groups have put their halves of the channels together.
+template<int BM_, int BN_, int WM_, int WN_, int THREADS_, int LDS_BYTES_>
+struct HaloFinishCfg {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, THREADS = THREADS_, LDS_BYTES = LDS_BYTES_;
+  static constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
+};
+
+// KG: groups of four wavefronts.  A tile that has its CU to itself (the halo of 128 channels and more fills the LDS)
+// would run one wavefront per SIMD, which has nothing to issue while it waits for its fragments or at the barrier:
+// a 64-channel step of the 128x128 tile took 0.57 us against 0.21 us of MFMAs.  Two groups share the tile: group g
+// multiplies channels 32g..32g+31 of every step, the same 64 x 64 per wavefront and as many bytes read from LDS, and
+// at the end each gives the other half of its sums through LDS.  Pairs under RowSync by the device's clock, one group ->
+// two, in us: 8x28x28x128 32.7 -> 30.7, 8x14x14x256 39.2 -> 35.2, 32x14x14x256 48.5 -> 46.6, 8x7x7x512 39.1 -> 35.5,
+// 32x7x7x512 54.6 -> 51.5; in one launch without runs 14x14x256 68.2 -> 56.3.  A step still takes 0.5 us: with the
+// barrier between the two products and the first fragments of a step read ahead of it (a ring of four chunks where it
+// fits) 48.3 at 32x14x14x256, and with tiles beginning at different steps of their range 47.2.
+template<int BM_, int BN_, int WM_, int WN_, int STAGES_, int OCC_, int KG_ = 1>
 struct Halo3x3Cfg {
-  static constexpr int BM = BM_, BN = BN_, BK = 64, WM = WM_, WN = WN_, STAGES = STAGES_, OCC = OCC_;
-  static constexpr int THREADS = kThreads;
-  static constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32, KS = BK / 16;
+  static constexpr int BM = BM_, BN = BN_, BK = 64, WM = WM_, WN = WN_, STAGES = STAGES_, OCC = OCC_, KG = KG_;
+  static constexpr int WAVES = 4 * KG, THREADS = WAVES * 64;
+  static constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32, KS = BK / 16 / KG;      // KS: 16-channel products per wavefront and step
   static constexpr int B_ROW_BYTES = BK * 2, B_CPR = B_ROW_BYTES / 16;
-  static constexpr int B_STAGE = BN * B_ROW_BYTES, B_LOADS = B_STAGE / 1024 / 4;
+  static constexpr int B_STAGE = BN * B_ROW_BYTES, B_LOADS = B_STAGE / 1024 / WAVES;
   static constexpr int B_BYTES = STAGES * B_STAGE;
-  static constexpr int LDS_BYTES = B_BYTES;        // what the epilogue may use (finishTile)
-  static_assert(WM * WN == 4 && B_CPR == 8 && B_LOADS >= 1, "four wavefronts, 64-channel filter chunks");
+  // The halves of two groups: of the wavefront's two rows of MFMA tiles, or of its two columns where it has one row.
+  static constexpr bool HALVE_ROWS = TM == 2;
+  static constexpr int EXCHANGE_BYTES = KG == 1 ? 0 : BM * BN * 4;
+  // what the epilogue may use (finishTile): with two groups also the halo's place, for the share of a tile a run of
+  // two adds up itself
+  static constexpr int FINISH_BYTES = KG == 1 ? B_BYTES : (BM * (BN * 2 + 16) + 1023) / 1024 * 1024 + (BM / 2) * BN * 4;
+  using Finish = HaloFinishCfg<BM, BN, KG == 2 && HALVE_ROWS ? 2 * WM : WM, KG == 2 && !HALVE_ROWS ? 2 * WN : WN, THREADS, FINISH_BYTES>;
+  static_assert(WM * WN == 4 && B_CPR == 8 && B_LOADS >= 1, "four wavefronts per group, 64-channel filter chunks");
+  static_assert(KG == 1 || (KG == 2 && (TM == 2 || (TM == 1 && TN == 2))), "two groups exchange halves of a wavefront's tile");
   // Bytes of LDS a launch needs for images of width W with C channels.
   static uint32_t ldsBytes(uint32_t W, uint32_t C) {
     const uint32_t haloBytes = (BM + 2 * W + 3) * C * 2;      // the run of input pixels and one pixel of zeros behind it
-    return B_BYTES + (haloBytes + 1023) / 1024 * 1024;
+    const uint32_t bytes = B_BYTES + (haloBytes + 1023) / 1024 * 1024, finish = FINISH_BYTES > EXCHANGE_BYTES ? FINISH_BYTES : EXCHANGE_BYTES;
+    return bytes > finish ? bytes : finish;
   }
 };
 
@@ -63,12 +92,14 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / C::WN, wn = wave % C::WN;
+  const int group = C::KG == 1 ? 0 : wave >> 2, inGroup = wave & 3;
+  const int wm = inGroup / C::WN, wn = inGroup % C::WN;
   const uint32_t hi = lane >> 5;
   const cusync::DynStage& stage = p.stage;
 
   const uint32_t Cc = p.cvC, W = p.cvW, H = p.cvH;
   const uint32_t pixBytes = Cc * 2, cprMask = Cc / 8 - 1;             // C is a power of two
+  const uint32_t swzShift = Cc == 64 ? 1 : 0;
   const uint32_t pixShift = 31 - __builtin_clz(pixBytes);
   const uint32_t haloPix = C::BM + 2 * W + 2;
   const uint32_t haloLoads = ((haloPix + 1) * pixBytes + 1023) / 1024;       // 1 KiB pieces; pixel haloPix is the pixel of zeros
@@ -80,21 +111,21 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
   const uint32_t ldsHalo = ldsBase + C::B_BYTES;
   const char* halo = smem + C::B_BYTES;
 
-  // Filter stage: [BN rows = output channels][BK halfs], chunk c of row n at slot c ^ (n & 7).
+  // Filter stage: [BN rows = output channels][BK halfs], chunk c of row n at slot c ^ (n/2 & 7).
   uint32_t bLoadRow[C::B_LOADS], bLoadChunk[C::B_LOADS];
 #pragma unroll
   for (int q = 0; q < C::B_LOADS; q++) {
     const uint32_t slot = (wave * C::B_LOADS + q) * 64 + lane;
     bLoadRow[q] = slot / C::B_CPR;
-    bLoadChunk[q] = (slot % C::B_CPR) ^ (bLoadRow[q] & 7);
+    bLoadChunk[q] = (slot % C::B_CPR) ^ ((bLoadRow[q] >> 1) & 7);
   }
   // fragment of MFMA tile j, k-step kk: row wn*WTN + 32j + lane%32 (a multiple of 32 more does not change
-  // row & 7), chunk 2kk + hi
+  // row/2 & 7), chunk 2kk + hi
   uint32_t bFrag[C::KS];
   {
     const uint32_t row = wn * C::WTN + (lane & 31);
 #pragma unroll
-    for (int kk = 0; kk < C::KS; kk++) bFrag[kk] = row * C::B_ROW_BYTES + (((2 * kk + hi) ^ (row & 7)) * 16);
+    for (int kk = 0; kk < C::KS; kk++) bFrag[kk] = row * C::B_ROW_BYTES + (((2 * (group * C::KS + kk) + hi) ^ ((row >> 1) & 7)) * 16);
   }
 
   const uint32_t numTiles = stage.numTiles();
@@ -151,10 +182,10 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
 
     // Halo: input pixels m0 - (W+1) .. m0 + BM + W, 1 KiB per load; pixels before the first or after the
     // last image are sent out of range and arrive as zeros.
-    for (uint32_t q = wave; q < haloLoads; q += 4) {
+    for (uint32_t q = wave; q < haloLoads; q += C::WAVES) {
       const uint32_t byteOff = q * 1024 + lane * 16;
       const uint32_t pl = byteOff >> pixShift, slot = (byteOff & (pixBytes - 1)) >> 4;
-      const uint32_t chunk = slot ^ (pl & cprMask);
+      const uint32_t chunk = slot ^ ((pl >> swzShift) & cprMask);
       const uint32_t flat = m0 + pl - (W + 1);                       // wraps below zero for the first tile
       const bool inside = m0 + pl >= W + 1 && flat < p.M && pl < haloPix;
       loadToLds(rA, __builtin_amdgcn_readfirstlane(ldsHalo + q * 1024), inside ? (flat * Cc + chunk * 8) * 2 : kOutOfRange);
@@ -196,7 +227,7 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
       for (int i = 0; i < C::TM; i++) {
         const uint32_t pl = (uint32_t)((int32_t)(aPixel0 + i * 32) + shift);
         aBase[i] = (tapMask[i] >> tap) & 1 ? pl << pixShift : zeroPixel;
-        aSwz[i] = pl & cprMask;      // any slot of the pixel of zeros will do
+        aSwz[i] = (pl >> swzShift) & cprMask;      // any slot of the pixel of zeros will do
       }
       // The fragments of 16 channels are requested kFragsAhead products of 16 channels before they are used.
       half8 fb[C::KS][C::TN], fa[C::KS][C::TM];
@@ -205,7 +236,7 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
         for (int j = 0; j < C::TN; j++) fb[kk][j] = *reinterpret_cast<const half8*>(sb + bFrag[kk] + j * 32 * C::B_ROW_BYTES);
 #pragma unroll
         for (int i = 0; i < C::TM; i++) {
-          const uint32_t chunk = cc * (C::BK / 8) + 2 * kk + hi;
+          const uint32_t chunk = cc * (C::BK / 8) + 2 * (group * C::KS + kk) + hi;
           fa[kk][i] = *reinterpret_cast<const half8*>(halo + aBase[i] + ((chunk ^ aSwz[i]) << 4));
         }
       };
@@ -228,7 +259,40 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
     waitVmcnt<0>();
     const unsigned long long tl2 = p.timeline ? wall_clock64() : 0;
     if (tid == 0) nextRaw = stage.drawBegin(dryXcds, noDraws);     // settled after the epilogue
-    const bool completed = finishTile<C, SPLIT>(p, acc, t, wm, wn, lane, &sLast, smem);
+    using F = typename C::Finish;
+    bool completed;
+    if constexpr (C::KG == 1) {
+      completed = finishTile<F, SPLIT>(p, acc, t, wm, wn, lane, &sLast, smem);
+    } else {
+      // Group g keeps half g of the sums, its own and the other group's: sixteen bytes per lane and piece, every
+      // lane's values in a place of their own.
+      floatx16 sums[F::TM][F::TN];
+      constexpr int HALF = F::TM * F::TN;
+      static_assert(F::TM == 1, "half of two rows, or one of two columns, of MFMA tiles");
+      auto place = [&](int to, int h, int g) { return smem + (((inGroup * 2 + to) * HALF + h) * 4 + g) * 1024 + lane * 16; };
+      auto part = [&](int half, int h) { return C::HALVE_ROWS ? acc[half][h] : acc[0][half]; };
+      __syncthreads();             // every wavefront is out of the steps and its loads have landed
+#pragma unroll
+      for (int h = 0; h < HALF; h++) {
+        floatx16 give;
+        if (group == 0) { give = part(1, h); sums[0][h] = part(0, h); }
+        else { give = part(0, h); sums[0][h] = part(1, h); }
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          *reinterpret_cast<floatx4*>(place(1 - group, h, g)) = floatx4{give[4 * g], give[4 * g + 1], give[4 * g + 2], give[4 * g + 3]};
+      }
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < HALF; h++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const floatx4 v = *reinterpret_cast<const floatx4*>(place(group, h, g));
+#pragma unroll
+          for (int e = 0; e < 4; e++) sums[0][h][4 * g + e] += v[e];
+        }
+      if constexpr (C::HALVE_ROWS) completed = finishTile<F, SPLIT>(p, sums, t, 2 * wm + group, wn, lane, &sLast, smem);
+      else completed = finishTile<F, SPLIT>(p, sums, t, wm, 2 * wn + group, lane, &sLast, smem);
+    }
     cusync_dim3 done = {m0, n0, 0};
     if (completed && stage.isProducer()) stage.post(done, 1, stage.storesThrough());
     else __syncthreads();
@@ -238,7 +302,7 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
 }
 
 template<class C, bool SPLIT = false>
-__global__ __launch_bounds__(kThreads, C::OCC) void convHalo3x3Kernel(GemmParams p) {
+__global__ __launch_bounds__(C::THREADS, C::OCC) void convHalo3x3Kernel(GemmParams p) {
   convHalo3x3Layer<C, SPLIT>(p);
 }
 
@@ -256,7 +320,7 @@ struct ConvChainParams {
 };
 
 template<class C>
-__global__ __launch_bounds__(kThreads, C::OCC) void convHalo3x3ChainKernel(ConvChainParams cp) {
+__global__ __launch_bounds__(C::THREADS, C::OCC) void convHalo3x3ChainKernel(ConvChainParams cp) {
   for (uint32_t l = 0; l < cp.layers; l++) {
     convHalo3x3Layer<C, false>(cp.layer[l]);
     __syncthreads();        // everyone has read the last ticket of this layer before the next one's is written

@@ -106,6 +106,22 @@ def test_conv_matches_oracle(tile, geom):
     assert_close(got, orc.conv2d_nhwc(x, w, pad, stride), "y")
 
 
+@pytest.mark.parametrize("tile", [api.CONV_TILE.HALO_128x128x64, api.CONV_TILE.HALO_64x128x64])
+@pytest.mark.parametrize("geom", [(1, 1, 3, 128, 8), (1, 8, 8, 128, 128), (1, 5, 13, 128, 136), (3, 7, 7, 512, 264), (1, 129, 1, 256, 128)])
+@pytest.mark.parametrize("split_k", [1, 2, 4])
+def test_two_groups_of_wavefronts_share_a_tile(tile, geom, split_k):
+    """Each group sums half of every step's channels: with integers the sums are exact (at most 9 * 512 * 4 < 2^24, and
+    the oracle rounds them to halfs as the kernel does), so a channel left out or counted twice shows bit by bit."""
+    print("conv groups", tile, geom, split_k, flush=True)
+    N, H, W, Cc, K = geom
+    if not fits(tile, Cc, W=W):
+        pytest.skip("geometry outside the halo tile's domain")
+    rng = np.random.default_rng(Cc + K)
+    x, w = rng.integers(-2, 3, (N, H, W, Cc)).astype(np.float16), rng.integers(-2, 3, (K, 3, 3, Cc)).astype(np.float16)
+    got = run_conv(x, w, tile, launches=2, split_k=split_k)
+    assert np.array_equal(got.view(np.uint16), orc.conv2d_nhwc(x, w).view(np.uint16))
+
+
 HALO_TILES = [api.CONV_TILE.HALO_256x64x64, api.CONV_TILE.HALO_128x128x64, api.CONV_TILE.HALO_64x128x64]
 
 
