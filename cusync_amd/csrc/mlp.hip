@@ -332,10 +332,13 @@ bool choose(const cusync_mlp_config& given, Choice* o) {
   const bool llama = c.model == CUSYNC_MLP_LLAMA;
   // one_launch < 0: where one launch measured ahead of two on the GPT-3 shard (1 to 64 rows under either policy:
   // 1-5 us of 67-83; 512 to 1024 rows: 1-3 us of 172-284; behind at 256 rows and from 1025 on, and at every size of
-  // the LLaMA shard, whose GEMM2 wants a tile of its own) and the tiles are the table's
+  // the LLaMA shard, whose GEMM2 wants a tile of its own, but for StridedSync up to 32 rows, where both take 32x128) and
+  // the tiles are the table's.  LLaMA under StridedSync, by the device's clock in us, two launches -> one, inner 2752 /
+  // 2816: 1 row 37.3 -> 34.7 / 39.2 -> 36.1, 16 rows 38.3 -> 35.3 / 40.2 -> 37.0, 32 rows 39.2 -> 36.4 / 41.6 -> 38.3
+  // (a third of that under RowSync, which keeps its two launches).
   const bool automatic = c.one_launch < 0;
-  if (automatic) c.one_launch = c.sync != CUSYNC_SYNC_STREAM && !llama && c.tile1 < 0 && c.tile2 < 0 &&
-                                (c.batch <= 64 || (c.batch >= 512 && c.batch <= 1024));
+  if (automatic) c.one_launch = c.sync != CUSYNC_SYNC_STREAM && c.tile1 < 0 && c.tile2 < 0 &&
+                                (llama ? c.sync == CUSYNC_SYNC_STRIDED && c.batch <= 32 : c.batch <= 64 || (c.batch >= 512 && c.batch <= 1024));
   const uint32_t k1 = c.hidden, n1 = llama ? 2 * c.inner : c.inner, k2 = c.inner, n2 = c.hidden;
   const bool swiglu = llama && c.activation;
   // where silu(gate) * up is computed: 2 = GEMM1's epilogue (the built-in choice), -1 = a stage of its own, 1 = GEMM2's A loader

@@ -215,6 +215,20 @@ def test_llama_mlp_in_one_launch(batch, sync):
     check_against_oracle(api.MODEL.LLAMA, x, w1, w2, h, y, inner=2752, fused=True)
 
 
+@pytest.mark.parametrize("inner", [2752, 2816])
+@pytest.mark.parametrize("batch,one", [(1, 1), (32, 1), (33, 0)])
+def test_llama_strided_takes_one_launch_up_to_32_rows(batch, inner, one):
+    import ctypes as C
+    from cusync_amd import _lib
+    print("llama strided launches", batch, inner, flush=True)
+    x, w1, w2, h, y, prod, cons, tiles, _ = run_mlp(api.MODEL.LLAMA, batch, 8192, inner, api.SYNC.STRIDED, runs=3, one_launch=-1)
+    cfg = _lib.MlpConfig(api.MODEL.LLAMA, batch, 8192, inner, api.SYNC.STRIDED, -1, -1, -1, 1, 0, 0, 0, 0, -1, 0, 0)
+    v = [C.c_int(-1) for _ in range(5)]
+    assert _lib.load().cusync_mlp_choice(C.byref(cfg), *[C.byref(i) for i in v]) == 0 and v[4].value == one
+    assert cons.spin_timeouts == 0 and prod.spin_timeouts == 0
+    check_against_oracle(api.MODEL.LLAMA, x, w1, w2, h, y, inner=inner, fused=True)
+
+
 def test_mlp_in_one_launch_rejects():
     w1, w2, dw1, dw2 = weights(api.MODEL.GPT3, 12288, 6144)
     with pytest.raises(RuntimeError):       # two different tiles cannot share a launch
