@@ -159,7 +159,7 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
         const uint32_t kv = h * kPieceKeys + 4 * hi;
 #pragma unroll
         for (int r = 0; r < 16; r++)
-          if (kv + 8 * (r / 4) + (r % 4) > limit) sc[r] = kMasked;
+          if (kv + 8 * (r / 4) + (r % 4) > limit) sc[r] = kUnseen;
       }
       float pieceMax = sc[0];
 #pragma unroll

@@ -52,7 +52,11 @@ constexpr int kRowBytes = kHD * 2;                  // one K or V row of a head
 constexpr int kStageBytes = kBKV * kRowBytes;       // one K or one V block
 constexpr int ldsBytes(int stages) { return stages * 2 * kStageBytes; }      // `stages` blocks of K and of V
 constexpr int kBlockLoads = 8;                      // 1 KiB direct loads per wavefront and block (four of K, four of V)
-constexpr float kMasked = -1.0e30f;
+constexpr float kMasked = -1.0e30f;                 // running maximum of a query that has seen no key yet
+// Score of a key its query does not see.  The weight is exp2(fma(score, scale, -max * scale)): -infinity makes it 0 whatever
+// the maximum.  With kMasked here, a query that sees none of a piece's keys and has seen none before would get exp2 of the
+// rounding error of kMasked * scale, which is of the order of 1e21: 0 or infinity, by its sign.
+constexpr float kUnseen = -__builtin_inff();
 
 struct AttnParams {
   cusync::DynStage stage;
@@ -305,7 +309,7 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
         for (int a = 0; a < 2; a++)
 #pragma unroll
           for (int r = 0; r < 16; r++)
-            if (kvBase + 32 * a + 8 * (r / 4) + (r % 4) > limit) sacc[a][r] = kMasked;
+            if (kvBase + 32 * a + 8 * (r / 4) + (r % 4) > limit) sacc[a][r] = kUnseen;
       }
       float blockMax = kMasked;
 #pragma unroll

@@ -254,7 +254,7 @@ def test_attention_layer_with_cache(S, cached):
 
 # ---- key range split over several workgroups --------------------------------------------------------------
 
-def run_attention_split(qkv, cached, heads, causal, blocks, launches=2, max_workgroups=0):
+def run_attention_split(qkv, cached, heads, causal, blocks, launches=2, max_workgroups=0, scale=0.0):
     import torch
     L = _lib.load()
     S = qkv.shape[0] - cached
@@ -269,7 +269,7 @@ def run_attention_split(qkv, cached, heads, causal, blocks, launches=2, max_work
         do.fill_(float("nan"))
         torch.cuda.synchronize()
         rc = api.attention(st, S, heads, dq.data_ptr(), qkv.shape[1], do.data_ptr(), heads * 128, causal=causal, cached_rows=cached,
-                           kv_split_blocks=blocks, workspace=ws.data_ptr(), max_workgroups=max_workgroups)
+                           kv_split_blocks=blocks, workspace=ws.data_ptr(), max_workgroups=max_workgroups, scale=scale)
         assert rc == api.ERR.SUCCESS, api.last_error()
         assert L.cusync_rt_device_sync() == 0, api.last_error()
     assert st.read_state().tile_counter == 0
