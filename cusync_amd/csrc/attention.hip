@@ -96,6 +96,7 @@ struct cusync_attn_layer {
   hipStream_t stream[3];
   hipEvent_t done[3];              // behind the run's last launch on each stream (see rt::waitEnd)
   uint32_t timeoutsSeen;           // sum of the stages' give-up counters when the last run returned
+  bool broken;                     // a run failed behind a launch (see rt::abandonRun)
 };
 
 extern "C" void cusync_attn_layer_destroy(cusync_attn_layer* L);
@@ -400,6 +401,7 @@ void cusync_attn_layer_destroy(cusync_attn_layer* L) {
 cusync_error cusync_attn_layer_run(cusync_attn_layer* L, const void* x, void* qkv, void* o, void* y, int runs,
                                    double* times_us, double* stage_us) {
   if (!L || !x || !qkv || !o || !y) return CUSYNC_ERROR_NOT_INITIALIZED;
+  if (L->broken) return cusync::rt::refuseBroken("attn layer");
   const bool overlapped = L->cfg.sync != CUSYNC_SYNC_STREAM;
   const uint32_t S = L->cfg.seq, E = L->E, H = L->cfg.hidden;
   for (int r = 0; r < runs; r++) {
@@ -421,18 +423,21 @@ cusync_error cusync_attn_layer_run(cusync_attn_layer* L, const void* x, void* qk
 
     hipStream_t s0 = L->stream[0], s1 = overlapped ? L->stream[1] : s0, s2 = overlapped ? L->stream[2] : s0;
     cusync_error e;
+    if (r == 0 && ((e = cusync_gemm_can_implement(&a1)) != CUSYNC_SUCCESS || (e = cusync_attention_can_implement(&a2)) != CUSYNC_SUCCESS ||
+                   (e = cusync_gemm_can_implement(&a3)) != CUSYNC_SUCCESS)) return e;      // before anything is launched
+    auto failed = [&](cusync_error why) { return cusync::rt::abandonRun(L->stream, 3, &L->broken, why); };
     if ((e = cusync_gemm_run(&a1, s0)) != CUSYNC_SUCCESS) return e;
     // overlapped: each consumer's stream is held back until every workgroup of its producer has started: from the
     // host when the producer's launch took every workgroup slot of the device (a wait kernel's wave would keep its
     // last workgroup off the device), by the wait kernel otherwise.
-    if (overlapped && (e = cusync_hold_back(&L->st[0], s1)) != CUSYNC_SUCCESS) return e;
-    if ((e = cusync_attention_run(&a2, s1)) != CUSYNC_SUCCESS) return e;
-    if (overlapped && (e = cusync_hold_back(&L->st[1], s2)) != CUSYNC_SUCCESS) return e;
-    if ((e = cusync_gemm_run(&a3, s2)) != CUSYNC_SUCCESS) return e;
+    if (overlapped && (e = cusync_hold_back(&L->st[0], s1)) != CUSYNC_SUCCESS) return failed(e);
+    if ((e = cusync_attention_run(&a2, s1)) != CUSYNC_SUCCESS) return failed(e);
+    if (overlapped && (e = cusync_hold_back(&L->st[1], s2)) != CUSYNC_SUCCESS) return failed(e);
+    if ((e = cusync_gemm_run(&a3, s2)) != CUSYNC_SUCCESS) return failed(e);
     hipStream_t on[3] = {s0, s1, s2};
-    for (int i = overlapped ? 0 : 2; i < 3; i++) if (CUSYNC_HIP(hipEventRecord(L->done[i], on[i]))) return CUSYNC_ERROR_DEVICE;
+    for (int i = overlapped ? 0 : 2; i < 3; i++) if (CUSYNC_HIP(hipEventRecord(L->done[i], on[i]))) return failed(CUSYNC_ERROR_DEVICE);
     for (int i = 2; i >= (overlapped ? 0 : 2); i--)
-      if ((e = cusync::rt::waitEnd(L->st[i], on[i], "attn layer")) != CUSYNC_SUCCESS) return e;
+      if ((e = cusync::rt::waitEnd(L->st[i], on[i], "attn layer")) != CUSYNC_SUCCESS) return failed(e);
     if (times_us) times_us[r] = cusync::rt::stampsUs(L->st[0], false, L->st[2]);
     if (!overlapped && stage_us)
       for (int i = 0; i < 3; i++) stage_us[3 * r + i] = cusync::rt::stampsUs(L->st[i ? i - 1 : 0], i > 0, L->st[i]);

@@ -285,6 +285,7 @@ struct cusync_conv_chain {
   std::vector<void*> ws;             // per layer: partial sums and counters of the runs a tile's steps are cut into
   int splitK = 1;
   uint32_t timeoutsSeen = 0;         // sum of the stages' give-up counters when the last run returned
+  bool broken = false;               // a run failed behind a launch (see rt::abandonRun)
 };
 
 namespace {
@@ -442,6 +443,7 @@ void cusync_conv_chain_destroy(cusync_conv_chain* c) {
 cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* const* ys, int runs,
                                    double* times_us, double* layer_us) {
   if (!c || !x || !ys) return CUSYNC_ERROR_NOT_INITIALIZED;
+  if (c->broken) return cusync::rt::refuseBroken("conv chain");
   const uint32_t n = c->cfg.layers;
   const bool overlapped = c->cfg.sync != CUSYNC_SYNC_STREAM;
   auto layerArgs = [&](uint32_t i) {
@@ -459,6 +461,12 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
     a.workspace = c->splitK > 1 ? c->ws[i] : nullptr;
     return a;
   };
+  for (uint32_t i = 0; runs > 0 && i < n; i++) {      // before anything is launched
+    const cusync_conv2d_args a = layerArgs(i);
+    const cusync_error e = cusync_conv2d_can_implement(&a);
+    if (e != CUSYNC_SUCCESS) return e;
+  }
+  auto failed = [&](cusync_error why) { return cusync::rt::abandonRun(c->stream.data(), (int)c->stream.size(), &c->broken, why); };
   if (overlapped && c->cfg.fused) {
     // all layers in one launch on the first stream
     ConvTile* ti = convTile(c->cfg.tile);
@@ -472,14 +480,12 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
       cp.layers = n;
       for (uint32_t i = 0; i < n; i++) {
         const cusync_conv2d_args a = layerArgs(i);
-        const cusync_error e = cusync_conv2d_can_implement(&a);
-        if (e != CUSYNC_SUCCESS) return e;
         cp.layer[i] = convParams(&a, ti, launched);
       }
       hipLaunchKernelGGL(ti->chainKernel, dim3(launched), dim3(ti->threads), lds, c->stream[0], cp);
-      if (CUSYNC_HIP(hipGetLastError()) || CUSYNC_HIP(hipEventRecord(c->done[0], c->stream[0]))) return CUSYNC_ERROR_DEVICE;
+      if (CUSYNC_HIP(hipGetLastError()) || CUSYNC_HIP(hipEventRecord(c->done[0], c->stream[0]))) return failed(CUSYNC_ERROR_DEVICE);
       const cusync_error e = cusync::rt::waitEnd(c->st[n - 1], c->stream[0], "conv chain");
-      if (e != CUSYNC_SUCCESS) return e;
+      if (e != CUSYNC_SUCCESS) return failed(e);
       if (times_us) times_us[r] = cusync::rt::stampsUs(c->st[0], false, c->st[n - 1]);
       for (uint32_t i = 0; i < n; i++) c->st[i].iter += 1;
     }
@@ -493,13 +499,13 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
       // overlapped: layer i's stream is held back until layer i - 1 is on the device: by the reference's wait kernel
       // where that layer's launch left workgroup slots free (392 tiles on 512 slots for the benchmark shapes), so
       // that the wait kernel's wave takes nothing from the producer; from this thread where the launch took them all.
-      if (overlapped && i > 0 && (e = cusync_hold_back(&c->st[i - 1], s)) != CUSYNC_SUCCESS) return e;
-      if ((e = cusync_conv2d_run(&a, s)) != CUSYNC_SUCCESS) return e;
+      if (overlapped && i > 0 && (e = cusync_hold_back(&c->st[i - 1], s)) != CUSYNC_SUCCESS) return failed(e);
+      if ((e = cusync_conv2d_run(&a, s)) != CUSYNC_SUCCESS) return i ? failed(e) : e;
     }
-    for (uint32_t i = 0; i < (overlapped ? n : 1); i++) if (CUSYNC_HIP(hipEventRecord(c->done[i], c->stream[i]))) return CUSYNC_ERROR_DEVICE;
+    for (uint32_t i = 0; i < (overlapped ? n : 1); i++) if (CUSYNC_HIP(hipEventRecord(c->done[i], c->stream[i]))) return failed(CUSYNC_ERROR_DEVICE);
     for (uint32_t i = n; i-- > (overlapped ? 0 : n - 1);) {
       const cusync_error e = cusync::rt::waitEnd(c->st[i], c->stream[overlapped ? i : 0], "conv chain");
-      if (e != CUSYNC_SUCCESS) return e;
+      if (e != CUSYNC_SUCCESS) return failed(e);
     }
     if (times_us) times_us[r] = cusync::rt::stampsUs(c->st[0], false, c->st[n - 1]);
     if (!overlapped && layer_us)

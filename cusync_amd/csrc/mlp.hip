@@ -32,6 +32,7 @@ struct cusync_mlp {
   cusync_stage_desc prod, cons;
   hipStream_t sProd, sCons;
   hipEvent_t done[3];                // behind the run's last launch on sProd, sCons, sMid (see rt::waitEnd)
+  bool broken;                       // a run failed behind a launch (see rt::abandonRun)
   // LLaMA with silu(gate) * up as GEMM1's epilogue: w1p holds W1 with the gate and up columns interleaved in
   // groups of eight, the intermediate is [batch][inner]
   bool fused;
@@ -576,11 +577,18 @@ void cusync_mlp_destroy(cusync_mlp* m) {
 cusync_error cusync_mlp_run_split(cusync_mlp* m, const void* x, void* h, void* y, int runs,
                                   double* times_us, double* gemm1_us, double* gemm2_us) {
   if (!m || !x || !h || !y) return CUSYNC_ERROR_NOT_INITIALIZED;
+  if (m->broken) return cusync::rt::refuseBroken("mlp");
   const bool overlapped = m->prod.out.kind != CUSYNC_POLICY_NOSYNC;
+  auto failed = [&](cusync_error why) {
+    const hipStream_t streams[3] = {m->sProd, m->sCons, m->sMid};
+    return cusync::rt::abandonRun(streams, 3, &m->broken, why);
+  };
   for (int r = 0; r < runs; r++) {
     cusync_gemm_args a1 = gemmArgs(m, 0, x, h, y);
     cusync_gemm_args a2 = gemmArgs(m, 1, x, h, y);
     cusync_error e;
+    if (r == 0 && ((e = cusync_gemm_can_implement(&a1)) != CUSYNC_SUCCESS ||
+                   (e = cusync_gemm_can_implement(&a2)) != CUSYNC_SUCCESS)) return e;      // before anything is launched
     if (overlapped && m->cfg.one_launch) {
       // both GEMMs in one launch: same stages and semaphores, no wait kernel, no second launch
       const cusync_gemm_args both[2] = {a1, a2};
@@ -593,25 +601,25 @@ cusync_error cusync_mlp_run_split(cusync_mlp* m, const void* x, void* h, void* y
       // of the CUs would keep the last producer workgroup off the device until another retires); for any other
       // the reference's wait kernel goes into the consumer's stream, unordered like the reference's.
       if (m->actStage) {        // GEMM1 -> activation -> GEMM2, a stream and a hold-back per edge
-        if ((e = cusync_hold_back(&m->prod, m->sMid)) != CUSYNC_SUCCESS) return e;
-        if ((e = runActStage(m, h, m->sMid)) != CUSYNC_SUCCESS) return e;
-        if ((e = cusync_invoke_wait_kernel(&m->mid, m->sCons)) != CUSYNC_SUCCESS) return e;
+        if ((e = cusync_hold_back(&m->prod, m->sMid)) != CUSYNC_SUCCESS) return failed(e);
+        if ((e = runActStage(m, h, m->sMid)) != CUSYNC_SUCCESS) return failed(e);
+        if ((e = cusync_invoke_wait_kernel(&m->mid, m->sCons)) != CUSYNC_SUCCESS) return failed(e);
       } else if ((e = cusync_hold_back(&m->prod, m->sCons)) != CUSYNC_SUCCESS) {
-        return e;
+        return failed(e);
       }
-      if ((e = cusync_gemm_run(&a2, m->sCons)) != CUSYNC_SUCCESS) return e;
+      if ((e = cusync_gemm_run(&a2, m->sCons)) != CUSYNC_SUCCESS) return failed(e);
     } else {
-      if (m->actStage && (e = runActStage(m, h, m->sProd)) != CUSYNC_SUCCESS) return e;     // counted with GEMM2
-      if ((e = cusync_gemm_run(&a2, m->sProd)) != CUSYNC_SUCCESS) return e;
+      if (m->actStage && (e = runActStage(m, h, m->sProd)) != CUSYNC_SUCCESS) return failed(e);     // counted with GEMM2
+      if ((e = cusync_gemm_run(&a2, m->sProd)) != CUSYNC_SUCCESS) return failed(e);
     }
     // Every launch of the run reports its end, the consumer's last: the stages are then free for the next run.
     const bool ownStreams = overlapped && !m->cfg.one_launch;
     if (CUSYNC_HIP(hipEventRecord(m->done[0], m->sProd)) || (ownStreams && CUSYNC_HIP(hipEventRecord(m->done[1], m->sCons))) ||
-        (ownStreams && m->actStage && CUSYNC_HIP(hipEventRecord(m->done[2], m->sMid)))) return CUSYNC_ERROR_DEVICE;
-    if ((e = cusync::rt::waitEnd(m->cons, ownStreams ? m->sCons : m->sProd, "mlp")) != CUSYNC_SUCCESS) return e;
+        (ownStreams && m->actStage && CUSYNC_HIP(hipEventRecord(m->done[2], m->sMid)))) return failed(CUSYNC_ERROR_DEVICE);
+    if ((e = cusync::rt::waitEnd(m->cons, ownStreams ? m->sCons : m->sProd, "mlp")) != CUSYNC_SUCCESS) return failed(e);
     if (ownStreams) {
-      if ((e = cusync::rt::waitEnd(m->prod, m->sProd, "mlp")) != CUSYNC_SUCCESS) return e;
-      if (m->actStage && (e = cusync::rt::waitEnd(m->mid, m->sMid, "mlp")) != CUSYNC_SUCCESS) return e;
+      if ((e = cusync::rt::waitEnd(m->prod, m->sProd, "mlp")) != CUSYNC_SUCCESS) return failed(e);
+      if (m->actStage && (e = cusync::rt::waitEnd(m->mid, m->sMid, "mlp")) != CUSYNC_SUCCESS) return failed(e);
     }
     if (times_us) times_us[r] = cusync::rt::stampsUs(m->prod, false, m->cons);
     if (!overlapped && gemm1_us) gemm1_us[r] = cusync::rt::stampsUs(m->prod, false, m->prod);

@@ -110,6 +110,17 @@ double stampsUs(const cusync_stage_desc& from, bool fromEnd, const cusync_stage_
   return (double)ticks * 0.01;
 }
 
+cusync_error abandonRun(const hipStream_t* streams, int count, bool* broken, cusync_error e) {
+  for (int i = 0; i < count; i++) if (streams[i]) (void)hipStreamSynchronize(streams[i]);
+  *broken = true;
+  return e;
+}
+
+cusync_error refuseBroken(const char* what) {
+  setError(std::string(what) + ": an earlier run of this handle failed on the device; destroy it and create another");
+  return CUSYNC_ERROR_DEVICE;
+}
+
 }  // namespace rt
 }  // namespace cusync
 

@@ -37,6 +37,13 @@ void noteLaunch(const cusync_stage_desc& stage, bool fillsDevice);
 // 8.3 (6.1 instead of 17.3 for a chain on two streams); the record costs the run nothing, the kernels are under way.
 cusync_error waitEnd(const cusync_stage_desc& s, hipStream_t stream, const char* what);
 double stampsUs(const cusync_stage_desc& from, bool fromEnd, const cusync_stage_desc& to);
+// A handle checks the arguments of all its stages before the first launch of a run, so that a run that is refused has
+// launched nothing.  What fails behind a launch is the device's doing: some stages have then stamped and posted the
+// run's number and others have not, and a later run would find them done before they began.  The handle waits for what
+// it launched (abandonRun: the operands are the caller's again), keeps `broken` and refuses every run from then on
+// (refuseBroken).  The text of the failure stays.
+cusync_error abandonRun(const hipStream_t* streams, int count, bool* broken, cusync_error e);
+cusync_error refuseBroken(const char* what);
 // Adds up the counters of waits that gave up (cusync_stage_desc::spinTimeouts) of the stages given; null
 // entries and stages without a counter are skipped.  Returns false if a copy from the device failed.
 bool spinTimeoutsOf(const cusync_stage_desc* const* stages, int count, uint32_t* sum);

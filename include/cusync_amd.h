@@ -554,7 +554,10 @@ cusync_error cusync_mlp_reload_weights(cusync_mlp *mlp);
  * when the activation is GEMM1's epilogue, see cusync_mlp_config::swiglu_in_gemm2).  If times_us != NULL it receives one elapsed time
  * per run (TB/mlp.cu:691-708 measures it with events): from the moment the first kernel's first workgroup starts to the
  * moment the last kernel's last workgroup has its outputs in memory, by the device's 100 MHz clock.  The call returns
- * when that has happened for the last run; the outputs may be read, and every operand changed or freed, at once. */
+ * when that has happened for the last run; the outputs may be read, and every operand changed or freed, at once.
+ * An argument that one of the stages refuses is found before anything is launched.  After an error of the device behind
+ * the run's first launch the call has waited for what it launched, and the handle refuses further runs.  Both hold for
+ * cusync_conv_chain_run and cusync_attn_layer_run as well. */
 /* Returns CUSYNC_ERROR_DEVICE (text in cusync_rt_last_error) when a wait of one of the chain's stages, the wait
  * kernel's included, gave up after CUSYNC_SPIN_LIMIT polls during the call: the kernel went on with data that
  * had not been posted, so the outputs of the call are not valid.  The same holds for cusync_conv_chain_run and

@@ -63,6 +63,40 @@ def test_outputs_are_there_when_a_run_returns(kind, sync):
     handle.destroy()
 
 
+@pytest.mark.parametrize("sync", [api.SYNC.STREAM, api.SYNC.ROW, api.SYNC.TILE])
+@pytest.mark.parametrize("kind", [(api.MODEL.GPT3, 1, -1, 0), (api.MODEL.GPT3, 40, 0, 0), (api.MODEL.LLAMA, 300, -1, -1), "conv", "attention"])
+def test_a_refused_run_has_launched_nothing(kind, sync):
+    """A last output that is not aligned is found before the stages in front of it are launched: the outputs stay as they
+    were, and the next run counts its stages from where the last whole run left them."""
+    import torch
+    print("run refused", kind, sync, flush=True)
+    torch.cuda.synchronize()
+    handle, run, b, outputs = chain(kind, sync)
+    p = [t.data_ptr() for t in b]
+    if kind == "conv":
+        refused = lambda: handle.run(p[outputs], p[:outputs - 1] + [p[outputs - 1] + 2])
+    elif kind == "attention":
+        refused = lambda: handle.run(p[3], p[2], p[0], p[1] + 2)
+    else:
+        refused = lambda: handle.run(p[2], p[0], p[1] + 2)
+    run()
+    torch.cuda.synchronize()
+    want = [t.clone() for t in b[:outputs]]
+    for _ in range(3):
+        for t in b[:outputs]:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with pytest.raises(api.CuSyncError):
+            refused()
+        torch.cuda.synchronize()
+        assert all(bool(torch.isnan(t).all()) for t in b[:outputs])
+        run()
+        torch.cuda.synchronize()
+        for t, w in zip(b, want):
+            assert torch.equal(t.view(torch.int16), w.view(torch.int16))
+    handle.destroy()
+
+
 def test_split_times_add_up():
     import torch
     torch.cuda.synchronize()
