@@ -128,7 +128,8 @@ const char *cusync_rt_last_error(void);            /* text of the last failed HI
  * kernels, the 3x3 convolution kernel with the input tile in LDS and the attention kernel append one record of eight 64-bit words per finished tile behind a record count in word 0: role and
  * workgroup and XCD, tile, and the 100 MHz clock at five points of the tile (drawn, first loads issued, main loop
  * done, posted, kernel entry).  This is how the per-workgroup timelines in profiles/ were taken.  NULL switches it
- * off again; when off the kernels pay one test per tile.  No counterpart in the reference. */
+ * off again; when off the kernels pay one test per tile.  The records are in memory when a chain handle's run returns;
+ * after a launch that does not synchronise, when its stream has been synchronised.  No counterpart in the reference. */
 cusync_error cusync_rt_set_timeline(void *device_buffer, size_t bytes);
 int cusync_rt_device_count(void);
 int cusync_rt_device_info(int *num_cus, int *clock_khz, size_t *lds_per_cu, size_t *hbm_bytes,

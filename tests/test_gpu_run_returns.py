@@ -63,6 +63,41 @@ def test_outputs_are_there_when_a_run_returns(kind, sync):
     handle.destroy()
 
 
+@pytest.mark.parametrize("sync", [api.SYNC.STREAM, api.SYNC.ROW])
+@pytest.mark.parametrize("kind", [(api.MODEL.GPT3, 1, -1, 0), (api.MODEL.GPT3, 700, -1, 0), "conv", "attention"])
+def test_diagnosis_records_are_there_when_a_run_returns(kind, sync):
+    import torch
+    from cusync_amd import _lib
+    print("records", kind, sync, flush=True)
+    L = _lib.load()
+    torch.cuda.synchronize()
+    handle, run, b, outputs = chain(kind, sync)
+    # (attention: not the third stage, whose 64x128x64 tile is register-staged and keeps no records)
+    tiles = sum(int(np.prod(handle.stage_state(i).grid)) for i in range(outputs))
+    other = torch.cuda.Stream()
+    try:
+        for _ in range(10):
+            buf = torch.zeros(1 + 8 * (tiles + 8), dtype=torch.int64, device="cuda")
+            early = torch.empty_like(buf)
+            torch.cuda.synchronize()
+            assert L.cusync_rt_set_timeline(buf.data_ptr(), buf.numel() * 8) == api.ERR.SUCCESS
+            run()
+            with torch.cuda.stream(other):        # a stream that knows nothing of the chain's
+                early.copy_(buf, non_blocking=True)
+            other.synchronize()
+            L.cusync_rt_set_timeline(None, 0)
+            torch.cuda.synchronize()
+            assert torch.equal(early, buf)
+            r = buf.cpu().numpy()
+            assert r[0] == tiles
+            rec = r[1:1 + 8 * tiles].reshape(-1, 8)
+            assert (rec[:, 2:] > 0).all() and (rec[:, 5] >= rec[:, 2]).all()
+    finally:
+        L.cusync_rt_set_timeline(None, 0)
+    torch.cuda.synchronize()
+    handle.destroy()
+
+
 @pytest.mark.parametrize("sync", [api.SYNC.STREAM, api.SYNC.ROW, api.SYNC.TILE])
 @pytest.mark.parametrize("kind", [(api.MODEL.GPT3, 1, -1, 0), (api.MODEL.GPT3, 40, 0, 0), (api.MODEL.LLAMA, 300, -1, -1), "conv", "attention"])
 def test_a_refused_run_has_launched_nothing(kind, sync):
