@@ -37,30 +37,34 @@ struct ConvTile {
   int residentPerCU;
   void (*chainKernel)(ConvChainParams);     // several layers in one launch; halo tiles only
   void (*splitKernel)(GemmParams);          // the same tile with its steps cut into runs (split_k > 1); halo tiles only
+  uint32_t (*haloLds)(uint32_t W, uint32_t C);      // a launch's LDS for images of width W with C channels; halo tiles only
 };
 
 #define CUSYNC_CONV_TILE(BM, BN, BK, WM, WN, ST, OCC) \
   { BM, BN, BK, kThreads, (size_t)DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>::LDS_BYTES, \
-    gemmDmaKernel<DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>, kAConv>, -1, nullptr, nullptr }
+    gemmDmaKernel<DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>, kAConv>, -1, nullptr, nullptr, nullptr }
+#define CUSYNC_HALO_TILE(CFG) \
+  { CFG::BM, CFG::BN, CFG::BK, CFG::THREADS, 0, convHalo3x3Kernel<CFG>, -1, convHalo3x3ChainKernel<CFG>, convHalo3x3Kernel<CFG, true>, CFG::ldsBytes }
 
 using HaloA = Halo3x3Cfg<256, 64, 4, 1, 4, 2>;     // 64 output channels per tile: four waves of 64 x 64 stacked
 using HaloB = Halo3x3Cfg<128, 128, 2, 2, 3, 2, 2>;    // 128 output channels per tile
 using HaloC = Halo3x3Cfg<64, 128, 2, 2, 3, 2, 2>;     // 64 pixels: what fits beside the halo of 512-channel pixels (7 x 7 images)
+using HaloCPair = Halo3x3Cfg<64, 128, 2, 2, 3, 2>;    // the same tile where two of them fit a CU (convTileFor)
 
-ConvTile g_convTiles[CUSYNC_CONV_TILE_COUNT] = {
+constexpr int kHaloCPair = CUSYNC_CONV_TILE_COUNT;
+ConvTile g_convTiles[CUSYNC_CONV_TILE_COUNT + 1] = {
   CUSYNC_CONV_TILE(128, 64, 32, 2, 2, 4, 3),    // CUSYNC_CONV_TILE_128x64x32
   CUSYNC_CONV_TILE(128, 128, 32, 2, 2, 4, 2),   // CUSYNC_CONV_TILE_128x128x32
   CUSYNC_CONV_TILE(256, 64, 32, 4, 1, 3, 2),    // CUSYNC_CONV_TILE_256x64x32
   // the halo tiles: 3x3 / pad 1 / stride 1 only; LDS size depends on the image width and channels
-  { HaloA::BM, HaloA::BN, HaloA::BK, HaloA::THREADS, 0, convHalo3x3Kernel<HaloA>, -1, convHalo3x3ChainKernel<HaloA>, convHalo3x3Kernel<HaloA, true> },   // CUSYNC_CONV_TILE_HALO_256x64x64
-  { HaloB::BM, HaloB::BN, HaloB::BK, HaloB::THREADS, 0, convHalo3x3Kernel<HaloB>, -1, convHalo3x3ChainKernel<HaloB>, convHalo3x3Kernel<HaloB, true> },   // CUSYNC_CONV_TILE_HALO_128x128x64
-  { HaloC::BM, HaloC::BN, HaloC::BK, HaloC::THREADS, 0, convHalo3x3Kernel<HaloC>, -1, convHalo3x3ChainKernel<HaloC>, convHalo3x3Kernel<HaloC, true> },   // CUSYNC_CONV_TILE_HALO_64x128x64
+  CUSYNC_HALO_TILE(HaloA),      // CUSYNC_CONV_TILE_HALO_256x64x64
+  CUSYNC_HALO_TILE(HaloB),      // CUSYNC_CONV_TILE_HALO_128x128x64
+  CUSYNC_HALO_TILE(HaloC),      // CUSYNC_CONV_TILE_HALO_64x128x64
+  CUSYNC_HALO_TILE(HaloCPair),
 };
 
-bool isHalo(int tile) { return tile >= CUSYNC_CONV_TILE_HALO_256x64x64 && tile <= CUSYNC_CONV_TILE_HALO_64x128x64; }
-uint32_t haloLds(int tile, uint32_t W, uint32_t C) {
-  return tile == CUSYNC_CONV_TILE_HALO_256x64x64 ? HaloA::ldsBytes(W, C) : tile == CUSYNC_CONV_TILE_HALO_128x128x64 ? HaloB::ldsBytes(W, C) : HaloC::ldsBytes(W, C);
-}
+bool isHalo(int tile) { return tile >= 0 && tile < CUSYNC_CONV_TILE_COUNT && g_convTiles[tile].haloLds; }
+uint32_t haloLds(int tile, uint32_t W, uint32_t C) { return g_convTiles[tile].haloLds(W, C); }
 constexpr uint32_t kMaxLds = 160 * 1024 - 1024;      // what one workgroup may ask for (the kernel has 8 bytes of static LDS)
 
 // The halo kernel needs 3x3, pad 1, stride 1, a power-of-two channel count of at least 64, and its tile plus
@@ -76,13 +80,25 @@ ConvTile* convTile(int tile) {
   return &g_convTiles[tile];
 }
 
+// The kernels that images of width W with C channels run with.  The 64x128 tile has one group of four wavefronts where
+// two tiles fit a CU's LDS (64 channels, and 128 up to a width of 28): the other tile's wavefronts then fill the gaps
+// that the second group is there for, and a CU holds one tile of two groups only (with runs its kernel has 217 registers
+// per lane, and the launches of a tile share one count).  One convolution, one group / two groups, in us: 32x28x28x64 to
+// 64 channels 11.6 / 18.9, 32x56x56x64 35.6 / 49.8, 32x28x28x128 to 128 17.2 / 26.0; with fewer tiles than CUs level at
+// 64 channels and 4 to 5 % behind at 128.  (The 128x128 tile at 64 channels, where two fit as well, is level: two groups
+// from 4 % ahead to 4 % behind.)
+ConvTile* convTileFor(int tile, uint32_t W, uint32_t C) {
+  if (tile == CUSYNC_CONV_TILE_HALO_64x128x64 && 2 * (HaloCPair::ldsBytes(W, C) + 1024) <= 160 * 1024) return &g_convTiles[kHaloCPair];
+  return convTile(tile);
+}
+
 int g_convNumCUs = 0;
-uint32_t g_haloLds[CUSYNC_CONV_TILE_COUNT] = {};      // LDS size the cached occupancy of a halo kernel was computed for
+uint32_t g_haloLds[CUSYNC_CONV_TILE_COUNT + 1] = {};      // LDS size the cached occupancy of a halo kernel was computed for
 
 int residentConv(ConvTile* ti, size_t lds) {
   std::lock_guard<std::mutex> lock(g_convMutex);
   const int idx = (int)(ti - g_convTiles);
-  const bool halo = isHalo(idx);
+  const bool halo = ti->haloLds != nullptr;
   if (ti->residentPerCU < 0 || (halo && g_haloLds[idx] != lds)) {
     int dev = 0;
     hipDeviceProp_t prop;
@@ -248,16 +264,16 @@ cusync_error cusync_conv2d_can_implement(const cusync_conv2d_args* a) {
 }
 
 int cusync_conv2d_max_resident(int tile) {
-  ConvTile* ti = convTile(tile);
+  ConvTile* ti = convTileFor(tile, 56, 64);
   if (!ti) return 0;
-  return residentConv(ti, isHalo(tile) ? haloLds(tile, 56, 64) : ti->lds);     // the halo tiles: for 56 x 56 x 64 images
+  return residentConv(ti, ti->haloLds ? ti->haloLds(56, 64) : ti->lds);     // the halo tiles: for 56 x 56 x 64 images
 }
 
 cusync_error cusync_conv2d_run(const cusync_conv2d_args* a, void* stream) {
   cusync_error e = cusync_conv2d_can_implement(a);
   if (e != CUSYNC_SUCCESS) return e;
-  ConvTile* ti = convTile(a->tile);
-  const size_t lds = isHalo(a->tile) ? haloLds(a->tile, a->W, a->C) : ti->lds;
+  ConvTile* ti = convTileFor(a->tile, a->W, a->C);
+  const size_t lds = ti->haloLds ? ti->haloLds(a->W, a->C) : ti->lds;
   const int resident = residentConv(ti, lds);
   if (resident <= 0) { cusync::rt::setError("conv2d: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
   const cusync_stage_desc& s = a->stage;
@@ -349,8 +365,8 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
   c->splitK = 1;
   if (cfg->split_k > 1) c->splitK = cfg->split_k;
   else if (cfg->split_k == 0 && isHalo(c->cfg.tile) && !(c->cfg.fused && cfg->sync != CUSYNC_SYNC_STREAM)) {
-    ConvTile* ti = convTile(c->cfg.tile);
-    const int resident = residentConv(ti, haloLds(c->cfg.tile, cfg->W, cfg->C));
+    ConvTile* ti = convTileFor(c->cfg.tile, cfg->W, cfg->C);
+    const int resident = residentConv(ti, ti->haloLds(cfg->W, cfg->C));
     const uint32_t tiles = g.x * g.y, steps = 9 * (cfg->C / 64);
     uint32_t s = resident > 0 && tiles * 2 <= (uint32_t)g_convNumCUs ? std::min<uint32_t>((uint32_t)resident / tiles, steps / 9) : 1u;
     if (tm >= 128) s = s >= 4 ? 4 : s == 3 ? 2 : s;      // a 128-row tile's four pieces divide among two or four runs
@@ -469,8 +485,8 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
   auto failed = [&](cusync_error why) { return cusync::rt::abandonRun(c->stream.data(), (int)c->stream.size(), &c->broken, why); };
   if (overlapped && c->cfg.fused) {
     // all layers in one launch on the first stream
-    ConvTile* ti = convTile(c->cfg.tile);
-    const size_t lds = haloLds(c->cfg.tile, c->cfg.W, c->cfg.C);
+    ConvTile* ti = convTileFor(c->cfg.tile, c->cfg.W, c->cfg.C);
+    const size_t lds = ti->haloLds(c->cfg.W, c->cfg.C);
     const int resident = residentConv(ti, lds);
     if (resident <= 0) { cusync::rt::setError("conv chain: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
     const cusync_dim3& g = c->st[0].grid;

@@ -122,6 +122,24 @@ def test_two_groups_of_wavefronts_share_a_tile(tile, geom, split_k):
     assert np.array_equal(got.view(np.uint16), orc.conv2d_nhwc(x, w).view(np.uint16))
 
 
+def test_two_64_row_tiles_share_a_cu():
+    # 64 channels: two tiles fit a CU's LDS, and one group of wavefronts per tile leaves registers for both
+    assert _lib.load().cusync_conv2d_max_resident(api.CONV_TILE.HALO_64x128x64) == 2 * api.device_info()["cus"]
+
+
+# widths on both sides of the line up to which two 64-row tiles of 128 channels fit a CU, and 64 channels
+@pytest.mark.parametrize("geom", [(2, 9, 28, 128, 136), (2, 9, 29, 128, 136), (9, 28, 28, 64, 264)])
+@pytest.mark.parametrize("split_k", [1, 2, 5])
+def test_groups_per_64_row_tile(geom, split_k):
+    """Integers: exact sums (at most 9 * 128 * 4 < 2^24), rounded to halfs by the oracle as by the kernel."""
+    print("conv pair of tiles", geom, split_k, flush=True)
+    N, H, W, Cc, K = geom
+    rng = np.random.default_rng(W + K)
+    x, w = rng.integers(-2, 3, (N, H, W, Cc)).astype(np.float16), rng.integers(-2, 3, (K, 3, 3, Cc)).astype(np.float16)
+    got = run_conv(x, w, api.CONV_TILE.HALO_64x128x64, launches=2, split_k=split_k)
+    assert np.array_equal(got.view(np.uint16), orc.conv2d_nhwc(x, w).view(np.uint16))
+
+
 HALO_TILES = [api.CONV_TILE.HALO_256x64x64, api.CONV_TILE.HALO_128x128x64, api.CONV_TILE.HALO_64x128x64]
 
 
