@@ -68,8 +68,6 @@ enum { kAPlain = 0, kAConv = 1 };
 // [1] tile x | y << 16 | z << 32 | tiles this workgroup did before << 48
 // [2..6] constant-rate 100 MHz clock: tile drawn, first loads issued (the waits of the first chunks are over),
 //        main loop done, epilogue and post done, and the clock at kernel entry of this workgroup;  [7] launched
-// Written through to memory like the outputs: a chain handle's run returns on the stage's end stamp, before the kernel's
-// end writes this XCD's L2 back, and the caller reads the records then.
 __device__ __forceinline__ void recordTileAt(unsigned long long* timeline, uint32_t timelineCap, const cusync::DynStage& stage,
                                              uint32_t launched, const cusync_dim3& t, uint32_t round,
                                              unsigned long long tEntry, unsigned long long t0, unsigned long long t1,
@@ -80,12 +78,9 @@ __device__ __forceinline__ void recordTileAt(unsigned long long* timeline, uint3
   unsigned long long* r = timeline + 1 + slot * 8;
   const uint32_t role = (stage.isProducer() ? 1u : 0u) | (stage.isConsumer() ? 2u : 0u);
   const uint32_t xcc = __builtin_amdgcn_s_getreg((3 << 11) | 20);       // HW_REG_XCC_ID, bits 0..3
-  const unsigned long long v[8] = {
-    role | ((unsigned long long)cusync::DynStage::workgroupIndex() << 8) | ((unsigned long long)xcc << 40),
-    t.x | ((unsigned long long)t.y << 16) | ((unsigned long long)t.z << 32) | ((unsigned long long)round << 48),
-    t0, t1, t2, t3, tEntry, launched};
-#pragma unroll
-  for (int i = 0; i < 8; i++) __hip_atomic_store(r + i, v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  r[0] = role | ((unsigned long long)cusync::DynStage::workgroupIndex() << 8) | ((unsigned long long)xcc << 40);
+  r[1] = t.x | ((unsigned long long)t.y << 16) | ((unsigned long long)t.z << 32) | ((unsigned long long)round << 48);
+  r[2] = t0; r[3] = t1; r[4] = t2; r[5] = t3; r[6] = tEntry; r[7] = launched;
 }
 __device__ __forceinline__ void recordTile(const GemmParams& p, const cusync_dim3& t, uint32_t round,
                                            unsigned long long tEntry, unsigned long long t0, unsigned long long t1,

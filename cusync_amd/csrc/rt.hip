@@ -90,7 +90,14 @@ cusync_error waitEnd(const cusync_stage_desc& s, hipStream_t stream, const char*
   const unsigned long long want = (uint32_t)s.iter & 0xffffu;
   auto looked = std::chrono::steady_clock::now();
   for (uint32_t spins = 1;; spins++) {
-    if ((stampOf(s, 1) & 0xffffu) == want) return CUSYNC_SUCCESS;
+    if ((stampOf(s, 1) & 0xffffu) == want) {
+      // Diagnosis records are plain stores: in memory when the kernel's end has written the XCDs' L2 back, not yet when
+      // the stamp is.  (Written through where they are made, or written back in front of the stamp, they change the
+      // code around them also where they are off: the 128x128 convolution tile 27.2 -> 28.0 us at 8x14x14x256, the
+      // 64x128 tile 33.2 -> 34.3 at 32x7x7x512.)
+      if (g_timeline && check(hipStreamSynchronize(stream), "hipStreamSynchronize", __FILE__, __LINE__)) return CUSYNC_ERROR_DEVICE;
+      return CUSYNC_SUCCESS;
+    }
     __builtin_ia32_pause();      // the stamp arrives over the bus
     if (spins % 1024 == 0 && std::chrono::steady_clock::now() - looked > std::chrono::milliseconds(2)) {
       // A launch that failed on the device leaves no stamp: what does its stream say?

@@ -162,8 +162,7 @@ struct DynStage {
     if ((d.flags & CUSYNC_STAGE_STAMPS_START) && workgroupIndex() == 0) stamp(0);
   }
   // When a workgroup has no tile left, called by all its threads.  Every wavefront has its stores acknowledged, the
-  // barrier collects the wavefronts, and the count (relaxed: the stores, of outputs and of the diagnosis records, went
-  // through to memory) tells the last workgroup.
+  // barrier collects the wavefronts, and the count (relaxed: the stores went through to memory) tells the last workgroup.
   __device__ __forceinline__ void leave(uint32_t launched) const {
     if (!(d.flags & CUSYNC_STAGE_STAMPS_END)) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
