@@ -21,7 +21,8 @@
 // stored at chunk ^ (pixel & (C/8 - 1)); where a pixel is 128 bytes (C = 64), and in the filter's 128-byte rows, two
 // neighbours cover all banks once and take one position: chunk ^ (pixel/2 & 7).  (With neighbours in different
 // positions, rows r and r + 8 share their banks: pairs under RowSync 38.7 -> 37.6 us at 32x28x28x128, 51.5 -> 49.8 at
-// 32x7x7x512, level at the other stages.)
+// 32x7x7x512, level at the other stages.  The 256x64 tile at 128 channels, which the chain takes only when told to, pays
+// 2 to 4 % for the shift by nothing: one convolution 62.9 -> 65.6 us at 32x56x56x128.)
 //
 // Every wavefront (of a group) owns a 64 x 64 piece of the tile (two by two MFMA tiles), 32 x 64 of the 64-pixel tile: with
 // 64 x 32 the kernel spent its time on LDS reads, three 16-byte reads per two
