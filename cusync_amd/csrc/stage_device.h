@@ -26,8 +26,10 @@ struct DynStage {
   // True when every producer tile starts and ends on a 128-byte line of the
   // buffer the consumer reads (set by the launcher).  Then a line of that buffer
   // can only enter this XCD's caches after the semaphore guarding it was seen,
-  // because the kernel began with clean caches and never touches a tile before
-  // its wait; the wait can skip the cache invalidation that would also throw
+  // because the kernel began with clean caches and never touches a line that
+  // holds part of a producer's tile before its wait (cached rows in front of the
+  // producer's, which the attention kernels read before it, are lines of their
+  // own then); the wait can skip the cache invalidation that would also throw
   // away the weights the XCD's workgroups share.
   bool lineAligned;
   // allStatic(launched) of the launch this object goes to, worked out by the launcher (set by prepare()): in the

@@ -1,10 +1,14 @@
 """The attention kernel of up to 32 query rows with a split key range, at the edges of its range."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle as orc
+import test_gpu_attention as attention
+from cusync_amd import _lib, api
 from test_gpu_attention import run_attention_split
-from util import assert_close, normal_f16
+from util import assert_close, empty_dev, normal_f16, to_dev, to_host, uniform_f16
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +48,56 @@ def test_masked_keys_weigh_nothing(S, cached, heads, blocks, scale):
     got, grid = run_attention_split(qkv, cached, heads, True, blocks, scale=scale)
     assert grid[2] > 1
     assert_close(got, reference(qkv, cached, heads, scale), "O")
+
+
+# as the second stage of the chain under every policy, with a piece that holds cached and new rows
+@pytest.mark.parametrize("S,cached", [(7, 130), (17, 300), (32, 2031)])
+def test_few_rows_in_the_layer(S, cached):
+    attention.test_attention_layer_with_cache(S, cached)
+
+
+@pytest.mark.parametrize("sync", ["row", "tile", "consecutive"])
+@pytest.mark.parametrize("S,cached,blocks,more", [(17, 300, 1, 0), (17, 300, 1, 8), (32, 2031, 6, 8), (1, 130, 1, 8)])
+def test_few_rows_behind_a_projection(S, cached, blocks, more, sync):
+    """A consumer that reads the cached rows before it waits.  With a row pitch or a base that is not whole 128-byte lines
+    (`more` halfs) the last cached row shares a line with the first new one, which the wait then has to invalidate."""
+    import torch
+    print("attention few consumer", S, cached, blocks, more, sync, flush=True)
+    L = _lib.load()
+    hidden, heads, tile = 4096, 3, api.TILE.D32x128x64
+    E, ld = heads * 128, 3 * heads * 128 + more
+    w = normal_f16((hidden, 3 * E), 41)
+    xs = [uniform_f16((S, hidden), 42 + r) for r in range(3)]
+    cache = normal_f16((cached, 3 * E), 40, std=1.0)
+    flat = torch.full((more + (cached + S) * ld,), float("nan"), dtype=torch.float16, device="cuda")
+    qkv = flat[more:].view(cached + S, ld)
+    qkv[:cached, :3 * E] = to_dev(cache)
+    o, dw, dxs = empty_dev((S, E)), to_dev(w), [to_dev(x) for x in xs]
+    tm, tn, _ = api.tile_shape(tile)
+    grid = api.gemm_grid(tile, S, 3 * E)
+    pol = {"row": api.row_sync(tm, grid[0]), "tile": api.tile_sync(api.ORDER.TRANSPOSE_XY, tm, tn),
+           "consecutive": api.consecutive_sync(api.ORDER.TRANSPOSE_XY, 8 * E, tm, tn)}[sync]
+    prod = api.Stage(grid, (1, 1, 1), api.no_sync(), pol)
+    cons = api.Stage(api.attention_grid(S, heads, cached, blocks), (1, 1, 1), pol, api.no_sync())
+    assert cons.grid()[2] > 1 and api.set_producer_consumer_pair(prod, cons) == api.ERR.SUCCESS
+    ws = torch.zeros(api.attention_workspace_size(S, heads, cached, blocks), dtype=torch.uint8, device="cuda")
+    s0, s1 = torch.cuda.Stream(), torch.cuda.Stream()
+    for x, dx in zip(xs, dxs):
+        qkv[cached:] = float("nan")
+        o.fill_(float("nan"))
+        torch.cuda.synchronize()
+        assert api.gemm(prod, S, 3 * E, hidden, dx.data_ptr(), hidden, dw.data_ptr(), 3 * E, qkv[cached:].data_ptr(), ld, tile,
+                        stream=s0.cuda_stream) == api.ERR.SUCCESS, api.last_error()
+        assert L.cusync_hold_back(C.byref(prod.desc), s1.cuda_stream) == api.ERR.SUCCESS, api.last_error()
+        assert api.attention(cons, S, heads, qkv.data_ptr(), ld, o.data_ptr(), E, cached_rows=cached, kv_split_blocks=blocks,
+                             workspace=ws.data_ptr(), stream=s1.cuda_stream) == api.ERR.SUCCESS, api.last_error()
+        torch.cuda.synchronize()
+        prod.incrementIter()
+        cons.incrementIter()
+        full = np.ascontiguousarray(to_host(qkv)[:, :3 * E])
+        assert np.array_equal(full[:cached].view(np.uint16), cache.view(np.uint16))
+        assert_close(full[cached:], orc.gemm(x, w), "new rows")
+        assert_close(to_host(o), orc.attention_kv(full, cached, heads, 128, True), "O")
+    assert prod.read_state().spin_timeouts == 0 and cons.read_state().spin_timeouts == 0
+    prod.destroy()
+    cons.destroy()

@@ -19,8 +19,8 @@ def chain(kind, sync):
         ys = [empty_dev((N, H, H, C)) for _ in ws]
         h = api.ConvChain(N, H, H, C, [w.data_ptr() for w in ws], sync)
         return h, lambda: h.run(x.data_ptr(), [y.data_ptr() for y in ys]), ys + [x] + ws, len(ys)
-    if kind == "attention":
-        S, cached, hidden, heads = 40, 300, 1024, 3
+    if kind in ("attention", "attention of few rows"):
+        S, cached, hidden, heads = 40 if kind == "attention" else 17, 300, 1024, 3
         E = heads * 128
         x, wqkv, wo = to_dev(uniform_f16((S, hidden), 1)), to_dev(normal_f16((hidden, 3 * E), 2)), to_dev(normal_f16((E, hidden), 3))
         qkv, o, y = to_dev(normal_f16((cached + S, 3 * E), 4, std=1.0)), empty_dev((S, E)), empty_dev((S, hidden))
@@ -37,7 +37,8 @@ def chain(kind, sync):
 
 @pytest.mark.parametrize("sync", [api.SYNC.STREAM, api.SYNC.ROW, api.SYNC.TILE])
 @pytest.mark.parametrize("kind", [(api.MODEL.GPT3, 1, -1, 0), (api.MODEL.GPT3, 40, 0, 0), (api.MODEL.GPT3, 700, -1, 0), (api.MODEL.LLAMA, 300, -1, 0),
-                                  (api.MODEL.LLAMA, 300, -1, -1), (api.MODEL.LLAMA, 300, -1, 1), "conv", "attention"])
+                                  (api.MODEL.LLAMA, 300, -1, -1), (api.MODEL.LLAMA, 300, -1, 1), "conv", "attention",
+                                  "attention of few rows"])
 def test_outputs_are_there_when_a_run_returns(kind, sync):
     import torch
     print("run returns", kind, sync, flush=True)
