@@ -440,10 +440,10 @@ def main():
                 "default_launches": {k: 1 if v else 2 for k, v in default_one.items()},
                 "rowsync_default_us": round(m["rowsync_one_launch" if default_one["rowsync"] and "rowsync_one_launch" in m else "rowsync"][0], 2),
                 "tilesync_default_us": round(m["tilesync_one_launch" if default_one["tilesync"] and "tilesync_one_launch" in m else "tilesync"][0], 2),
-                # medians of 60 steps in the driver's process: the launcher objects' loop by its events, and the handle beside
-                # it by the device's clock, which leaves out the 4 to 6 us that lie between the events and the kernels
+                # medians of 60 steps in the driver's process: the launcher objects' loop by its own events, and the loop
+                # against the handle beside it, both by the host's clock from the first call to the step's end
                 "launcher_rowsync_us": launcher[(b, "rowsync")]["launcher_us"], "launcher_tilesync_us": launcher[(b, "tilesync")]["launcher_us"],
-                "launcher_vs_handle_pct": {k: round(launcher[(b, k)]["launcher_us"] / launcher[(b, k)]["handle_us"] * 100 - 100, 2)
+                "launcher_vs_handle_pct": {k: round(launcher[(b, k)]["launcher_host_us"] / launcher[(b, k)]["handle_host_us"] * 100 - 100, 2)
                                            for k in ("rowsync", "tilesync")},
                 "best_policy": min(in_place, key=lambda k: m[k][0]),
                 "best_gain_pct": round(100 - best / s_us * 100, 2),

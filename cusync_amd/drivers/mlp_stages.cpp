@@ -20,11 +20,16 @@
 //
 // Output per batch size and policy: START-OVERLAPPED: / one {"Total": us} per timed run / END-OVERLAPPED: as the
 // reference prints them (mlp.cu:707, 1079-1084), then one summary object
-//   {"batch", "sync", "tile1", "tile2", "split_k1", "split_k2", "launcher_us", "handle_us", "runs", "above_1p05"}
+//   {"batch", "sync", "tile1", "tile2", "split_k1", "split_k2", "launcher_us", "handle_us", "launcher_host_us",
+//    "handle_host_us", "runs", "above_1p05"}
 // (medians over all timed runs; handle_us: the cusync_mlp_* handle on the same buffers, its rounds of --runs runs
-// alternating with the launchers' so that both see the same clocks; above_1p05: launcher runs slower than 1.05 x
-// their median).
+// alternating with the launchers' so that both see the same clocks.  launcher_us is the loop's own measure, events around
+// the two launches; handle_us the handle's, the device's clock from the first workgroup's start to the last one's end,
+// some 4 to 6 us less for the same kernels.  The host's clock measures both alike: launcher_host_us from the loop's
+// first call to its event wait's return, handle_host_us a call of cusync_mlp_run.  above_1p05: launcher runs slower than
+// 1.05 x their median).
 #include <algorithm>
+#include <chrono>
 #include <type_traits>
 
 #include "cusync/cusync.h"
@@ -53,6 +58,8 @@ void writeHalfs(const std::string& path, const std::vector<uint16_t>& v) {
   if (!f || fwrite(v.data(), 2, v.size(), f) != v.size()) { fprintf(stderr, "cannot write %s\n", path.c_str()); exit(EXIT_FAILURE); }
   fclose(f);
 }
+
+double nowUs() { return std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
 
 double median(std::vector<double> v) {
   if (v.empty()) return 0;
@@ -93,14 +100,16 @@ struct CuSyncGPT3 {
     RT_CHECK(cusync_rt_event_create(&end));
   }
 
-  void run(void* producer_stream, void* consumer_stream, int iters, std::vector<double>* times) {
+  void run(void* producer_stream, void* consumer_stream, int iters, std::vector<double>* times, std::vector<double>* host) {
     for (int r = 0; r < iters; r++) {
+      const double t0 = nowUs();
       RT_CHECK(cusync_rt_event_record(start, producer_stream));
       STATUS_CHECK(gemm_op1.run(true, NULL, producer_stream));
       prod.invokeWaitKernel(consumer_stream);
       STATUS_CHECK(gemm_op2.run(true, NULL, consumer_stream));
       RT_CHECK(cusync_rt_event_record(end, consumer_stream));
       RT_CHECK(cusync_rt_event_sync(end));
+      if (host) host->push_back(nowUs() - t0);
       double us = 0;
       RT_CHECK(cusync_rt_event_elapsed_us(start, end, &us));
       if (times) times->push_back(us);
@@ -125,7 +134,7 @@ struct Request {
   int split_k1, split_k2, runs, rounds, warmup;
   bool withHandle;
 };
-struct Result { std::vector<double> launcher, handle; };
+struct Result { std::vector<double> launcher, handle, launcherHost, handleHost; };
 
 // The set-up of mlp.cu:1020-1062 for one pair of tile shapes and one policy.
 template<int Tile1, int Tile2, bool Row>
@@ -168,14 +177,16 @@ Result runPair(MLPParameters& mlpParams, const Request& rq) {
       if (!handle) { fprintf(stderr, "cusync_mlp_create failed: %s\n", cusync_rt_last_error()); exit(EXIT_FAILURE); }
       DRV_CHECK(cusync_mlp_run(handle, mlpParams.x, mlpParams.xw1, mlpParams.xw12, rq.warmup, nullptr));
     }
-    chain.run(producer_stream, consumer_stream, rq.warmup, nullptr);
-    std::vector<double> t(rq.runs);
+    chain.run(producer_stream, consumer_stream, rq.warmup, nullptr, nullptr);
     for (int round = 0; round < rq.rounds; round++) {
-      if (handle) {
-        DRV_CHECK(cusync_mlp_run(handle, mlpParams.x, mlpParams.xw1, mlpParams.xw12, rq.runs, t.data()));
-        out.handle.insert(out.handle.end(), t.begin(), t.end());
+      for (int i = 0; handle && i < rq.runs; i++) {
+        double us = 0;
+        const double t0 = nowUs();
+        DRV_CHECK(cusync_mlp_run(handle, mlpParams.x, mlpParams.xw1, mlpParams.xw12, 1, &us));
+        out.handleHost.push_back(nowUs() - t0);
+        out.handle.push_back(us);
       }
-      chain.run(producer_stream, consumer_stream, rq.runs, &out.launcher);       // last: what --check reads is the launchers' output
+      chain.run(producer_stream, consumer_stream, rq.runs, &out.launcher, &out.launcherHost);       // last: what --check reads is the launchers' output
     }
     if (handle) cusync_mlp_destroy(handle);
   }
@@ -290,8 +301,10 @@ int main(int argc, char** argv) {
       int above = 0;
       for (double t : res.launcher) above += t > 1.05 * med;
       printf("{\"batch\": %d, \"sync\": \"%s\", \"tile1\": %d, \"tile2\": %d, \"split_k1\": %d, \"split_k2\": %d, \"launcher_us\": %.2f, "
-             "\"handle_us\": %s, \"runs\": %zu, \"above_1p05\": %d}\n", batch, row ? "rowsync" : "tilesync", tile1, tile2, rq.split_k1, rq.split_k2,
-             med, res.handle.empty() ? "null" : std::to_string(median(res.handle)).c_str(), res.launcher.size(), above);
+             "\"handle_us\": %s, \"launcher_host_us\": %.2f, \"handle_host_us\": %s, \"runs\": %zu, \"above_1p05\": %d}\n",
+             batch, row ? "rowsync" : "tilesync", tile1, tile2, rq.split_k1, rq.split_k2, med,
+             res.handle.empty() ? "null" : std::to_string(median(res.handle)).c_str(), median(res.launcherHost),
+             res.handle.empty() ? "null" : std::to_string(median(res.handleHost)).c_str(), res.launcher.size(), above);
       fflush(stdout);
 
       if (!dump.empty()) {

@@ -102,6 +102,7 @@ def test_mlp_stages_driver_against_oracle(tmp_path):
     assert [(r["batch"], r["sync"]) for r in rows] == [(256, "rowsync"), (256, "tilesync"), (2048, "rowsync"), (2048, "tilesync")]
     for r in rows:
         assert r["runs"] == 5 and r["launcher_us"] > 0 and r["handle_us"] > 0
+        assert r["launcher_host_us"] > r["launcher_us"] and r["handle_host_us"] > r["handle_us"]      # the host's clock holds the whole step
     for b in batches:
         got = {}
         for sync in ("rowsync", "tilesync"):
