@@ -277,7 +277,12 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   // times are alike, so the blocks are cut into about as many splits as a split has blocks, within one workgroup per
   // CU.  With several row tiles not below eight blocks (the chain under RowSync in us, half the range -> this: 16 rows
   // behind 2048 66.5 -> 60.6, behind 8192 94.9 -> 67.5; 64 behind 2048 85.8 -> 75.4; 128 behind 8192 164.5 -> 107.2;
-  // 256 behind 4096 132 -> 109; 512 behind 2048 143 -> 135; 1 behind 512 57.1 -> 56.4).
+  // 256 behind 4096 132 -> 109; 512 behind 2048 143 -> 135; 1 behind 512 57.1 -> 56.4).  Where the row tiles of all heads
+  // leave no CU for a second split (12 heads: from 1281 rows on) the range stays whole, which is ahead of two halves
+  // where the stages overlap and the cache is not much longer than the rows, and behind them in stream order at 12 heads
+  // (a pass, whole / two halves: under RowSync 2048 rows behind 64 352 / 364, behind 2048 384 / 409, behind 8192
+  // 502 / 526, 1408 behind 8192 418 / 408; in stream order 2048 behind 64 367 / 343, behind 2048 406 / 392, 1408 behind
+  // 2048 328 / 299; 64 heads, 512 rows behind 64: 194 / 217 and 203 / 210).
   const uint32_t kvBlocks = (cfg->cached_rows + cfg->seq + kBKV - 1) / kBKV;
   uint32_t perSplit = kvBlocks >= 8 ? (kvBlocks + 1) / 2 : 0u;
   if (cfg->cached_rows) {

@@ -335,8 +335,9 @@ bool choose(const cusync_mlp_config& given, Choice* o) {
   // 1-5 us of 67-83; 512 to 1024 rows: 1-3 us of 172-284; behind at 256 rows and from 1025 on, and at every size of
   // the LLaMA shard, whose GEMM2 wants a tile of its own, but for StridedSync up to 32 rows, where both take 32x128) and
   // the tiles are the table's.  LLaMA under StridedSync, by the device's clock in us, two launches -> one, inner 2752 /
-  // 2816: 1 row 37.3 -> 34.7 / 39.2 -> 36.1, 16 rows 38.3 -> 35.3 / 40.2 -> 37.0, 32 rows 39.2 -> 36.4 / 41.6 -> 38.3
-  // (a third of that under RowSync, which keeps its two launches).
+  // 2816: 1 row 37.3 -> 34.7 / 39.2 -> 36.1, 16 rows 38.3 -> 35.3 / 40.2 -> 37.0, 32 rows 39.2 -> 36.4 / 41.6 -> 38.3.
+  // The other two policies keep their two launches, though one is ahead of them as well: 16 rows, inner 2752, TileSync
+  // 39.5 -> 36.2 (a pass by the host's clock 47.7 -> 45.4), RowSync 39.3 -> 37.1 (47.2 -> 46.3).
   const bool automatic = c.one_launch < 0;
   if (automatic) c.one_launch = c.sync != CUSYNC_SYNC_STREAM && c.tile1 < 0 && c.tile2 < 0 &&
                                 (llama ? c.sync == CUSYNC_SYNC_STRIDED && c.batch <= 32 : c.batch <= 64 || (c.batch >= 512 && c.batch <= 1024));
