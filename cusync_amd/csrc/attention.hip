@@ -53,6 +53,15 @@ bool deepPipeline(const cusync_attention_args* a) {
   return g_attnNumCUs > 0 && a->stage.grid.x * a->stage.grid.y * a->stage.grid.z > (uint32_t)g_attnNumCUs;
 }
 
+// The few-row form holds as much LDS as the deep one.  Under AvoidWaitKernel, whose caller has seen to it that all stages
+// fit on the device at once (cusync_attention_max_resident counts the shallow form), and whose consumer may reach the
+// device first and leave the attention no CU of its own, it runs only where the deep form would have.
+Form chooseForm(const cusync_attention_args* a) {
+  const bool deep = deepPipeline(a);
+  if (a->seq <= (uint32_t)kFewRows && a->stage.grid.z > 1 && (deep || !(a->stage.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL))) return kFew;
+  return deep ? kDeep : kShallow;
+}
+
 int residentAttention(Form form) {
   std::lock_guard<std::mutex> lock(g_attnMutex);
   int& perCU = g_attnResidentPerCU[form];
@@ -182,7 +191,7 @@ int cusync_attention_max_resident(void) { return residentAttention(kShallow); }
 cusync_error cusync_attention_run(const cusync_attention_args* a, void* stream) {
   cusync_error e = cusync_attention_can_implement(a);
   if (e != CUSYNC_SUCCESS) return e;
-  const Form form = a->seq <= (uint32_t)kFewRows && a->stage.grid.z > 1 ? kFew : deepPipeline(a) ? kDeep : kShallow;
+  const Form form = chooseForm(a);
   const int resident = residentAttention(form);
   if (resident <= 0) { setError("attention: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
   const cusync_stage_desc& s = a->stage;

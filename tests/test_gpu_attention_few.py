@@ -28,6 +28,31 @@ def test_few_rows_split_key_range(S, cached, heads, blocks, causal):
     assert np.array_equal(got.view(np.uint16), one.view(np.uint16))       # the result does not depend on arrival order
 
 
+def test_few_rows_of_a_stage_that_may_start_last():
+    """Under AvoidWaitKernel a stage that is no larger than its caller counted on: bit for bit the kernel of more rows, whose
+    last 17 of 33 these are."""
+    import torch
+    print("attention few AvoidWaitKernel", flush=True)
+    heads, total, blocks = 3, 317, 1
+    qkv = normal_f16((total, 3 * heads * 128), 35, std=1.0)
+    dq, outs = to_dev(qkv), {}
+    # a stage that posts (to nobody), so that it is not alone on its stream
+    post = api.tile_sync(api.ORDER.TRANSPOSE_XY, 128, 128)
+    for S, opts in ((17, api.OPT.AVOID_WAIT_KERNEL), (33, 0), (17, 0)):
+        cached = total - S
+        o = empty_dev((S, heads * 128), fill=float("nan"))
+        ws = torch.zeros(api.attention_workspace_size(S, heads, cached, blocks), dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        st = api.Stage(api.attention_grid(S, heads, cached, blocks), (1, 1, 1), api.no_sync(), post, opts=opts)
+        assert api.attention(st, S, heads, dq.data_ptr(), 3 * heads * 128, o.data_ptr(), heads * 128, cached_rows=cached,
+                             kv_split_blocks=blocks, workspace=ws.data_ptr()) == api.ERR.SUCCESS, api.last_error()
+        torch.cuda.synchronize()
+        st.destroy()
+        outs[S, opts] = to_host(o)
+        assert_close(outs[S, opts], orc.attention_kv(qkv, cached, heads, 128, True), "O")
+    assert np.array_equal(outs[17, api.OPT.AVOID_WAIT_KERNEL].view(np.uint16), outs[33, 0][16:].view(np.uint16))
+
+
 def reference(qkv, cached, heads, scale):
     """Causal attention in float64, the result rounded to halfs."""
     q, k, v = (qkv[:, i * heads * 128:(i + 1) * heads * 128].reshape(-1, heads, 128).transpose(1, 0, 2).astype(np.float64) for i in range(3))
