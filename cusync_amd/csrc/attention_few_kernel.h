@@ -28,6 +28,7 @@ constexpr int kPieceKeys = 32, kPieceBytes = 2 * kPieceKeys * kRowBytes, kPieceL
 constexpr int kFewLdsBytes = 4 * 2 * kPieceBytes;
 
 __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) {
+  constexpr uint32_t from = 0;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   __shared__ uint32_t sTicket, sLast;
   __shared__ float sStat[2][4][64];
@@ -70,15 +71,17 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
 
   uint32_t dryXcds = 0, nextRaw = 0;
   const unsigned long long tlEntry = p.timeline ? wall_clock64() : 0;
-  if (tid == 0) stage.enter();
+  const unsigned long long entered = stage.enter();
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   const bool noDraws = stage.noDraws;
   for (uint32_t round = 0;; round++) {
+    const AttnParams p = cusync::argumentsHere<AttnParams>(from);
+    const cusync::DynStage& stage = p.stage;
     if (tid == 0) sTicket = round == 0 ? stage.firstTicket(p.launched, dryXcds, noDraws) : stage.drawFinish(nextRaw, p.launched, round, dryXcds, noDraws);
     __syncthreads();
     const uint32_t ticket = sTicket;
     if (ticket >= numTiles) {
-      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
       break;
     }
     const cusync_dim3 t = stage.ticketToTile(ticket);
@@ -111,7 +114,7 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
     };
     issue(first, 0);
     issue(first + 4, 1);
-    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
     if (consumer) waitRows(head * kHD);
     half8 qf[8];
 #pragma unroll
@@ -193,7 +196,8 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
     }
     waitVmcnt<0>();
     const unsigned long long tl2 = p.timeline ? wall_clock64() : 0;
-    if (tid == 0) nextRaw = stage.drawBegin(dryXcds, noDraws);
+    const AttnParams e = cusync::argumentsHere<AttnParams>(from);
+    if (tid == 0) nextRaw = e.stage.drawBegin(dryXcds, noDraws);
     rowSum += __shfl_xor(rowSum, 32);
 
     // Four running results into one: wavefront w's [tt][g][lane] values behind one another, 16 KB each.
@@ -204,7 +208,7 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
       for (int g = 0; g < 4; g++)
         *reinterpret_cast<floatx4*>(smem + ((wave * 16 + tt * 4 + g) * 64 + lane) * 16) =
             floatx4{o[tt][4 * g], o[tt][4 * g + 1], o[tt][4 * g + 2], o[tt][4 * g + 3]};
-    sStat[0][wave][lane] = rowMax * p.scaleLog2;       // (scaled: a wavefront without keys keeps a value far below any score)
+    sStat[0][wave][lane] = rowMax * e.scaleLog2;       // (scaled: a wavefront without keys keeps a value far below any score)
     sStat[1][wave][lane] = rowSum;
     __syncthreads();
     float m = sStat[0][0][lane], sum = 0.0f;
@@ -224,11 +228,11 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
     bool completed = true;
     if (splits > 1) {
       // this split's share into the workspace, written through (see attentionKernel); the last to arrive adds them up
-      const size_t slot = (size_t)head * stage.d.grid.z;
-      const __amdgpu_buffer_rsrc_t rPart = makeRsrc(p.partO, p.partBytes);
+      const size_t slot = (size_t)head * e.stage.d.grid.z;
+      const __amdgpu_buffer_rsrc_t rPart = makeRsrc(e.partO, e.partBytes);
       auto offO = [&](uint32_t z, int g) { return (uint32_t)(((slot + z) * (64 * kThreads) + (g * kThreads + tid) * 4) * sizeof(float)); };
       auto offS = [&](uint32_t z, int which) {
-        return (uint32_t)(((char*)p.partStat - (char*)p.partO) + ((slot + z) * (2 * kThreads) + which * kThreads + lane) * sizeof(float));
+        return (uint32_t)(((char*)e.partStat - (char*)e.partO) + ((slot + z) * (2 * kThreads) + which * kThreads + lane) * sizeof(float));
       };
 #pragma unroll
       for (int g = 0; g < 4; g++)
@@ -239,10 +243,10 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
       }
       waitVmcnt<0>();
       __syncthreads();
-      uint32_t* counter = p.arrivals + head;
+      uint32_t* counter = e.arrivals + head;
       if (tid == 0) {
-        const bool last = stage.countIn(counter) == splits - 1;
-        if (last) { cusync::dev::storeRelaxed(counter, 0); stage.countSeen(); }
+        const bool last = e.stage.countIn(counter) == splits - 1;
+        if (last) { cusync::dev::storeRelaxed(counter, 0); e.stage.countSeen(); }
         sLast = last;
       }
       __syncthreads();
@@ -287,24 +291,25 @@ __global__ __launch_bounds__(kThreads, 1) void attentionFewKernel(AttnParams p) 
         }
       }
     }
-    if (completed && myq < p.S) {
+    if (completed && myq < e.S) {
       const float inv = 1.0f / sum;
-      const __amdgpu_buffer_rsrc_t rOut = makeRsrc(p.out, p.S * p.ldo * 2);
-      const uint32_t dst = (myq * p.ldo + head * kHD + 32 * wave + 4 * hi) * 2;
+      const __amdgpu_buffer_rsrc_t rOut = makeRsrc(e.out, e.S * e.ldo * 2);
+      const uint32_t dst = (myq * e.ldo + head * kHD + 32 * wave + 4 * hi) * 2;
 #pragma unroll
       for (int g = 0; g < 4; g++) {
         half4 v;
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = (half_t)(mine[g][e] * inv);
+        for (int c = 0; c < 4; c++) v[c] = (half_t)(mine[g][c] * inv);
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, v), rOut, (int)(dst + 16 * g), 0, 16 /* sc1 */);
       }
     }
     const cusync_dim3 done = {0, head * kHD, 0};
-    if (completed && stage.isProducer()) stage.post(done, 1, stage.storesThrough());
+    if (completed && e.stage.isProducer()) e.stage.post(done, 1, e.stage.storesThrough());
     else __syncthreads();
-    if (tid == 0) recordTileAt(p.timeline, p.timelineCap, stage, p.launched, t, round, tlEntry, tl0, tl1, tl2, p.timeline ? wall_clock64() : 0);
+    if (tid == 0) recordTileAt(e.timeline, e.timelineCap, e.stage, e.launched, t, round, tlEntry, tl0, tl1, tl2, e.timeline ? wall_clock64() : 0);
   }
-  stage.leave(p.launched);
+  const AttnParams atEnd = cusync::argumentsHere<AttnParams>(from);
+  atEnd.stage.leave(atEnd.launched);
 }
 
 }  // namespace attn

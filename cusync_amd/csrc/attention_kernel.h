@@ -81,6 +81,7 @@ struct AttnParams {
 // to itself) or 2 (64 KB, room for another kernel's workgroups beside it).
 template<int kStages>
 __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
+  constexpr uint32_t from = 0;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   __shared__ uint32_t sTicket, sLast;
 
@@ -145,15 +146,17 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
   // being computed and settled when the tile is done.
   uint32_t dryXcds = 0, nextRaw = 0;
   const unsigned long long tlEntry = p.timeline ? wall_clock64() : 0;
-  if (tid == 0) stage.enter();
+  const unsigned long long entered = stage.enter();
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   const bool noDraws = stage.noDraws;     // every tile is some workgroup's static first tile
   for (uint32_t round = 0;; round++) {
+    const AttnParams p = cusync::argumentsHere<AttnParams>(from);
+    const cusync::DynStage& stage = p.stage;
     if (tid == 0) sTicket = round == 0 ? stage.firstTicket(p.launched, dryXcds, noDraws) : stage.drawFinish(nextRaw, p.launched, round, dryXcds, noDraws);
     __syncthreads();
     const uint32_t ticket = sTicket;
     if (ticket >= numTiles) {
-      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
       break;
     }
     cusync_dim3 t = stage.ticketToTile(ticket);
@@ -171,7 +174,7 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
     const uint32_t splits = p.chunk ? (nblk + p.chunk - 1) / p.chunk : 1;
     if (t.z >= splits) {                               // this row tile needs fewer splits than the grid has
       if (tid == 0) nextRaw = stage.drawBegin(dryXcds, noDraws);
-      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
       __syncthreads();
       continue;
     }
@@ -236,7 +239,7 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
     waitKV(jBegin, min(jBegin + (uint32_t)kStages - 2, jEnd - 1));
 #pragma unroll
     for (uint32_t a = 0; a < kStages - 1; a++) issue(jBegin + a, a, jBegin + a < jEnd);
-    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
     // Q fragments stay in registers for the whole tile: k-step s is head-dim 16s + 8hi .. + 7 of row myq.
     if (!(stage.d.in.kind == CUSYNC_POLICY_ROWSYNC && p.cached == 0 && seenRows[0] >= qEnd)) waitRows(q0, qEnd, head * kHD);
     half8 qf[8];
@@ -378,7 +381,8 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
     waitVmcnt<0>();        // the loads issued past the end of the range may still be on their way into LDS
 
     const unsigned long long tl2 = p.timeline ? wall_clock64() : 0;
-    if (tid == 0) nextRaw = stage.drawBegin(dryXcds, noDraws);     // settled after the epilogue
+    const AttnParams e = cusync::argumentsHere<AttnParams>(from);
+    if (tid == 0) nextRaw = e.stage.drawBegin(dryXcds, noDraws);     // settled after the epilogue
     rowSum += __shfl_xor(rowSum, 32);
     bool completed = true;
     if (splits > 1) {
@@ -386,8 +390,8 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
       // written through to memory as they are stored: left dirty in this XCD's L2 they would be written back by the
       // release below together with everything else that is dirty there, which was measured at 14-20 us per tile
       // when the tiles of half a launch finish together.
-      const size_t slot = ((size_t)head * stage.d.grid.y + t.y) * stage.d.grid.z;
-      const __amdgpu_buffer_rsrc_t rPart = makeRsrc(p.partO, p.partBytes);
+      const size_t slot = ((size_t)head * e.stage.d.grid.y + t.y) * e.stage.d.grid.z;
+      const __amdgpu_buffer_rsrc_t rPart = makeRsrc(e.partO, e.partBytes);
       const uint32_t offO = (uint32_t)(((slot + t.z) * (64 * kThreads) + tid * 4) * sizeof(float));
 #pragma unroll
       for (int tt = 0; tt < 4; tt++)
@@ -396,19 +400,19 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
           const floatx4 v = floatx4{o[tt][4 * g], o[tt][4 * g + 1], o[tt][4 * g + 2], o[tt][4 * g + 3]};
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, v), rPart, (int)(offO + (tt * 4 + g) * (kThreads * 16)), 0, 16 /* sc1 */);
         }
-      const uint32_t offS = (uint32_t)(((char*)p.partStat - (char*)p.partO) + ((slot + t.z) * (2 * kThreads) + tid) * sizeof(float));
-      const float scaledMax = rowMax * p.scaleLog2;      // the running maximum is kept unscaled
+      const uint32_t offS = (uint32_t)(((char*)e.partStat - (char*)e.partO) + ((slot + t.z) * (2 * kThreads) + tid) * sizeof(float));
+      const float scaledMax = rowMax * e.scaleLog2;      // the running maximum is kept unscaled
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, scaledMax), rPart, (int)offS, 0, 16);
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, rowSum), rPart, (int)(offS + kThreads * sizeof(float)), 0, 16);
       // The count below is the first thread's, and a workgroup barrier does not wait for stores to memory: every
       // wavefront sees its own through first.
       waitVmcnt<0>();
       __syncthreads();
-      uint32_t* counter = p.arrivals + head * stage.d.grid.y + t.y;
+      uint32_t* counter = e.arrivals + head * e.stage.d.grid.y + t.y;
       if (tid == 0) {
-        const uint32_t before = stage.countIn(counter);      // relaxed: the shares were written through and are acknowledged
+        const uint32_t before = e.stage.countIn(counter);      // relaxed: the shares were written through and are acknowledged
         const bool last = before == splits - 1;
-        if (last) { cusync::dev::storeRelaxed(counter, 0); stage.countSeen(); }
+        if (last) { cusync::dev::storeRelaxed(counter, 0); e.stage.countSeen(); }
         sLast = last;
       }
       __syncthreads();
@@ -419,7 +423,7 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
         // an acquire fence, which would empty this XCD's L2 under the workgroups still walking their keys; and they
         // are issued two splits at a time: a round trip to memory per split and two more for the row statistics is
         // what this step used to consist of (15 us for two splits).
-        auto statOff = [&](uint32_t z) { return (uint32_t)(((char*)p.partStat - (char*)p.partO) + ((slot + z) * (2 * kThreads) + tid) * sizeof(float)); };
+        auto statOff = [&](uint32_t z) { return (uint32_t)(((char*)e.partStat - (char*)e.partO) + ((slot + z) * (2 * kThreads) + tid) * sizeof(float)); };
         auto loadStat = [&](uint32_t off) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rPart, (int)off, 0, 16 /* sc1 */)); };
         float m = kMasked;
         for (uint32_t z = 0; z < splits; z += 4) {
@@ -457,7 +461,7 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
               for (int g = 0; g < 4; g++) {
                 const floatx4 f = __builtin_bit_cast(floatx4, v[q][tt * 4 + g]);
 #pragma unroll
-                for (int e = 0; e < 4; e++) o[tt][4 * g + e] += w * f[e];
+                for (int c = 0; c < 4; c++) o[tt][4 * g + c] += w * f[c];
               }
           }
         }
@@ -465,17 +469,17 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
     }
     // Normalise and store: register r of tile tt is head-dim 32tt + 8(r/4) + 4hi + r%4 of query myq.
     const float inv = 1.0f / rowSum;
-    if (completed && myq < p.S) {
+    if (completed && myq < e.S) {
       // written through like the partial results: a post, or another tile's release, then finds nothing to write back
-      const __amdgpu_buffer_rsrc_t rOut = makeRsrc(p.out, p.S * p.ldo * 2);
-      const uint32_t dst = (myq * p.ldo + head * kHD + 4 * hi) * 2;
+      const __amdgpu_buffer_rsrc_t rOut = makeRsrc(e.out, e.S * e.ldo * 2);
+      const uint32_t dst = (myq * e.ldo + head * kHD + 4 * hi) * 2;
 #pragma unroll
       for (int tt = 0; tt < 4; tt++)
 #pragma unroll
         for (int g = 0; g < 4; g++) {
           half4 v;
 #pragma unroll
-          for (int e = 0; e < 4; e++) v[e] = (half_t)(o[tt][4 * g + e] * inv);
+          for (int c = 0; c < 4; c++) v[c] = (half_t)(o[tt][4 * g + c] * inv);
           __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, v), rOut, (int)(dst + (32 * tt + 8 * g) * 2), 0, 16 /* sc1 */);
         }
     }
@@ -483,11 +487,12 @@ __global__ __launch_bounds__(kThreads, 2) void attentionKernel(AttnParams p) {
     // All waves must be past their last LDS read before the next tile's loads
     // land in stage 0; the post (or this barrier) provides that.
     cusync_dim3 done = {q0, head * kHD, 0};
-    if (completed && stage.isProducer()) stage.post(done, 1, stage.storesThrough());
+    if (completed && e.stage.isProducer()) e.stage.post(done, 1, e.stage.storesThrough());
     else __syncthreads();
-    if (tid == 0) recordTileAt(p.timeline, p.timelineCap, stage, p.launched, t, round, tlEntry, tl0, tl1, tl2, p.timeline ? wall_clock64() : 0);
+    if (tid == 0) recordTileAt(e.timeline, e.timelineCap, e.stage, e.launched, t, round, tlEntry, tl0, tl1, tl2, e.timeline ? wall_clock64() : 0);
   }
-  stage.leave(p.launched);
+  const AttnParams atEnd = cusync::argumentsHere<AttnParams>(from);
+  atEnd.stage.leave(atEnd.launched);
 }
 
 }  // namespace attn

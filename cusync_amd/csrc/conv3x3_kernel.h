@@ -86,7 +86,7 @@ struct Halo3x3Cfg {
 // are (finishTile); the layers whose tiles are fewer than half the CUs are run that way.  A kernel without it does
 // not carry the exchange's code.
 template<class C, bool SPLIT>
-__device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
+__device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p, uint32_t from = 0) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   __shared__ uint32_t sTicket, sLast;
 
@@ -105,7 +105,7 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
   const uint32_t haloPix = C::BM + 2 * W + 2;
   const uint32_t haloLoads = ((haloPix + 1) * pixBytes + 1023) / 1024;       // 1 KiB pieces; pixel haloPix is the pixel of zeros
   const uint32_t zeroPixel = haloPix << pixShift;
-  const uint32_t chunksPerTap = Cc / C::BK, steps = 9 * chunksPerTap;
+  const uint32_t chunksPerTapLog = pixShift - 7, chunksPerTap = 1u << chunksPerTapLog, steps = 9 * chunksPerTap;
   const uint4v rA = rawRsrc(p.A, p.M * Cc * 2);
   const uint4v rB = rawRsrc(p.B, p.N * p.ldb * 2);
   const uint32_t ldsBase = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
@@ -135,15 +135,17 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
 
   uint32_t dryXcds = 0, nextRaw = 0;
   const unsigned long long tlEntry = p.timeline ? wall_clock64() : 0;
-  if (tid == 0) stage.enter();
+  const unsigned long long entered = stage.enter();
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   const bool noDraws = stage.noDraws;     // every tile is some workgroup's static first tile
   for (uint32_t round = 0;; round++) {
+    const GemmParams p = cusync::argumentsHere<GemmParams>(from);
+    const cusync::DynStage& stage = p.stage;
     if (tid == 0) sTicket = round == 0 ? stage.firstTicket(p.launched, dryXcds, noDraws) : stage.drawFinish(nextRaw, p.launched, round, dryXcds, noDraws);
     __syncthreads();
     const uint32_t ticket = sTicket;
     if (ticket >= numTiles) {
-      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
       break;
     }
     const cusync_dim3 t = stage.ticketToTile(ticket);
@@ -203,7 +205,7 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
     };
 #pragma unroll
     for (uint32_t it = 0; it < C::STAGES - 1; it++) issueB(itBegin + it);
-    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
     const unsigned long long tl1 = p.timeline ? wall_clock64() : 0;
 
     floatx16 acc[C::TM][C::TN];
@@ -220,7 +222,7 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
       __builtin_amdgcn_s_barrier();                   // ... for everyone; everyone is done with chunk it-1
       asm volatile("" ::: "memory");
       issueB(it + C::STAGES - 1);
-      const uint32_t tap = it / chunksPerTap, cc = it % chunksPerTap;
+      const uint32_t tap = it >> chunksPerTapLog, cc = it & (chunksPerTap - 1);
       const int32_t shift = ((int32_t)(tap / 3) - 1) * (int32_t)W + (int32_t)(tap % 3) - 1;
       const char* sb = smem + ((it - itBegin) % C::STAGES) * C::B_STAGE;
       uint32_t aBase[C::TM], aSwz[C::TM];
@@ -259,11 +261,12 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
     // epilogue is about to reuse.
     waitVmcnt<0>();
     const unsigned long long tl2 = p.timeline ? wall_clock64() : 0;
-    if (tid == 0) nextRaw = stage.drawBegin(dryXcds, noDraws);     // settled after the epilogue
+    const GemmParams e = cusync::argumentsHere<GemmParams>(from);
+    if (tid == 0) nextRaw = e.stage.drawBegin(dryXcds, noDraws);     // settled after the epilogue
     using F = typename C::Finish;
     bool completed;
     if constexpr (C::KG == 1) {
-      completed = finishTile<F, SPLIT>(p, acc, t, wm, wn, lane, &sLast, smem);
+      completed = finishTile<F, SPLIT>(e, acc, t, wm, wn, lane, &sLast, smem);
     } else {
       // Group g keeps half g of the sums, its own and the other group's: sixteen bytes per lane and piece, every
       // lane's values in a place of their own.
@@ -291,15 +294,16 @@ __device__ __forceinline__ void convHalo3x3Layer(const GemmParams& p) {
 #pragma unroll
           for (int e = 0; e < 4; e++) sums[0][h][4 * g + e] += v[e];
         }
-      if constexpr (C::HALVE_ROWS) completed = finishTile<F, SPLIT>(p, sums, t, 2 * wm + group, wn, lane, &sLast, smem);
-      else completed = finishTile<F, SPLIT>(p, sums, t, wm, 2 * wn + group, lane, &sLast, smem);
+      if constexpr (C::HALVE_ROWS) completed = finishTile<F, SPLIT>(e, sums, t, 2 * wm + group, wn, lane, &sLast, smem);
+      else completed = finishTile<F, SPLIT>(e, sums, t, wm, 2 * wn + group, lane, &sLast, smem);
     }
     cusync_dim3 done = {m0, n0, 0};
-    if (completed && stage.isProducer()) stage.post(done, 1, stage.storesThrough());
+    if (completed && e.stage.isProducer()) e.stage.post(done, 1, e.stage.storesThrough());
     else __syncthreads();
-    if (tid == 0) recordTile(p, t, round, tlEntry, tl0, tl1, tl2, p.timeline ? wall_clock64() : 0);
+    if (tid == 0) recordTile(e, t, round, tlEntry, tl0, tl1, tl2, e.timeline ? wall_clock64() : 0);
   }
-  stage.leave(p.launched);
+  const GemmParams atEnd = cusync::argumentsHere<GemmParams>(from);
+  atEnd.stage.leave(atEnd.launched);
 }
 
 template<class C, bool SPLIT = false>
@@ -323,7 +327,7 @@ struct ConvChainParams {
 template<class C>
 __global__ __launch_bounds__(C::THREADS, C::OCC) void convHalo3x3ChainKernel(ConvChainParams cp) {
   for (uint32_t l = 0; l < cp.layers; l++) {
-    convHalo3x3Layer<C, false>(cp.layer[l]);
+    convHalo3x3Layer<C, false>(cp.layer[l], l * sizeof(GemmParams));
     __syncthreads();        // everyone has read the last ticket of this layer before the next one's is written
   }
 }

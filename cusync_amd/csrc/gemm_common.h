@@ -203,7 +203,7 @@ struct TileStore {
   char* lds;
   uint32_t m0, n0;
   int wm, wn, lane;
-  uint32_t tid;        // threadIdx.x, opaque to the compiler where the K loop is assembly (see the constructor)
+  uint32_t tid;        // threadIdx.x, opaque to the compiler (see the constructor)
   bool through;
   __amdgpu_buffer_rsrc_t rD;
   static constexpr uint32_t kAllRows = (1u << C::WM) - 1;
@@ -212,13 +212,11 @@ struct TileStore {
       : p(p_), lds(lds_), m0(t.y * C::BM), n0(t.x * C::BN), wm(wm_), wn(wn_), lane(lane_), tid(threadIdx.x), through(p_.stage.storesThrough()),
         rD(makeRsrc(p_.D, p_.M * p_.ldd * 2)) {
     // Everything the copy-out computes per thread (piece index -> row, column, offset) depends on the thread index
-    // only, so the compiler works it out once, ahead of the tile loop, and keeps it live across the K loop: where
-    // that loop is assembly with most registers named, those values wait in scratch and every tile's epilogue
-    // reloads them.  Made opaque here, they are computed where they are used.
-    if constexpr (IsAssemblyTile<C>::value) {
-      asm volatile("" : "+v"(tid));
-      asm volatile("" : "+v"(lane));
-    }
+    // only, so the compiler works it out once, ahead of the tile loop, in front of the launch's first loads, and keeps
+    // it live across the K loop: where that loop is assembly with most registers named, those values wait in scratch
+    // and every tile's epilogue reloads them.  Made opaque here, they are computed where they are used.
+    asm volatile("" : "+v"(tid));
+    asm volatile("" : "+v"(lane));
   }
 
   template<class V>

@@ -161,7 +161,7 @@ struct WideOperands {
 // and the kernel parked ten more registers per lane in scratch for it); it would gain at 2048 rows, 595 -> 588 us,
 // where the two launches are ahead anyway.
 template<class C, int AMODE, bool CHUNKS, bool ROUNDS>
-__device__ __forceinline__ void gemmDmaTiles(const GemmParams& p) {
+__device__ __forceinline__ void gemmDmaTiles(const GemmParams& p, uint32_t from = 0) {
   constexpr bool conv = AMODE == kAConv;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   __shared__ uint32_t sTicket, sLast;
@@ -187,15 +187,17 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p) {
   // being computed and settled when the tile is done.
   uint32_t dryXcds = 0, nextRaw = 0;
   const unsigned long long tlEntry = p.timeline ? wall_clock64() : 0;
-  if (tid == 0) stage.enter();
+  const unsigned long long entered = stage.enter();
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   const bool noDraws = stage.noDraws;     // every tile is some workgroup's static first tile
   for (uint32_t round = 0;; round++) {
+    const GemmParams p = cusync::argumentsHere<GemmParams>(from);
+    const cusync::DynStage& stage = p.stage;
     if (tid == 0) sTicket = round == 0 ? stage.firstTicket(p.launched, dryXcds, noDraws) : stage.drawFinish(nextRaw, p.launched, round, dryXcds, noDraws);
     __syncthreads();
     const uint32_t ticket = sTicket;
     if (ticket >= numTiles) {
-      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
       break;
     }
     const cusync_dim3 t = stage.ticketToTile(ticket);
@@ -296,7 +298,7 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p) {
     }
 
     // ---- consumer side (same protocol as the staged kernel) ------------------
-    uint32_t nextColTile = (kBegin & ~(p.waitRound - 1)) / tnq;     // the first chunk's line may begin in the tile before
+    uint32_t nextColTile = chunkSync ? (kBegin & ~(p.waitRound - 1)) / tnq : 0;     // the first chunk's line may begin in the tile before
     const bool oneRowBlock = chunkSync && (m0 / tmq == (mEnd - 1) / tmq);
     uint32_t readyEnd = 0;        // column tiles of the producer below this one are known to be posted (for all row blocks of this tile)
     auto waitRows = [&](uint32_t col, uint32_t z) { stage.waitWaveRows(m0, mEnd - 1, tmq, col, z); };
@@ -525,7 +527,7 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p) {
     if constexpr (C::STAGES > 3) { if constexpr (perChunk) { if (nk > 2) waitChunk(kBegin + 2 * C::BK); } issueAll(Parity<2>{}, 2); }
     if constexpr (C::STAGES > 4) { if constexpr (perChunk) { if (nk > 3) waitChunk(kBegin + 3 * C::BK); } issueAll(Parity<3>{}, 3); }
     static_assert(C::STAGES >= 2 && C::STAGES <= 5, "prologue written for 2..5 stages");
-    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
     const unsigned long long tl1 = p.timeline ? wall_clock64() : 0;
 
     if constexpr (C::PINGPONG && C::BN == 384) {
@@ -639,17 +641,19 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p) {
     // epilogue is about to reuse.
     waitVmcnt<0>();
     const unsigned long long tl2 = p.timeline ? wall_clock64() : 0;
-    if (tid == 0) nextRaw = stage.drawBegin(dryXcds, noDraws);     // settled after the epilogue
-    const bool completed = finishTile<C, !conv>(p, acc, t, wm, wn, lane, &sLast, smem);
+    const GemmParams e = cusync::argumentsHere<GemmParams>(from);
+    if (tid == 0) nextRaw = e.stage.drawBegin(dryXcds, noDraws);     // settled after the epilogue
+    const bool completed = finishTile<C, !conv>(e, acc, t, wm, wn, lane, &sLast, smem);
 
     // All waves must be past their last LDS read before the next tile's loads
     // land in stage 0; the post (or this barrier) provides that.
-    cusync_dim3 done = {m0, outputColumn(p, n0), t.z};
-    if (completed && stage.isProducer()) stage.post(done, postsPerTile(p), stage.storesThrough());
+    cusync_dim3 done = {m0, outputColumn(e, n0), t.z};
+    if (completed && e.stage.isProducer()) e.stage.post(done, postsPerTile(e), e.stage.storesThrough());
     else __syncthreads();
-    if (tid == 0) recordTile(p, t, round, tlEntry, tl0, tl1, tl2, p.timeline ? wall_clock64() : 0);
+    if (tid == 0) recordTile(e, t, round, tlEntry, tl0, tl1, tl2, e.timeline ? wall_clock64() : 0);
   }
-  stage.leave(p.launched);
+  const GemmParams atEnd = cusync::argumentsHere<GemmParams>(from);
+  atEnd.stage.leave(atEnd.launched);
 }
 
 template<class C, int AMODE = kAPlain, bool CHUNKS = true>
@@ -667,7 +671,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_PER_SIMD) void gemmDmaKernel(G
 template<class C>
 __global__ __launch_bounds__(C::THREADS, C::WAVES_PER_SIMD) void gemmDmaChainKernel(GemmChainParams cp) {
   for (uint32_t g = 0; g < cp.count; g++) {
-    gemmDmaTiles<C, kAPlain, true, false>(cp.gemm[g]);
+    gemmDmaTiles<C, kAPlain, true, false>(cp.gemm[g], g * sizeof(GemmParams));
     __syncthreads();        // everyone has read the last ticket of this GEMM before the next one's is written
   }
 }

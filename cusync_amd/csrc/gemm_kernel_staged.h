@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kThreads) void gemmKernel(GemmParams p) {
   // first tile's loads are under way; the draw of the next ticket is issued while a tile is
   // being computed and settled when the tile is done.
   uint32_t dryXcds = 0, nextRaw = 0;
-  if (tid == 0) stage.enter();
+  const unsigned long long entered = stage.enter();
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   const bool noDraws = stage.noDraws;     // every tile is some workgroup's static first tile
   for (uint32_t round = 0;; round++) {
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kThreads) void gemmKernel(GemmParams p) {
     __syncthreads();
     const uint32_t ticket = sTicket;
     if (ticket >= numTiles) {
-      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+      if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
       break;
     }
     const cusync_dim3 t = stage.ticketToTile(ticket);      // x = column tile, y = row tile
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kThreads) void gemmKernel(GemmParams p) {
 
     issue(Parity<0>{}, 0);
     if (nk > 1) issue(Parity<1>{}, 1);
-    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
     earlyPoll(kBegin + 2 * C::BK);
     stash(Parity<0>{});
     __syncthreads();

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kActThreads) void swigluStageKernel(ActParams p) {
     if (tid == 0) sTicket = round == 0 ? stage.firstTicket(p.launched, dryXcds, noDraws) : stage.drawFinish(nextRaw, p.launched, round, dryXcds, noDraws);
     __syncthreads();
     const uint32_t ticket = sTicket;
-    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched);
+    if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, 0);
     if (ticket >= numTiles) break;
     const cusync_dim3 t = stage.ticketToTile(ticket);
     const uint32_t m0 = t.y * kActM, c0 = t.x * kActN;

@@ -18,8 +18,23 @@
 #include <hip/hip_runtime.h>
 #include "../../include/cusync/device-functions.h"
 #include "policy_eval.h"
+#include "tile_deal.h"
 
 namespace cusync {
+
+// The kernel's arguments, `from` bytes into them, read at this place in the program: a kernel that may work through
+// several tiles takes them anew for each tile and again for each epilogue, so that what is loaded, and what is worked out
+// of it, is what the code behind this place needs.  Taken once, ahead of the tile loop, everything that does not change
+// from tile to tile was (a thousand instructions in front of the first tile, two hundred of them parking the results: 2.5 to
+// 3.5 us of every launch, against 1.2 to 1.6 now).  By value: through a reference they are read again behind every
+// statement that may write memory, in the K loops above all.
+template<class Params>
+__device__ __forceinline__ Params argumentsHere(uint32_t from = 0) {
+  typedef const char __attribute__((address_space(4)))* Arguments;
+  Arguments base = (Arguments)__builtin_amdgcn_kernarg_segment_ptr() + from;
+  asm volatile("" : "+s"(base));
+  return *(const Params*)base;
+}
 
 struct DynStage {
   cusync_stage_desc d;
@@ -32,8 +47,8 @@ struct DynStage {
   // own then); the wait can skip the cache invalidation that would also throw
   // away the weights the XCD's workgroups share.
   bool lineAligned;
-  // allStatic(launched) of the launch this object goes to, worked out by the launcher (set by prepare()): in the
-  // kernel it is a loop of eight rounds of integer divisions that every wavefront would run before its first load.
+  // The launch this object goes to has a workgroup for every tile (set by prepare()): nobody then needs a dispenser, a
+  // look at the others or the count of workgroups that ran dry, and a workgroup leaves after its tile without an atomic.
   bool noDraws;
   // Diagnosis (set by the launcher from CUSYNC_FORCE_RELEASE): every post, and every count the k-slices and key-range
   // splits hand partial results over with, is a release at device scope (and the counts' readers acquire), as the
@@ -64,17 +79,7 @@ struct DynStage {
   // then takes tickets until the tiles run out.  All of the following are
   // called by the first thread of a workgroup only.
   //
-  // Each of the eight XCDs has its own L2, so which workgroup gets which tile
-  // decides how much of the operands is re-fetched from memory.  The tiles are
-  // therefore dealt per XCD.  With at least eight column tiles XCD x owns the
-  // column tiles [x*gx/8, (x+1)*gx/8) of every row, in row-major order: its
-  // workgroups share the same few B column panels (and, row by row, the same
-  // A panels) in their L2.  With fewer column tiles (a convolution with 64
-  // output channels has one) XCD x owns the row tiles [x*gy/8, (x+1)*gy/8)
-  // instead, so that the rows of A it reads — for a convolution each input
-  // pixel is read by up to R*S neighbouring rows — stay in its L2.  The
-  // ticket is the tile's position in the row-major schedule; it still goes
-  // through the stage's ticket -> tile table.
+  // tile_deal.h says how the tiles are dealt to the XCDs.
   //
   // A device-wide atomic takes the better part of a microsecond, several when
   // hundreds of workgroups hit one address at kernel start, and a kernel of a
@@ -96,35 +101,8 @@ struct DynStage {
   //    length is dry for good, the others are tried in turn, so the end of the
   //    launch stays balanced.  The last workgroup to find everything dry
   //    re-arms the dispensers for the next run.
-  __host__ __device__ __forceinline__ bool dealtByRows() const { return d.grid.x < 8; }
-  __host__ __device__ __forceinline__ uint32_t xcdTiles(uint32_t x) const {
-    const uint32_t span = dealtByRows() ? d.grid.y : d.grid.x;
-    return ((x + 1) * span / 8 - x * span / 8) * (dealtByRows() ? d.grid.x : d.grid.y) * d.grid.z;
-  }
-  // Positions of XCD x's list that are handed out statically to the first tiles of the workgroups.
-  __host__ __device__ __forceinline__ uint32_t xcdStatic(uint32_t x, uint32_t launched) const {
-    const uint32_t wgs = launched > x ? (launched - x + 7) / 8 : 0;
-    const uint32_t tiles = xcdTiles(x);
-    return wgs < tiles ? wgs : tiles;
-  }
-  __device__ __forceinline__ uint32_t xcdTicket(uint32_t x, uint32_t l) const {
-    const uint32_t span = dealtByRows() ? d.grid.y : d.grid.x;
-    const uint32_t lo = x * span / 8, width = (x + 1) * span / 8 - lo;
-    if (!dealtByRows()) return lo + l % width + (l / width) * d.grid.x;
-    const uint32_t perSlice = width * d.grid.x;          // this XCD's tiles in one k-slice
-    return (l / perSlice) * d.grid.x * d.grid.y + lo * d.grid.x + l % perSlice;
-  }
-  // True when the static first tiles already are all tiles (a launch of one round whose workgroups spread
-  // evenly over the lists): nobody then needs a dispenser, a look at the others or the count of workgroups
-  // that ran dry, and a workgroup leaves after its tile without a single atomic.
-  __host__ __device__ __forceinline__ bool allStatic(uint32_t launched) const {
-    if (!customOrder()) return false;
-    bool all = true;
-    for (uint32_t x = 0; x < 8; x++) all = all && xcdStatic(x, launched) == xcdTiles(x);
-    return all;
-  }
-  // Host side, once the descriptor and lineAligned are in place: what the kernel would otherwise work out per wavefront.
-  __host__ void prepare(uint32_t launched) { noDraws = allStatic(launched); }
+  // Host side, once the descriptor is in place.
+  __host__ void prepare(uint32_t launched) { noDraws = customOrder() && launched >= d.grid.x * d.grid.y * d.grid.z; }
   static __device__ __forceinline__ uint32_t workgroupIndex() {
     return blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
   }
@@ -137,8 +115,10 @@ struct DynStage {
     return dev::ticketAdd(d.startCounter, 1);
   }
   // The workgroup that started last raises the wait-kernel flag.
-  __device__ __forceinline__ void finishStart(uint32_t token, uint32_t launched) const {
+  __device__ __forceinline__ void finishStart(uint32_t token, uint32_t launched, unsigned long long entered) const {
+    if (entered) stamp(0, entered);
     if (!isProducer() || (d.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL)) return;
+    asm volatile("" : "+v"(token));        // looked at here and not before: the count's round trip is over by now
     if (token == launched - 1) {
       dev::storeRelaxed(d.startCounter, 0);
       // The flag says that every producer workgroup is on the device and publishes no data (a consumer reads the
@@ -154,14 +134,16 @@ struct DynStage {
   // the last, the host's wait for it and another for every stream beside it: a pass of the GPT-3 MLP at one row 76.8 ->
   // 70.5 us with the stamps, of the 56x56x64 convolution pair on two streams 55.4 -> 40.9, of attention on three
   // (16 rows behind 2048) 89.9 -> 67.5.
-  __device__ __forceinline__ void stamp(uint32_t which) const {
-    const unsigned long long v = (wall_clock64() << 16) | ((uint32_t)d.iter & 0xffffu);
+  __device__ __forceinline__ void stamp(uint32_t which, unsigned long long clock) const {
+    const unsigned long long v = (clock << 16) | ((uint32_t)d.iter & 0xffffu);
     __hip_atomic_store(reinterpret_cast<unsigned long long*>(d.spinTimeouts + CUSYNC_HOST_STAMP_OFFSET) + which, v,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
-  // At kernel entry, called by the first thread of every workgroup.
-  __device__ __forceinline__ void enter() const {
-    if ((d.flags & CUSYNC_STAGE_STAMPS_START) && workgroupIndex() == 0) stamp(0);
+  // At kernel entry: the clock for the stamp of the launch's start, 0 where this workgroup makes none.  finishStart()
+  // stores it, behind the first loads: a wavefront's counter of memory operations goes down in order, so what is loaded
+  // after a store to the host's memory waits for its way over the bus, and the first workgroup held up its tile by 2.4 us.
+  __device__ __forceinline__ unsigned long long enter() const {
+    return (d.flags & CUSYNC_STAGE_STAMPS_START) && workgroupIndex() == 0 ? wall_clock64() : 0;
   }
   // When a workgroup has no tile left, called by all its threads.  Every wavefront has its stores acknowledged, the
   // barrier collects the wavefronts, and the count (relaxed: the stores went through to memory) tells the last workgroup.
@@ -174,7 +156,7 @@ struct DynStage {
       if (countIn(left) == launched - 1) {
         dev::storeRelaxed(left, 0);
         countSeen();
-        stamp(1);
+        stamp(1, wall_clock64());
       }
     }
   }
@@ -195,8 +177,8 @@ struct DynStage {
     constexpr uint32_t kLine = 32;          // counters are 128 bytes apart
     const uint32_t mine = homeList();
     if (raw != 0xffffffffu) {
-      const uint32_t l = raw + xcdStatic(mine, launched);
-      if (l < xcdTiles(mine)) return xcdTicket(mine, l);
+      const uint32_t l = raw + deal::listStatic(d.grid, mine, launched);
+      if (l < deal::listTiles(d.grid, mine)) return deal::listTicket(d.grid, mine, l);
     }
     dry |= 1u << mine;
     uint32_t seen[8];
@@ -204,12 +186,12 @@ struct DynStage {
     for (uint32_t x = 0; x < 8; x++) seen[x] = dev::loadRelaxed(&d.xcdTickets[x * kLine]);
 #pragma unroll
     for (uint32_t x = 0; x < 8; x++)
-      if (seen[x] + xcdStatic(x, launched) >= xcdTiles(x)) dry |= 1u << x;
+      if (seen[x] + deal::listStatic(d.grid, x, launched) >= deal::listTiles(d.grid, x)) dry |= 1u << x;
     for (uint32_t s = 1; s < 8; s++) {
       const uint32_t x = (mine + s) & 7u;
       if (dry & (1u << x)) continue;
-      const uint32_t l = dev::ticketAdd(&d.xcdTickets[x * kLine], 1) + xcdStatic(x, launched);
-      if (l < xcdTiles(x)) return xcdTicket(x, l);
+      const uint32_t l = dev::ticketAdd(&d.xcdTickets[x * kLine], 1) + deal::listStatic(d.grid, x, launched);
+      if (l < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, l);
       dry |= 1u << x;
     }
     const uint32_t finished = dev::ticketAdd(&d.xcdTickets[8 * kLine], 1);
@@ -222,7 +204,8 @@ struct DynStage {
   __device__ __forceinline__ uint32_t firstTicket(uint32_t launched, uint32_t& dry, bool noDraws = false) const {
     if (!customOrder()) return workgroupIndex();
     const uint32_t b = workgroupIndex(), x = b & 7u, pos = b >> 3;
-    if (pos < xcdTiles(x)) return xcdTicket(x, pos);
+    if (noDraws) return deal::onlyTicket(d.grid, launched, b);
+    if (pos < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, pos);
     return drawFinish(drawBegin(dry, noDraws), launched, 0, dry, noDraws);
   }
 

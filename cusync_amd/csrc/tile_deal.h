@@ -1,0 +1,67 @@
+// Which tile a workgroup of a persistent launch begins with: host and device code, so that it can be checked on the CPU.
+//
+// Each of the eight XCDs has its own L2, so which workgroup gets which tile decides how much of the operands is
+// re-fetched from memory.  The tiles are therefore dealt in eight lists, one per XCD.  With at least eight column tiles
+// list x holds the column tiles [x*gx/8, (x+1)*gx/8) of every row, in row-major order: its workgroups share the same few
+// B column panels (and, row by row, the same A panels) in their L2.  With fewer column tiles (a convolution with 64
+// output channels has one) it holds the row tiles [x*gy/8, (x+1)*gy/8) instead, so that the rows of A it reads (for a
+// convolution each input pixel is read by up to R*S neighbouring rows) stay in its L2.  A ticket is the tile's position
+// in the row-major schedule; it still goes through the stage's ticket -> tile table.
+//
+// Workgroups are dispatched to the XCDs round-robin: workgroup b works on list b % 8 and begins with position b / 8 of it.
+#pragma once
+
+#include "policy_eval.h"
+
+namespace cusync {
+namespace deal {
+
+constexpr uint32_t kNoTicket = 0xffffffffu;
+
+CUSYNC_HD bool byRows(const cusync_dim3& grid) { return grid.x < 8; }
+CUSYNC_HD uint32_t listTiles(const cusync_dim3& grid, uint32_t x) {
+  const uint32_t span = byRows(grid) ? grid.y : grid.x;
+  return ((x + 1) * span / 8 - x * span / 8) * (byRows(grid) ? grid.x : grid.y) * grid.z;
+}
+CUSYNC_HD uint32_t listWorkgroups(uint32_t x, uint32_t launched) { return launched > x ? (launched - x + 7) / 8 : 0; }
+// Positions of list x that are handed out statically to the first tiles of the workgroups.
+CUSYNC_HD uint32_t listStatic(const cusync_dim3& grid, uint32_t x, uint32_t launched) {
+  const uint32_t wgs = listWorkgroups(x, launched), tiles = listTiles(grid, x);
+  return wgs < tiles ? wgs : tiles;
+}
+// Ticket of position l of list x.
+CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l) {
+  const uint32_t span = byRows(grid) ? grid.y : grid.x;
+  const uint32_t lo = x * span / 8, width = (x + 1) * span / 8 - lo;
+  if (!byRows(grid)) return lo + l % width + (l / width) * grid.x;
+  const uint32_t perSlice = width * grid.x;          // this list's tiles in one k-slice
+  return (l / perSlice) * grid.x * grid.y + lo * grid.x + l % perSlice;
+}
+
+// A launch of at least as many workgroups as tiles needs no dispenser: every tile is some workgroup's first one.  Where
+// the lists do not come out even (98 tiles of a convolution: lists of 12 to 14 for 12 or 13 workgroups each) the
+// workgroups beyond their own list's length take, in order, the positions that other lists have left over.  Drawn from
+// the dispensers instead, those workgroups began 2.5 us after the others, every workgroup paid two round trips to learn
+// that nothing is left, and the k-slices of a tile could not share their reduction (slicesShareReduction).
+CUSYNC_HD uint32_t leftOver(const cusync_dim3& grid, uint32_t launched, uint32_t b) {
+  const uint32_t mine = b & 7u;
+  uint32_t s = b / 8 - listTiles(grid, mine);        // how many workgroups without a place of their own come before this one
+  for (uint32_t x = 0; x < mine; x++) {
+    const uint32_t tiles = listTiles(grid, x), wgs = listWorkgroups(x, launched);
+    if (wgs > tiles) s += wgs - tiles;
+  }
+  for (uint32_t x = 0; x < 8; x++) {
+    const uint32_t tiles = listTiles(grid, x), wgs = listWorkgroups(x, launched);
+    const uint32_t left = tiles > wgs ? tiles - wgs : 0;
+    if (s < left) return listTicket(grid, x, wgs + s);
+    s -= left;
+  }
+  return kNoTicket;                                  // more workgroups than tiles
+}
+// The only ticket of workgroup b of such a launch.
+CUSYNC_HD uint32_t onlyTicket(const cusync_dim3& grid, uint32_t launched, uint32_t b) {
+  return b / 8 < listTiles(grid, b & 7u) ? listTicket(grid, b & 7u, b / 8) : leftOver(grid, launched, b);
+}
+
+}  // namespace deal
+}  // namespace cusync

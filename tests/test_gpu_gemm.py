@@ -171,6 +171,21 @@ def test_gemm_split_k_with_the_reduction_shared_among_the_slices(tile, split):
     assert_close(shared, orc.gemm(a, b, orc.EPI_GELU), "shared reduction, %d slices, tile %d" % (split, tile))
 
 
+@pytest.mark.parametrize("tile,M,N,split", [(api.TILE.D128x192x64, 300, 9 * 192, 2), (api.TILE.T256x192x64, 1000, 13 * 192, 4),
+                                            (api.TILE.T256x192x64, 700, 3 * 192, 2), (api.TILE.D32x128x64, 20, 11 * 128, 3)])
+def test_gemm_tiles_that_do_not_divide_among_the_xcds(tile, M, N, split):
+    # a workgroup per tile, but the eight lists the tiles are dealt in are of unequal length: the workgroups beyond their
+    # list's end take what other lists have left over, without a dispenser, and the k-slices share their reduction
+    print("uneven lists tile", tile, M, N, "slices", split, flush=True)
+    K = 512
+    a = uniform_f16((M, K), 41)
+    b = normal_f16((K, N), 42, std=0.05)
+    plain = run_gemm(a, b, tile, split_k=split)
+    shared = run_gemm(a, b, tile, split_k=split, shared_reduction=1, launches=3)
+    assert np.array_equal(plain.view(np.uint16), shared.view(np.uint16))
+    assert_close(shared, orc.gemm(a, b), "uneven lists, %d slices, tile %d" % (split, tile))
+
+
 def test_gemm_split_k_is_deterministic():
     a = uniform_f16((64, 4096), 23)
     b = normal_f16((4096, 256), 24, std=0.05)
