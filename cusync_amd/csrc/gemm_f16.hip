@@ -90,6 +90,9 @@ int residentWorkgroups(int tile) {
       if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ti->kernel[v], (int)ti->threads, ti->lds))) return 0;
       perCU = std::min(perCU, n);
     }
+    if (ti->chainKernelAhead &&
+        (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ti->chainKernelAhead), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ti->ldsChainAhead)) ||
+         CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&ti->chainAheadResidentPerCU, ti->chainKernelAhead, (int)ti->threads, ti->ldsChainAhead)))) return 0;
     const void* others[5] = { reinterpret_cast<const void*>(ti->chainKernel), reinterpret_cast<const void*>(ti->kernelNoChunkWaits),
                               reinterpret_cast<const void*>(ti->kernelOnce), reinterpret_cast<const void*>(ti->kernelOnceNoChunkWaits),
                               reinterpret_cast<const void*>(ti->chainKernelOnce) };
@@ -211,6 +214,7 @@ static GemmParams gemmParams(const cusync_gemm_args* a, const TileInfo* ti, uint
   p.stage.lineAligned = !cusync::rt::forceAcquire() && s.in.kind != CUSYNC_POLICY_NOSYNC && (uintptr_t)a->A % 128 == 0 &&
                         (a->lda * 2) % 128 == 0 && (wholeLineTiles || canRound);
   p.stage.releaseAll = cusync::rt::forceRelease();
+  p.stage.turn = 0;
   p.waitRound = p.stage.lineAligned && !wholeLineTiles ? 64 : 1;
   p.stage.prepare(launched);
   p.M = a->M; p.N = a->N; p.K = a->K;
@@ -370,6 +374,7 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
   const int resident = residentWorkgroups(args[0].tile);
   if (resident <= 0) { setError("gemm: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
   uint32_t launched = (uint32_t)resident, mostTiles = 0;
+  bool oneRow = true;
   for (int i = 0; i < count; i++) {
     const cusync_gemm_args& a = args[i];
     if (a.tile != args[0].tile) { setError("gemm chain: all GEMMs must use the same tile"); return CUSYNC_ERROR_NOT_INITIALIZED; }
@@ -378,19 +383,25 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
     if (e != CUSYNC_SUCCESS) return e;
     if (a.stage.in.kind != CUSYNC_POLICY_NOSYNC && i == 0) { setError("gemm chain: the first GEMM cannot wait on a stage outside the launch"); return CUSYNC_ERROR_NOT_INITIALIZED; }
     mostTiles = std::max<uint32_t>(mostTiles, a.stage.grid.x * a.stage.grid.y * a.stage.grid.z);
+    oneRow = oneRow && a.stage.grid.y == 1;
     if (a.max_workgroups > 0) launched = std::min<uint32_t>(launched, (uint32_t)a.max_workgroups);
   }
   // As many workgroups as the GEMM with most tiles has (and the device holds at once).  A workgroup without a tile
   // of GEMM i goes straight on to GEMM i+1 and waits there for tiles that running workgroups hold.
   launched = std::min<uint32_t>(launched, mostTiles);
+  // Grids of one row read B once.  Where each tile has a CU to itself, the workgroup takes all of the CU's LDS for loads in
+  // flight and fetches B ahead of the wait for its producer (DmaCfg::AHEAD): GPT-3 MLP in one launch, without -> with,
+  // TileSync: 64 rows 82.6 -> 80.7 us, 1 row 72.1 -> 71.1.  With more tiles two smaller workgroups share a CU and fill each
+  // other's gaps (inner width 49 152, 384 tiles, 1 row: 392 us, one workgroup to a CU 409).
+  const bool ahead = oneRow && ti->chainAheadResidentPerCU > 0 && mostTiles <= (uint32_t)(ti->chainAheadResidentPerCU * g_numCUs);
+  const auto kernel = ahead ? ti->chainKernelAhead : oneRow && ti->chainKernelOnce ? ti->chainKernelOnce : ti->chainKernel;
   GemmChainParams cp = {};
   cp.count = (uint32_t)count;
-  bool once = ti->chainKernelOnce != nullptr;
   for (int i = 0; i < count; i++) {
     cp.gemm[i] = gemmParams(&args[i], ti, launched);
-    once = once && args[i].stage.grid.y == 1;
+    cp.gemm[i].stage.turn = (uint32_t)i;
   }
-  hipLaunchKernelGGL(once ? ti->chainKernelOnce : ti->chainKernel, dim3(launched), dim3(ti->threads), ti->lds, (hipStream_t)stream, cp);
+  hipLaunchKernelGGL(kernel, dim3(launched), dim3(ti->threads), ahead ? ti->ldsChainAhead : ti->lds, (hipStream_t)stream, cp);
   if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
   return CUSYNC_SUCCESS;
 }

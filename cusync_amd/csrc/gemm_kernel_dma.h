@@ -52,7 +52,7 @@ namespace cusync {
 namespace gemm {
 
 template<int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_, int WAVES_PER_SIMD_ = 1, bool BT_ = false, bool PIPE_ = false, bool PINGPONG_ = false,
-         bool ONCE_ = false>
+         bool ONCE_ = false, bool AHEAD_ = false>
 struct DmaCfg {
   // B is read by one row tile only (a grid of one row): its loads carry the non-temporal hint.  A launch of few rows
   // is bound by streaming the weights, and a probe that only reads 151 MB takes 26.2 us with the hint and 29.0 without
@@ -61,6 +61,13 @@ struct DmaCfg {
   // L2 lines the neighbours were about to ask for: 96 rows on 64-row tiles 96.9 -> 106.2 us, LLaMA at 512 rows
   // 103.3 -> 119.8.
   static constexpr bool ONCE = ONCE_;
+  // B is fetched ahead of A: a consumer's weights do not depend on its producer, so three of the four wavefronts send out
+  // their share of the first STAGES - 1 chunks of B before the producer is waited for, while the fourth polls (a
+  // wavefront's loads return in order: the poll would come back behind its own), and the memory is not idle between the
+  // producer's last weights and the consumer's first.  All of the producer tiles are waited for at once.  GPT-3 MLP in one
+  // launch, 64 rows: 83.0 -> 80.6 us; attention of 16 rows behind 2048, whose output projection is such a launch:
+  // 68.0 -> 66.0.
+  static constexpr bool AHEAD = AHEAD_;
   static constexpr bool PIPE = PIPE_;                      // barrier in the middle of a chunk, fragments prefetched across chunks
   static constexpr bool PINGPONG = PINGPONG_;              // K loop in assembly, operands in whole cache lines (see above)
   static constexpr bool BT = BT_;                          // B given as [N][K] (k contiguous), e.g. KRSC filters
@@ -104,6 +111,8 @@ struct DmaCfg {
 
 template<int BM, int BN, int BK, int WM, int WN, int STAGES, int WAVES_PER_SIMD>
 using DmaCfgOnce = DmaCfg<BM, BN, BK, WM, WN, STAGES, WAVES_PER_SIMD, false, false, false, true>;
+template<int BM, int BN, int BK, int WM, int WN, int STAGES, int WAVES_PER_SIMD>
+using DmaCfgAhead = DmaCfg<BM, BN, BK, WM, WN, STAGES, WAVES_PER_SIMD, false, false, false, true, true>;
 
 // One direct load: 64 lanes x 16 bytes from buffer `rsrc` at per-lane byte offset
 // `voff` into LDS at ldsAddr + 16*lane.  ldsAddr must be wave-uniform.
@@ -435,17 +444,18 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p, uint32_t from 
 
     // Iteration kt on stage S = kt % STAGES.  Chunks kt+1 .. kt+STAGES-2 are the
     // ones this wave still has in flight behind chunk kt.
-    auto step = [&](auto SP, uint32_t kt) {
+    auto stepAt = [&](auto SP, auto INFLIGHT, uint32_t kt) {
       constexpr int S = decltype(SP)::value;
-      waitVmcnt<(C::STAGES - 2) * C::LOADS>();
+      waitVmcnt<decltype(INFLIGHT)::value>();
       __builtin_amdgcn_s_barrier();      // chunk kt is in LDS for everyone; everyone is done with chunk kt-1
       asm volatile("" ::: "memory");
       const uint32_t ktLoad = kt + C::STAGES - 1;
-      if constexpr (conv || !ROUNDS) { if (ktLoad < nk) waitChunk(kBegin + ktLoad * C::BK); }
+      if constexpr ((conv || !ROUNDS) && !C::AHEAD) { if (ktLoad < nk) waitChunk(kBegin + ktLoad * C::BK); }
       __builtin_amdgcn_sched_barrier(0);
       compute(SP, Parity<(S + C::STAGES - 1) % C::STAGES>{}, ktLoad);
       __builtin_amdgcn_sched_barrier(0);
     };
+    auto step = [&](auto SP, uint32_t kt) { stepAt(SP, Parity<(C::STAGES - 2) * C::LOADS>{}, kt); };
 
     // ---- pipelined order -----------------------------------------------------------
     half8 pfa[2][C::TM], pfb[2][C::TN];
@@ -503,7 +513,7 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p, uint32_t from 
       __builtin_amdgcn_sched_barrier(0);
     };
 
-    if (consumer) {
+    if (consumer && !C::AHEAD) {
       cusync_dim3 w = {m0, 0, 1};
       if (stage.needsWait(w)) {
         if (wave == 0) { if constexpr (conv) cvWaitRows(0, 1); else waitRows(0, 1); }
@@ -519,14 +529,34 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p, uint32_t from 
     constexpr bool perChunk = conv || !ROUNDS;
     auto waitThrough = [&](uint32_t kt) { waitChunk(kBegin + min(kt, nk - 1) * C::BK); };
     // (the assembly K loop has no place for waits: a stage of a tile policy waits for all its producer tiles here)
-    if constexpr (C::PINGPONG) waitThrough(nk - 1);
-    else if constexpr (perChunk) waitChunk(kBegin);
-    else waitThrough(C::STAGES - 2);
-    if constexpr (!C::PINGPONG) issueAll(Parity<0>{}, 0);
-    if constexpr (C::STAGES > 2 && !C::PINGPONG) { if constexpr (perChunk) { if (nk > 1) waitChunk(kBegin + C::BK); } issueAll(Parity<1>{}, 1); }
-    if constexpr (C::STAGES > 3) { if constexpr (perChunk) { if (nk > 2) waitChunk(kBegin + 2 * C::BK); } issueAll(Parity<2>{}, 2); }
-    if constexpr (C::STAGES > 4) { if constexpr (perChunk) { if (nk > 3) waitChunk(kBegin + 3 * C::BK); } issueAll(Parity<3>{}, 3); }
-    static_assert(C::STAGES >= 2 && C::STAGES <= 5, "prologue written for 2..5 stages");
+    if constexpr (C::AHEAD) {
+      // (see DmaCfg::AHEAD; the first round of the loop counts with this order)
+      auto issueB = [&] { staticFor<C::STAGES - 1>([&](auto SP) { staticFor<C::B_LOADS>([&](auto QP) { issueOne(SP, QP, decltype(SP)::value); }); }); };
+      if (!consumer || wave != 0) issueB();
+      if (consumer) {
+        if (wave == 0) {
+          const cusync_dim3 w = {m0, 0, 1};
+          if (stage.needsWait(w)) waitRows(0, 1);
+          waitThrough(nk - 1);
+        }
+        __syncthreads();
+        if (wave == 0) issueB();
+      }
+      staticFor<C::STAGES - 1>([&](auto SP) {
+        staticFor<C::A_LOADS>([&](auto QP) { issueOne(SP, Parity<C::B_LOADS + decltype(QP)::value>{}, decltype(SP)::value); });
+      });
+    } else {
+      if constexpr (C::PINGPONG) waitThrough(nk - 1);
+      else if constexpr (perChunk) waitChunk(kBegin);
+      else waitThrough(C::STAGES - 2);
+      if constexpr (!C::PINGPONG) {
+        staticFor<C::STAGES - 1>([&](auto SP) {
+          constexpr uint32_t kt = decltype(SP)::value;
+          if constexpr (perChunk && kt > 0) { if (nk > kt) waitChunk(kBegin + kt * C::BK); }
+          issueAll(SP, kt);
+        });
+      }
+    }
     if (tid == 0 && round == 0) stage.finishStart(startToken, p.launched, entered);
     const unsigned long long tl1 = p.timeline ? wall_clock64() : 0;
 
@@ -627,13 +657,22 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p, uint32_t from 
         if (C::STAGES > 4 && kt + 4 < nk) stepP(Parity<4 % C::STAGES>{}, kt + 4);
       }
     } else {
-      for (uint32_t kt = 0; kt < nk; kt += C::STAGES) {
-        if constexpr (!perChunk) waitThrough(kt + 2 * C::STAGES - 2);      // the loads this round issues
-        step(Parity<0>{}, kt);
-        if (kt + 1 < nk) step(Parity<1 % C::STAGES>{}, kt + 1);
-        if (C::STAGES > 2 && kt + 2 < nk) step(Parity<2 % C::STAGES>{}, kt + 2);
-        if (C::STAGES > 3 && kt + 3 < nk) step(Parity<3 % C::STAGES>{}, kt + 3);
-        if (C::STAGES > 4 && kt + 4 < nk) step(Parity<4 % C::STAGES>{}, kt + 4);
+      uint32_t kt = 0;
+      if constexpr (C::AHEAD) {
+        // First round: behind A of chunk i the prologue issued A of the chunks after it only, B of all of them before.
+        staticFor<C::STAGES>([&](auto SP) {
+          constexpr int I = decltype(SP)::value;
+          constexpr int BEHIND = I < C::STAGES - 2 ? (C::STAGES - 2 - I) * C::A_LOADS + I * C::LOADS : (C::STAGES - 2) * C::LOADS;
+          if (I < nk) stepAt(SP, Parity<BEHIND>{}, I);
+        });
+        kt = C::STAGES;
+      }
+      for (; kt < nk; kt += C::STAGES) {
+        if constexpr (!perChunk && !C::AHEAD) waitThrough(kt + 2 * C::STAGES - 2);      // the loads this round issues
+        staticFor<C::STAGES>([&](auto SP) {
+          constexpr uint32_t I = decltype(SP)::value;
+          if (I == 0 || kt + I < nk) step(SP, kt + I);
+        });
       }
     }
 
@@ -671,7 +710,7 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_PER_SIMD) void gemmDmaKernel(G
 template<class C>
 __global__ __launch_bounds__(C::THREADS, C::WAVES_PER_SIMD) void gemmDmaChainKernel(GemmChainParams cp) {
   for (uint32_t g = 0; g < cp.count; g++) {
-    gemmDmaTiles<C, kAPlain, true, false>(cp.gemm[g], g * sizeof(GemmParams));
+    gemmDmaTiles<C, kAPlain, true, C::AHEAD>(cp.gemm[g], g * sizeof(GemmParams));
     __syncthreads();        // everyone has read the last ticket of this GEMM before the next one's is written
   }
 }

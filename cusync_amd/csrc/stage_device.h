@@ -55,6 +55,9 @@ struct DynStage {
   // plain protocol has it, also where the stores were written through and acknowledged and the library normally
   // raises them relaxed.  Results must not change; only the write-backs and invalidations come back.
   bool releaseAll;
+  // How many positions further on the lists of tiles are begun (see deal::listTicket): the place of a GEMM in a launch of
+  // several, 0 elsewhere.
+  uint32_t turn;
 
   __device__ __forceinline__ bool isProducer() const { return d.out.kind != CUSYNC_POLICY_NOSYNC; }
   // Whether this stage's kernels write their output through to memory as they store it (sc1): a producer's do, so
@@ -178,7 +181,7 @@ struct DynStage {
     const uint32_t mine = homeList();
     if (raw != 0xffffffffu) {
       const uint32_t l = raw + deal::listStatic(d.grid, mine, launched);
-      if (l < deal::listTiles(d.grid, mine)) return deal::listTicket(d.grid, mine, l);
+      if (l < deal::listTiles(d.grid, mine)) return deal::listTicket(d.grid, mine, l, turn);
     }
     dry |= 1u << mine;
     uint32_t seen[8];
@@ -191,7 +194,7 @@ struct DynStage {
       const uint32_t x = (mine + s) & 7u;
       if (dry & (1u << x)) continue;
       const uint32_t l = dev::ticketAdd(&d.xcdTickets[x * kLine], 1) + deal::listStatic(d.grid, x, launched);
-      if (l < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, l);
+      if (l < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, l, turn);
       dry |= 1u << x;
     }
     const uint32_t finished = dev::ticketAdd(&d.xcdTickets[8 * kLine], 1);
@@ -204,8 +207,8 @@ struct DynStage {
   __device__ __forceinline__ uint32_t firstTicket(uint32_t launched, uint32_t& dry, bool noDraws = false) const {
     if (!customOrder()) return workgroupIndex();
     const uint32_t b = workgroupIndex(), x = b & 7u, pos = b >> 3;
-    if (noDraws) return deal::onlyTicket(d.grid, launched, b);
-    if (pos < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, pos);
+    if (noDraws) return deal::onlyTicket(d.grid, launched, b, turn);
+    if (pos < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, pos, turn);
     return drawFinish(drawBegin(dry, noDraws), launched, 0, dry, noDraws);
   }
 

@@ -29,8 +29,13 @@ CUSYNC_HD uint32_t listStatic(const cusync_dim3& grid, uint32_t x, uint32_t laun
   const uint32_t wgs = listWorkgroups(x, launched), tiles = listTiles(grid, x);
   return wgs < tiles ? wgs : tiles;
 }
-// Ticket of position l of list x.
-CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l) {
+// Ticket of position l of list x.  `turn`: the list is begun that many positions further on.  A workgroup of a launch of
+// several GEMMs has the same position in each one's list, so without a turn the tiles it gets have much the same columns:
+// where the weights' rows are a multiple of 1 KiB apart all rows of a column tile lie in one class of memory channels, one
+// class in four is a quarter slower, and the workgroups that finish such a tile last would begin another one.  (GPT-3 MLP at
+// one row: 48 and 96 column tiles, lists of 6 and 12.)
+CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l, uint32_t turn = 0) {
+  if (turn) l = (l + turn) % listTiles(grid, x);
   const uint32_t span = byRows(grid) ? grid.y : grid.x;
   const uint32_t lo = x * span / 8, width = (x + 1) * span / 8 - lo;
   if (!byRows(grid)) return lo + l % width + (l / width) * grid.x;
@@ -43,7 +48,7 @@ CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l) {
 // workgroups beyond their own list's length take, in order, the positions that other lists have left over.  Drawn from
 // the dispensers instead, those workgroups began 2.5 us after the others, every workgroup paid two round trips to learn
 // that nothing is left, and the k-slices of a tile could not share their reduction (slicesShareReduction).
-CUSYNC_HD uint32_t leftOver(const cusync_dim3& grid, uint32_t launched, uint32_t b) {
+CUSYNC_HD uint32_t leftOver(const cusync_dim3& grid, uint32_t launched, uint32_t b, uint32_t turn = 0) {
   const uint32_t mine = b & 7u;
   uint32_t s = b / 8 - listTiles(grid, mine);        // how many workgroups without a place of their own come before this one
   for (uint32_t x = 0; x < mine; x++) {
@@ -53,14 +58,14 @@ CUSYNC_HD uint32_t leftOver(const cusync_dim3& grid, uint32_t launched, uint32_t
   for (uint32_t x = 0; x < 8; x++) {
     const uint32_t tiles = listTiles(grid, x), wgs = listWorkgroups(x, launched);
     const uint32_t left = tiles > wgs ? tiles - wgs : 0;
-    if (s < left) return listTicket(grid, x, wgs + s);
+    if (s < left) return listTicket(grid, x, wgs + s, turn);
     s -= left;
   }
   return kNoTicket;                                  // more workgroups than tiles
 }
 // The only ticket of workgroup b of such a launch.
-CUSYNC_HD uint32_t onlyTicket(const cusync_dim3& grid, uint32_t launched, uint32_t b) {
-  return b / 8 < listTiles(grid, b & 7u) ? listTicket(grid, b & 7u, b / 8) : leftOver(grid, launched, b);
+CUSYNC_HD uint32_t onlyTicket(const cusync_dim3& grid, uint32_t launched, uint32_t b, uint32_t turn = 0) {
+  return b / 8 < listTiles(grid, b & 7u) ? listTicket(grid, b & 7u, b / 8, turn) : leftOver(grid, launched, b, turn);
 }
 
 }  // namespace deal

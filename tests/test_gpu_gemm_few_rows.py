@@ -45,3 +45,59 @@ def test_one_row_tile_and_the_next(tile, rows, more, split_k):
     # up to `rows` rows the weights are read by one row tile (non-temporal loads), one row more and by two
     print("few rows", tile, rows + more, split_k, flush=True)
     exact_gemm(tile, rows + more, 328, 520, split_k)
+
+
+@pytest.mark.parametrize("tile", [api.TILE.D32x128x64, api.TILE.D64x128x64, api.TILE.D64x192x64])
+@pytest.mark.parametrize("K", [8, 64, 72, 200, 320, 392, 456])
+def test_fewer_chunks_than_stages(tile, K):
+    # the prologue sends out all of B's first chunks ahead of A's: one chunk of K, as many as the pipeline has stages, one more
+    print("few chunks", tile, K, flush=True)
+    exact_gemm(tile, 20, 328, K, 1)
+
+
+@pytest.mark.parametrize("policy_kind", ["row", "tile"])
+@pytest.mark.parametrize("tile", [api.TILE.D32x128x64, api.TILE.D64x128x64, api.TILE.D64x192x64])
+@pytest.mark.parametrize("K,N1,N2,split2", [(72, 328, 1992, 1), (72, 328, 33288, 1), (520, 1416, 4104, 2), (328, 2568, 520, 3)])
+def test_one_row_of_tiles_in_one_launch(policy_kind, tile, K, N1, N2, split2):
+    # two GEMMs of one row of tiles in one launch: the second one's lists begin a position further on, its weights are
+    # fetched before the first one's tiles are waited for (not with more tiles than CUs); lists of unequal length, N and K
+    # not multiples of the tile
+    import torch
+    L = _lib.load()
+    rows = api.tile_shape(tile)[0]
+    for M in (1, rows):
+        print("one launch", policy_kind, tile, M, K, N1, N2, split2, flush=True)
+        rng = np.random.default_rng(tile + M + K)
+        a, b = rng.integers(-1, 2, (M, K)).astype(np.float16), rng.integers(-1, 2, (K, N1)).astype(np.float16)
+        d = rng.integers(-1, 2, (N1, N2)).astype(np.float16)
+        da, db, dd = to_dev(a), to_dev(b), to_dev(d)
+        dc, de = empty_dev((M, N1), fill=float("nan")), empty_dev((M, N2), fill=float("nan"))
+        grids = [api.gemm_grid(tile, M, N1, 1), api.gemm_grid(tile, M, N2, split2)]
+        tm, tn, _ = api.tile_shape(tile)
+        pol = api.tile_sync(api.ORDER.TRANSPOSE_XY, tm, tn) if policy_kind == "tile" else api.row_sync(tm, grids[0][0])
+        st = [api.Stage(grids[0], (1, 1, 1), api.no_sync(), pol), api.Stage(grids[1], (1, 1, 1), pol, api.no_sync())]
+        assert api.set_producer_consumer_pair(st[0], st[1]) == api.ERR.SUCCESS
+        args = (_lib.GemmArgs * 2)(
+            api.gemm_args(st[0], M, N1, K, da.data_ptr(), K, db.data_ptr(), N1, dc.data_ptr(), N1, tile),
+            api.gemm_args(st[1], M, N2, N1, dc.data_ptr(), N1, dd.data_ptr(), N2, de.data_ptr(), N2, tile, split_k=split2))
+        ws = None
+        if split2 > 1:
+            ws = torch.zeros(L.cusync_gemm_workspace_size(C.byref(args[1])), dtype=torch.uint8, device="cuda")
+            args[1].workspace = ws.data_ptr()
+        c = a.astype(np.float64) @ b.astype(np.float64)
+        assert np.abs(c).max() < 2048          # exact in fp16
+        e = (c @ d.astype(np.float64)).astype(np.float16)
+        for it in range(3):
+            for t in (dc, de):
+                t.fill_(float("nan"))
+            torch.cuda.synchronize()
+            assert L.cusync_gemm_chain_run(args, 2, None) == api.ERR.SUCCESS, api.last_error()
+            assert L.cusync_rt_device_sync() == 0, api.last_error()
+            for k in range(2):
+                st[k].incrementIter()
+                args[k].stage = st[k].desc
+            assert np.array_equal(to_host(dc), c.astype(np.float16)) and np.array_equal(to_host(de), e), it
+        states = [s_.read_state() for s_ in st]
+        for s_ in st:
+            s_.destroy()
+        assert all(s_.spin_timeouts == 0 and s_.tile_counter == 0 for s_ in states)

@@ -1,5 +1,5 @@
 """How a launch of at least as many workgroups as tiles hands its tiles out (cusync_amd/csrc/tile_deal.h), host code only:
-every tile is exactly one workgroup's, whatever the grid, and the workgroups beyond the tiles get none."""
+every tile is exactly one workgroup's, whatever the grid, and the workgroups beyond the tiles get none; also where the lists are begun some positions further on, as those of a later GEMM of one launch are."""
 import os
 import subprocess
 
@@ -10,17 +10,17 @@ SRC = r"""
 #include <vector>
 #include "tile_deal.h"
 using namespace cusync::deal;
-static int check(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t more) {
+static int check(uint32_t gx, uint32_t gy, uint32_t gz, uint32_t more, uint32_t turn) {
   const cusync_dim3 grid = {gx, gy, gz};
   const uint32_t tiles = gx * gy * gz, launched = tiles + more;
   std::vector<int> taken(tiles, 0);
   uint32_t without = 0, inPlace = 0;
   for (uint32_t b = 0; b < launched; b++) {
-    const uint32_t t = onlyTicket(grid, launched, b);
+    const uint32_t t = onlyTicket(grid, launched, b, turn);
     if (t == kNoTicket) { without++; continue; }
     if (t >= tiles || taken[t]++) { std::printf("grid %u %u %u + %u: ticket %u of workgroup %u\n", gx, gy, gz, more, t, b); return 1; }
     // a workgroup within its list's length begins with its list's position, as in a launch of several rounds
-    if (b / 8 < listTiles(grid, b % 8)) { inPlace++; if (t != listTicket(grid, b % 8, b / 8)) { std::printf("grid %u %u %u: workgroup %u is not in its list\n", gx, gy, gz, b); return 1; } }
+    if (b / 8 < listTiles(grid, b % 8)) { inPlace++; if (t != listTicket(grid, b % 8, b / 8, turn)) { std::printf("grid %u %u %u: workgroup %u is not in its list\n", gx, gy, gz, b); return 1; } }
   }
   if (without != more) { std::printf("grid %u %u %u + %u: %u workgroups without a tile\n", gx, gy, gz, more, without); return 1; }
   return 0;
@@ -30,10 +30,11 @@ int main() {
     for (uint32_t gy = 1; gy <= 14; gy++)
       for (uint32_t gz = 1; gz <= 5; gz++)
         for (uint32_t more : {0u, 1u, 7u, 8u, 30u})
-          if (check(gx, gy, gz, more)) return 1;
+          for (uint32_t turn : {0u, 1u, 3u})
+            if (check(gx, gy, gz, more, turn)) return 1;
   // launches of the chains: 14 x 14 x 256 at batch 32, LLaMA's GEMM1, the QKV projection, attention, one column of 392 tiles
   const uint32_t chains[][3] = {{2, 49, 2}, {29, 4, 2}, {29, 8, 1}, {36, 1, 4}, {43, 1, 4}, {12, 1, 6}, {12, 4, 2}, {1, 392, 1}, {64, 4, 1}};
-  for (auto& c : chains) if (check(c[0], c[1], c[2], 0)) return 1;
+  for (auto& c : chains) for (uint32_t turn = 0; turn < 8; turn++) if (check(c[0], c[1], c[2], 0, turn)) return 1;
   std::printf("ok\n");
   return 0;
 }
