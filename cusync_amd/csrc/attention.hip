@@ -248,23 +248,35 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   L->E = cfg->heads * kHD;
   // Per-row-count choice, from the tuner's measurements (cusync_amd/tile_sizes_db.py, gpt3_attention_mi355x) and
   // sweeps between its row counts.  Widths that are multiples of 192 (4608 = 24 x 192, 12288 = 64 x 192) take the
-  // 192-wide direct-to-LDS tiles.  QKV projection (24 column tiles): 64x192x64 in k-slices while the projection
-  // streams the weights, up to 320 rows (five row tiles in two slices are 240 workgroups: 56 us against 69 for
-  // 128x192); 128x192 with a CU to itself up to 1024 rows, except from 641 to 768 rows, which are three whole row
-  // tiles of 256x192 in two slices (105 against 124 us); 256x192 above.  Output projection (64 column tiles):
-  // 64x192x64 up to 256 rows, 128x192 alone up to 512, 256x192 up to 1024, and above that 128x192 at two workgroups
-  // per CU, whose tiles fill the last round better (1280 rows: 79 -> 69 us, 1536: 80 -> 72, level at 2048).
+  // 192-wide direct-to-LDS tiles.  QKV projection (24 column tiles), in as many k-slices as fill the device
+  // (pickSplitToFill): 32x128 and 64x128 up to 32 and 64 rows, 64x192 up to 192, 128x192 up to 384, each with a CU to
+  // itself, 256x192 above.  Output projection (64 column tiles): 64x192x64 up to 256 rows, 128x192 alone up to 512,
+  // 256x192 up to 1024, and above that 128x192 at two workgroups per CU, whose tiles fill the last round better (1280
+  // rows: 79 -> 69 us, 1536: 80 -> 72, level at 2048).
   // Other widths: tiles that follow the row count up to 128 rows, 128x128 up to 1024 rows, 128x256 above.
   const int small = cfg->seq <= 32 ? CUSYNC_TILE_D32x128x64 : cfg->seq <= 64 ? CUSYNC_TILE_64x128x64 : CUSYNC_TILE_128x128x64;
   const int dflt = cfg->seq <= 128 ? small : cfg->seq <= 1024 ? CUSYNC_TILE_128x128x32 : CUSYNC_TILE_128x256x32;
   const uint32_t S = cfg->seq;
-  // (with the 256x192 tile's K loop in assembly, 256x192 in k-slices also leads from 321 to 512 rows and from 769 to
-  // 1024: the QKV projection 73 -> 67 us at 384 rows, 131 -> 115 at 896, 137 -> 120 at 1024; from 513 to 640 rows its
-  // third row tile is mostly padding and 128x192 stays, 87 against 102 us)
+  // A tile is taken early or late where its k-slices bring four fifths of the CUs to work and the neighbour's do not (us):
+  // 64x128 up to 64 rows against 64x192 in eight slices, 48 rows 32.0 -> 29.6, 64 rows 32.5 -> 30.6; 128x192x64 from 257 to
+  // 384 rows, three row tiles in three slices, against 64x192 in two up to 320 rows (270 rows 65.5 -> 59.0) and 256x192 in
+  // four above (384 rows 69.2 -> 62.0); 256x192 from 513 rows, three slices of three row tiles, against 128x192 with a CU to
+  // itself in two (600 rows 100 -> 89) and against two slices of its own (768 rows 108 -> 92).  Where it does not fill,
+  // the narrower rule stays: 64x192 up to 320 rows, 128x192 alone from 513 to 640.
   // (two full row tiles of 128, 193 to 256 rows: 128x192 with the operands fetched 64 columns of K at a time, the QKV
-  // projection 55 -> 52 us at 256 rows, 51 -> 49.5 at 224; level below, and at 320 rows its third row tile costs 17 us)
-  const int wide1 = S <= 32 ? small : S > 192 && S <= 256 && cfg->hidden % 64 == 0 ? CUSYNC_TILE_D128x192x64
-                    : S <= 320 ? CUSYNC_TILE_D64x192x64 : S > 512 && S <= 640 ? CUSYNC_TILE_128x192x32_ALONE
+  // projection 55 -> 52 us at 256 rows, 51 -> 49.5 at 224; level below)
+  auto workgroups = [&](int tile) {
+    uint32_t tm = 0, bk = 0;
+    cusync_gemm_tile_shape(tile, &tm, nullptr, &bk);
+    const cusync_dim3 flat = cusync_gemm_grid(tile, S, 3 * L->E, 1);
+    return flat.x * flat.y * (uint32_t)cusync::gemm::pickSplitToFill(flat.x * flat.y, tm, cfg->hidden, bk, cusync_gemm_max_resident(tile));
+  };
+  auto fills = [&](int tile) { const uint32_t n = workgroups(tile); return n * 5 >= 256 * 4 && n <= 256; };
+  const bool lines = cfg->hidden % 64 == 0;
+  const bool widthsAgree = cfg->sync != CUSYNC_SYNC_STRIDED || L->E % 192 == 0;     // (ConsecutiveSync refuses the same widths whichever tile is taken)
+  const int wide1 = S <= 32 ? small : S <= 64 ? (!fills(CUSYNC_TILE_D64x192x64) && fills(CUSYNC_TILE_D64x128x64) && widthsAgree ? CUSYNC_TILE_D64x128x64 : CUSYNC_TILE_D64x192x64)
+                    : S <= 192 ? CUSYNC_TILE_D64x192x64 : S <= 384 && lines && (S <= 256 || fills(CUSYNC_TILE_D128x192x64)) ? CUSYNC_TILE_D128x192x64
+                    : S <= 320 ? CUSYNC_TILE_D64x192x64 : S > 512 && S <= 640 && !fills(CUSYNC_TILE_256x192x32) ? CUSYNC_TILE_128x192x32_ALONE
                     : CUSYNC_TILE_256x192x32;
   const int wide3 = S <= 32 ? small : S <= 256 ? CUSYNC_TILE_D64x192x64 : S <= 512 ? CUSYNC_TILE_128x192x32_ALONE
                     : S <= 1024 ? CUSYNC_TILE_256x192x32 : CUSYNC_TILE_128x192x32;
@@ -274,6 +286,8 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   L->tile3 = cfg->tile3 >= 0 ? cfg->tile3 : cfg->hidden % 192 == 0 ? inLines(wide3, L->E) : dflt;
   // (above 1024 rows the output projection's five to eight row tiles of 256x384, at most one per CU, beat 128x192 at
   // two workgroups per CU: the chain under RowSync 216 -> 212 us at 1280 rows, 267 -> 255 at 1536, 327 -> 311 at 2048)
+  if (cfg->tile1 < 0 && L->tile1 == CUSYNC_TILE_256x192x64 && (3 * L->E) % 384 == 0 &&
+      cusync::gemm::wideInThreeSlices(3 * L->E / 384 * ((S + 255) / 256), cfg->hidden, cusync_gemm_max_resident(CUSYNC_TILE_256x384x32))) L->tile1 = CUSYNC_TILE_256x384x32;
   if (cfg->tile3 < 0 && S > 1024 && cfg->hidden % 384 == 0 && L->E % 64 == 0) L->tile3 = CUSYNC_TILE_256x384x32;
   L->ws1 = L->ws3 = L->ws2 = nullptr;
   // Key ranges of 8 blocks (512 rows) or more are cut in two: under a causal mask the last row tiles walk the
@@ -313,7 +327,7 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   cusync_gemm_tile_shape(L->tile3, nullptr, nullptr, &bk3);
   const cusync_dim3 flat1 = cusync_gemm_grid(L->tile1, cfg->seq, 3 * L->E, 1);
   const cusync_dim3 flat3 = cusync_gemm_grid(L->tile3, cfg->seq, cfg->hidden, 1);
-  L->split1 = cusync::gemm::pickSplit(0, flat1.x * flat1.y, cfg->hidden, bk1, cusync_gemm_max_resident(L->tile1));
+  L->split1 = cusync::gemm::pickSplitToFill(flat1.x * flat1.y, tm1, cfg->hidden, bk1, cusync_gemm_max_resident(L->tile1));
   L->split3 = cusync::gemm::pickSplit(0, flat3.x * flat3.y, L->E, bk3, cusync_gemm_max_resident(L->tile3));
   const cusync_dim3 g1 = cusync_gemm_grid(L->tile1, cfg->seq, 3 * L->E, L->split1);
   const cusync_dim3 g2 = cusync_attention_grid_split(cfg->seq, cfg->heads, cfg->cached_rows, L->kvSplit);

@@ -413,11 +413,12 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
   constexpr uint32_t kPieces = C::TM * C::WM;                                   // 32-row pieces of a tile
   constexpr uint32_t kEpiBytes = (C::WM * 32 * (C::BN * 2 + 16) + 1023) / 1024 * 1024;
   constexpr uint32_t kPieceBytes = C::WN * C::TN * 4 * 1024;                    // 32 rows x BN columns of fp32
-  const uint32_t perSlice = C::BM >= 128 && p.coopReduce ? kPieces / p.splitK : 0;
-  const bool ownInLds = C::BM >= 128 && p.coopReduce && kEpiBytes + perSlice * kPieceBytes <= (uint32_t)C::LDS_BYTES;
-  auto ownedPiece = [&](int i) { return ((uint32_t)i * C::WM + (uint32_t)wm) / (perSlice ? perSlice : 1u) == t.z; };      // uniform per wavefront; asked under the shared reduction only
+  const bool shared = C::BM >= 128 && p.coopReduce;
+  const uint32_t firstPiece = shared ? t.z * kPieces / p.splitK : 0, endPiece = shared ? (t.z + 1) * kPieces / p.splitK : 0;
+  const bool ownInLds = shared && kEpiBytes + (kPieces + p.splitK - 1) / p.splitK * kPieceBytes <= (uint32_t)C::LDS_BYTES;
+  auto ownedPiece = [&](int i) { const uint32_t u = (uint32_t)i * C::WM + (uint32_t)wm; return u >= firstPiece && u < endPiece; };      // uniform per wavefront; asked under the shared reduction only
   auto ownSlot = [&](int i, int j, int g) {
-    const uint32_t o = (uint32_t)i * C::WM + (uint32_t)wm - t.z * perSlice;
+    const uint32_t o = (uint32_t)i * C::WM + (uint32_t)wm - firstPiece;
     return lds + kEpiBytes + ((o * C::WN + (uint32_t)wn) * (C::TN * 4) + (uint32_t)(j * 4 + g)) * 1024 + (uint32_t)lane * 16;
   };
   if (ownInLds) __syncthreads();         // every wavefront is out of the main loop and its loads have landed
@@ -440,10 +441,10 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
   uint32_t* counter = p.arrivals + tileIndex;
 
   // (the launcher shares the reduction only among tiles of 128 rows and more: the smaller ones do not carry the code)
-  if (C::BM >= 128 && p.coopReduce) {
+  if (shared) {
     // ---- every slice adds up and stores its share ---------------------------------------------------------
     // The tile is cut into BM/32 pieces of 32 rows (piece u = i * WM + wm: MFMA row tile i of wave row wm); slice z
-    // takes the pieces [z * U/S, (z + 1) * U/S).  A piece is summed over the slices in index order (this slice's
+    // takes the pieces [z * U/S, (z + 1) * U/S), of unequal number where S does not divide U.  A piece is summed over the slices in index order (this slice's
     // own term read back like the others: see above), so the result is the same, bit for bit, whichever way and
     // in whatever order of arrival the tile is put together.
     uint32_t* departures = p.arrivals + p.stage.d.grid.x * p.stage.d.grid.y + tileIndex;
@@ -458,7 +459,6 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
 #pragma unroll 1
     for (int i = 0; i < C::TM; i++) {
       const bool owned = ownedPiece(i);
-      const uint32_t firstPiece = t.z * perSlice, endPiece = firstPiece + perSlice;
       // wave rows of this pass that belong to this slice
       uint32_t rows = 0;
 #pragma unroll

@@ -48,6 +48,8 @@ namespace {
 
 using cusync::rt::setError;
 using cusync::gemm::pickSplit;
+using cusync::gemm::pickSplitToFill;
+using cusync::gemm::wideInThreeSlices;
 using cusync::gemm::half_t;
 using cusync::gemm::uint4v;
 
@@ -265,6 +267,9 @@ void pickTiles(const cusync_mlp_config& c, int sync, bool swiglu, bool fused, in
   // (1025 to 1536 rows, five or six row tiles: 160 or 192 tiles of 256x384 in one round against 128x192 at two
   // workgroups per CU in one and a half: 1056 rows 397 -> 347 us, 1152: 404 -> 353, 1280: 407 -> 365, 1536: 444 -> 400)
   if (big && c.batch > 1024 && !swiglu && k2 % 64 == 0 && n2 % 384 == 0 && !c.one_launch) b = CUSYNC_TILE_256x384x32;
+  // (five row tiles, 1025 to 1280 rows: GEMM1 in three slices of 256x384, see wideInThreeSlices)
+  if (a == CUSYNC_TILE_256x192x64 && n1 % 384 == 0 && !c.one_launch && c.split_k1 <= 0 && sync != CUSYNC_SYNC_STRIDED &&
+      wideInThreeSlices(n1 / 384 * ((c.batch + 255) / 256), k1, cusync_gemm_max_resident(CUSYNC_TILE_256x384x32))) a = CUSYNC_TILE_256x384x32;
   *t1 = c.tile1 >= 0 ? c.tile1 : a;
   *t2 = c.tile2 >= 0 ? c.tile2 : b;
   // both GEMMs in one launch share a kernel: the consumer takes the producer's tile
@@ -336,8 +341,8 @@ bool choose(const cusync_mlp_config& given, Choice* o) {
   // the LLaMA shard, whose GEMM2 wants a tile of its own, but for StridedSync up to 32 rows, where both take 32x128) and
   // the tiles are the table's.  LLaMA under StridedSync, by the device's clock in us, two launches -> one, inner 2752 /
   // 2816: 1 row 37.3 -> 34.7 / 39.2 -> 36.1, 16 rows 38.3 -> 35.3 / 40.2 -> 37.0, 32 rows 39.2 -> 36.4 / 41.6 -> 38.3.
-  // The other two policies keep their two launches, though one is ahead of them as well: 16 rows, inner 2752, TileSync
-  // 39.5 -> 36.2 (a pass by the host's clock 47.7 -> 45.4), RowSync 39.3 -> 37.1 (47.2 -> 46.3).
+  // The other two policies keep their two launches: with GEMM1 in five slices there is nothing left to gain (20 rows, a pass
+  // by the host's clock: TileSync in two launches 44.8, StridedSync in one 45.0).
   const bool automatic = c.one_launch < 0;
   if (automatic) c.one_launch = c.sync != CUSYNC_SYNC_STREAM && c.tile1 < 0 && c.tile2 < 0 &&
                                 (llama ? c.sync == CUSYNC_SYNC_STRIDED && c.batch <= 32 : c.batch <= 64 || (c.batch >= 512 && c.batch <= 1024));
@@ -362,14 +367,14 @@ bool choose(const cusync_mlp_config& given, Choice* o) {
     o->oneLaunch = false;
     pickTiles(c, o->sync, o->aMode2 == CUSYNC_A_SWIGLU, o->fused, &o->tile1, &o->tile2);
   }
-  uint32_t bk1 = 0, bk2 = 0;
-  if (cusync_gemm_tile_shape(o->tile1, nullptr, nullptr, &bk1) || cusync_gemm_tile_shape(o->tile2, nullptr, nullptr, &bk2)) {
+  uint32_t tm1 = 0, bk1 = 0, bk2 = 0;
+  if (cusync_gemm_tile_shape(o->tile1, &tm1, nullptr, &bk1) || cusync_gemm_tile_shape(o->tile2, nullptr, nullptr, &bk2)) {
     setError("mlp: unknown tile id");
     return false;
   }
   const cusync_dim3 flat1 = cusync_gemm_grid(o->tile1, c.batch, n1, 1);
   const cusync_dim3 flat2 = cusync_gemm_grid(o->tile2, c.batch, n2, 1);
-  o->split1 = pickSplit(c.split_k1, flat1.x * flat1.y, k1, bk1, cusync_gemm_max_resident(o->tile1));
+  o->split1 = c.split_k1 > 0 ? c.split_k1 : pickSplitToFill(flat1.x * flat1.y, tm1, k1, bk1, cusync_gemm_max_resident(o->tile1));
   o->split2 = pickSplit(c.split_k2, flat2.x * flat2.y, k2, bk2, cusync_gemm_max_resident(o->tile2));
   return true;
 }

@@ -29,17 +29,51 @@ inline int pickSplit(int requested, uint32_t tiles, uint32_t K, uint32_t bk, int
   return s;
 }
 
+// The same for GEMMs whose columns do not come in powers of two (the attention chain's QKV projection: 36 column tiles of
+// 128, 24 of 192).  Doubling stops at half to three quarters of the CUs there, so single slices are added until four
+// fifths of the CUs have work.  From eight slices on it does not pay: what they add up grows with every slice (48 rows on
+// 64x192 tiles, 24 of them: 31.9 / 32.3 / 33.1 us with 8 / 9 / 10).  QKV projection, doubling -> this: 16 rows (36 tiles, 4 -> 6
+// slices) 29.7 -> 26.0 us, 128 rows (48, 4 -> 5) 43.9 -> 40.5, 190 rows (72, 2 -> 3) 67.4 -> 51.9, 768 rows (72, 2 -> 3)
+// 108.0 -> 93.7; level between four and seven slices once 200 CUs are busy (36 tiles, 16 rows: 26.9 / 26.0 / 26.1 us with 5 / 6 / 7).
+// Nor from four slices on where the tiles have 128 rows and more and the slices share the reduction: five of them share it
+// unevenly (48 tiles, the attention chain in stream order: 256 rows 102.6 us with four, 106.6 with five; 512 rows 137.5, 141.5).
+inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t bk, int resident) {
+  const uint32_t target = (uint32_t)std::min(resident, 256);
+  uint32_t s = (uint32_t)pickSplit(0, tiles, K, bk, resident);
+  if (tileM >= 128 && s >= 4) return (int)s;
+  for (uint32_t more = s + 1; s < 8 && tiles * s * 5 < target * 4 && more < 8 && tiles * more <= target && K / more >= 8 * bk; more++)
+    if (everySliceHasAChunk(K, bk, more)) s = more;
+  return (int)s;
+}
+
+// Whether 256x384 tiles in three slices take over from 256x192 tiles in one: where the 256x192 tiles are too many for two
+// slices on 256 CUs and leave a fifth of them or more idle in one (137 to 170 of them), half as many tiles in three slices
+// keep four fifths or more busy, with two thirds of the work each and less of it loads.  `tiles`: of 256x384.  GEMMs of
+// 256x192 -> 256x384, us: 12 288 to 4 608 columns (12 tiles of 384), 1300 rows 186 -> 154, 1500: 190 -> 167, 1700: 200 -> 194;
+// to 6 144 columns, 1100 rows 191 -> 172, 1280: 200 -> 181.  Outside that range it falls behind (6 144 columns, 1500 rows, 96
+// tiles in two slices: 215 -> 220).  Every slice has to be a whole number of 64 columns of K long.
+inline bool wideInThreeSlices(uint32_t tiles, uint32_t K, int resident) {
+  const uint32_t per = (K / 32 + 2) / 3 * 32;
+  return resident >= 256 && tiles * 3 <= 256 && tiles * 3 * 5 >= 256 * 4 && tiles * 2 * 2 > 256 && K % 64 == 0 && per % 64 == 0 && everySliceHasAChunk(K, 32, 3);
+}
+
 // Whether the k-slices of a tile add it up together (each waits for its siblings, then sums and stores a share of
 // the tile) instead of leaving all of it to the slice that arrives last.  The waiting slices hold their CUs, so
 // every slice of the launch must have a workgroup of its own from the start (one round, all of them dealt a
 // static first tile) and nothing may keep a sibling off the device: under AvoidWaitKernel the consumer's launch
 // can reach the device before its producer's and take the slots the siblings need, the resident slices would
 // spin until their bound runs out, so there the last-arriver form is kept, whose workgroups retire and free
-// their slots.  Tiles of 128 rows and more whose 32-row pieces divide among the slices only.
+// their slots.  Tiles of 128 rows and more with a 32-row piece for every slice only.
+inline bool slicesCanShareReduction(int splitK, bool requested, bool directToLdsTile, bool everyTileStatic, uint32_t launched,
+                                    uint32_t tiles, uint32_t tileM, bool avoidWaitKernel) {
+  return splitK > 1 && requested && directToLdsTile && everyTileStatic && launched == tiles && tileM >= 128 &&
+         tileM / 32 >= (uint32_t)splitK && !avoidWaitKernel;
+}
+// The same for a kernel whose pieces have to divide among the slices (the 3x3 convolution's runs).
 inline bool slicesShareReduction(int splitK, bool requested, bool directToLdsTile, bool everyTileStatic, uint32_t launched,
                                  uint32_t tiles, uint32_t tileM, bool avoidWaitKernel) {
-  return splitK > 1 && requested && directToLdsTile && everyTileStatic && launched == tiles && tileM >= 128 &&
-         (tileM / 32) % (uint32_t)splitK == 0 && !avoidWaitKernel;
+  return slicesCanShareReduction(splitK, requested, directToLdsTile, everyTileStatic, launched, tiles, tileM, avoidWaitKernel) &&
+         (tileM / 32) % (uint32_t)splitK == 0;
 }
 
 }  // namespace gemm

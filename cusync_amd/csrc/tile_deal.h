@@ -47,7 +47,7 @@ CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l, u
 // the lists do not come out even (98 tiles of a convolution: lists of 12 to 14 for 12 or 13 workgroups each) the
 // workgroups beyond their own list's length take, in order, the positions that other lists have left over.  Drawn from
 // the dispensers instead, those workgroups began 2.5 us after the others, every workgroup paid two round trips to learn
-// that nothing is left, and the k-slices of a tile could not share their reduction (slicesShareReduction).
+// that nothing is left, and the k-slices of a tile could not share their reduction (slicesCanShareReduction).
 CUSYNC_HD uint32_t leftOver(const cusync_dim3& grid, uint32_t launched, uint32_t b, uint32_t turn = 0) {
   const uint32_t mine = b & 7u;
   uint32_t s = b / 8 - listTiles(grid, mine);        // how many workgroups without a place of their own come before this one

@@ -181,6 +181,20 @@ def test_attention_layer_gpt3_shard(S):
     check_layer(S, 12288, 12, sampled=True)
 
 
+# the first and last rows of the ranges in which the projection takes another tile or number of k-slices
+@pytest.mark.parametrize("S", [33, 64, 190, 257, 384, 513, 640, 1281, 1792])
+def test_attention_layer_where_the_projection_changes_tiles(S):
+    print("attn layer edges", S, flush=True)
+    check_layer(S, 12288, 12, sampled=True)
+
+
+# other widths, where those tiles do not fill the device or only some of them do
+@pytest.mark.parametrize("S,hidden,heads", [(48, 2048, 9), (300, 4096, 15), (600, 2048, 3), (1300, 2048, 12)])
+def test_attention_layer_of_other_widths(S, hidden, heads):
+    print("attn layer widths", S, hidden, heads, flush=True)
+    check_layer(S, hidden, heads, sampled=True)
+
+
 # ---- key/value cache variant (src/ml-bench/transformer/attention.cu:265-276, 289) ----------------
 
 def run_attention_kv(qkv, cached, heads, causal=True):

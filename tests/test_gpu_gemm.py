@@ -158,7 +158,7 @@ def test_gemm_split_k(tile, split):
                                         (api.TILE.D128x192x64, 2), (api.TILE.D128x192x64, 4)])      # as the 256-row MLP runs it
 def test_gemm_split_k_with_the_reduction_shared_among_the_slices(tile, split):
     # every k-slice has a workgroup of its own, so the slices of a tile each add up and store a share of it (where
-    # the tile has 128 rows or more and its 32-row pieces divide among them: not for 3 slices, not for the 64- and
+    # the tile has 128 rows or more and a 32-row piece for each of them: not for the 64- and
     # 32-row tiles, which fall back to the last slice doing all of it).  Same sums in the same order: bit-identical to the unshared reduction, launch
     # after launch (the counters re-arm), ragged edges included.
     print("shared reduction tile", tile, "slices", split, flush=True)
@@ -169,6 +169,20 @@ def test_gemm_split_k_with_the_reduction_shared_among_the_slices(tile, split):
     shared = run_gemm(a, b, tile, split_k=split, epilogue=api.EPI.GELU, shared_reduction=1, launches=3)
     assert np.array_equal(plain.view(np.uint16), shared.view(np.uint16))
     assert_close(shared, orc.gemm(a, b, orc.EPI_GELU), "shared reduction, %d slices, tile %d" % (split, tile))
+
+
+@pytest.mark.parametrize("tile,split", [(api.TILE.T256x192x64, 3), (api.TILE.T256x192x64, 5), (api.TILE.T256x192x64, 7), (api.TILE.T256x384x32, 3),
+                                        (api.TILE.D128x192x64, 3), (api.TILE.T256x256x32, 6)])
+def test_gemm_shared_reduction_of_unequal_shares(tile, split):
+    # the tile's eight (four) 32-row pieces do not divide among the slices: some add up one more than others
+    print("unequal shares tile", tile, "slices", split, flush=True)
+    M, N, K = 300, 392, 2048
+    a = uniform_f16((M, K), 33)
+    b = normal_f16((K, N), 34, std=0.05)
+    plain = run_gemm(a, b, tile, split_k=split)
+    shared = run_gemm(a, b, tile, split_k=split, shared_reduction=1, launches=3)
+    assert np.array_equal(plain.view(np.uint16), shared.view(np.uint16))
+    assert_close(shared, orc.gemm(a, b), "unequal shares, %d slices, tile %d" % (split, tile))
 
 
 @pytest.mark.parametrize("tile,M,N,split", [(api.TILE.D128x192x64, 300, 9 * 192, 2), (api.TILE.T256x192x64, 1000, 13 * 192, 4),

@@ -120,6 +120,10 @@ def test_gpt3_mlp_full_size(batch):
         assert np.array_equal(prod.sems, expected_sems(prod, tiles, 3)) and prod.kernel_executed == 3
 
 
+def test_gpt3_mlp_of_five_row_tiles():
+    test_gpt3_mlp_full_size(1025)       # GEMM1 in three k-slices of 256x384, the last row tile of one row
+
+
 def test_gpt3_without_activation_matches_reference_check_build():
     # the reference's --check build has no GeLU (TB/mlp.cu:148-151)
     x, w1, w2, h, y, _, _, _, _ = run_mlp(api.MODEL.GPT3, 64, sync=api.SYNC.TILE, activation=0, **GPT3)

@@ -76,3 +76,57 @@ def test_split_choice(tmp_path):
     # the slices of a tile wait for each other only where nothing can keep a sibling off the device: never for a stage
     # under AvoidWaitKernel, whose consumer may be dispatched ahead of its producer
     assert shares == [1, 0, 0, 0, 0, 0, 0, 0, 0]
+
+
+FILL = r"""
+#include <cstdio>
+#include "split_choice.h"
+using namespace cusync::gemm;
+int main() {
+  for (uint32_t tiles = 1; tiles <= 300; tiles++)
+    for (uint32_t K : {64u, 1536u, 2752u, 6144u, 8192u, 12288u})
+      for (int resident : {0, 256, 512})
+        for (uint32_t tileM : {64u, 256u})
+          std::printf("F %u %u %d %u %d %d\n", tiles, K, resident, tileM, pickSplit(0, tiles, K, 64, resident), pickSplitToFill(tiles, tileM, K, 64, resident));
+  for (uint32_t tiles = 1; tiles <= 300; tiles++)
+    for (uint32_t K : {64u, 96u, 2752u, 4096u, 8192u, 12288u}) std::printf("W %u %u %d %d\n", tiles, K, wideInThreeSlices(tiles, K, 256) ? 1 : 0, wideInThreeSlices(tiles, K, 0) ? 1 : 0);
+  for (int slices = 1; slices <= 10; slices++)
+    for (uint32_t tileM : {32u, 64u, 128u, 256u})
+      std::printf("S %d %u %d %d\n", slices, tileM, slicesCanShareReduction(slices, true, true, true, 240, 240, tileM, false) ? 1 : 0,
+                  slicesCanShareReduction(slices, true, true, true, 240, 240, tileM, true) || slicesCanShareReduction(slices, false, true, true, 240, 240, tileM, false) ||
+                  slicesCanShareReduction(slices, true, false, true, 240, 240, tileM, false) || slicesCanShareReduction(slices, true, true, false, 240, 240, tileM, false) ||
+                  slicesCanShareReduction(slices, true, true, true, 200, 240, tileM, false) ? 1 : 0);
+}
+"""
+
+
+def test_slices_that_fill_the_device(tmp_path):
+    src = tmp_path / "fill_test.cpp"
+    src.write_text(FILL)
+    exe = tmp_path / "fill_test"
+    subprocess.check_call(["g++", "-std=c++17", "-Wall", "-I", os.path.join(ROOT, "cusync_amd", "csrc"), str(src), "-o", str(exe)])
+    lines = [f.split() for f in subprocess.check_output([str(exe)], text=True).split("\n") if f]
+    fill = {}
+    for f in lines:
+        v = [int(x) for x in f[1:]]
+        if f[0] == "F":
+            tiles, K, resident, tileM, doubled, got = v
+            fill[(tiles, K, resident, tileM)] = got
+            assert doubled <= got and (got == doubled or got < 8) and (got == doubled or doubled < 4 or tileM < 128)
+            if got != doubled:                                # never a second round, never without need, never a slice without work
+                assert tiles * got <= min(resident, 256) and tiles * (got - 1) * 5 < min(resident, 256) * 4 and K >= 8 * 64 * got
+            chunks = -(-K // 64)
+            assert (got - 1) * -(-chunks // got) < chunks
+        elif f[0] == "W":
+            tiles, K, got, without = v
+            per = -(-K // 32 // 3) * 32
+            assert not without and (not got or (205 <= tiles * 3 <= 256 and tiles * 4 > 256 and per % 64 == 0 and 2 * per < K))
+            if K == 12288:
+                assert got == int(69 <= tiles <= 85)
+        else:
+            assert v[2] == int(1 < v[0] <= v[1] // 32 and v[1] >= 128) and not v[3]
+    # the QKV projection's 36 and 24 column tiles, LLaMA's 43, and launches the doubling fills already
+    want = {(36, 12288): 6, (48, 12288): 5, (72, 12288): 3, (96, 12288): 2, (24, 12288): 8, (120, 12288): 2, (43, 8192): 5, (58, 8192): 4, (64, 6144): 4}
+    for (tiles, K), s in want.items():
+        assert fill[(tiles, K, 256, 64)] == s, (tiles, K)
+    assert fill[(48, 12288, 256, 256)] == 4 and fill[(72, 12288, 256, 256)] == 3
