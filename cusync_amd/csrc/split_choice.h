@@ -37,12 +37,13 @@ inline int pickSplit(int requested, uint32_t tiles, uint32_t K, uint32_t bk, int
 // 108.0 -> 93.7; level between four and seven slices once 200 CUs are busy (36 tiles, 16 rows: 26.9 / 26.0 / 26.1 us with 5 / 6 / 7).
 // Nor from four slices on where the tiles have 128 rows and more and the slices share the reduction: five of them share it
 // unevenly (48 tiles, the attention chain in stream order: 256 rows 102.6 us with four, 106.6 with five; 512 rows 137.5, 141.5).
+// (A slice is a whole number of 64 columns of K long: the 256x384x32 tile takes no other.)
 inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t bk, int resident) {
   const uint32_t target = (uint32_t)std::min(resident, 256);
   uint32_t s = (uint32_t)pickSplit(0, tiles, K, bk, resident);
   if (tileM >= 128 && s >= 4) return (int)s;
   for (uint32_t more = s + 1; s < 8 && tiles * s * 5 < target * 4 && more < 8 && tiles * more <= target && K / more >= 8 * bk; more++)
-    if (everySliceHasAChunk(K, bk, more)) s = more;
+    if (everySliceHasAChunk(K, bk, more) && ((K + bk - 1) / bk + more - 1) / more * bk % 64 == 0) s = more;
   return (int)s;
 }
 

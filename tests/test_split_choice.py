@@ -89,6 +89,11 @@ int main() {
         for (uint32_t tileM : {64u, 256u})
           std::printf("F %u %u %d %u %d %d\n", tiles, K, resident, tileM, pickSplit(0, tiles, K, 64, resident), pickSplitToFill(tiles, tileM, K, 64, resident));
   for (uint32_t tiles = 1; tiles <= 300; tiles++)
+    for (uint32_t K = 64; K <= 16384; K += 64) {       // 32 columns of K to a chunk, as the 256x384 tile has
+      const int doubled = pickSplit(0, tiles, K, 32, 256), got = pickSplitToFill(tiles, 256, K, 32, 256);
+      if (got != doubled && (K / 32 + got - 1) / got * 32 % 64) std::printf("B %u %u %d\n", tiles, K, got);
+    }
+  for (uint32_t tiles = 1; tiles <= 300; tiles++)
     for (uint32_t K : {64u, 96u, 2752u, 4096u, 8192u, 12288u}) std::printf("W %u %u %d %d\n", tiles, K, wideInThreeSlices(tiles, K, 256) ? 1 : 0, wideInThreeSlices(tiles, K, 0) ? 1 : 0);
   for (int slices = 1; slices <= 10; slices++)
     for (uint32_t tileM : {32u, 64u, 128u, 256u})
@@ -117,6 +122,8 @@ def test_slices_that_fill_the_device(tmp_path):
                 assert tiles * got <= min(resident, 256) and tiles * (got - 1) * 5 < min(resident, 256) * 4 and K >= 8 * 64 * got
             chunks = -(-K // 64)
             assert (got - 1) * -(-chunks // got) < chunks
+        elif f[0] == "B":
+            assert False, "a slice that is not a whole number of 64 columns: %s" % f
         elif f[0] == "W":
             tiles, K, got, without = v
             per = -(-K // 32 // 3) * 32
