@@ -52,10 +52,12 @@ inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t 
 // keep four fifths or more busy, with two thirds of the work each and less of it loads.  `tiles`: of 256x384.  GEMMs of
 // 256x192 -> 256x384, us: 12 288 to 4 608 columns (12 tiles of 384), 1300 rows 186 -> 154, 1500: 190 -> 167, 1700: 200 -> 194;
 // to 6 144 columns, 1100 rows 191 -> 172, 1280: 200 -> 181.  Outside that range it falls behind (6 144 columns, 1500 rows, 96
-// tiles in two slices: 215 -> 220).  Every slice has to be a whole number of 64 columns of K long.
+// tiles in two slices: 215 -> 220).  The launch takes its slice count from pickSplitToFill, which has to make it three: with
+// K below 768 or three slices that are not whole numbers of 64 columns it gives one or two, which is another launch than the
+// one measured, or one the tile refuses (K = 576: two slices of nine chunks).
 inline bool wideInThreeSlices(uint32_t tiles, uint32_t K, int resident) {
-  const uint32_t per = (K / 32 + 2) / 3 * 32;
-  return resident >= 256 && tiles * 3 <= 256 && tiles * 3 * 5 >= 256 * 4 && tiles * 2 * 2 > 256 && K % 64 == 0 && per % 64 == 0 && everySliceHasAChunk(K, 32, 3);
+  return resident >= 256 && tiles * 3 <= 256 && tiles * 3 * 5 >= 256 * 4 && tiles * 2 * 2 > 256 && K % 64 == 0 &&
+         pickSplitToFill(tiles, 256, K, 32, resident) == 3;
 }
 
 // Whether the k-slices of a tile add it up together (each waits for its siblings, then sums and stores a share of

@@ -124,6 +124,15 @@ def test_gpt3_mlp_of_five_row_tiles():
     test_gpt3_mlp_full_size(1025)       # GEMM1 in three k-slices of 256x384, the last row tile of one row
 
 
+@pytest.mark.parametrize("hidden", [576, 704, 768])
+def test_gpt3_mlp_of_five_row_tiles_and_a_short_k(hidden):
+    # the fewest columns of K that 256x384 takes three slices of, and two K below it, whose GEMM1 has to take another tile
+    print("short k", hidden, flush=True)
+    x, w1, w2, h, y, prod, cons, tiles, _ = run_mlp(api.MODEL.GPT3, 1100, hidden, 6144, api.SYNC.ROW)
+    assert cons.spin_timeouts == 0 and (tiles[0] == api.TILE.T256x384x32) == (hidden == 768)
+    check_against_oracle(api.MODEL.GPT3, x, w1, w2, h, y, 6144)
+
+
 def test_gpt3_without_activation_matches_reference_check_build():
     # the reference's --check build has no GeLU (TB/mlp.cu:148-151)
     x, w1, w2, h, y, _, _, _, _ = run_mlp(api.MODEL.GPT3, 64, sync=api.SYNC.TILE, activation=0, **GPT3)

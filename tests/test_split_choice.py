@@ -94,6 +94,11 @@ int main() {
       if (got != doubled && (K / 32 + got - 1) / got * 32 % 64) std::printf("B %u %u %d\n", tiles, K, got);
     }
   for (uint32_t tiles = 1; tiles <= 300; tiles++)
+    for (uint32_t K = 32; K <= 16384; K += 32) {       // the launch takes its slice count from pickSplitToFill: it has to be the three the tile was chosen for
+      const int got = pickSplitToFill(tiles, 256, K, 32, 256);
+      if (wideInThreeSlices(tiles, K, 256) && (got != 3 || K % 64 || (K / 32 + 2) / 3 % 2)) std::printf("B %u %u %d\n", tiles, K, got);
+    }
+  for (uint32_t tiles = 1; tiles <= 300; tiles++)
     for (uint32_t K : {64u, 96u, 2752u, 4096u, 8192u, 12288u}) std::printf("W %u %u %d %d\n", tiles, K, wideInThreeSlices(tiles, K, 256) ? 1 : 0, wideInThreeSlices(tiles, K, 0) ? 1 : 0);
   for (int slices = 1; slices <= 10; slices++)
     for (uint32_t tileM : {32u, 64u, 128u, 256u})
@@ -123,7 +128,7 @@ def test_slices_that_fill_the_device(tmp_path):
             chunks = -(-K // 64)
             assert (got - 1) * -(-chunks // got) < chunks
         elif f[0] == "B":
-            assert False, "a slice that is not a whole number of 64 columns: %s" % f
+            assert False, "256x384x32: slices that are not whole numbers of 64 columns, or not the three the tile was chosen for: %s" % f
         elif f[0] == "W":
             tiles, K, got, without = v
             per = -(-K // 32 // 3) * 32
