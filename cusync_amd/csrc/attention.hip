@@ -269,7 +269,7 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
     uint32_t tm = 0, bk = 0;
     cusync_gemm_tile_shape(tile, &tm, nullptr, &bk);
     const cusync_dim3 flat = cusync_gemm_grid(tile, S, 3 * L->E, 1);
-    return flat.x * flat.y * (uint32_t)cusync::gemm::pickSplitToFill(flat.x * flat.y, tm, cfg->hidden, bk, cusync_gemm_max_resident(tile));
+    return flat.x * flat.y * (uint32_t)cusync::gemm::pickSplitToFill(flat.x * flat.y, tm, cfg->hidden, bk, cusync_gemm_max_resident(tile), cusync::gemm::sliceUnit(tile));
   };
   auto fills = [&](int tile) { const uint32_t n = workgroups(tile); return n * 5 >= 256 * 4 && n <= 256; };
   const bool lines = cfg->hidden % 64 == 0;
@@ -327,8 +327,8 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   cusync_gemm_tile_shape(L->tile3, nullptr, nullptr, &bk3);
   const cusync_dim3 flat1 = cusync_gemm_grid(L->tile1, cfg->seq, 3 * L->E, 1);
   const cusync_dim3 flat3 = cusync_gemm_grid(L->tile3, cfg->seq, cfg->hidden, 1);
-  L->split1 = cusync::gemm::pickSplitToFill(flat1.x * flat1.y, tm1, cfg->hidden, bk1, cusync_gemm_max_resident(L->tile1));
-  L->split3 = cusync::gemm::pickSplit(0, flat3.x * flat3.y, L->E, bk3, cusync_gemm_max_resident(L->tile3));
+  L->split1 = cusync::gemm::pickSplitToFill(flat1.x * flat1.y, tm1, cfg->hidden, bk1, cusync_gemm_max_resident(L->tile1), cusync::gemm::sliceUnit(L->tile1));
+  L->split3 = cusync::gemm::pickSplit(0, flat3.x * flat3.y, L->E, bk3, cusync_gemm_max_resident(L->tile3), cusync::gemm::sliceUnit(L->tile3));
   const cusync_dim3 g1 = cusync_gemm_grid(L->tile1, cfg->seq, 3 * L->E, L->split1);
   const cusync_dim3 g2 = cusync_attention_grid_split(cfg->seq, cfg->heads, cfg->cached_rows, L->kvSplit);
   const cusync_dim3 g3 = cusync_gemm_grid(L->tile3, cfg->seq, cfg->hidden, L->split3);

@@ -49,6 +49,7 @@ namespace {
 using cusync::rt::setError;
 using cusync::gemm::pickSplit;
 using cusync::gemm::pickSplitToFill;
+using cusync::gemm::sliceUnit;
 using cusync::gemm::wideInThreeSlices;
 using cusync::gemm::half_t;
 using cusync::gemm::uint4v;
@@ -374,8 +375,8 @@ bool choose(const cusync_mlp_config& given, Choice* o) {
   }
   const cusync_dim3 flat1 = cusync_gemm_grid(o->tile1, c.batch, n1, 1);
   const cusync_dim3 flat2 = cusync_gemm_grid(o->tile2, c.batch, n2, 1);
-  o->split1 = c.split_k1 > 0 ? c.split_k1 : pickSplitToFill(flat1.x * flat1.y, tm1, k1, bk1, cusync_gemm_max_resident(o->tile1));
-  o->split2 = pickSplit(c.split_k2, flat2.x * flat2.y, k2, bk2, cusync_gemm_max_resident(o->tile2));
+  o->split1 = c.split_k1 > 0 ? c.split_k1 : pickSplitToFill(flat1.x * flat1.y, tm1, k1, bk1, cusync_gemm_max_resident(o->tile1), sliceUnit(o->tile1));
+  o->split2 = pickSplit(c.split_k2, flat2.x * flat2.y, k2, bk2, cusync_gemm_max_resident(o->tile2), sliceUnit(o->tile2));
   return true;
 }
 

@@ -4,6 +4,8 @@
 #include <stdint.h>
 #include <algorithm>
 
+#include "../../include/cusync_amd.h"
+
 namespace cusync {
 namespace gemm {
 
@@ -21,11 +23,21 @@ inline bool everySliceHasAChunk(uint32_t K, uint32_t bk, uint32_t slices) {
   return slices >= 1 && slices <= chunks && (slices - 1) * ((chunks + slices - 1) / slices) < chunks;
 }
 
-inline int pickSplit(int requested, uint32_t tiles, uint32_t K, uint32_t bk, int resident) {
+// Columns of K in a slice, and whether they come in whole numbers of `unit`.
+inline bool sliceInUnits(uint32_t K, uint32_t bk, uint32_t slices, uint32_t unit) {
+  return ((K + bk - 1) / bk + slices - 1) / slices * bk % unit == 0;
+}
+
+// The number of columns of K a slice has to be a whole number of: 64 for the 256x384x32 tile, which refuses others.  (768 output
+// columns at 1100 rows are ten of its tiles, and two slices of K = 1088 would have 17 chunks of 32 each.)
+inline uint32_t sliceUnit(int tile) { return tile == CUSYNC_TILE_256x384x32 ? 64 : 1; }
+
+inline int pickSplit(int requested, uint32_t tiles, uint32_t K, uint32_t bk, int resident, uint32_t unit = 1) {
   if (requested > 0) return requested;
   const uint32_t target = (uint32_t)std::min(resident, 256);
   int s = 1;
-  while (tiles * (uint32_t)s * 2 <= target && K / ((uint32_t)s * 2) >= 8 * bk && everySliceHasAChunk(K, bk, (uint32_t)s * 2)) s *= 2;
+  while (tiles * (uint32_t)s * 2 <= target && K / ((uint32_t)s * 2) >= 8 * bk && everySliceHasAChunk(K, bk, (uint32_t)s * 2) &&
+         sliceInUnits(K, bk, (uint32_t)s * 2, unit)) s *= 2;
   return s;
 }
 
@@ -37,13 +49,13 @@ inline int pickSplit(int requested, uint32_t tiles, uint32_t K, uint32_t bk, int
 // 108.0 -> 93.7; level between four and seven slices once 200 CUs are busy (36 tiles, 16 rows: 26.9 / 26.0 / 26.1 us with 5 / 6 / 7).
 // Nor from four slices on where the tiles have 128 rows and more and the slices share the reduction: five of them share it
 // unevenly (48 tiles, the attention chain in stream order: 256 rows 102.6 us with four, 106.6 with five; 512 rows 137.5, 141.5).
-// (A slice is a whole number of 64 columns of K long: the 256x384x32 tile takes no other.)
-inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t bk, int resident) {
+// (An added slice is a whole number of 64 columns of K long whatever the tile.)
+inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t bk, int resident, uint32_t unit = 1) {
   const uint32_t target = (uint32_t)std::min(resident, 256);
-  uint32_t s = (uint32_t)pickSplit(0, tiles, K, bk, resident);
+  uint32_t s = (uint32_t)pickSplit(0, tiles, K, bk, resident, unit);
   if (tileM >= 128 && s >= 4) return (int)s;
   for (uint32_t more = s + 1; s < 8 && tiles * s * 5 < target * 4 && more < 8 && tiles * more <= target && K / more >= 8 * bk; more++)
-    if (everySliceHasAChunk(K, bk, more) && ((K + bk - 1) / bk + more - 1) / more * bk % 64 == 0) s = more;
+    if (everySliceHasAChunk(K, bk, more) && sliceInUnits(K, bk, more, 64)) s = more;
   return (int)s;
 }
 
@@ -54,10 +66,10 @@ inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t 
 // to 6 144 columns, 1100 rows 191 -> 172, 1280: 200 -> 181.  Outside that range it falls behind (6 144 columns, 1500 rows, 96
 // tiles in two slices: 215 -> 220).  The launch takes its slice count from pickSplitToFill, which has to make it three: with
 // K below 768 or three slices that are not whole numbers of 64 columns it gives one or two, which is another launch than the
-// one measured, or one the tile refuses (K = 576: two slices of nine chunks).
+// one measured.
 inline bool wideInThreeSlices(uint32_t tiles, uint32_t K, int resident) {
   return resident >= 256 && tiles * 3 <= 256 && tiles * 3 * 5 >= 256 * 4 && tiles * 2 * 2 > 256 && K % 64 == 0 &&
-         pickSplitToFill(tiles, 256, K, 32, resident) == 3;
+         pickSplitToFill(tiles, 256, K, 32, resident, 64) == 3;
 }
 
 // Whether the k-slices of a tile add it up together (each waits for its siblings, then sums and stores a share of

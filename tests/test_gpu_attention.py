@@ -189,7 +189,7 @@ def test_attention_layer_where_the_projection_changes_tiles(S):
 
 
 # other widths, where those tiles do not fill the device or only some of them do
-@pytest.mark.parametrize("S,hidden,heads", [(48, 2048, 9), (300, 4096, 15), (600, 2048, 3), (1300, 2048, 12), (1300, 576, 12)])
+@pytest.mark.parametrize("S,hidden,heads", [(48, 2048, 9), (300, 4096, 15), (600, 2048, 3), (1300, 2048, 12), (1300, 576, 12), (1100, 3840, 9)])
 def test_attention_layer_of_other_widths(S, hidden, heads):
     print("attn layer widths", S, hidden, heads, flush=True)
     check_layer(S, hidden, heads, sampled=True)

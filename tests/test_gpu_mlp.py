@@ -133,6 +133,14 @@ def test_gpt3_mlp_of_five_row_tiles_and_a_short_k(hidden):
     check_against_oracle(api.MODEL.GPT3, x, w1, w2, h, y, 6144)
 
 
+def test_gpt3_mlp_whose_second_gemm_has_an_odd_number_of_chunks_in_two_slices():
+    # GEMM2 on 256x384 tiles, K = 1088: 34 chunks of 32, and slices of 17 are none that tile takes
+    print("odd chunks", flush=True)
+    x, w1, w2, h, y, prod, cons, tiles, _ = run_mlp(api.MODEL.GPT3, 1100, 768, 1088, api.SYNC.ROW)
+    assert cons.spin_timeouts == 0 and tiles[1] == api.TILE.T256x384x32
+    check_against_oracle(api.MODEL.GPT3, x, w1, w2, h, y, 1088)
+
+
 def test_gpt3_without_activation_matches_reference_check_build():
     # the reference's --check build has no GeLU (TB/mlp.cu:148-151)
     x, w1, w2, h, y, _, _, _, _ = run_mlp(api.MODEL.GPT3, 64, sync=api.SYNC.TILE, activation=0, **GPT3)

@@ -89,13 +89,14 @@ int main() {
         for (uint32_t tileM : {64u, 256u})
           std::printf("F %u %u %d %u %d %d\n", tiles, K, resident, tileM, pickSplit(0, tiles, K, 64, resident), pickSplitToFill(tiles, tileM, K, 64, resident));
   for (uint32_t tiles = 1; tiles <= 300; tiles++)
-    for (uint32_t K = 64; K <= 16384; K += 64) {       // 32 columns of K to a chunk, as the 256x384 tile has
-      const int doubled = pickSplit(0, tiles, K, 32, 256), got = pickSplitToFill(tiles, 256, K, 32, 256);
-      if (got != doubled && (K / 32 + got - 1) / got * 32 % 64) std::printf("B %u %u %d\n", tiles, K, got);
+    for (uint32_t K = 64; K <= 16384; K += 64) {       // 32 columns of K to a chunk, as the 256x384 tile has: no slice it refuses, added or doubled
+      const uint32_t unit = sliceUnit(CUSYNC_TILE_256x384x32);
+      for (int got : {pickSplit(0, tiles, K, 32, 256, unit), pickSplitToFill(tiles, 256, K, 32, 256, unit), pickSplitToFill(tiles, 64, K, 32, 256, unit)})
+        if ((K / 32 + got - 1) / got * 32 % 64) std::printf("B %u %u %d\n", tiles, K, got);
     }
   for (uint32_t tiles = 1; tiles <= 300; tiles++)
     for (uint32_t K = 32; K <= 16384; K += 32) {       // the launch takes its slice count from pickSplitToFill: it has to be the three the tile was chosen for
-      const int got = pickSplitToFill(tiles, 256, K, 32, 256);
+      const int got = pickSplitToFill(tiles, 256, K, 32, 256, sliceUnit(CUSYNC_TILE_256x384x32));
       if (wideInThreeSlices(tiles, K, 256) && (got != 3 || K % 64 || (K / 32 + 2) / 3 % 2)) std::printf("B %u %u %d\n", tiles, K, got);
     }
   for (uint32_t tiles = 1; tiles <= 300; tiles++)
