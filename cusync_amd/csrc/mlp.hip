@@ -270,7 +270,7 @@ void pickTiles(const cusync_mlp_config& c, int sync, bool swiglu, bool fused, in
   if (big && c.batch > 1024 && !swiglu && k2 % 64 == 0 && n2 % 384 == 0 && !c.one_launch) b = CUSYNC_TILE_256x384x32;
   // (five row tiles, 1025 to 1280 rows: GEMM1 in three slices of 256x384, see wideInThreeSlices)
   if (a == CUSYNC_TILE_256x192x64 && n1 % 384 == 0 && !c.one_launch && c.split_k1 <= 0 && sync != CUSYNC_SYNC_STRIDED &&
-      wideInThreeSlices(n1 / 384 * ((c.batch + 255) / 256), k1, cusync_gemm_max_resident(CUSYNC_TILE_256x384x32))) a = CUSYNC_TILE_256x384x32;
+      wideInThreeSlices(n1 / 384 * ((c.batch + 255) / 256), k1, cusync_gemm_max_resident(CUSYNC_TILE_256x384x32), (uint32_t)std::max(0, c.max_wg1))) a = CUSYNC_TILE_256x384x32;
   *t1 = c.tile1 >= 0 ? c.tile1 : a;
   *t2 = c.tile2 >= 0 ? c.tile2 : b;
   // both GEMMs in one launch share a kernel: the consumer takes the producer's tile
@@ -375,7 +375,7 @@ bool choose(const cusync_mlp_config& given, Choice* o) {
   }
   const cusync_dim3 flat1 = cusync_gemm_grid(o->tile1, c.batch, n1, 1);
   const cusync_dim3 flat2 = cusync_gemm_grid(o->tile2, c.batch, n2, 1);
-  o->split1 = c.split_k1 > 0 ? c.split_k1 : pickSplitToFill(flat1.x * flat1.y, tm1, k1, bk1, cusync_gemm_max_resident(o->tile1), sliceUnit(o->tile1));
+  o->split1 = c.split_k1 > 0 ? c.split_k1 : pickSplitToFill(flat1.x * flat1.y, tm1, k1, bk1, cusync_gemm_max_resident(o->tile1), sliceUnit(o->tile1), (uint32_t)std::max(0, c.max_wg1));
   o->split2 = pickSplit(c.split_k2, flat2.x * flat2.y, k2, bk2, cusync_gemm_max_resident(o->tile2), sliceUnit(o->tile2));
   return true;
 }

@@ -41,6 +41,9 @@ inline int pickSplit(int requested, uint32_t tiles, uint32_t K, uint32_t bk, int
   return s;
 }
 
+// Rounds a launch of `workgroups` takes under a limit of `cap` of them (0: no limit, one round).
+inline uint32_t roundsOf(uint32_t workgroups, uint32_t cap) { return cap ? (workgroups + cap - 1) / cap : 1; }
+
 // The same for GEMMs whose columns do not come in powers of two (the attention chain's QKV projection: 36 column tiles of
 // 128, 24 of 192).  Doubling stops at half to three quarters of the CUs there, so single slices are added until four
 // fifths of the CUs have work.  From eight slices on it does not pay: what they add up grows with every slice (48 rows on
@@ -50,12 +53,16 @@ inline int pickSplit(int requested, uint32_t tiles, uint32_t K, uint32_t bk, int
 // Nor from four slices on where the tiles have 128 rows and more and the slices share the reduction: five of them share it
 // unevenly (48 tiles, the attention chain in stream order: 256 rows 102.6 us with four, 106.6 with five; 512 rows 137.5, 141.5).
 // (An added slice is a whole number of 64 columns of K long whatever the tile.)
-inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t bk, int resident, uint32_t unit = 1) {
+// `cap`: the caller's limit of workgroups for the launch, 0 without one.  Under a limit a slice is added only where the rounds
+// it costs leave less work behind one another.  LLaMA MLP, GEMM1 of 43 tiles, 40 rows under RowSync, four slices / five: at
+// most 200 workgroups, where the fifth is a second round, 50.2 / 55.8 us; 100, three rounds of fifths, 62 / 67; 160, two
+// rounds either way, 61.6 / 56.6.
+inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t bk, int resident, uint32_t unit = 1, uint32_t cap = 0) {
   const uint32_t target = (uint32_t)std::min(resident, 256);
   uint32_t s = (uint32_t)pickSplit(0, tiles, K, bk, resident, unit);
   if (tileM >= 128 && s >= 4) return (int)s;
   for (uint32_t more = s + 1; s < 8 && tiles * s * 5 < target * 4 && more < 8 && tiles * more <= target && K / more >= 8 * bk; more++)
-    if (everySliceHasAChunk(K, bk, more) && sliceInUnits(K, bk, more, 64)) s = more;
+    if (everySliceHasAChunk(K, bk, more) && sliceInUnits(K, bk, more, 64) && roundsOf(tiles * more, cap) * s < roundsOf(tiles * s, cap) * more) s = more;
   return (int)s;
 }
 
@@ -66,10 +73,12 @@ inline int pickSplitToFill(uint32_t tiles, uint32_t tileM, uint32_t K, uint32_t 
 // to 6 144 columns, 1100 rows 191 -> 172, 1280: 200 -> 181.  Outside that range it falls behind (6 144 columns, 1500 rows, 96
 // tiles in two slices: 215 -> 220).  The launch takes its slice count from pickSplitToFill, which has to make it three: with
 // K below 768 or three slices that are not whole numbers of 64 columns it gives one or two, which is another launch than the
-// one measured.
-inline bool wideInThreeSlices(uint32_t tiles, uint32_t K, int resident) {
-  return resident >= 256 && tiles * 3 <= 256 && tiles * 3 * 5 >= 256 * 4 && tiles * 2 * 2 > 256 && K % 64 == 0 &&
-         pickSplitToFill(tiles, 256, K, 32, resident, 64) == 3;
+// one measured.  Under a limit of workgroups the slices have to be ahead by rounds as well, two thirds of
+// the work in each (1100 rows, 80 tiles, the pair, 256x192 in one slice / this: at most 200 workgroups 386 / 468 us, 160: 384 / 428, 128:
+// 532 / 429, 64: 694 / 632; at 100, where the rounds are level, 522 / 501, and 513 / 548 where GEMM2 has the limit too).
+inline bool wideInThreeSlices(uint32_t tiles, uint32_t K, int resident, uint32_t cap = 0) {
+  return resident >= 256 && tiles * 3 <= 256 && tiles * 3 * 5 >= 256 * 4 && tiles * 2 * 2 > 256 && K % 64 == 0 && 2 * roundsOf(tiles * 3, cap) < 3 * roundsOf(tiles * 2, cap) &&
+         pickSplitToFill(tiles, 256, K, 32, resident, 64, cap) == 3;
 }
 
 // Whether the k-slices of a tile add it up together (each waits for its siblings, then sums and stores a share of

@@ -133,6 +133,16 @@ def test_gpt3_mlp_of_five_row_tiles_and_a_short_k(hidden):
     check_against_oracle(api.MODEL.GPT3, x, w1, w2, h, y, 6144)
 
 
+@pytest.mark.parametrize("limit", [239, 128])
+def test_gpt3_mlp_of_five_row_tiles_under_a_limit_of_workgroups(limit):
+    # one workgroup short of a round of three slices, GEMM1 keeps 256x192; at 128 two rounds of them are ahead of two of 256x192
+    print("limit", limit, flush=True)
+    x, w1, w2, h, y, prod, cons, tiles, _ = run_mlp(api.MODEL.GPT3, 1100, 12288, 6144, api.SYNC.ROW, max_wg1=limit)
+    assert cons.spin_timeouts == 0 and tiles[0] == (api.TILE.T256x192x64 if limit == 239 else api.TILE.T256x384x32)
+    assert tiles[2] == (1 if limit == 239 else 3)
+    check_against_oracle(api.MODEL.GPT3, x, w1, w2, h, y, 6144)
+
+
 def test_gpt3_mlp_whose_second_gemm_has_an_odd_number_of_chunks_in_two_slices():
     # GEMM2 on 256x384 tiles, K = 1088: 34 chunks of 32, and slices of 17 are none that tile takes
     print("odd chunks", flush=True)

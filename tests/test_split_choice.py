@@ -101,6 +101,15 @@ int main() {
     }
   for (uint32_t tiles = 1; tiles <= 300; tiles++)
     for (uint32_t K : {64u, 96u, 2752u, 4096u, 8192u, 12288u}) std::printf("W %u %u %d %d\n", tiles, K, wideInThreeSlices(tiles, K, 256) ? 1 : 0, wideInThreeSlices(tiles, K, 0) ? 1 : 0);
+  // a limit of workgroups: never more work behind one another than without the added slices, and the tile as measured
+  for (uint32_t tiles = 1; tiles <= 256; tiles++)
+    for (uint32_t cap = 1; cap <= 300; cap++) {
+      const uint32_t doubled = (uint32_t)pickSplit(0, tiles, 12288, 64, 256), got = (uint32_t)pickSplitToFill(tiles, 64, 12288, 64, 256, 1, cap);
+      if (got != doubled && roundsOf(tiles * got, cap) * doubled >= roundsOf(tiles * doubled, cap) * got) std::printf("C %u %u %u\n", tiles, cap, got);
+      if (cap >= 256 && got != (uint32_t)pickSplitToFill(tiles, 64, 12288, 64, 256)) std::printf("C %u %u %u\n", tiles, cap, got);
+      if (wideInThreeSlices(tiles, 12288, 256, cap) && pickSplitToFill(tiles, 256, 12288, 32, 256, 64, cap) != 3) std::printf("C %u %u wide\n", tiles, cap);
+    }
+  for (uint32_t cap : {0u, 300u, 240u, 239u, 200u, 160u, 128u, 100u}) std::printf("L %u %d %d\n", cap, wideInThreeSlices(80, 12288, 256, cap) ? 1 : 0, pickSplitToFill(43, 64, 8192, 64, 256, 1, cap));
   for (int slices = 1; slices <= 10; slices++)
     for (uint32_t tileM : {32u, 64u, 128u, 256u})
       std::printf("S %d %u %d %d\n", slices, tileM, slicesCanShareReduction(slices, true, true, true, 240, 240, tileM, false) ? 1 : 0,
@@ -117,7 +126,7 @@ def test_slices_that_fill_the_device(tmp_path):
     exe = tmp_path / "fill_test"
     subprocess.check_call(["g++", "-std=c++17", "-Wall", "-I", os.path.join(ROOT, "cusync_amd", "csrc"), str(src), "-o", str(exe)])
     lines = [f.split() for f in subprocess.check_output([str(exe)], text=True).split("\n") if f]
-    fill = {}
+    fill, limits = {}, {}
     for f in lines:
         v = [int(x) for x in f[1:]]
         if f[0] == "F":
@@ -130,6 +139,10 @@ def test_slices_that_fill_the_device(tmp_path):
             assert (got - 1) * -(-chunks // got) < chunks
         elif f[0] == "B":
             assert False, "256x384x32: slices that are not whole numbers of 64 columns, or not the three the tile was chosen for: %s" % f
+        elif f[0] == "C":
+            assert False, "more rounds than without the added slices: %s" % f
+        elif f[0] == "L":
+            limits[v[0]] = (v[1], v[2])
         elif f[0] == "W":
             tiles, K, got, without = v
             per = -(-K // 32 // 3) * 32
@@ -143,3 +156,5 @@ def test_slices_that_fill_the_device(tmp_path):
     for (tiles, K), s in want.items():
         assert fill[(tiles, K, 256, 64)] == s, (tiles, K)
     assert fill[(48, 12288, 256, 256)] == 4 and fill[(72, 12288, 256, 256)] == 3
+    # GPT-3 at five row tiles, whether in three slices of 256x384; LLaMA's 43 tiles, slices
+    assert limits == {0: (1, 5), 300: (1, 5), 240: (1, 5), 239: (0, 5), 200: (0, 4), 160: (0, 5), 128: (1, 5), 100: (0, 4)}
