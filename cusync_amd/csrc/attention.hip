@@ -265,6 +265,8 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   // the narrower rule stays: 64x192 up to 320 rows, 128x192 alone from 513 to 640.
   // (two full row tiles of 128, 193 to 256 rows: 128x192 with the operands fetched 64 columns of K at a time, the QKV
   // projection 55 -> 52 us at 256 rows, 51 -> 49.5 at 224; level below)
+  // (where K is a multiple of 64, the 256x192 tile that fetches both operands 64 columns at a time, K loop in assembly)
+  auto inLines = [](int tile, uint32_t K) { return tile == CUSYNC_TILE_256x192x32 && K % 64 == 0 ? (int)CUSYNC_TILE_256x192x64 : tile; };
   auto workgroups = [&](int tile) {
     uint32_t tm = 0, bk = 0;
     cusync_gemm_tile_shape(tile, &tm, nullptr, &bk);
@@ -276,12 +278,10 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   const bool widthsAgree = cfg->sync != CUSYNC_SYNC_STRIDED || L->E % 192 == 0;     // (ConsecutiveSync refuses the same widths whichever tile is taken)
   const int wide1 = S <= 32 ? small : S <= 64 ? (!fills(CUSYNC_TILE_D64x192x64) && fills(CUSYNC_TILE_D64x128x64) && widthsAgree ? CUSYNC_TILE_D64x128x64 : CUSYNC_TILE_D64x192x64)
                     : S <= 192 ? CUSYNC_TILE_D64x192x64 : S <= 384 && lines && (S <= 256 || fills(CUSYNC_TILE_D128x192x64)) ? CUSYNC_TILE_D128x192x64
-                    : S <= 320 ? CUSYNC_TILE_D64x192x64 : S > 512 && S <= 640 && !fills(CUSYNC_TILE_256x192x32) ? CUSYNC_TILE_128x192x32_ALONE
+                    : S <= 320 ? CUSYNC_TILE_D64x192x64 : S > 512 && S <= 640 && !fills(inLines(CUSYNC_TILE_256x192x32, cfg->hidden)) ? CUSYNC_TILE_128x192x32_ALONE
                     : CUSYNC_TILE_256x192x32;
   const int wide3 = S <= 32 ? small : S <= 256 ? CUSYNC_TILE_D64x192x64 : S <= 512 ? CUSYNC_TILE_128x192x32_ALONE
                     : S <= 1024 ? CUSYNC_TILE_256x192x32 : CUSYNC_TILE_128x192x32;
-  // (where K is a multiple of 64, the 256x192 tile that fetches both operands 64 columns at a time, K loop in assembly)
-  auto inLines = [](int tile, uint32_t K) { return tile == CUSYNC_TILE_256x192x32 && K % 64 == 0 ? (int)CUSYNC_TILE_256x192x64 : tile; };
   L->tile1 = cfg->tile1 >= 0 ? cfg->tile1 : (3 * L->E) % 192 == 0 ? inLines(wide1, cfg->hidden) : dflt;
   L->tile3 = cfg->tile3 >= 0 ? cfg->tile3 : cfg->hidden % 192 == 0 ? inLines(wide3, L->E) : dflt;
   // (above 1024 rows the output projection's five to eight row tiles of 256x384, at most one per CU, beat 128x192 at

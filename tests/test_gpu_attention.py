@@ -195,6 +195,14 @@ def test_attention_layer_of_other_widths(S, hidden, heads):
     check_layer(S, hidden, heads, sampled=True)
 
 
+def test_attention_layer_whose_slices_are_too_short_to_fill_the_device():
+    # K = 1344 in three slices of 256x192x32 would fill the CUs, but the tile that runs takes K 64 columns at a time and gets two:
+    # 128x192 alone on its CU stays
+    print("attn layer short slices", flush=True)
+    assert run_layer(600, 1344, 12, api.SYNC.ROW, runs=1)[7][0] == api.TILE.T128x192x32_ALONE
+    check_layer(600, 1344, 12, sampled=True)
+
+
 # ---- key/value cache variant (src/ml-bench/transformer/attention.cu:265-276, 289) ----------------
 
 def run_attention_kv(qkv, cached, heads, causal=True):
