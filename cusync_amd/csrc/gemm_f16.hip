@@ -373,7 +373,7 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
   if (!ti || !ti->chainKernel) { setError("gemm chain: needs a direct-to-LDS tile"); return CUSYNC_ERROR_NOT_INITIALIZED; }
   const int resident = residentWorkgroups(args[0].tile);
   if (resident <= 0) { setError("gemm: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
-  uint32_t launched = (uint32_t)resident, mostTiles = 0;
+  uint32_t launched = (uint32_t)resident, mostTiles = 0, pitches = 0;
   bool oneRow = true;
   for (int i = 0; i < count; i++) {
     const cusync_gemm_args& a = args[i];
@@ -384,6 +384,7 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
     if (a.stage.in.kind != CUSYNC_POLICY_NOSYNC && i == 0) { setError("gemm chain: the first GEMM cannot wait on a stage outside the launch"); return CUSYNC_ERROR_NOT_INITIALIZED; }
     mostTiles = std::max<uint32_t>(mostTiles, a.stage.grid.x * a.stage.grid.y * a.stage.grid.z);
     oneRow = oneRow && a.stage.grid.y == 1;
+    pitches |= a.ldb * (uint32_t)sizeof(half_t);
     if (a.max_workgroups > 0) launched = std::min<uint32_t>(launched, (uint32_t)a.max_workgroups);
   }
   // As many workgroups as the GEMM with most tiles has (and the device holds at once).  A workgroup without a tile
@@ -395,11 +396,12 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
   // other's gaps (inner width 49 152, 384 tiles, 1 row: 392 us, one workgroup to a CU 409).
   const bool ahead = oneRow && ti->chainAheadResidentPerCU > 0 && mostTiles <= (uint32_t)(ti->chainAheadResidentPerCU * g_numCUs);
   const auto kernel = ahead ? ti->chainKernelAhead : oneRow && ti->chainKernelOnce ? ti->chainKernelOnce : ti->chainKernel;
+  const bool turn = cusync::deal::listsTurn(oneRow, mostTiles, launched, (uint32_t)g_numCUs, pitches);
   GemmChainParams cp = {};
   cp.count = (uint32_t)count;
   for (int i = 0; i < count; i++) {
     cp.gemm[i] = gemmParams(&args[i], ti, launched);
-    cp.gemm[i].stage.turn = (uint32_t)i;
+    cp.gemm[i].stage.turn = turn ? (uint32_t)i : 0;
   }
   hipLaunchKernelGGL(kernel, dim3(launched), dim3(ti->threads), ahead ? ti->ldsChainAhead : ti->lds, (hipStream_t)stream, cp);
   if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;

@@ -55,8 +55,8 @@ struct DynStage {
   // plain protocol has it, also where the stores were written through and acknowledged and the library normally
   // raises them relaxed.  Results must not change; only the write-backs and invalidations come back.
   bool releaseAll;
-  // How many positions further on the lists of tiles are begun (see deal::listTicket): the place of a GEMM in a launch of
-  // several, 0 elsewhere.
+  // How many positions further on the lists of tiles are begun: the place of a GEMM in a launch of several where deal::listsTurn
+  // says so, 0 elsewhere, above all in launches that draw from the dispensers.
   uint32_t turn;
 
   __device__ __forceinline__ bool isProducer() const { return d.out.kind != CUSYNC_POLICY_NOSYNC; }
@@ -181,7 +181,7 @@ struct DynStage {
     const uint32_t mine = homeList();
     if (raw != 0xffffffffu) {
       const uint32_t l = raw + deal::listStatic(d.grid, mine, launched);
-      if (l < deal::listTiles(d.grid, mine)) return deal::listTicket(d.grid, mine, l, turn);
+      if (l < deal::listTiles(d.grid, mine)) return deal::listTicket(d.grid, mine, l);
     }
     dry |= 1u << mine;
     uint32_t seen[8];
@@ -194,7 +194,7 @@ struct DynStage {
       const uint32_t x = (mine + s) & 7u;
       if (dry & (1u << x)) continue;
       const uint32_t l = dev::ticketAdd(&d.xcdTickets[x * kLine], 1) + deal::listStatic(d.grid, x, launched);
-      if (l < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, l, turn);
+      if (l < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, l);
       dry |= 1u << x;
     }
     const uint32_t finished = dev::ticketAdd(&d.xcdTickets[8 * kLine], 1);
@@ -208,7 +208,7 @@ struct DynStage {
     if (!customOrder()) return workgroupIndex();
     const uint32_t b = workgroupIndex(), x = b & 7u, pos = b >> 3;
     if (noDraws) return deal::onlyTicket(d.grid, launched, b, turn);
-    if (pos < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, pos, turn);
+    if (pos < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, pos);
     return drawFinish(drawBegin(dry, noDraws), launched, 0, dry, noDraws);
   }
 

@@ -29,11 +29,7 @@ CUSYNC_HD uint32_t listStatic(const cusync_dim3& grid, uint32_t x, uint32_t laun
   const uint32_t wgs = listWorkgroups(x, launched), tiles = listTiles(grid, x);
   return wgs < tiles ? wgs : tiles;
 }
-// Ticket of position l of list x.  `turn`: the list is begun that many positions further on.  A workgroup of a launch of
-// several GEMMs has the same position in each one's list, so without a turn the tiles it gets have much the same columns:
-// where the weights' rows are a multiple of 1 KiB apart all rows of a column tile lie in one class of memory channels, one
-// class in four is a quarter slower, and the workgroups that finish such a tile last would begin another one.  (GPT-3 MLP at
-// one row: 48 and 96 column tiles, lists of 6 and 12.)
+// Ticket of position l of list x.  `turn`: the list is begun that many positions further on (see listsTurn).
 CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l, uint32_t turn = 0) {
   if (turn) l = (l + turn) % listTiles(grid, x);
   const uint32_t span = byRows(grid) ? grid.y : grid.x;
@@ -41,6 +37,20 @@ CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l, u
   if (!byRows(grid)) return lo + l % width + (l / width) * grid.x;
   const uint32_t perSlice = width * grid.x;          // this list's tiles in one k-slice
   return (l / perSlice) * grid.x * grid.y + lo * grid.x + l % perSlice;
+}
+
+// Whether the later GEMMs of a launch of several begin their lists a position further on each.  A workgroup has the same
+// position in each one's list, so without the turn the tiles it gets have much the same columns.  Where the rows of the
+// weights are a multiple of 1 KiB apart, all rows of a column tile lie in one class of memory channels, one class in four is
+// a quarter slower, and the workgroups that finish such a tile last would begin another one.  GPT-3 MLP in one launch (48 and
+// 96 column tiles, lists of 6 and 12), a pass without -> with the turn, us: TileSync 1 row 70.5 -> 68.9, 16 rows 71.9 -> 70.1, 64
+// rows 80.2 -> 79.8, inner width 24576, 1 row 217.3 -> 215.0; RowSync 1 row 70.9 -> 70.4, 16 rows 72.3 -> 71.5.
+// Not where tiles share CUs, which costs under TileSync what is not explained (inner width 49152, 384 tiles: 1 row 385.6 -> 407.5,
+// 32 rows 410.9 -> 433.6; RowSync level).  Not where several row tiles read the same weights (512 to 1024 rows: level), nor at
+// other row pitches (LLaMA, 11008 bytes, StridedSync: 1 row 43.6 -> 43.9, 16 rows 44.6 -> 44.9).
+// `pitches`: the row pitches of all the GEMMs' weights in bytes, or'ed.
+inline bool listsTurn(bool oneRowOfTiles, uint32_t mostTiles, uint32_t launched, uint32_t numCUs, uint32_t pitches) {
+  return oneRowOfTiles && mostTiles <= launched && mostTiles <= numCUs && pitches % 1024 == 0;
 }
 
 // A launch of at least as many workgroups as tiles needs no dispenser: every tile is some workgroup's first one.  Where

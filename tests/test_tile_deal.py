@@ -35,6 +35,13 @@ int main() {
   // launches of the chains: 14 x 14 x 256 at batch 32, LLaMA's GEMM1, the QKV projection, attention, one column of 392 tiles
   const uint32_t chains[][3] = {{2, 49, 2}, {29, 4, 2}, {29, 8, 1}, {36, 1, 4}, {43, 1, 4}, {12, 1, 6}, {12, 4, 2}, {1, 392, 1}, {64, 4, 1}};
   for (auto& c : chains) for (uint32_t turn = 0; turn < 8; turn++) if (check(c[0], c[1], c[2], 0, turn)) return 1;
+  // the lists turn for one row of tiles with a CU for each, the weights' rows a multiple of 1 KiB apart
+  const struct { bool oneRow; uint32_t tiles, launched, pitches; bool turns; } launches[] = {
+    {true, 240, 240, 12288 | 24576, true}, {true, 256, 256, 12288 | 24576, true}, {true, 192, 192, 49152 | 24576, true},
+    {true, 384, 384, 98304 | 24576, false}, {true, 240, 100, 12288 | 24576, false}, {false, 128, 128, 12288 | 24576, false},
+    {true, 215, 215, 11008 | 16384, false}, {true, 240, 240, 12544 | 24832, false}};
+  for (auto& l : launches)
+    if (listsTurn(l.oneRow, l.tiles, l.launched, 256, l.pitches) != l.turns) { std::printf("turn: %u tiles, %u workgroups, pitches %u\n", l.tiles, l.launched, l.pitches); return 1; }
   std::printf("ok\n");
   return 0;
 }
