@@ -90,17 +90,15 @@ int residentWorkgroups(int tile) {
       if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ti->kernel[v], (int)ti->threads, ti->lds))) return 0;
       perCU = std::min(perCU, n);
     }
-    if (ti->chainKernelAhead &&
-        (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ti->chainKernelAhead), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ti->ldsChainAhead)) ||
-         CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&ti->chainAheadResidentPerCU, ti->chainKernelAhead, (int)ti->threads, ti->ldsChainAhead)))) return 0;
-    const void* others[5] = { reinterpret_cast<const void*>(ti->chainKernel), reinterpret_cast<const void*>(ti->kernelNoChunkWaits),
-                              reinterpret_cast<const void*>(ti->kernelOnce), reinterpret_cast<const void*>(ti->kernelOnceNoChunkWaits),
-                              reinterpret_cast<const void*>(ti->chainKernelOnce) };
-    for (const void* k : others) {
-      if (!k) continue;
+    const struct { const void* kernel; size_t lds; } others[6] = {
+      { reinterpret_cast<const void*>(ti->chainKernel), ti->lds }, { reinterpret_cast<const void*>(ti->kernelNoChunkWaits), ti->lds },
+      { reinterpret_cast<const void*>(ti->kernelOnce), ti->lds }, { reinterpret_cast<const void*>(ti->kernelOnceNoChunkWaits), ti->lds },
+      { reinterpret_cast<const void*>(ti->chainKernelOnce), ti->lds }, { reinterpret_cast<const void*>(ti->chainKernelAhead), ti->ldsChainAhead } };
+    for (const auto& k : others) {
+      if (!k.kernel) continue;
       int n = 0;
-      if (CUSYNC_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)std::max<size_t>(ti->lds, g_ldsPerCU / 2))) ||
-          CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, (int)ti->threads, ti->lds))) return 0;
+      if (CUSYNC_HIP(hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)std::max<size_t>(k.lds, g_ldsPerCU / 2))) ||
+          CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k.kernel, (int)ti->threads, k.lds))) return 0;
       perCU = std::min(perCU, n);
     }
     ti->residentPerCU = perCU;
@@ -390,11 +388,11 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
   // As many workgroups as the GEMM with most tiles has (and the device holds at once).  A workgroup without a tile
   // of GEMM i goes straight on to GEMM i+1 and waits there for tiles that running workgroups hold.
   launched = std::min<uint32_t>(launched, mostTiles);
-  // Grids of one row read B once.  Where each tile has a CU to itself, the workgroup takes all of the CU's LDS for loads in
-  // flight and fetches B ahead of the wait for its producer (DmaCfg::AHEAD): GPT-3 MLP in one launch, without -> with,
-  // TileSync: 64 rows 82.6 -> 80.7 us, 1 row 72.1 -> 71.1.  With more tiles two smaller workgroups share a CU and fill each
-  // other's gaps (inner width 49 152, 384 tiles, 1 row: 392 us, one workgroup to a CU 409).
-  const bool ahead = oneRow && ti->chainAheadResidentPerCU > 0 && mostTiles <= (uint32_t)(ti->chainAheadResidentPerCU * g_numCUs);
+  // Grids of one row read B once.  Where each tile has a CU to itself the workgroup fetches B ahead of the wait for its
+  // producer (DmaCfg::AHEAD): GPT-3 MLP in one launch under RowSync, without -> with, 64 rows 81.7 -> 79.8 us, 1 row 71.0 -> 70.1.
+  // With more tiles it is level under RowSync and behind under TileSync (inner width 49 152, 384 tiles, 1 row: 403 and 403,
+  // 386 and 404).
+  const bool ahead = oneRow && ti->chainKernelAhead && mostTiles <= (uint32_t)g_numCUs;
   const auto kernel = ahead ? ti->chainKernelAhead : oneRow && ti->chainKernelOnce ? ti->chainKernelOnce : ti->chainKernel;
   const bool turn = cusync::deal::listsTurn(oneRow, mostTiles, launched, (uint32_t)g_numCUs, pitches);
   GemmChainParams cp = {};

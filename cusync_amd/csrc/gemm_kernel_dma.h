@@ -706,7 +706,10 @@ __global__ __launch_bounds__(C::THREADS, C::WAVES_PER_SIMD) void gemmDmaKernel(G
 // kernel or second launch sits between producer and consumer, which is what a chain of short GEMMs
 // (few rows: 30 us in the kernel, 10 us around it) pays most for.  Forward progress: the launch has
 // no more workgroups than stay resident, and a workgroup only moves on when the GEMM it is on has no
-// tile left to hand out, so every tile a consumer tile waits for is in the hands of a running workgroup.
+// tile left to hand out, so every tile a consumer tile waits for is in the hands of a running workgroup,
+// provided that the launch gets all its slots.  Beside another launch whose workgroups wait for each
+// other it does as long as both fit the device together; each could otherwise hold the slots the other's
+// first tiles need, until the bounded waits give up.
 template<class C>
 __global__ __launch_bounds__(C::THREADS, C::WAVES_PER_SIMD) void gemmDmaChainKernel(GemmChainParams cp) {
   for (uint32_t g = 0; g < cp.count; g++) {

@@ -29,7 +29,6 @@ struct TileInfo {
   void (*chainKernelOnce)(GemmChainParams);
   void (*chainKernelAhead)(GemmChainParams);
   size_t ldsChainAhead;
-  int chainAheadResidentPerCU;     // filled lazily, 0 without such a kernel
 };
 
 void fillStagedTiles(TileInfo* tiles);     // register-staged tiles (the only ones with a SwiGLU A operand)
@@ -41,13 +40,13 @@ void fillDmaTilesXWide(TileInfo* tiles);   // direct-to-LDS, 256x384, eight wave
 // Entry of a register-staged tile.
 #define CUSYNC_TILE(BM, BN, BK, WM, WN) \
   TileInfo{ BM, BN, BK, kThreads, (size_t)TileCfg<BM, BN, BK, WM, WN>::LDS_BYTES, \
-    { gemmKernel<TileCfg<BM, BN, BK, WM, WN>, false>, gemmKernel<TileCfg<BM, BN, BK, WM, WN>, true> }, -1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0 }
+    { gemmKernel<TileCfg<BM, BN, BK, WM, WN>, false>, gemmKernel<TileCfg<BM, BN, BK, WM, WN>, true> }, -1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0 }
 
 // Entry of a direct-to-LDS tile: no SwiGLU variant (that operand needs arithmetic on its way into LDS).
 #define CUSYNC_TILE_DMA(...) \
   TileInfo{ DmaCfg<__VA_ARGS__>::BM, DmaCfg<__VA_ARGS__>::BN, DmaCfg<__VA_ARGS__>::BK, DmaCfg<__VA_ARGS__>::THREADS, \
     (size_t)DmaCfg<__VA_ARGS__>::LDS_BYTES, { gemmDmaKernel<DmaCfg<__VA_ARGS__>>, nullptr }, -1, gemmDmaChainKernel<DmaCfg<__VA_ARGS__>>, \
-    nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0 }
+    nullptr, nullptr, nullptr, nullptr, nullptr, 0 }
 
 // Entry of a few-row direct-to-LDS tile: also the kernel compiled without the per-chunk waits.  A launch of these
 // tiles is short (40 us), and the wait code a kernel carries without running it (stream order, RowSync) costs it
@@ -59,7 +58,7 @@ void fillDmaTilesXWide(TileInfo* tiles);   // direct-to-LDS, 256x384, eight wave
     (size_t)DmaCfg<__VA_ARGS__>::LDS_BYTES, { gemmDmaKernel<DmaCfg<__VA_ARGS__>>, nullptr }, -1, gemmDmaChainKernel<DmaCfg<__VA_ARGS__>>, \
     gemmDmaKernel<DmaCfg<__VA_ARGS__>, kAPlain, false>, gemmDmaKernel<DmaCfgOnce<__VA_ARGS__>>, \
     gemmDmaKernel<DmaCfgAhead<__VA_ARGS__>, kAPlain, false>, gemmDmaChainKernel<DmaCfgOnce<__VA_ARGS__>>, \
-    gemmDmaChainKernel<AHEAD>, (size_t)AHEAD::LDS_BYTES, 0 }
+    gemmDmaChainKernel<AHEAD>, (size_t)AHEAD::LDS_BYTES }
 
 }  // namespace gemm
 }  // namespace cusync

@@ -45,8 +45,8 @@ CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l, u
 // a quarter slower, and the workgroups that finish such a tile last would begin another one.  GPT-3 MLP in one launch (48 and
 // 96 column tiles, lists of 6 and 12), a pass without -> with the turn, us: TileSync 1 row 70.5 -> 68.9, 16 rows 71.9 -> 70.1, 64
 // rows 80.2 -> 79.8, inner width 24576, 1 row 217.3 -> 215.0; RowSync 1 row 70.9 -> 70.4, 16 rows 72.3 -> 71.5.
-// Not where tiles share CUs, which costs under TileSync what is not explained (inner width 49152, 384 tiles: 1 row 385.6 -> 407.5,
-// 32 rows 410.9 -> 433.6; RowSync level).  Not where several row tiles read the same weights (512 to 1024 rows: level), nor at
+// Not where there are more tiles than CUs or workgroups, which costs under TileSync what is not explained (inner width 49152,
+// 384 tiles: 1 row 385.6 -> 407.5, 32 rows 410.9 -> 433.6; RowSync level).  Not where several row tiles read the same weights (512 to 1024 rows: level), nor at
 // other row pitches (LLaMA, 11008 bytes, StridedSync: 1 row 43.6 -> 43.9, 16 rows 44.6 -> 44.9).
 // `pitches`: the row pitches of all the GEMMs' weights in bytes, or'ed.
 inline bool listsTurn(bool oneRowOfTiles, uint32_t mostTiles, uint32_t launched, uint32_t numCUs, uint32_t pitches) {

@@ -340,7 +340,12 @@ cusync_error cusync_gemm_run_static_workspace(const cusync_gemm_args *args, void
  * posts, exactly as in separate launches (the stages are created and paired the same way), but no kernel boundary,
  * wait kernel or second launch sits in between.  No counterpart in the reference, whose consumer is always a launch
  * of its own; here a first dispatch on another stream starts 15-20 us after the producer did, which chains of
- * short kernels cannot afford.  args[0] must not wait on a stage outside the launch. */
+ * short kernels cannot afford.  args[0] must not wait on a stage outside the launch.
+ * The workgroups wait for tiles of others of the same launch, so all of them (the tiles of the GEMM with most, up to
+ * max_workgroups) need a slot on the device at once.  Two such launches in flight together, from two streams or two
+ * processes, must fit the device together (cusync_gemm_max_resident(tile) workgroups of one tile shape): where they do
+ * not, each may hold the slots the other's first tiles need until the bounded waits give up.  The same goes for the
+ * launches of shared_reduction. */
 cusync_error cusync_gemm_chain_run(const cusync_gemm_args *args, int count, void *stream);
 
 /* ------------------------------------------------------------------------- */
@@ -516,7 +521,8 @@ typedef struct cusync_mlp_config {
   int32_t split_k1, split_k2;  /* k-slices per GEMM (--split-k1/--split-k2, TB/mlp.cu:880-931); 0 = pick so that
                                   the launch fills the device */
   int32_t max_wg1, max_wg2;    /* workgroups per launch of each GEMM; 0 = built-in choice, -1 = as many as stay resident */
-  int32_t one_launch;          /* 1 (with a CuSync mode): both GEMMs in one launch, cusync_gemm_chain_run; needs the same
+  int32_t one_launch;          /* 1 (with a CuSync mode): both GEMMs in one launch, cusync_gemm_chain_run (which says what two of
+                                  them in flight at once need); needs the same
                                   direct-to-LDS tile for both and a plain A operand in GEMM2.  0: one launch per GEMM on
                                   two streams, as the reference runs them.  -1: whichever measured faster for this
                                   model and batch size with the table's tiles (cusync_mlp_choice reports it) */

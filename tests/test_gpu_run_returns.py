@@ -144,3 +144,45 @@ def test_split_times_add_up():
     total, g1, g2 = m.run(x.data_ptr(), h.data_ptr(), y.data_ptr(), runs=5, split=True)
     m.destroy()
     assert np.allclose(np.array(g1) + np.array(g2), total, atol=0.02) and min(g1) > 0 and min(g2) > 0
+
+
+def test_two_launches_of_several_gemms_at_once():
+    # two handles run from two host threads, both GEMMs of each in one launch whose workgroups wait for each other; 64x128 tiles
+    # leave a CU to two workgroups in every kernel, and two times 240 fit the device
+    import threading
+    import torch
+    from cusync_amd import _lib
+    print("two launches at once", flush=True)
+    L = _lib.load()
+    assert [L.cusync_gemm_max_resident(t) // L.cusync_gemm_max_resident(api.TILE.T256x192x64) for t in
+            (api.TILE.D32x128x64, api.TILE.D64x128x64, api.TILE.D64x192x64)] == [1, 2, 1]
+    hidden, inner, rows = 12288, 6144, 64
+    w1, w2 = to_dev(normal_f16((hidden, inner), 2, std=0.02)), to_dev(normal_f16((inner, hidden), 3, std=0.02))
+    bufs = [(to_dev(uniform_f16((rows, hidden), 4 + k)), empty_dev((rows, inner)), empty_dev((rows, hidden))) for k in range(2)]
+    torch.cuda.synchronize()
+    tile = api.TILE.D64x128x64
+    handles = [api.Mlp(api.MODEL.GPT3, rows, hidden, inner, api.SYNC.ROW, w1.data_ptr(), w2.data_ptr(), tile1=tile, tile2=tile, one_launch=True) for _ in bufs]
+    alone, failed = [], []
+    for h, (x, mid, y) in zip(handles, bufs):
+        assert int(np.prod(h.stage_state(0).grid)) <= L.cusync_gemm_max_resident(tile) // 2
+        h.run(x.data_ptr(), mid.data_ptr(), y.data_ptr())
+        alone.append(y.clone())
+        y.fill_(float("nan"))
+    torch.cuda.synchronize()
+
+    def work(h, x, mid, y):
+        try:
+            for _ in range(50):
+                h.run(x.data_ptr(), mid.data_ptr(), y.data_ptr())
+        except Exception as e:
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(h,) + b) for h, b in zip(handles, bufs)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    for (x, mid, y), want, h in zip(bufs, alone, handles):
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+        h.destroy()
