@@ -372,7 +372,7 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
   const int resident = residentWorkgroups(args[0].tile);
   if (resident <= 0) { setError("gemm: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
   uint32_t launched = (uint32_t)resident, mostTiles = 0, pitches = 0;
-  bool oneRow = true;
+  bool oneRow = true, aheadPays = true;
   for (int i = 0; i < count; i++) {
     const cusync_gemm_args& a = args[i];
     if (a.tile != args[0].tile) { setError("gemm chain: all GEMMs must use the same tile"); return CUSYNC_ERROR_NOT_INITIALIZED; }
@@ -383,16 +383,17 @@ cusync_error cusync_gemm_chain_run(const cusync_gemm_args* args, int count, void
     mostTiles = std::max<uint32_t>(mostTiles, a.stage.grid.x * a.stage.grid.y * a.stage.grid.z);
     oneRow = oneRow && a.stage.grid.y == 1;
     pitches |= a.ldb * (uint32_t)sizeof(half_t);
+    const uint32_t chunks = (a.K + ti->bk - 1) / ti->bk, slices = (uint32_t)a.split_k;
+    aheadPays = aheadPays && fetchAheadPays(waitsPerChunk(a.stage), (chunks + slices - 1) / slices * ti->bk);
     if (a.max_workgroups > 0) launched = std::min<uint32_t>(launched, (uint32_t)a.max_workgroups);
   }
   // As many workgroups as the GEMM with most tiles has (and the device holds at once).  A workgroup without a tile
   // of GEMM i goes straight on to GEMM i+1 and waits there for tiles that running workgroups hold.
   launched = std::min<uint32_t>(launched, mostTiles);
   // Grids of one row read B once.  Where each tile has a CU to itself the workgroup fetches B ahead of the wait for its
-  // producer (DmaCfg::AHEAD): GPT-3 MLP in one launch under RowSync, without -> with, 64 rows 81.7 -> 79.8 us, 1 row 71.0 -> 70.1.
-  // With more tiles it is level under RowSync and behind under TileSync (inner width 49 152, 384 tiles, 1 row: 403 and 403,
-  // 386 and 404).
-  const bool ahead = oneRow && ti->chainKernelAhead && mostTiles <= (uint32_t)g_numCUs;
+  // producer (DmaCfg::AHEAD) if that pays: GPT-3 MLP in one launch under RowSync, without -> with, 64 rows 81.7 -> 79.8 us, 1 row
+  // 71.0 -> 70.1; with more tiles it is level (inner width 49 152, 384 tiles, 1 row: 403 and 403).
+  const bool ahead = oneRow && ti->chainKernelAhead && aheadPays && mostTiles <= (uint32_t)g_numCUs;
   const auto kernel = ahead ? ti->chainKernelAhead : oneRow && ti->chainKernelOnce ? ti->chainKernelOnce : ti->chainKernel;
   const bool turn = cusync::deal::listsTurn(oneRow, mostTiles, launched, (uint32_t)g_numCUs, pitches);
   GemmChainParams cp = {};

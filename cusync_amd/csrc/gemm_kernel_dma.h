@@ -64,9 +64,9 @@ struct DmaCfg {
   // B is fetched ahead of A: a consumer's weights do not depend on its producer, so three of the four wavefronts send out
   // their share of the first STAGES - 1 chunks of B before the producer is waited for, while the fourth polls (a
   // wavefront's loads return in order: the poll would come back behind its own), and the memory is not idle between the
-  // producer's last weights and the consumer's first.  All of the producer tiles are waited for at once.  GPT-3 MLP in one
-  // launch, 64 rows: 83.0 -> 80.6 us; attention of 16 rows behind 2048, whose output projection is such a launch:
-  // 68.0 -> 66.0.
+  // producer's last weights and the consumer's first.  All of the producer tiles are waited for at once, which under a policy
+  // with waits per chunk pays for short k-slices only (fetchAheadPays).  GPT-3 MLP in one launch, 64 rows: 81.5 -> 79.8 us;
+  // attention of 16 rows behind 2048, whose output projection is such a launch: 68.0 -> 66.0.
   static constexpr bool AHEAD = AHEAD_;
   static constexpr bool PIPE = PIPE_;                      // barrier in the middle of a chunk, fragments prefetched across chunks
   static constexpr bool PINGPONG = PINGPONG_;              // K loop in assembly, operands in whole cache lines (see above)
@@ -164,8 +164,8 @@ struct WideOperands {
 //
 // ROUNDS: a GEMM's chunk waits are made once per round of the pipeline (STAGES chunks ahead) instead of once per
 // chunk.  The wait's code is inlined where it is called; per chunk that is nine copies of it in the kernel, per
-// round two, and the TileSync consumer of the 2048-row MLP is 13 us (2 %) faster for it.  The kernel of several
-// GEMMs in one launch keeps the waits per chunk: compiled the other way the 512-row chain, where one launch is the
+// round two, and the TileSync consumer of the 2048-row MLP is 13 us (2 %) faster for it.  (With DmaCfg::AHEAD there is one
+// wait for all chunks.)  The other kernels of several GEMMs in one launch keep the waits per chunk: compiled the other way the 512-row chain, where one launch is the
 // best mode, took 212 instead of 208 us (and 222 instead of 212 while the k-slices' reduction was still unrolled
 // and the kernel parked ten more registers per lane in scratch for it); it would gain at 2048 rows, 595 -> 588 us,
 // where the two launches are ahead anyway.

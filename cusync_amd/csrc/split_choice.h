@@ -81,6 +81,14 @@ inline bool wideInThreeSlices(uint32_t tiles, uint32_t K, int resident, uint32_t
          pickSplitToFill(tiles, 256, K, 32, resident, 64, cap) == 3;
 }
 
+// Whether a GEMM that consumes another's tiles in the same launch gains from fetching its weights ahead of the wait, for which
+// all producer tiles of a k-slice are waited for at once (DmaCfg::AHEAD).  Under a policy that can be waited for chunk by chunk
+// a long slice begins on the first chunks while the last are still being made, and that is worth more: MLPs of 32x128 and
+// 64x192 tiles in one launch, TileSync and StridedSync, us with -> without, by columns of K in a slice of GEMM2: 688 43.7 -> 44.6,
+// 1536 47.4 -> 48.4 and 79.8 -> 81.2, 2304 100.7 -> 101.7; 2752 113.0 -> 112.2, 3072 68.9 -> 68.5 and 121.0 -> 120.5, 4608 94.1 ->
+// 93.4, 6144 116.6 -> 115.1 and 214.4 -> 210.5, 12288 214.5 -> 210.4.
+inline bool fetchAheadPays(bool waitsPerChunk, uint32_t kPerSlice) { return !waitsPerChunk || kPerSlice <= 2560; }
+
 // Whether the k-slices of a tile add it up together (each waits for its siblings, then sums and stores a share of
 // the tile) instead of leaving all of it to the slice that arrives last.  The waiting slices hold their CUs, so
 // every slice of the launch must have a workgroup of its own from the start (one round, all of them dealt a

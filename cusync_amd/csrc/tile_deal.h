@@ -47,7 +47,7 @@ CUSYNC_HD uint32_t listTicket(const cusync_dim3& grid, uint32_t x, uint32_t l, u
 // rows 80.2 -> 79.8, inner width 24576, 1 row 217.3 -> 215.0; RowSync 1 row 70.9 -> 70.4, 16 rows 72.3 -> 71.5.
 // Not where there are more tiles than CUs or workgroups, which costs under TileSync what is not explained (inner width 49152,
 // 384 tiles: 1 row 385.6 -> 407.5, 32 rows 410.9 -> 433.6; RowSync level).  Not where several row tiles read the same weights (512 to 1024 rows: level), nor at
-// other row pitches (LLaMA, 11008 bytes, StridedSync: 1 row 43.6 -> 43.9, 16 rows 44.6 -> 44.9).
+// other row pitches (LLaMA, 11008 bytes, StridedSync, 1 row 43.9 and 44.2, 16 rows 44.7 and 45.1: level).
 // `pitches`: the row pitches of all the GEMMs' weights in bytes, or'ed.
 inline bool listsTurn(bool oneRowOfTiles, uint32_t mostTiles, uint32_t launched, uint32_t numCUs, uint32_t pitches) {
   return oneRowOfTiles && mostTiles <= launched && mostTiles <= numCUs && pitches % 1024 == 0;

@@ -57,11 +57,11 @@ def test_fewer_chunks_than_stages(tile, K):
 
 @pytest.mark.parametrize("policy_kind", ["row", "tile"])
 @pytest.mark.parametrize("tile", [api.TILE.D32x128x64, api.TILE.D64x128x64, api.TILE.D64x192x64])
-@pytest.mark.parametrize("K,N1,N2,split2", [(72, 328, 1992, 1), (72, 328, 33288, 1), (520, 1416, 4104, 2), (328, 2568, 520, 3), (200, 1536, 3584, 2)])
+@pytest.mark.parametrize("K,N1,N2,split2", [(72, 328, 1992, 1), (72, 328, 33288, 1), (520, 1416, 4104, 2), (328, 2568, 520, 3), (200, 1536, 3584, 2), (72, 3080, 520, 1)])
 def test_one_row_of_tiles_in_one_launch(policy_kind, tile, K, N1, N2, split2):
-    # two GEMMs of one row of tiles in one launch: the second one's lists begin a position further on (where both have rows
-    # of weights that are a multiple of 1 KiB apart: the last case), its weights are fetched before the first one's tiles are waited for (not with more tiles than CUs); lists of unequal length, N and K
-    # not multiples of the tile
+    # two GEMMs of one row of tiles in one launch: the second one's lists begin a position further on (K = 200, whose weights'
+    # rows are multiples of 1 KiB apart), its weights are fetched before the first one's tiles are waited for (not with more
+    # tiles than CUs, nor under a tile policy with N1 = 3080); lists of unequal length, N and K not multiples of the tile
     import torch
     L = _lib.load()
     rows = api.tile_shape(tile)[0]

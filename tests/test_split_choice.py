@@ -110,6 +110,7 @@ int main() {
       if (wideInThreeSlices(tiles, 12288, 256, cap) && pickSplitToFill(tiles, 256, 12288, 32, 256, 64, cap) != 3) std::printf("C %u %u wide\n", tiles, cap);
     }
   for (uint32_t cap : {0u, 300u, 240u, 239u, 200u, 160u, 128u, 100u}) std::printf("L %u %d %d\n", cap, wideInThreeSlices(80, 12288, 256, cap) ? 1 : 0, pickSplitToFill(43, 64, 8192, 64, 256, 1, cap));
+  for (uint32_t k : {64u, 688u, 1536u, 2304u, 2752u, 3072u, 12288u}) std::printf("A %u %d %d\n", k, fetchAheadPays(false, k) ? 1 : 0, fetchAheadPays(true, k) ? 1 : 0);
   for (int slices = 1; slices <= 10; slices++)
     for (uint32_t tileM : {32u, 64u, 128u, 256u})
       std::printf("S %d %u %d %d\n", slices, tileM, slicesCanShareReduction(slices, true, true, true, 240, 240, tileM, false) ? 1 : 0,
@@ -141,6 +142,8 @@ def test_slices_that_fill_the_device(tmp_path):
             assert False, "256x384x32: slices that are not whole numbers of 64 columns, or not the three the tile was chosen for: %s" % f
         elif f[0] == "C":
             assert False, "more rounds than without the added slices: %s" % f
+        elif f[0] == "A":
+            assert v[1] == 1 and v[2] == int(v[0] <= 2304)        # a row is waited for as a whole; tile by tile, long slices begin early
         elif f[0] == "L":
             limits[v[0]] = (v[1], v[2])
         elif f[0] == "W":
