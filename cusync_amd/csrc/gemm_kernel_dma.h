@@ -61,7 +61,7 @@ struct DmaCfg {
   // L2 lines the neighbours were about to ask for: 96 rows on 64-row tiles 96.9 -> 106.2 us, LLaMA at 512 rows
   // 103.3 -> 119.8.
   static constexpr bool ONCE = ONCE_;
-  // B is fetched ahead of A: a consumer's weights do not depend on its producer, so three of the four wavefronts send out
+  // B is fetched ahead of A: under ReorderTileLoads a consumer's weights do not depend on its producer, so three of the four wavefronts send out
   // their share of the first STAGES - 1 chunks of B before the producer is waited for, while the fourth polls (a
   // wavefront's loads return in order: the poll would come back behind its own), and the memory is not idle between the
   // producer's last weights and the consumer's first.  All of the producer tiles are waited for at once, which under a policy
@@ -530,9 +530,11 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p, uint32_t from 
     auto waitThrough = [&](uint32_t kt) { waitChunk(kBegin + min(kt, nk - 1) * C::BK); };
     // (the assembly K loop has no place for waits: a stage of a tile policy waits for all its producer tiles here)
     if constexpr (C::AHEAD) {
-      // (see DmaCfg::AHEAD; the first round of the loop counts with this order)
+      // (see DmaCfg::AHEAD; the first round of the loop counts with this order).  Without ReorderTileLoads B comes behind the
+      // wait as well: it may be written on the producer's stream, and under AvoidWaitKernel nothing else orders it.
+      const bool early = !consumer || (stage.d.opts & CUSYNC_OPT_REORDER_TILE_LOADS);
       auto issueB = [&] { staticFor<C::STAGES - 1>([&](auto SP) { staticFor<C::B_LOADS>([&](auto QP) { issueOne(SP, QP, decltype(SP)::value); }); }); };
-      if (!consumer || wave != 0) issueB();
+      if (!consumer || (early && wave != 0)) issueB();
       if (consumer) {
         if (wave == 0) {
           const cusync_dim3 w = {m0, 0, 1};
@@ -540,7 +542,7 @@ __device__ __forceinline__ void gemmDmaTiles(const GemmParams& p, uint32_t from 
           waitThrough(nk - 1);
         }
         __syncthreads();
-        if (wave == 0) issueB();
+        if (wave == 0 || !early) issueB();
       }
       staticFor<C::STAGES - 1>([&](auto SP) {
         staticFor<C::A_LOADS>([&](auto QP) { issueOne(SP, Parity<C::B_LOADS + decltype(QP)::value>{}, decltype(SP)::value); });

@@ -281,7 +281,9 @@ typedef struct cusync_gemm_args {
   cusync_stage_desc stage;     /* Arguments::custage (cusyncgemm.h:293-350) */
   uint32_t M, N, K;            /* problem_size */
   const void *A; uint32_t lda; /* fp16 row-major [M,K] (or [M,2K] gate|up for CUSYNC_A_SWIGLU) */
-  const void *B; uint32_t ldb; /* fp16 row-major [K,N] */
+  const void *B; uint32_t ldb; /* fp16 row-major [K,N].  A consumer stage with CUSYNC_OPT_REORDER_TILE_LOADS may read it before its
+                                  producer has posted, and so may one with a register-staged tile whatever its options:
+                                  it must not be the producer's output then, and what writes it must be done before this launch */
   void *D; uint32_t ldd;       /* fp16 row-major [M,N] ([M,N/2] with CUSYNC_EPILOGUE_SWIGLU); D = epilogue(A*B), alpha = 1, beta = 0 */
   int32_t epilogue;            /* CUSYNC_EPILOGUE_* */
   int32_t a_mode;              /* CUSYNC_A_* */

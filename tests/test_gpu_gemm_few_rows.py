@@ -60,13 +60,13 @@ def test_fewer_chunks_than_stages(tile, K):
 @pytest.mark.parametrize("K,N1,N2,split2", [(72, 328, 1992, 1), (72, 328, 33288, 1), (520, 1416, 4104, 2), (328, 2568, 520, 3), (200, 1536, 3584, 2), (72, 3080, 520, 1)])
 def test_one_row_of_tiles_in_one_launch(policy_kind, tile, K, N1, N2, split2):
     # two GEMMs of one row of tiles in one launch: the second one's lists begin a position further on (K = 200, whose weights'
-    # rows are multiples of 1 KiB apart), its weights are fetched before the first one's tiles are waited for (not with more
+    # rows are multiples of 1 KiB apart), its weights are fetched, under ReorderTileLoads before the first one's tiles are waited for (not with more
     # tiles than CUs, nor under a tile policy with N1 = 3080); lists of unequal length, N and K not multiples of the tile
     import torch
     L = _lib.load()
     rows = api.tile_shape(tile)[0]
-    for M in (1, rows):
-        print("one launch", policy_kind, tile, M, K, N1, N2, split2, flush=True)
+    for M, opts in ((1, api.OPT.REORDER_TILE_LOADS), (rows, api.OPT.REORDER_TILE_LOADS), (rows, 0)):
+        print("one launch", policy_kind, tile, M, K, N1, N2, split2, opts, flush=True)
         rng = np.random.default_rng(tile + M + K)
         a, b = rng.integers(-1, 2, (M, K)).astype(np.float16), rng.integers(-1, 2, (K, N1)).astype(np.float16)
         d = rng.integers(-1, 2, (N1, N2)).astype(np.float16)
@@ -75,7 +75,7 @@ def test_one_row_of_tiles_in_one_launch(policy_kind, tile, K, N1, N2, split2):
         grids = [api.gemm_grid(tile, M, N1, 1), api.gemm_grid(tile, M, N2, split2)]
         tm, tn, _ = api.tile_shape(tile)
         pol = api.tile_sync(api.ORDER.TRANSPOSE_XY, tm, tn) if policy_kind == "tile" else api.row_sync(tm, grids[0][0])
-        st = [api.Stage(grids[0], (1, 1, 1), api.no_sync(), pol), api.Stage(grids[1], (1, 1, 1), pol, api.no_sync())]
+        st = [api.Stage(grids[0], (1, 1, 1), api.no_sync(), pol, opts=opts), api.Stage(grids[1], (1, 1, 1), pol, api.no_sync(), opts=opts)]
         assert api.set_producer_consumer_pair(st[0], st[1]) == api.ERR.SUCCESS
         args = (_lib.GemmArgs * 2)(
             api.gemm_args(st[0], M, N1, K, da.data_ptr(), K, db.data_ptr(), N1, dc.data_ptr(), N1, tile),
@@ -101,3 +101,41 @@ def test_one_row_of_tiles_in_one_launch(policy_kind, tile, K, N1, N2, split2):
         for s_ in st:
             s_.destroy()
         assert all(s_.spin_timeouts == 0 and s_.tile_counter == 0 for s_ in states)
+
+
+@pytest.mark.parametrize("policy_kind", ["row", "tile"])
+@pytest.mark.parametrize("tile", [api.TILE.D32x128x64, api.TILE.D64x128x64, api.TILE.D64x192x64])
+def test_weights_written_ahead_of_the_producer_on_its_stream(policy_kind, tile):
+    # a consumer under AvoidWaitKernel and without ReorderTileLoads reaches the device before its producer; its weights are
+    # written on the producer's stream, ahead of the producer: the wait for the producer's tiles is what orders them.  (The
+    # producer's stream is filled first: two streams may share a hardware queue, and the consumer must not be in front there.)
+    import torch
+    print("weights behind the wait", policy_kind, tile, flush=True)
+    M, K, N1, N2 = 20, 64, 512, 512
+    rng = np.random.default_rng(tile)
+    a, b = rng.integers(-1, 2, (M, K)).astype(np.float16), rng.integers(-1, 2, (K, N1)).astype(np.float16)
+    d = rng.integers(-1, 2, (N1, N2)).astype(np.float16)
+    da, db, src = to_dev(a), to_dev(b), to_dev(d)
+    w, c, e = empty_dev((N1, N2), fill=0.0), empty_dev((M, N1), fill=float("nan")), empty_dev((M, N2), fill=float("nan"))
+    filler = torch.zeros(64 << 20, device="cuda")
+    tm, tn, _ = api.tile_shape(tile)
+    g1, g2 = api.gemm_grid(tile, M, N1), api.gemm_grid(tile, M, N2)
+    pol = api.tile_sync(api.ORDER.TRANSPOSE_XY, tm, tn) if policy_kind == "tile" else api.row_sync(tm, g1[0])
+    prod = api.Stage(g1, (1, 1, 1), api.no_sync(), pol, opts=api.OPT.AVOID_WAIT_KERNEL)
+    cons = api.Stage(g2, (1, 1, 1), pol, api.no_sync(), opts=api.OPT.AVOID_WAIT_KERNEL)
+    assert api.set_producer_consumer_pair(prod, cons) == api.ERR.SUCCESS
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        for _ in range(24):                   # two milliseconds and more in which the consumer gets to the device and waits
+            filler.add_(1)
+        w.add_(src)
+    assert api.gemm(prod, M, N1, K, da.data_ptr(), K, db.data_ptr(), N1, c.data_ptr(), N1, tile, stream=first.cuda_stream) == api.ERR.SUCCESS, api.last_error()
+    assert api.gemm(cons, M, N2, N1, c.data_ptr(), N1, w.data_ptr(), N2, e.data_ptr(), N2, tile, stream=second.cuda_stream) == api.ERR.SUCCESS, api.last_error()
+    torch.cuda.synchronize()
+    ps, cs = prod.read_state(), cons.read_state()
+    prod.destroy(); cons.destroy()
+    assert ps.spin_timeouts == 0 and cs.spin_timeouts == 0
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.abs(want).max() < 2048
+    assert np.array_equal(to_host(e), (want @ d.astype(np.float64)).astype(np.float16))
