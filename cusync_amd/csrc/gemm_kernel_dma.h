@@ -105,7 +105,8 @@ struct DmaCfg {
   static_assert(LDS_BYTES * (WAVES_PER_SIMD * 4 / WAVES) <= 160 * 1024, "fits the LDS of one CU");
   static_assert((STAGES - 1) * LOADS < 64, "outstanding loads fit the vmcnt counter");
   static_assert(KS >= 2, "the loads of the next chunk ride on the LDS reads of k-step 1");
-  static_assert(!PIPE || (KS == 2 && STAGES >= 3), "the pipelined order is written for two k-steps per chunk");
+  static_assert(!PIPE || (KS == 2 && STAGES >= 3 && STAGES <= 5), "the pipelined order is written for two k-steps per chunk and up to five stages");
+  static_assert(!AHEAD || (ONCE && !PIPE && !PINGPONG), "the order of the first loads is written for the few-row tiles");
   static_assert(!PINGPONG || (WAVES == 8 && !PIPE && !BT && BM == 256 && ((BN == 384 && BK == 32) || (BN == 192 && BK == 64))), "the assembly K loops are written for two tiles");
 };
 

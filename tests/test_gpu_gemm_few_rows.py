@@ -65,8 +65,9 @@ def test_one_row_of_tiles_in_one_launch(policy_kind, tile, K, N1, N2, split2):
     import torch
     L = _lib.load()
     rows = api.tile_shape(tile)[0]
-    for M, opts in ((1, api.OPT.REORDER_TILE_LOADS), (rows, api.OPT.REORDER_TILE_LOADS), (rows, 0)):
-        print("one launch", policy_kind, tile, M, K, N1, N2, split2, opts, flush=True)
+    # (limit: workgroups that work through several tiles of each GEMM, most of them drawn)
+    for M, opts, limit in ((1, api.OPT.REORDER_TILE_LOADS, 0), (rows, api.OPT.REORDER_TILE_LOADS, 0), (rows, 0, 0), (rows, api.OPT.REORDER_TILE_LOADS, 3)):
+        print("one launch", policy_kind, tile, M, K, N1, N2, split2, opts, limit, flush=True)
         rng = np.random.default_rng(tile + M + K)
         a, b = rng.integers(-1, 2, (M, K)).astype(np.float16), rng.integers(-1, 2, (K, N1)).astype(np.float16)
         d = rng.integers(-1, 2, (N1, N2)).astype(np.float16)
@@ -78,7 +79,7 @@ def test_one_row_of_tiles_in_one_launch(policy_kind, tile, K, N1, N2, split2):
         st = [api.Stage(grids[0], (1, 1, 1), api.no_sync(), pol, opts=opts), api.Stage(grids[1], (1, 1, 1), pol, api.no_sync(), opts=opts)]
         assert api.set_producer_consumer_pair(st[0], st[1]) == api.ERR.SUCCESS
         args = (_lib.GemmArgs * 2)(
-            api.gemm_args(st[0], M, N1, K, da.data_ptr(), K, db.data_ptr(), N1, dc.data_ptr(), N1, tile),
+            api.gemm_args(st[0], M, N1, K, da.data_ptr(), K, db.data_ptr(), N1, dc.data_ptr(), N1, tile, max_workgroups=limit),
             api.gemm_args(st[1], M, N2, N1, dc.data_ptr(), N1, dd.data_ptr(), N2, de.data_ptr(), N2, tile, split_k=split2))
         ws = None
         if split2 > 1:
