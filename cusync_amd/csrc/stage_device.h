@@ -56,7 +56,9 @@ struct DynStage {
   // raises them relaxed.  Results must not change; only the write-backs and invalidations come back.
   bool releaseAll;
   // How many positions further on the lists of tiles are begun: the place of a GEMM in a launch of several where deal::listsTurn
-  // says so, 0 elsewhere, above all in launches that draw from the dispensers.
+  // says so, 0 elsewhere, above all in launches that draw from the dispensers.  (The draws are given it all the same: without
+  // it there the compiler arranges the kernels' start otherwise, 0.5 us a layer of 28x28x128 convolutions, pair of 22 images
+  // under RowSync 38.2 -> 39.5 us.)
   uint32_t turn;
 
   __device__ __forceinline__ bool isProducer() const { return d.out.kind != CUSYNC_POLICY_NOSYNC; }
@@ -181,7 +183,7 @@ struct DynStage {
     const uint32_t mine = homeList();
     if (raw != 0xffffffffu) {
       const uint32_t l = raw + deal::listStatic(d.grid, mine, launched);
-      if (l < deal::listTiles(d.grid, mine)) return deal::listTicket(d.grid, mine, l);
+      if (l < deal::listTiles(d.grid, mine)) return deal::listTicket(d.grid, mine, l, turn);
     }
     dry |= 1u << mine;
     uint32_t seen[8];
@@ -194,7 +196,7 @@ struct DynStage {
       const uint32_t x = (mine + s) & 7u;
       if (dry & (1u << x)) continue;
       const uint32_t l = dev::ticketAdd(&d.xcdTickets[x * kLine], 1) + deal::listStatic(d.grid, x, launched);
-      if (l < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, l);
+      if (l < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, l, turn);
       dry |= 1u << x;
     }
     const uint32_t finished = dev::ticketAdd(&d.xcdTickets[8 * kLine], 1);
@@ -208,7 +210,7 @@ struct DynStage {
     if (!customOrder()) return workgroupIndex();
     const uint32_t b = workgroupIndex(), x = b & 7u, pos = b >> 3;
     if (noDraws) return deal::onlyTicket(d.grid, launched, b, turn);
-    if (pos < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, pos);
+    if (pos < deal::listTiles(d.grid, x)) return deal::listTicket(d.grid, x, pos, turn);
     return drawFinish(drawBegin(dry, noDraws), launched, 0, dry, noDraws);
   }
 
