@@ -173,9 +173,6 @@ GemmParams convParams(const cusync_conv2d_args* a, const ConvTile* ti, uint32_t 
                         (s.in.kind == CUSYNC_POLICY_ROWSYNC || (s.in.tileN * 2) % 128 == 0);
   p.stage.releaseAll = cusync::rt::forceRelease();
   p.stage.prepare(launched);
-  // the runs of a tile share the adding up when each has a workgroup of its own from the start (see gemm_f16.hip)
-  p.coopReduce = slicesShareReduction((int)p.splitK, true, true, p.stage.noDraws, launched, s.grid.x * s.grid.y * s.grid.z,
-                                      ti->bm, (s.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL) != 0);
   return p;
 }
 

@@ -41,10 +41,17 @@ constexpr int kFragsAhead = 1;
 
 // How the accumulators leave a tile: as the kernel's wavefronts hold them, or (two groups, see KG) as they hold them
 // once the groups have put their halves of the channels together.
+//
+// The runs of a tile leave it to the one that arrives last to add them up.  Adding up and storing a share each, as the
+// k-slices of a GEMM do, makes every run wait for its siblings and the tile for two more round trips, and the sums it
+// spreads are few (64 KB a run, not 200): pairs and chains of four, us, shared -> last arriver: 32x14x14x256 in two runs,
+// pair under TileSync 51.3 -> 48.3, chain 94 -> 86; 12x14x14x256 in four runs, pair under RowSync 44.4 -> 39.9, chain under
+// TileSync 82.7 -> 72.5; 2x14x14x256 in four 39.7 -> 39.0.  It is ahead at every batch of 14x14 and 28x28 images.
 template<int BM_, int BN_, int WM_, int WN_, int THREADS_, int LDS_BYTES_>
 struct HaloFinishCfg {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, THREADS = THREADS_, LDS_BYTES = LDS_BYTES_;
   static constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
+  static constexpr bool LAST_SLICE_ADDS = true;
 };
 
 // KG: groups of four wavefronts.  A tile that has its CU to itself (the halo of 128 channels and more fills the LDS)
@@ -67,9 +74,9 @@ struct Halo3x3Cfg {
   // The halves of two groups: of the wavefront's two rows of MFMA tiles, or of its two columns where it has one row.
   static constexpr bool HALVE_ROWS = TM == 2;
   static constexpr int EXCHANGE_BYTES = KG == 1 ? 0 : BM * BN * 4;
-  // what the epilogue may use (finishTile): with two groups also the halo's place, for the share of a tile a run of
-  // two adds up itself
-  static constexpr int FINISH_BYTES = KG == 1 ? B_BYTES : (BM * (BN * 2 + 16) + 1023) / 1024 * 1024 + (BM / 2) * BN * 4;
+  // what the epilogue may use (finishTile): with two groups, whose wavefronts store twice as many rows at a time, also
+  // some of the halo's place
+  static constexpr int FINISH_BYTES = KG == 1 ? B_BYTES : (BM * (BN * 2 + 16) + 1023) / 1024 * 1024;
   using Finish = HaloFinishCfg<BM, BN, KG == 2 && HALVE_ROWS ? 2 * WM : WM, KG == 2 && !HALVE_ROWS ? 2 * WN : WN, THREADS, FINISH_BYTES>;
   static_assert(WM * WN == 4 && B_CPR == 8 && B_LOADS >= 1, "four wavefronts per group, 64-channel filter chunks");
   static_assert(KG == 1 || (KG == 2 && (TM == 2 || (TM == 1 && TN == 2))), "two groups exchange halves of a wavefront's tile");

@@ -43,7 +43,7 @@ struct GemmParams {
   // Split-K where every k-slice of the launch has a workgroup of its own from the start (one round, all resident):
   // the slices of a tile wait for each other and each adds up and stores a share of the tile (whole 32-row
   // pieces of it), instead of the slice that arrives last doing all of it while the others' CUs idle.  Set by the
-  // launcher; needs BM/32 to be a multiple of splitK.
+  // launcher; needs BM/32 to be no less than splitK.
   uint32_t coopReduce;
   uint32_t partialBytes;   // size of `partials`, for the buffer descriptor of the write-through stores
   uint32_t mPad;           // m-tiles * BM
@@ -186,6 +186,11 @@ __device__ __forceinline__ void schedPass() {
 // True for the tile configurations whose K loop is assembly (DmaCfg::PINGPONG).
 template<class C, class = void> struct IsAssemblyTile : std::false_type {};
 template<class C> struct IsAssemblyTile<C, std::enable_if_t<C::PINGPONG>> : std::true_type {};
+
+// Whether the slices of a tile may add it up together (finishTileSplit): tiles of 128 rows and more, and not where the
+// configuration says that the last slice does it alone.
+template<class C, class = void> struct SharesReduction { static constexpr bool value = C::BM >= 128; };
+template<class C> struct SharesReduction<C, std::enable_if_t<C::LAST_SLICE_ADDS>> : std::false_type {};
 
 // Stores of an output tile.  Final values go through LDS so that global memory sees whole rows: a lane holds 4
 // consecutive columns of 32 different rows, which stored directly would be 8-byte pieces scattered over 32 cache
@@ -413,7 +418,7 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
   constexpr uint32_t kPieces = C::TM * C::WM;                                   // 32-row pieces of a tile
   constexpr uint32_t kEpiBytes = (C::WM * 32 * (C::BN * 2 + 16) + 1023) / 1024 * 1024;
   constexpr uint32_t kPieceBytes = C::WN * C::TN * 4 * 1024;                    // 32 rows x BN columns of fp32
-  const bool shared = C::BM >= 128 && p.coopReduce;
+  const bool shared = SharesReduction<C>::value && p.coopReduce;
   const uint32_t firstPiece = shared ? t.z * kPieces / p.splitK : 0, endPiece = shared ? (t.z + 1) * kPieces / p.splitK : 0;
   const bool ownInLds = shared && kEpiBytes + (kPieces + p.splitK - 1) / p.splitK * kPieceBytes <= (uint32_t)C::LDS_BYTES;
   auto ownedPiece = [&](int i) { const uint32_t u = (uint32_t)i * C::WM + (uint32_t)wm; return u >= firstPiece && u < endPiece; };      // uniform per wavefront; asked under the shared reduction only
@@ -440,13 +445,13 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
   const uint32_t tileIndex = t.y * p.stage.d.grid.x + t.x;
   uint32_t* counter = p.arrivals + tileIndex;
 
-  // (the launcher shares the reduction only among tiles of 128 rows and more: the smaller ones do not carry the code)
+  // (the other tiles do not carry the code)
   if (shared) {
     // ---- every slice adds up and stores its share ---------------------------------------------------------
     // The tile is cut into BM/32 pieces of 32 rows (piece u = i * WM + wm: MFMA row tile i of wave row wm); slice z
-    // takes the pieces [z * U/S, (z + 1) * U/S), of unequal number where S does not divide U.  A piece is summed over the slices in index order (this slice's
-    // own term read back like the others: see above), so the result is the same, bit for bit, whichever way and
-    // in whatever order of arrival the tile is put together.
+    // takes the pieces [z * U/S, (z + 1) * U/S), of unequal number where S does not divide U.  A piece is summed over
+    // the slices in index order (this slice's own term read back like the others: see above), so the result is the
+    // same, bit for bit, whichever way and in whatever order of arrival the tile is put together.
     uint32_t* departures = p.arrivals + p.stage.d.grid.x * p.stage.d.grid.y + tileIndex;
     if (threadIdx.x == 0) {
       // not a release: the partial sums were written through and every wavefront has seen its own acknowledged

@@ -101,7 +101,7 @@ inline bool slicesCanShareReduction(int splitK, bool requested, bool directToLds
   return splitK > 1 && requested && directToLdsTile && everyTileStatic && launched == tiles && tileM >= 128 &&
          tileM / 32 >= (uint32_t)splitK && !avoidWaitKernel;
 }
-// The same for a kernel whose pieces have to divide among the slices (the 3x3 convolution's runs).
+// The same in equal shares, which none of the kernels needs.
 inline bool slicesShareReduction(int splitK, bool requested, bool directToLdsTile, bool everyTileStatic, uint32_t launched,
                                  uint32_t tiles, uint32_t tileM, bool avoidWaitKernel) {
   return slicesCanShareReduction(splitK, requested, directToLdsTile, everyTileStatic, launched, tiles, tileM, avoidWaitKernel) &&
