@@ -43,7 +43,8 @@ struct GemmParams {
   // Split-K where every k-slice of the launch has a workgroup of its own from the start (one round, all resident):
   // the slices of a tile wait for each other and each adds up and stores a share of the tile (whole 32-row
   // pieces of it), instead of the slice that arrives last doing all of it while the others' CUs idle.  Set by the
-  // launcher; needs BM/32 to be no less than splitK.
+  // launcher; needs BM/32 to be no less than splitK.  The number of polls a slice waits for its siblings before it gives
+  // the tile up (DynStage::gatherSlices); 0: the slice that arrives last adds up.
   uint32_t coopReduce;
   uint32_t partialBytes;   // size of `partials`, for the buffer descriptor of the write-through stores
   uint32_t mPad;           // m-tiles * BM
@@ -419,8 +420,8 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
   constexpr uint32_t kEpiBytes = (C::WM * 32 * (C::BN * 2 + 16) + 1023) / 1024 * 1024;
   constexpr uint32_t kPieceBytes = C::WN * C::TN * 4 * 1024;                    // 32 rows x BN columns of fp32
   const bool shared = SharesReduction<C>::value && p.coopReduce;
-  const uint32_t firstPiece = shared ? t.z * kPieces / p.splitK : 0, endPiece = shared ? (t.z + 1) * kPieces / p.splitK : 0;
-  const bool ownInLds = shared && kEpiBytes + (kPieces + p.splitK - 1) / p.splitK * kPieceBytes <= (uint32_t)C::LDS_BYTES;
+  uint32_t firstPiece = shared ? t.z * kPieces / p.splitK : 0, endPiece = shared ? (t.z + 1) * kPieces / p.splitK : 0;
+  bool ownInLds = shared && kEpiBytes + (kPieces + p.splitK - 1) / p.splitK * kPieceBytes <= (uint32_t)C::LDS_BYTES;
   auto ownedPiece = [&](int i) { const uint32_t u = (uint32_t)i * C::WM + (uint32_t)wm; return u >= firstPiece && u < endPiece; };      // uniform per wavefront; asked under the shared reduction only
   auto ownSlot = [&](int i, int j, int g) {
     const uint32_t o = (uint32_t)i * C::WM + (uint32_t)wm - firstPiece;
@@ -455,11 +456,44 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
     uint32_t* departures = p.arrivals + p.stage.d.grid.x * p.stage.d.grid.y + tileIndex;
     if (threadIdx.x == 0) {
       // not a release: the partial sums were written through and every wavefront has seen its own acknowledged
-      p.stage.countIn(counter);
-      if (!dev::pollUntilAtLeast(counter, p.splitK)) dev::countGiveUp(p.stage.d.spinTimeouts);     // the siblings are resident: bounded all the same
+      *sLast = p.stage.gatherSlices(counter, p.splitK, p.coopReduce);
       p.stage.countSeen();
     }
     __syncthreads();
+    const uint32_t how = __builtin_amdgcn_readfirstlane(*sLast);
+    if (how != DynStage::kSlicesShare) {
+      // Given up: what this slice kept for itself goes where the others' partial sums are; who finishes waits until the
+      // slices that left have got that far (they have arrived, so they are running) and takes all pieces.
+      if (ownInLds) {
+        // (addresses of its own, worked out here: kept from above they are registers the K loop goes without)
+        uint32_t tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const uint32_t first = (uint32_t)(((size_t)tileIndex * kTileFloats + (size_t)t.z * sliceStride) * sizeof(float)) + tid * 16;
+        const char* kept = lds + kEpiBytes + (tid & 63) * 16;
+#pragma unroll 1
+        for (int i = 0; i < C::TM; i++) {
+          if (!ownedPiece(i)) continue;
+          const uint32_t o = (uint32_t)i * C::WM + (uint32_t)wm - firstPiece;
+#pragma unroll 1
+          for (int n = 0; n < C::TN * 4; n++)
+            __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const uint4v*>(kept + ((o * C::WN + (uint32_t)wn) * (C::TN * 4) + (uint32_t)n) * 1024), rPart,
+                                                   (int)(first + (uint32_t)(i * C::TN * 4 + n) * (C::THREADS * 16)), 0, 16 /* sc1 */);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        ownInLds = false;
+      }
+      if (how == DynStage::kSliceLeaves) {
+        if (threadIdx.x == 0) p.stage.countIn(departures);
+        return false;
+      }
+      if (threadIdx.x == 0) {
+        if (!dev::pollUntilAtLeast(departures, p.splitK - 1)) dev::countGiveUp(p.stage.d.spinTimeouts);
+        p.stage.countSeen();
+      }
+      __syncthreads();
+      firstPiece = 0; endPiece = kPieces;
+    }
     // not unrolled: the sums do not live in the accumulators, so one copy of the pass serves every i
 #pragma unroll 1
     for (int i = 0; i < C::TM; i++) {
@@ -507,6 +541,7 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
       // A producer's stores must be out before the count that lets the last slice post: they were written through
       // and are acknowledged (the wait above), so the count needs no release, which would only start a write-back of
       // this XCD's L2.  No acquire either: nobody reads another slice's output.
+      // (the one that finishes a tile the others gave up has found theirs)
       const uint32_t before = p.stage.countIn(departures);
       const bool last = before == p.splitK - 1;
       if (last) { dev::storeRelaxed(counter, 0); dev::storeRelaxed(departures, 0); }
@@ -514,18 +549,18 @@ __device__ __forceinline__ bool finishTileSplit(const GemmParams& p, floatx16 (&
     }
     __syncthreads();
     return *sLast != 0;
+  } else {
+    if (threadIdx.x == 0) {
+      // neither release (the partial sums were written through and are acknowledged) nor acquire (the finishing slice
+      // reads them with device-coherent loads): either would work on this XCD's whole L2
+      const uint32_t before = p.stage.countIn(counter);
+      const bool last = before == p.splitK - 1;
+      if (last) { dev::storeRelaxed(counter, 0); p.stage.countSeen(); }
+      *sLast = last;
+    }
+    __syncthreads();
+    if (!*sLast) return false;
   }
-
-  if (threadIdx.x == 0) {
-    // neither release (the partial sums were written through and are acknowledged) nor acquire (the finishing slice
-    // reads them with device-coherent loads): either would work on this XCD's whole L2
-    const uint32_t before = p.stage.countIn(counter);
-    const bool last = before == p.splitK - 1;
-    if (last) { dev::storeRelaxed(counter, 0); p.stage.countSeen(); }
-    *sLast = last;
-  }
-  __syncthreads();
-  if (!*sLast) return false;
   // The slice that arrived last adds the slices in index order, one row of MFMA tiles at a time: all loads
   // of that row for one slice are issued together (TN * 4 of 16 bytes per thread).  One position at a time
   // would be a chain of round trips to memory as long as the GEMM itself; everything at once, accumulated

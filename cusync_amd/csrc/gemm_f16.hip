@@ -197,6 +197,11 @@ static size_t partialBytes(const cusync_gemm_args* a, const TileInfo* ti) {
   return (size_t)a->split_k * g.y * g.x * ti->bm * ti->bn * sizeof(float);
 }
 
+// Polls a k-slice waits for its siblings, of 1 to 1.5 us each: longer than the slices of a tile are apart by themselves (a
+// consumer's first slice is done up to 200 us before the producer has posted what the last one reads), and short beside the
+// second after which a wait gives up for good.
+constexpr uint32_t kSlicePatience = 1024;
+
 // Kernel parameters of one GEMM launched with `launched` workgroups.
 static GemmParams gemmParams(const cusync_gemm_args* a, const TileInfo* ti, uint32_t launched) {
   const cusync_stage_desc& s = a->stage;
@@ -235,9 +240,11 @@ static GemmParams gemmParams(const cusync_gemm_args* a, const TileInfo* ti, uint
   // apart, the same scheme (also cut finer, into 32x32 pieces) ended every launch 6-12 us later than the slice
   // that arrives last doing all of it.  Never under AvoidWaitKernel (see slicesCanShareReduction).
   const bool direct = ti->chainKernel != nullptr;
+  const char* patience = getenv("CUSYNC_SLICE_PATIENCE");
   p.coopReduce = slicesCanShareReduction(a->split_k, a->shared_reduction != 0, direct, p.stage.noDraws, launched,
-                                      s.grid.x * s.grid.y * s.grid.z, ti->bm, (s.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL) != 0) &&
-                 !getenv("CUSYNC_NO_COOP_REDUCE");
+                                         s.grid.x * s.grid.y * s.grid.z, ti->bm, (s.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL) != 0) &&
+                         !getenv("CUSYNC_NO_COOP_REDUCE")
+                     ? patience ? (uint32_t)std::max(1, atoi(patience)) : kSlicePatience : 0;
   return p;
 }
 

@@ -75,6 +75,25 @@ struct DynStage {
   }
   // ... and what its reader does before it touches the data (nothing: it reads with device-coherent loads).
   __device__ __forceinline__ void countSeen() const { if (releaseAll) dev::acquireFence(); }
+  // How the k-slices of a tile that share its reduction come together at their counter; called by the first thread of a
+  // slice's workgroup.  All in: everyone takes a share.  A slice that waited `patience` polls for its siblings gives the tile
+  // up for all of them, unless the last has arrived meanwhile: the slices there leave their CUs, and the one that arrives last
+  // finds the mark and does all of it.  So a launch ends whatever keeps its workgroups off the device for a while, another
+  // launch of this kind above all, whose waiting slices hold what these wait for and the other way round.
+  enum : uint32_t { kSlicesShare = 0, kSliceLeaves = 1, kSliceFinishes = 2, kSlicesGivenUp = 0x80000000u };
+  __device__ __forceinline__ uint32_t gatherSlices(uint32_t* counter, uint32_t slices, uint32_t patience) const {
+    const uint32_t before = countIn(counter);
+    uint32_t seen = dev::loadRelaxed(counter), polls = 0, naps = 1;      // (the first poll is on its way beside the count)
+    if (before == (kSlicesGivenUp | (slices - 1))) return kSliceFinishes;
+    for (;; seen = dev::loadRelaxed(counter)) {
+      if (seen == slices) return kSlicesShare;
+      if (seen & kSlicesGivenUp) return kSliceLeaves;
+      if (++polls >= patience &&
+          __hip_atomic_compare_exchange_strong(counter, &seen, seen | kSlicesGivenUp, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return kSliceLeaves;
+      for (uint32_t i = 0; i < naps; i++) __builtin_amdgcn_s_sleep(16);
+      if (naps < CUSYNC_MAX_NAPS) naps <<= 1;
+    }
+  }
   __device__ __forceinline__ bool isConsumer() const { return d.in.kind != CUSYNC_POLICY_NOSYNC; }
   __device__ __forceinline__ uint32_t numTiles() const { return d.grid.x * d.grid.y * d.grid.z; }
   __host__ __device__ __forceinline__ bool customOrder() const { return !(d.opts & CUSYNC_OPT_AVOID_CUSTOM_ORDER); }

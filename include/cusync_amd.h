@@ -297,9 +297,9 @@ typedef struct cusync_gemm_args {
                                   the tile.  1: where every k-slice of the launch has a workgroup of its own from the start
                                   (no more tiles than workgroups stay resident), tileM is at least 128 and tileM/32 no less than split_k, the
                                   slices of a tile wait for each other and each adds up and stores a share; same sums in
-                                  the same order, so bit-identical results.  The waiting slices hold their CUs: only for
-                                  launches whose workgroups no other kernel keeps off the device while it waits for them
-                                  (the chains of this library launch a consumer only after its producer is resident).
+                                  the same order, so bit-identical results.  The waiting slices hold their CUs; where other
+                                  launches keep their siblings off the device for a millisecond or two they leave, and
+                                  the slice that arrives last does the rest, so a launch ends whatever runs beside it.
                                   Ignored (the last-arriver form runs) for a stage with CUSYNC_OPT_AVOID_WAIT_KERNEL: without
                                   the hold-back a consumer's launch may reach the device first and keep sibling slices off it.
                                   No counterpart in the reference, whose split-K reduction is a kernel of its own
@@ -346,8 +346,7 @@ cusync_error cusync_gemm_run_static_workspace(const cusync_gemm_args *args, void
  * The workgroups wait for tiles of others of the same launch, so all of them (the tiles of the GEMM with most, up to
  * max_workgroups) need a slot on the device at once.  Two such launches in flight together, from two streams or two
  * processes, must fit the device together (cusync_gemm_max_resident(tile) workgroups of one tile shape): where they do
- * not, each may hold the slots the other's first tiles need until the bounded waits give up.  The same goes for the
- * launches of shared_reduction. */
+ * not, each may hold the slots the other's first tiles need until the bounded waits give up. */
 cusync_error cusync_gemm_chain_run(const cusync_gemm_args *args, int count, void *stream);
 
 /* ------------------------------------------------------------------------- */

@@ -185,6 +185,24 @@ def test_gemm_shared_reduction_of_unequal_shares(tile, split):
     assert_close(shared, orc.gemm(a, b), "unequal shares, %d slices, tile %d" % (split, tile))
 
 
+@pytest.mark.parametrize("tile,split", [(api.TILE.T256x192x64, 2), (api.TILE.T256x192x64, 3), (api.TILE.T256x192x64, 8), (api.TILE.T256x384x32, 2),
+                                        (api.TILE.T256x384x32, 4), (api.TILE.D128x192x64, 2), (api.TILE.D128x192x64, 3), (api.TILE.D128x192x64, 4),
+                                        (api.TILE.T256x256x32, 2), (api.TILE.T256x192x32, 4), (api.TILE.T256x128x32, 2), (api.TILE.T128x256x32, 2),
+                                        (api.TILE.T128x128x32, 4), (api.TILE.T128x192x32, 2), (api.TILE.T128x192x32_ALONE, 4)])
+@pytest.mark.parametrize("patience", ["1", "8"])
+def test_gemm_slices_that_give_up_waiting_for_their_siblings(tile, split, patience, monkeypatch):
+    # one poll, or a few: most tiles are given up and added up by the slice that arrives last, others still shared.  The same
+    # sums in the same order, launch after launch (the counters re-arm)
+    print("patience", patience, "tile", tile, "slices", split, flush=True)
+    M, N, K = 300, 392, 2048
+    a = uniform_f16((M, K), 35)
+    b = normal_f16((K, N), 36, std=0.05)
+    plain = run_gemm(a, b, tile, split_k=split, epilogue=api.EPI.GELU)
+    monkeypatch.setenv("CUSYNC_SLICE_PATIENCE", patience)
+    given_up = run_gemm(a, b, tile, split_k=split, epilogue=api.EPI.GELU, shared_reduction=1, launches=5)
+    assert np.array_equal(plain.view(np.uint16), given_up.view(np.uint16))
+
+
 @pytest.mark.parametrize("tile,M,N,split", [(api.TILE.D128x192x64, 300, 9 * 192, 2), (api.TILE.T256x192x64, 1000, 13 * 192, 4),
                                             (api.TILE.T256x192x64, 700, 3 * 192, 2), (api.TILE.D32x128x64, 20, 11 * 128, 3)])
 def test_gemm_tiles_that_do_not_divide_among_the_xcds(tile, M, N, split):

@@ -146,25 +146,12 @@ def test_split_times_add_up():
     assert np.allclose(np.array(g1) + np.array(g2), total, atol=0.02) and min(g1) > 0 and min(g2) > 0
 
 
-def test_two_launches_of_several_gemms_at_once():
-    # two handles run from two host threads, both GEMMs of each in one launch whose workgroups wait for each other; 64x128 tiles
-    # leave a CU to two workgroups in every kernel, and two times 240 fit the device
+def run_two_at_once(handles, bufs):
+    """50 passes of each handle from a host thread of its own; every output is what the handle gave alone."""
     import threading
     import torch
-    from cusync_amd import _lib
-    print("two launches at once", flush=True)
-    L = _lib.load()
-    assert [L.cusync_gemm_max_resident(t) // L.cusync_gemm_max_resident(api.TILE.T256x192x64) for t in
-            (api.TILE.D32x128x64, api.TILE.D64x128x64, api.TILE.D64x192x64)] == [1, 2, 1]
-    hidden, inner, rows = 12288, 6144, 64
-    w1, w2 = to_dev(normal_f16((hidden, inner), 2, std=0.02)), to_dev(normal_f16((inner, hidden), 3, std=0.02))
-    bufs = [(to_dev(uniform_f16((rows, hidden), 4 + k)), empty_dev((rows, inner)), empty_dev((rows, hidden))) for k in range(2)]
-    torch.cuda.synchronize()
-    tile = api.TILE.D64x128x64
-    handles = [api.Mlp(api.MODEL.GPT3, rows, hidden, inner, api.SYNC.ROW, w1.data_ptr(), w2.data_ptr(), tile1=tile, tile2=tile, one_launch=True) for _ in bufs]
     alone, failed = [], []
     for h, (x, mid, y) in zip(handles, bufs):
-        assert int(np.prod(h.stage_state(0).grid)) <= L.cusync_gemm_max_resident(tile) // 2
         h.run(x.data_ptr(), mid.data_ptr(), y.data_ptr())
         alone.append(y.clone())
         y.fill_(float("nan"))
@@ -186,3 +173,37 @@ def test_two_launches_of_several_gemms_at_once():
     for (x, mid, y), want, h in zip(bufs, alone, handles):
         assert torch.equal(y.view(torch.int16), want.view(torch.int16))
         h.destroy()
+
+
+def test_two_launches_of_several_gemms_at_once():
+    # both GEMMs of a handle in one launch whose workgroups wait for each other; 64x128 tiles leave a CU to two workgroups in
+    # every kernel, and two times 240 fit the device
+    import torch
+    from cusync_amd import _lib
+    print("two launches at once", flush=True)
+    L = _lib.load()
+    assert [L.cusync_gemm_max_resident(t) // L.cusync_gemm_max_resident(api.TILE.T256x192x64) for t in
+            (api.TILE.D32x128x64, api.TILE.D64x128x64, api.TILE.D64x192x64)] == [1, 2, 1]
+    hidden, inner, rows = 12288, 6144, 64
+    w1, w2 = to_dev(normal_f16((hidden, inner), 2, std=0.02)), to_dev(normal_f16((inner, hidden), 3, std=0.02))
+    bufs = [(to_dev(uniform_f16((rows, hidden), 4 + k)), empty_dev((rows, inner)), empty_dev((rows, hidden))) for k in range(2)]
+    torch.cuda.synchronize()
+    tile = api.TILE.D64x128x64
+    handles = [api.Mlp(api.MODEL.GPT3, rows, hidden, inner, api.SYNC.ROW, w1.data_ptr(), w2.data_ptr(), tile1=tile, tile2=tile, one_launch=True) for _ in bufs]
+    assert all(int(np.prod(h.stage_state(0).grid)) <= L.cusync_gemm_max_resident(tile) // 2 for h in handles)
+    run_two_at_once(handles, bufs)
+
+
+@pytest.mark.parametrize("rows", [300, 512])
+def test_two_launches_whose_slices_wait_for_each_other_at_once(rows):
+    # GEMM1 of a LLaMA MLP, 174 or 232 workgroups to a handle on 256 CUs: each handle's slices may hold the CUs the other's
+    # siblings need, and then give their tiles up
+    import torch
+    print("two launches of slices at once", rows, flush=True)
+    hidden, inner = 8192, 2752
+    w1, w2 = to_dev(normal_f16((hidden, 2 * inner), 2, std=0.02)), to_dev(normal_f16((inner, hidden), 3, std=0.02))
+    bufs = [(to_dev(uniform_f16((rows, hidden), 4 + k)), empty_dev((rows, inner)), empty_dev((rows, hidden))) for k in range(2)]
+    torch.cuda.synchronize()
+    handles = [api.Mlp(api.MODEL.LLAMA, rows, hidden, inner, api.SYNC.ROW, w1.data_ptr(), w2.data_ptr()) for _ in bufs]
+    assert handles[0].splits()[0] > 1
+    run_two_at_once(handles, bufs)
