@@ -133,7 +133,7 @@ struct DynStage {
   static __device__ __forceinline__ uint32_t homeList() { return workgroupIndex() & 7u; }
 
   // Counts this workgroup as started; give the result to finishStart() later
-  // (after other work has been issued, so that the round trip is hidden).
+  // (after the first loads have been issued, so that they are not behind the round trip).
   __device__ __forceinline__ uint32_t beginStart() const {
     if (!isProducer() || (d.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL)) return 0;
     return dev::ticketAdd(d.startCounter, 1);
@@ -142,7 +142,9 @@ struct DynStage {
   __device__ __forceinline__ void finishStart(uint32_t token, uint32_t launched, unsigned long long entered) const {
     if (entered) stamp(0, entered);
     if (!isProducer() || (d.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL)) return;
-    asm volatile("" : "+v"(token));        // looked at here and not before: the count's round trip is over by now
+    // Looked at here and not before.  The prologue's loads are inline assembly, which the compiler does not count, so the wait
+    // it places for the count is for everything this wavefront has sent out: its share of the prologue, and the stamp.
+    asm volatile("" : "+v"(token));
     if (token == launched - 1) {
       dev::storeRelaxed(d.startCounter, 0);
       // The flag says that every producer workgroup is on the device and publishes no data (a consumer reads the
@@ -165,7 +167,8 @@ struct DynStage {
   }
   // At kernel entry: the clock for the stamp of the launch's start, 0 where this workgroup makes none.  finishStart()
   // stores it, behind the first loads: a wavefront's counter of memory operations goes down in order, so what is loaded
-  // after a store to the host's memory waits for its way over the bus, and the first workgroup held up its tile by 2.4 us.
+  // after a store to the host's memory waits for its way over the bus, and the first workgroup's loads were 2.4 us late.
+  // (A producer's first wavefront still waits for that store before its first MFMA, in finishStart, with its loads under way.)
   __device__ __forceinline__ unsigned long long enter() const {
     return (d.flags & CUSYNC_STAGE_STAMPS_START) && workgroupIndex() == 0 ? wall_clock64() : 0;
   }
