@@ -23,6 +23,7 @@
 #include "rt_internal.h"
 #include "gemm_kernel_dma.h"
 #include "conv3x3_kernel.h"
+#include "conv3x3_solo_kernel.h"
 #include "split_choice.h"
 
 namespace {
@@ -43,6 +44,8 @@ struct ConvTile {
 #define CUSYNC_CONV_TILE(BM, BN, BK, WM, WN, ST, OCC) \
   { BM, BN, BK, kThreads, (size_t)DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>::LDS_BYTES, \
     gemmDmaKernel<DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>, kAConv>, -1, nullptr, nullptr, nullptr }
+#define CUSYNC_SOLO_TILE(CFG) \
+  { CFG::BM, 2 * CFG::BN, CFG::BK, CFG::THREADS, 0, convHaloSoloKernel<CFG, false>, -1, nullptr, convHaloSoloKernel<CFG, true>, CFG::ldsBytes }
 #define CUSYNC_HALO_TILE(CFG) \
   { CFG::BM, CFG::BN, CFG::BK, CFG::THREADS, 0, convHalo3x3Kernel<CFG>, -1, convHalo3x3ChainKernel<CFG>, convHalo3x3Kernel<CFG, true>, CFG::ldsBytes }
 
@@ -51,8 +54,10 @@ using HaloB = Halo3x3Cfg<128, 128, 2, 2, 3, 2, 2>;    // 128 output channels per
 using HaloC = Halo3x3Cfg<64, 128, 2, 2, 3, 2, 2>;     // 64 pixels: what fits beside the halo of 512-channel pixels (7 x 7 images)
 using HaloCPair = Halo3x3Cfg<64, 128, 2, 2, 3, 2>;    // the same tile where two of them fit a CU (convTileFor)
 
-constexpr int kHaloCPair = CUSYNC_CONV_TILE_COUNT;
-ConvTile g_convTiles[CUSYNC_CONV_TILE_COUNT + 1] = {
+using Solo128 = HaloSoloCfg<128, 2, 1>;     // 64 columns of the 128x128 and of the 64x128 tile (soloTileFor)
+using Solo64 = HaloSoloCfg<64, 2, 1>;
+constexpr int kHaloCPair = CUSYNC_CONV_TILE_COUNT, kSolo128 = kHaloCPair + 1, kSolo64 = kHaloCPair + 2, kConvKernels = kHaloCPair + 3;
+ConvTile g_convTiles[kConvKernels] = {
   CUSYNC_CONV_TILE(128, 64, 32, 2, 2, 4, 3),    // CUSYNC_CONV_TILE_128x64x32
   CUSYNC_CONV_TILE(128, 128, 32, 2, 2, 4, 2),   // CUSYNC_CONV_TILE_128x128x32
   CUSYNC_CONV_TILE(256, 64, 32, 4, 1, 3, 2),    // CUSYNC_CONV_TILE_256x64x32
@@ -61,6 +66,8 @@ ConvTile g_convTiles[CUSYNC_CONV_TILE_COUNT + 1] = {
   CUSYNC_HALO_TILE(HaloB),      // CUSYNC_CONV_TILE_HALO_128x128x64
   CUSYNC_HALO_TILE(HaloC),      // CUSYNC_CONV_TILE_HALO_64x128x64
   CUSYNC_HALO_TILE(HaloCPair),
+  CUSYNC_SOLO_TILE(Solo128),
+  CUSYNC_SOLO_TILE(Solo64),
 };
 
 bool isHalo(int tile) { return tile >= 0 && tile < CUSYNC_CONV_TILE_COUNT && g_convTiles[tile].haloLds; }
@@ -93,7 +100,7 @@ ConvTile* convTileFor(int tile, uint32_t W, uint32_t C) {
 }
 
 int g_convNumCUs = 0;
-uint32_t g_haloLds[CUSYNC_CONV_TILE_COUNT + 1] = {};      // LDS size the cached occupancy of a halo kernel was computed for
+uint32_t g_haloLds[kConvKernels] = {};      // LDS size the cached occupancy of a halo kernel was computed for
 
 int residentConv(ConvTile* ti, size_t lds) {
   std::lock_guard<std::mutex> lock(g_convMutex);
@@ -127,6 +134,18 @@ int residentConv(ConvTile* ti, size_t lds) {
     if (halo) g_haloLds[idx] = (uint32_t)lds;
   }
   return ti->residentPerCU * g_convNumCUs;
+}
+
+// The kernel of conv3x3_solo_kernel.h, where a tile's split_k workgroups can be its two halves of columns times one, two or four
+// runs and every one of the launch's `parts` has a workgroup from the start; null elsewhere (three runs, five, a cap, several
+// rounds: the tile's own kernel with its steps in runs).  Where both can run, this one is ahead at every size measured: pairs
+// under RowSync, us, runs -> this, 128x128 tile in two 1x14x14x256 45 -> 33, 32x14x14x256 47 -> 36, in four 8x14x14x256 39.2 -> 34.0;
+// 64x128 tile in two 32x7x7x512 49.6 -> 42.2, in four 16x7x7x512 40.3 -> 37.1, in eight 2x7x7x512 34.4 -> 30.4.
+ConvTile* soloTileFor(int tile, int split, uint32_t parts, uint32_t W, uint32_t C) {
+  if ((split != 2 && split != 4 && split != 8) || (tile != CUSYNC_CONV_TILE_HALO_128x128x64 && tile != CUSYNC_CONV_TILE_HALO_64x128x64)) return nullptr;
+  ConvTile* ti = &g_convTiles[tile == CUSYNC_CONV_TILE_HALO_128x128x64 ? kSolo128 : kSolo64];
+  const uint32_t lds = ti->haloLds(W, C);
+  return lds <= kMaxLds && parts <= (uint32_t)residentConv(ti, lds) ? ti : nullptr;
 }
 
 uint32_t outExtent(uint32_t in, uint32_t filter, uint32_t pad, uint32_t stride) { return (in + 2 * pad - filter) / stride + 1; }
@@ -269,17 +288,18 @@ int cusync_conv2d_max_resident(int tile) {
 cusync_error cusync_conv2d_run(const cusync_conv2d_args* a, void* stream) {
   cusync_error e = cusync_conv2d_can_implement(a);
   if (e != CUSYNC_SUCCESS) return e;
-  ConvTile* ti = convTileFor(a->tile, a->W, a->C);
+  const uint32_t tiles = a->stage.grid.x * a->stage.grid.y * a->stage.grid.z;
+  ConvTile* ti = soloTileFor(a->tile, a->split_k, tiles, a->W, a->C);
+  if (!ti || (a->max_workgroups > 0 && (uint32_t)a->max_workgroups < tiles)) ti = convTileFor(a->tile, a->W, a->C);
   const size_t lds = ti->haloLds ? ti->haloLds(a->W, a->C) : ti->lds;
   const int resident = residentConv(ti, lds);
   if (resident <= 0) { cusync::rt::setError("conv2d: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
-  const cusync_stage_desc& s = a->stage;
-  const uint32_t tiles = s.grid.x * s.grid.y * s.grid.z;
   uint32_t launched = std::min<uint32_t>(tiles, (uint32_t)resident);
   if (a->max_workgroups > 0) launched = std::min<uint32_t>(launched, (uint32_t)a->max_workgroups);
 
   GemmParams p = convParams(a, ti, launched);
-  hipLaunchKernelGGL(a->split_k > 1 ? ti->splitKernel : ti->kernel, dim3(launched), dim3(ti->threads), lds, (hipStream_t)stream, p);
+  const bool solo = ti == &g_convTiles[kSolo128] || ti == &g_convTiles[kSolo64];
+  hipLaunchKernelGGL(a->split_k > (solo ? 2 : 1) ? ti->splitKernel : ti->kernel, dim3(launched), dim3(ti->threads), lds, (hipStream_t)stream, p);
   if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
   cusync::rt::noteLaunch(a->stage, launched >= (uint32_t)resident);
   return CUSYNC_SUCCESS;
@@ -337,6 +357,22 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
   if (cfg->layers < 1 || cfg->layers > 16) { setError("conv chain: 1 to 16 layers"); return nullptr; }
   cusync_conv_chain* c = new cusync_conv_chain();
   c->cfg = *cfg;
+  // The built-in choice, 128 channels and more: two workgroups to a tile, its halves of columns (soloTileFor), where all of the
+  // launch are resident; 64 rows a tile before 128, which leaves fewer CUs idle and makes each workgroup's serial way shorter
+  // (pairs under RowSync, us, 128 -> 64 rows: 1x14x14x256 32.8 -> 26.2, 20x14x14x256 34.5 -> 30.7, 8x28x28x128 27.8 -> 24.5).  Tiles of
+  // 512 channels are cut into runs as well while every one still has a workgroup and 18 units (2x7x7x512 34.2 -> 30.5 in four
+  // runs a half, 16x7x7x512 40.8 -> 37.1 in two); at 256 channels a cut costs in the exchange what it saves (8x14x14x256 27.2 -> 28.4).
+  c->splitK = 0;
+  if (c->cfg.tile < 0 && cfg->split_k == 0 && !(cfg->fused && cfg->sync != CUSYNC_SYNC_STREAM) && cfg->C % 128 == 0) {
+    for (int tile : {CUSYNC_CONV_TILE_HALO_64x128x64, CUSYNC_CONV_TILE_HALO_128x128x64}) {
+      const cusync_dim3 g = cusync_conv2d_grid_split(tile, cfg->N, cfg->H, cfg->W, cfg->C, 3, 3, 1, 1, 2);
+      if (g.x * g.y == 0 || !haloEligible(tile, cfg->W, cfg->C, 3, 3, 1, 1) || !soloTileFor(tile, 2, g.x * g.y * g.z, cfg->W, cfg->C)) continue;
+      c->cfg.tile = tile; c->splitK = 2;
+      const uint32_t units = 9 * (cfg->C / 64);
+      while (units > 36 && c->splitK < 8 && units / c->splitK >= 18 && soloTileFor(tile, c->splitK * 2, g.x * g.y * c->splitK * 2, cfg->W, cfg->C)) c->splitK *= 2;
+      break;
+    }
+  }
   if (c->cfg.tile < 0)
     c->cfg.tile = cfg->C % 128 == 0 && haloEligible(CUSYNC_CONV_TILE_HALO_128x128x64, cfg->W, cfg->C, 3, 3, 1, 1) ? CUSYNC_CONV_TILE_HALO_128x128x64
                   : haloEligible(CUSYNC_CONV_TILE_HALO_256x64x64, cfg->W, cfg->C, 3, 3, 1, 1) ? CUSYNC_CONV_TILE_HALO_256x64x64
@@ -359,9 +395,8 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
   // 1x7x7x512 82 -> 43 in eight; with shorter runs the exchange costs more than the idle CUs: 1x56x56x64 35 -> 50
   // in nine runs of one step), and a number the 32-row pieces of a 128-row tile divide among, so that the runs
   // share the adding up.
-  c->splitK = 1;
-  if (cfg->split_k > 1) c->splitK = cfg->split_k;
-  else if (cfg->split_k == 0 && isHalo(c->cfg.tile) && !(c->cfg.fused && cfg->sync != CUSYNC_SYNC_STREAM)) {
+  if (cfg->split_k > 0) c->splitK = cfg->split_k;
+  else if (c->splitK == 0 && isHalo(c->cfg.tile) && !(c->cfg.fused && cfg->sync != CUSYNC_SYNC_STREAM)) {
     ConvTile* ti = convTileFor(c->cfg.tile, cfg->W, cfg->C);
     const int resident = residentConv(ti, ti->haloLds(cfg->W, cfg->C));
     const uint32_t tiles = g.x * g.y, steps = 9 * (cfg->C / 64);
@@ -370,6 +405,7 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
     while (s > 1 && (steps + s - 1) / s * (s - 1) >= steps) s--;      // no run without steps
     c->splitK = (int)std::max(1u, s);
   }
+  c->splitK = std::max(1, c->splitK);
   if (c->splitK > 1 && (!isHalo(c->cfg.tile) || (c->cfg.fused && cfg->sync != CUSYNC_SYNC_STREAM))) {
     setError("conv chain: cutting a tile's steps into runs needs a halo tile and one launch per layer");
     delete c;
@@ -393,6 +429,7 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
       post.kind = CUSYNC_POLICY_ROWSYNC; post.order = CUSYNC_ORDER_TRANSPOSE_XY;
       post.tileM = tm; post.tileN = 1; post.waitValue = g.x; post.postValue = 1;
       wait = post;
+      opts = CUSYNC_OPT_REORDER_TILE_LOADS;      // the filters are the chain's own inputs, written by no layer
       break;
     case CUSYNC_SYNC_TILE:
       post.kind = CUSYNC_POLICY_TILESYNC; post.order = CUSYNC_ORDER_TRANSPOSE_XY;

@@ -78,5 +78,19 @@ CUSYNC_HD uint32_t onlyTicket(const cusync_dim3& grid, uint32_t launched, uint32
   return b / 8 < listTiles(grid, b & 7u) ? listTicket(grid, b & 7u, b / 8, turn) : leftOver(grid, launched, b, turn);
 }
 
+// The tile of workgroup b of such a launch where only the rows matter for locality (a convolution's): the tiles in the order
+// row by row, all columns and parts of a row together, are cut into eight runs whose lengths differ by one at most.  Every
+// list has a tile for each of its workgroups then, and the tile is two divisions away from the index.
+CUSYNC_HD cusync_dim3 evenTile(const cusync_dim3& grid, uint32_t tiles, uint32_t b) {
+  const uint32_t x = b & 7u, rest = tiles & 7u, at = x * (tiles >> 3) + (x < rest ? x : rest) + (b >> 3);
+  const uint32_t perRow = grid.x * grid.z;
+  cusync_dim3 t;
+  t.y = at / perRow;
+  const uint32_t in = at - t.y * perRow;
+  t.z = in / grid.x;
+  t.x = in - t.z * grid.x;
+  return t;
+}
+
 }  // namespace deal
 }  // namespace cusync

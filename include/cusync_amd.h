@@ -373,13 +373,14 @@ typedef struct cusync_conv2d_args {
   uint32_t K, R, S;            /* filter w[K,R,S,C]  fp16 KRSC, cross-correlation (CV/resnet.cu:678) */
   uint32_t pad, stride;        /* same in both directions; output y[N,P,Q,K], P = (H+2*pad-R)/stride+1 */
   const void *x;
-  const void *w;
+  const void *w;               /* a consumer stage with CUSYNC_OPT_REORDER_TILE_LOADS may read it before its wait for the producer */
   void *y;
   int32_t epilogue;            /* CUSYNC_EPILOGUE_* (the ResNet pair uses RELU after the first convolution) */
   int32_t tile;                /* CUSYNC_CONV_TILE_* */
   int32_t max_workgroups;      /* 0 = as many as stay resident */
   int32_t split_k;             /* Conv2dProblemSize::split_k_slices (CV/resnet.cu:246, 689, 765): 0 or 1 = none; n (halo tiles):
-                                  the R*S*C/64 steps of a tile in n runs, grid z = n, partial sums added in run order */
+                                  a tile is n workgroups', grid z = n: the R*S*C/64 steps in n runs, partial sums added in run
+                                  order, or (128x128 and 64x128 tiles, n = 2, 4, 8, all resident) n/2 runs of each half of the columns */
   void *workspace;             /* split_k > 1: cusync_conv2d_workspace_size bytes, 16-byte aligned; its counters (the last
                                   2 * tiles words) zero before the first run, the kernel leaves them zero */
 } cusync_conv2d_args;
@@ -414,8 +415,8 @@ typedef struct cusync_conv_chain_config {
   int32_t fused;               /* 1 (sync ROW or TILE, halo tiles, at most 8 layers): all layers in ONE launch whose workgroups
                                   work through layer 0, then layer 1, ... with the same semaphores between them; no wait
                                   kernel and no second launch between a producer and its consumer */
-  int32_t split_k;             /* --split_k_slices (CV/resnet.cu:329): runs a tile's steps are cut into; 1 = none; 0 = the
-                                  library picks (runs only for layers whose tiles leave more than half the CUs idle) */
+  int32_t split_k;             /* --split_k_slices (CV/resnet.cu:329): workgroups a tile is divided among; 1 = one; 0 = the
+                                  library picks (more only for layers whose tiles leave CUs idle) */
 } cusync_conv_chain_config;
 
 typedef struct cusync_conv_chain cusync_conv_chain;
