@@ -24,6 +24,7 @@
 #include "gemm_kernel_dma.h"
 #include "conv3x3_kernel.h"
 #include "conv3x3_solo_kernel.h"
+#include "conv3x3_rows_kernel.h"
 #include "split_choice.h"
 
 namespace {
@@ -146,6 +147,31 @@ ConvTile* soloTileFor(int tile, int split, uint32_t parts, uint32_t W, uint32_t 
   ConvTile* ti = &g_convTiles[tile == CUSYNC_CONV_TILE_HALO_128x128x64 ? kSolo128 : kSolo64];
   const uint32_t lds = ti->haloLds(W, C);
   return lds <= kMaxLds && parts <= (uint32_t)residentConv(ti, lds) ? ti : nullptr;
+}
+
+using RowsKernel = void (*)(GemmParams);
+RowsKernel rowsKernel(int epilogue) { return epilogue == CUSYNC_EPILOGUE_RELU ? convRowsKernel<CUSYNC_EPILOGUE_RELU> : convRowsKernel<CUSYNC_EPILOGUE_NONE>; }
+
+// The device's CUs, once convRowsKernel has its LDS allowance; 0 after an error.
+int rowsCUs() {
+  static const int cus = [] {
+    int dev = 0;
+    hipDeviceProp_t prop;
+    if (CUSYNC_HIP(hipGetDevice(&dev)) || CUSYNC_HIP(hipGetDeviceProperties(&prop, dev))) return 0;
+    for (int epilogue : {CUSYNC_EPILOGUE_NONE, CUSYNC_EPILOGUE_RELU})
+      if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(rowsKernel(epilogue)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds))) return 0;
+    return prop.multiProcessorCount;
+  }();
+  return cus;
+}
+
+// Rows of the product per workgroup of convRowsKernel (conv3x3_rows_kernel.h) for a layer of 64 channels, a workgroup per CU: whole
+// sixteens, no fewer than four wavefronts have work for; 0 where its input tile and the filter do not fit the LDS.
+uint32_t rowsPerWorkgroup(uint32_t N, uint32_t H, uint32_t W) {
+  const uint32_t M = N * H * W, cus = (uint32_t)rowsCUs();
+  if (!cus) return 0;
+  const uint32_t rows = std::max<uint32_t>(ConvRowsCfg::WAVES * ConvRowsCfg::T, ((M + cus - 1) / cus + ConvRowsCfg::T - 1) / ConvRowsCfg::T * ConvRowsCfg::T);
+  return ConvRowsCfg::ldsBytes(rows, W) <= kMaxLds ? rows : 0;
 }
 
 uint32_t outExtent(uint32_t in, uint32_t filter, uint32_t pad, uint32_t stride) { return (in + 2 * pad - filter) / stride + 1; }
@@ -317,6 +343,7 @@ struct cusync_conv_chain {
   std::vector<hipEvent_t> done;      // behind the run's last launch on each stream (see rt::waitEnd)
   std::vector<void*> ws;             // per layer: partial sums and counters of the runs a tile's steps are cut into
   int splitK = 1;
+  uint32_t rows = 0;                 // rows of the product per workgroup of convRowsKernel, 0: the tile's own kernel
   uint32_t timeoutsSeen = 0;         // sum of the stages' give-up counters when the last run returned
   bool broken = false;               // a run failed behind a launch (see rt::abandonRun)
 };
@@ -336,6 +363,18 @@ cusync_policy_desc noSyncDesc() {
   p.kind = CUSYNC_POLICY_NOSYNC;
   p.tileM = p.tileN = 1; p.R = p.S = 1;
   return p;
+}
+
+// One layer by rows (conv3x3_rows_kernel.h).  The arguments are checked.
+cusync_error runRows(const cusync_conv2d_args* a, uint32_t rows, void* counters, hipStream_t stream) {
+  const uint32_t launched = (a->N * a->H * a->W + rows - 1) / rows;
+  GemmParams p = convParams(a, convTile(a->tile), launched);
+  p.kPerSlice = rows;
+  p.arrivals = (uint32_t*)counters;
+  hipLaunchKernelGGL(rowsKernel(a->epilogue), dim3(launched), dim3(ConvRowsCfg::THREADS), ConvRowsCfg::ldsBytes(rows, a->W), stream, p);
+  if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
+  cusync::rt::noteLaunch(a->stage, launched >= (uint32_t)rowsCUs());
+  return CUSYNC_SUCCESS;
 }
 
 void freeChain(cusync_conv_chain* c) {
@@ -378,6 +417,12 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
                   : haloEligible(CUSYNC_CONV_TILE_HALO_256x64x64, cfg->W, cfg->C, 3, 3, 1, 1) ? CUSYNC_CONV_TILE_HALO_256x64x64
                   : cfg->C % 128 == 0 && haloEligible(CUSYNC_CONV_TILE_HALO_64x128x64, cfg->W, cfg->C, 3, 3, 1, 1) ? CUSYNC_CONV_TILE_HALO_64x128x64
                   : cfg->C % 128 == 0 ? CUSYNC_CONV_TILE_128x128x32 : CUSYNC_CONV_TILE_256x64x32;
+  // 64 channels, the built-in choice: tiles of 256 rows for the policies, the rows themselves dealt evenly to the CUs.
+  if (cfg->tile < 0 && cfg->split_k <= 1 && cfg->C == ConvRowsCfg::CHANNELS && c->cfg.tile == CUSYNC_CONV_TILE_HALO_256x64x64 &&
+      !(cfg->fused && cfg->sync != CUSYNC_SYNC_STREAM)) {
+    c->rows = rowsPerWorkgroup(cfg->N, cfg->H, cfg->W);
+    c->splitK = 1;
+  }
   uint32_t tm = 0, tn = 0;
   if (cusync_conv2d_tile_shape(c->cfg.tile, &tm, &tn, nullptr)) { setError("conv chain: unknown tile id"); delete c; return nullptr; }
   if (c->cfg.fused && cfg->sync != CUSYNC_SYNC_STREAM &&
@@ -471,12 +516,12 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
   c->st[0].flags |= CUSYNC_STAGE_STAMPS_START;
   for (uint32_t i = 0; i < cfg->layers; i++)
     if (!oneLaunch || i + 1 == cfg->layers) c->st[i].flags |= CUSYNC_STAGE_STAMPS_END;
-  if (c->splitK > 1) {
+  if (c->splitK > 1 || c->rows) {
     cusync_conv2d_args a;
     memset(&a, 0, sizeof a);
     a.N = cfg->N; a.H = cfg->H; a.W = cfg->W; a.C = cfg->C; a.K = cfg->C; a.R = a.S = 3; a.pad = 1; a.stride = 1;
     a.tile = c->cfg.tile; a.split_k = c->splitK;
-    const size_t bytes = cusync_conv2d_workspace_size(&a);
+    const size_t bytes = c->rows ? (size_t)g.x * g.y * sizeof(uint32_t) : cusync_conv2d_workspace_size(&a);
     for (uint32_t i = 0; i < cfg->layers; i++) {
       void* w = nullptr;
       if (CUSYNC_HIP(hipMalloc(&w, bytes)) || CUSYNC_HIP(hipMemset(w, 0, bytes))) { if (w) (void)hipFree(w); freeChain(c); return nullptr; }
@@ -550,7 +595,7 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
       // where that layer's launch left workgroup slots free (392 tiles on 512 slots for the benchmark shapes), so
       // that the wait kernel's wave takes nothing from the producer; from this thread where the launch took them all.
       if (overlapped && i > 0 && (e = cusync_hold_back(&c->st[i - 1], s)) != CUSYNC_SUCCESS) return failed(e);
-      if ((e = cusync_conv2d_run(&a, s)) != CUSYNC_SUCCESS) return i ? failed(e) : e;
+      if ((e = c->rows ? runRows(&a, c->rows, c->ws[i], s) : cusync_conv2d_run(&a, s)) != CUSYNC_SUCCESS) return i ? failed(e) : e;
     }
     for (uint32_t i = 0; i < (overlapped ? n : 1); i++) if (CUSYNC_HIP(hipEventRecord(c->done[i], c->stream[i]))) return failed(CUSYNC_ERROR_DEVICE);
     for (uint32_t i = n; i-- > (overlapped ? 0 : n - 1);) {

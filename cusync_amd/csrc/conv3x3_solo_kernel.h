@@ -78,6 +78,10 @@ __device__ __forceinline__ void convHaloSoloTile(const GemmParams& p) {
 
   const unsigned long long tlEntry = p.timeline ? wall_clock64() : 0;
   const unsigned long long entered = stage.enter();
+  // What a wavefront loads behind the start count arrives behind it, 1 to 3 us when hundreds of workgroups count at once: the one
+  // that counts leaves the halo to the others.
+  const bool counts = stage.countsStart();
+  const uint32_t loaders = counts ? C::KG - 1 : C::KG, loader = counts ? wave - 1 : wave;       // (all ones where it has nothing to load)
   const uint32_t startToken = tid == 0 ? stage.beginStart() : 0;
   cusync_dim3 t;
   if (stage.noDraws && (stage.d.flags & CUSYNC_STAGE_IDENTITY_ORDER)) t = deal::evenTile(stage.d.grid, p.launched, blockIdx.x);
@@ -121,7 +125,7 @@ __device__ __forceinline__ void convHaloSoloTile(const GemmParams& p) {
     }
   }
   // Halo, as in conv3x3_kernel.h.
-  for (uint32_t q = wave; q < haloLoads; q += C::KG) {
+  for (uint32_t q = loader; q < haloLoads; q += loaders) {
     const uint32_t byteOff = q * 1024 + lane * 16;
     const uint32_t pl = byteOff >> pixShift, slot = (byteOff & (pixBytes - 1)) >> 4;
     const uint32_t chunk = slot ^ ((pl >> swzShift) & cprMask);

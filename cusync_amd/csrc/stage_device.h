@@ -134,14 +134,15 @@ struct DynStage {
 
   // Counts this workgroup as started; give the result to finishStart() later
   // (after the first loads have been issued, so that they are not behind the round trip).
+  __device__ __forceinline__ bool countsStart() const { return isProducer() && !(d.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL); }
   __device__ __forceinline__ uint32_t beginStart() const {
-    if (!isProducer() || (d.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL)) return 0;
+    if (!countsStart()) return 0;
     return dev::ticketAdd(d.startCounter, 1);
   }
   // The workgroup that started last raises the wait-kernel flag.
   __device__ __forceinline__ void finishStart(uint32_t token, uint32_t launched, unsigned long long entered) const {
     if (entered) stamp(0, entered);
-    if (!isProducer() || (d.opts & CUSYNC_OPT_AVOID_WAIT_KERNEL)) return;
+    if (!countsStart()) return;
     // Looked at here and not before.  The prologue's loads are inline assembly, which the compiler does not count, so the wait
     // it places for the count is for everything this wavefront has sent out: its share of the prologue, and the stamp.
     asm volatile("" : "+v"(token));
@@ -388,16 +389,18 @@ struct DynStage {
     // for stores to memory.  Every wavefront sees its own stores of the tile through before it reaches the barrier.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) {
-      const uint32_t idx = dyn::tileIndex(d.out, tile, d.grid) * CUSYNC_SEM_STRIDE;
-      const uint32_t v = dyn::postValue(d.out) * times;
-      if (writtenThrough && !releaseAll) {
-        if (d.opts & CUSYNC_OPT_NO_ATOMIC_ADD) dev::storeRelaxed(&d.tileStatusWrite[idx], v * (uint32_t)d.iter);
-        else __hip_atomic_fetch_add((uint32_t*)&d.tileStatusWrite[idx], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      } else {
-        if (d.opts & CUSYNC_OPT_NO_ATOMIC_ADD) dev::releaseStore(&d.tileStatusWrite[idx], v * (uint32_t)d.iter);
-        else dev::releaseAdd(&d.tileStatusWrite[idx], v);
-      }
+    if (threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) raise(tile, times, writtenThrough);
+  }
+  // The post itself, by one thread, once all stores of the tile are known to be out.
+  __device__ __forceinline__ void raise(const cusync_dim3& tile, uint32_t times, bool writtenThrough) const {
+    const uint32_t idx = dyn::tileIndex(d.out, tile, d.grid) * CUSYNC_SEM_STRIDE;
+    const uint32_t v = dyn::postValue(d.out) * times;
+    if (writtenThrough && !releaseAll) {
+      if (d.opts & CUSYNC_OPT_NO_ATOMIC_ADD) dev::storeRelaxed(&d.tileStatusWrite[idx], v * (uint32_t)d.iter);
+      else __hip_atomic_fetch_add((uint32_t*)&d.tileStatusWrite[idx], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      if (d.opts & CUSYNC_OPT_NO_ATOMIC_ADD) dev::releaseStore(&d.tileStatusWrite[idx], v * (uint32_t)d.iter);
+      else dev::releaseAdd(&d.tileStatusWrite[idx], v);
     }
   }
 };
