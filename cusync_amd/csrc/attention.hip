@@ -18,6 +18,7 @@
 #include "attention_kernel.h"
 #include "attention_few_kernel.h"
 #include "split_choice.h"
+#include "gemm_resident.h"
 
 namespace {
 
@@ -97,6 +98,7 @@ struct cusync_attn_layer {
   uint32_t E;                      // heads * head_dim
   int tile1, tile3;
   int split1, split3;              // k-slices of the two projections
+  uint32_t resident3;              // the output projection holds its weights in registers (gemm_resident.h), this many columns a workgroup; 0: it does not
   void* ws1;
   void* ws3;                       // their split-K workspaces (null without slices)
   uint32_t kvSplit;                // key/value blocks per attention workgroup, 0 = no split
@@ -329,9 +331,16 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   const cusync_dim3 flat3 = cusync_gemm_grid(L->tile3, cfg->seq, cfg->hidden, 1);
   L->split1 = cusync::gemm::pickSplitToFill(flat1.x * flat1.y, tm1, cfg->hidden, bk1, cusync_gemm_max_resident(L->tile1), cusync::gemm::sliceUnit(L->tile1));
   L->split3 = cusync::gemm::pickSplit(0, flat3.x * flat3.y, L->E, bk3, cusync_gemm_max_resident(L->tile3), cusync::gemm::sliceUnit(L->tile3));
+  // Few rows: the output projection reads its weights while the attention, on a few CUs, is under way.  Not under
+  // AvoidWaitKernel, where its workgroups might hold what the stages in front of it need.
+  const int givenOpts = cfg->opts >= 0 ? cfg->opts : 0;
   const cusync_dim3 g1 = cusync_gemm_grid(L->tile1, cfg->seq, 3 * L->E, L->split1);
   const cusync_dim3 g2 = cusync_attention_grid_split(cfg->seq, cfg->heads, cfg->cached_rows, L->kvSplit);
-  const cusync_dim3 g3 = cusync_gemm_grid(L->tile3, cfg->seq, cfg->hidden, L->split3);
+  if (cfg->tile3 < 0 && !(givenOpts & CUSYNC_OPT_AVOID_WAIT_KERNEL) && cusync::gemm::weightsFitRegisters(cfg->seq, cfg->hidden, L->E)) {
+    L->resident3 = cusync::gemm::residentColumns(cfg->hidden, cfg->sync == CUSYNC_SYNC_STREAM ? 0 : g2.x * g2.y * g2.z);
+    L->split3 = 1;
+  }
+  const cusync_dim3 g3 = L->resident3 ? cusync::gemm::residentGrid(cfg->hidden, L->resident3) : cusync_gemm_grid(L->tile3, cfg->seq, cfg->hidden, L->split3);
 
   cusync_policy_desc sync1 = noSync(), sync2 = noSync();
   int opts = 0;
@@ -451,8 +460,10 @@ cusync_error cusync_attn_layer_run(cusync_attn_layer* L, const void* x, void* qk
 
     hipStream_t s0 = L->stream[0], s1 = overlapped ? L->stream[1] : s0, s2 = overlapped ? L->stream[2] : s0;
     cusync_error e;
+    cusync_gemm_args checked3 = a3;
+    if (L->resident3) checked3.stage.grid = cusync_gemm_grid(L->tile3, S, H, 1);      // everything else is the tiles' to check
     if (r == 0 && ((e = cusync_gemm_can_implement(&a1)) != CUSYNC_SUCCESS || (e = cusync_attention_can_implement(&a2)) != CUSYNC_SUCCESS ||
-                   (e = cusync_gemm_can_implement(&a3)) != CUSYNC_SUCCESS)) return e;      // before anything is launched
+                   (e = cusync_gemm_can_implement(&checked3)) != CUSYNC_SUCCESS)) return e;      // before anything is launched
     auto failed = [&](cusync_error why) { return cusync::rt::abandonRun(L->stream, 3, &L->broken, why); };
     if ((e = cusync_gemm_run(&a1, s0)) != CUSYNC_SUCCESS) return e;
     // overlapped: each consumer's stream is held back until every workgroup of its producer has started: from the
@@ -461,7 +472,7 @@ cusync_error cusync_attn_layer_run(cusync_attn_layer* L, const void* x, void* qk
     if (overlapped && (e = cusync_hold_back(&L->st[0], s1)) != CUSYNC_SUCCESS) return failed(e);
     if ((e = cusync_attention_run(&a2, s1)) != CUSYNC_SUCCESS) return failed(e);
     if (overlapped && (e = cusync_hold_back(&L->st[1], s2)) != CUSYNC_SUCCESS) return failed(e);
-    if ((e = cusync_gemm_run(&a3, s2)) != CUSYNC_SUCCESS) return failed(e);
+    if ((e = L->resident3 ? cusync::gemm::residentRun(&a3, L->resident3, s2) : cusync_gemm_run(&a3, s2)) != CUSYNC_SUCCESS) return failed(e);
     hipStream_t on[3] = {s0, s1, s2};
     for (int i = overlapped ? 0 : 2; i < 3; i++) if (CUSYNC_HIP(hipEventRecord(L->done[i], on[i]))) return failed(CUSYNC_ERROR_DEVICE);
     for (int i = 2; i >= (overlapped ? 0 : 2); i--)
