@@ -6,13 +6,13 @@
 namespace cusync {
 namespace gemm {
 
-// K up to 1536 is what the registers hold.  Up to 128 rows, where it is still ahead (128 rows, 12 heads, hidden 12288, under RowSync
-// 84.0 -> 82.4 us, behind 1000 98.6 -> 96.9) while each 16 rows more cost it 1.7 us and the tiles none.  Columns for half the CUs
-// at least and one round at most: hidden 8192, 16 rows behind 1000 51.7 -> 47.0, 16384 68.5 -> 59.9; with 3 heads, whose K is a
-// quarter, 39.4 -> 38.9.
+// K up to 1536 is what the registers hold.  Up to 112 rows: each 16 rows more cost it 1.7 us (2 with 128 columns) and the tiles none
+// (12 heads, hidden 12288, under RowSync, tiles / this: 112 rows behind 2000 93.7 / 92.4, behind 4000 99.3 / 97.9; 128 rows behind 2000
+// 94.6 / 95.5, behind 8000 107.7 / 108.7, without a cache 84.0 / 82.4).  Columns for half the CUs at least and one round at most: hidden
+// 8192, 16 rows behind 1000 51.7 -> 47.0, 16384 68.5 -> 59.9; with 3 heads, whose K is a quarter, 39.4 -> 38.9.
 inline bool weightsFitRegisters(uint32_t M, uint32_t N, uint32_t K) {
   const uint32_t tiles = (N + 63) / 64;
-  return M <= 128 && K <= 1536 && tiles >= 128 && tiles <= 256;
+  return M <= 112 && K <= 1536 && tiles >= 128 && tiles <= 256;
 }
 // Columns of a workgroup: 64, which reads its weights in half the time, where each has a CU of its own beside the `others`
 // workgroups of the stage in front of it (32 rows behind 100 under RowSync, 48 of them, 128 columns / 64: 57.2 / 56.0 us, in stream

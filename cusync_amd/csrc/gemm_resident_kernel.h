@@ -11,7 +11,7 @@
 //
 // The layer, 12 heads, hidden 12288, us, tiles in k-slices -> this: 16 rows behind 2048 under RowSync 60.8 -> 55.0, TileSync 58.6 ->
 // 53.3; 32 behind 2048 62.3 -> 58.3; 1 behind 64 53.0 -> 47.1; without a cache under RowSync 16 rows 53.7 -> 51.1, 64 64.9 -> 61.1,
-// 96 82.0 -> 77.7, 128 84.0 -> 82.4; in stream order 48 rows 67.8 -> 63.0, 80 rows 82.5 -> 79.2.
+// 96 82.0 -> 77.7, 112 83.1 -> 79.9; in stream order 48 rows 67.8 -> 63.0, 80 rows 82.5 -> 79.2.
 //
 // A workgroup has a CU's LDS to itself although it would do with half: two to a CU, half the CUs read all the weights, and 16 rows
 // behind 2048 took 61.4 us.
@@ -26,7 +26,7 @@ namespace gemm {
 template<int BN_>
 struct ResidentCfg {
   static constexpr int BN = BN_, COLS = BN / 16, ROWS = 16, WAVES = 8, THREADS = WAVES * 64, KS = 32, STEPS = 6;
-  static constexpr uint32_t MAX_ROWS = 128, MAX_K = WAVES * STEPS * KS;
+  static constexpr uint32_t MAX_ROWS = 112, MAX_K = WAVES * STEPS * KS;
   static constexpr int A_BYTES = STEPS * 1024;                    // of a wavefront: 16 rows of its k, a KiB per k-step
   static constexpr int BUFFERS = 2;                               // 16 rows being multiplied, 16 on their way
   static constexpr int PITCH = BN + 4;                            // floats
