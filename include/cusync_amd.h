@@ -498,6 +498,8 @@ void cusync_attn_layer_destroy(cusync_attn_layer *layer);
 cusync_error cusync_attn_layer_run(cusync_attn_layer *layer, const void *x, void *qkv, void *o, void *y, int runs,
                                    double *times_us, double *stage_us);
 const cusync_stage_desc *cusync_attn_layer_stage(const cusync_attn_layer *layer, int which);
+/* The projections' tiles.  With tile3 left to the layer, up to 112 rows the output projection can hold its weights in registers instead:
+ * its grid is then 64 or 128 columns to a workgroup, without k-slices, and tile3 the one it takes the place of. */
 int cusync_attn_layer_tiles(const cusync_attn_layer *layer, int *tile1, int *tile3);
 
 /* ------------------------------------------------------------------------- */
