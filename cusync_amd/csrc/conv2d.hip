@@ -142,7 +142,10 @@ int residentConv(ConvTile* ti, size_t lds) {
 // rounds: the tile's own kernel with its steps in runs).  Where both can run, this one is ahead at every size measured: pairs
 // under RowSync, us, runs -> this, 128x128 tile in two 1x14x14x256 45 -> 33, 32x14x14x256 47 -> 36, in four 8x14x14x256 39.2 -> 34.0;
 // 64x128 tile in two 32x7x7x512 49.6 -> 42.2, in four 16x7x7x512 40.3 -> 37.1, in eight 2x7x7x512 34.4 -> 30.4.
-ConvTile* soloTileFor(int tile, int split, uint32_t parts, uint32_t W, uint32_t C) {
+// Not under AvoidWaitKernel (`opts`): its caller has seen to it that all stages fit on the device at once, by the tile and what
+// cusync_conv2d_max_resident says of it, and here a workgroup has a CU to itself.
+ConvTile* soloTileFor(int tile, int split, uint32_t parts, uint32_t W, uint32_t C, int opts) {
+  if (opts & CUSYNC_OPT_AVOID_WAIT_KERNEL) return nullptr;
   if ((split != 2 && split != 4 && split != 8) || (tile != CUSYNC_CONV_TILE_HALO_128x128x64 && tile != CUSYNC_CONV_TILE_HALO_64x128x64)) return nullptr;
   ConvTile* ti = &g_convTiles[tile == CUSYNC_CONV_TILE_HALO_128x128x64 ? kSolo128 : kSolo64];
   const uint32_t lds = ti->haloLds(W, C);
@@ -315,7 +318,7 @@ cusync_error cusync_conv2d_run(const cusync_conv2d_args* a, void* stream) {
   cusync_error e = cusync_conv2d_can_implement(a);
   if (e != CUSYNC_SUCCESS) return e;
   const uint32_t tiles = a->stage.grid.x * a->stage.grid.y * a->stage.grid.z;
-  ConvTile* ti = soloTileFor(a->tile, a->split_k, tiles, a->W, a->C);
+  ConvTile* ti = soloTileFor(a->tile, a->split_k, tiles, a->W, a->C, a->stage.opts);
   if (!ti || (a->max_workgroups > 0 && (uint32_t)a->max_workgroups < tiles)) ti = convTileFor(a->tile, a->W, a->C);
   const size_t lds = ti->haloLds ? ti->haloLds(a->W, a->C) : ti->lds;
   const int resident = residentConv(ti, lds);
@@ -401,14 +404,19 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
   // (pairs under RowSync, us, 128 -> 64 rows: 1x14x14x256 32.8 -> 26.2, 20x14x14x256 34.5 -> 30.7, 8x28x28x128 27.8 -> 24.5).  Tiles of
   // 512 channels are cut into runs as well while every one still has a workgroup and 18 units (2x7x7x512 34.2 -> 30.5 in four
   // runs a half, 16x7x7x512 40.8 -> 37.1 in two); at 256 channels a cut costs in the exchange what it saves (8x14x14x256 27.2 -> 28.4).
+  // Under AvoidWaitKernel neither this nor the rows below: both take a CU for each of more workgroups than the tile's own
+  // kernel has (a pair of 8x28x28x128 is 392 of them and fits as 196), and a consumer that comes first would hold its producer's.
+  // (Whatever the sync, so that results do not depend on it.)
+  const int givenOpts = cfg->opts >= 0 ? cfg->opts : 0;
+  const bool ownKernels = !(givenOpts & CUSYNC_OPT_AVOID_WAIT_KERNEL) && !(cfg->fused && cfg->sync != CUSYNC_SYNC_STREAM);
   c->splitK = 0;
-  if (c->cfg.tile < 0 && cfg->split_k == 0 && !(cfg->fused && cfg->sync != CUSYNC_SYNC_STREAM) && cfg->C % 128 == 0) {
+  if (c->cfg.tile < 0 && cfg->split_k == 0 && ownKernels && cfg->C % 128 == 0) {
     for (int tile : {CUSYNC_CONV_TILE_HALO_64x128x64, CUSYNC_CONV_TILE_HALO_128x128x64}) {
       const cusync_dim3 g = cusync_conv2d_grid_split(tile, cfg->N, cfg->H, cfg->W, cfg->C, 3, 3, 1, 1, 2);
-      if (g.x * g.y == 0 || !haloEligible(tile, cfg->W, cfg->C, 3, 3, 1, 1) || !soloTileFor(tile, 2, g.x * g.y * g.z, cfg->W, cfg->C)) continue;
+      if (g.x * g.y == 0 || !haloEligible(tile, cfg->W, cfg->C, 3, 3, 1, 1) || !soloTileFor(tile, 2, g.x * g.y * g.z, cfg->W, cfg->C, givenOpts)) continue;
       c->cfg.tile = tile; c->splitK = 2;
       const uint32_t units = 9 * (cfg->C / 64);
-      while (units > 36 && c->splitK < 8 && units / c->splitK >= 18 && soloTileFor(tile, c->splitK * 2, g.x * g.y * c->splitK * 2, cfg->W, cfg->C)) c->splitK *= 2;
+      while (units > 36 && c->splitK < 8 && units / c->splitK >= 18 && soloTileFor(tile, c->splitK * 2, g.x * g.y * c->splitK * 2, cfg->W, cfg->C, givenOpts)) c->splitK *= 2;
       break;
     }
   }
@@ -418,8 +426,7 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
                   : cfg->C % 128 == 0 && haloEligible(CUSYNC_CONV_TILE_HALO_64x128x64, cfg->W, cfg->C, 3, 3, 1, 1) ? CUSYNC_CONV_TILE_HALO_64x128x64
                   : cfg->C % 128 == 0 ? CUSYNC_CONV_TILE_128x128x32 : CUSYNC_CONV_TILE_256x64x32;
   // 64 channels, the built-in choice: tiles of 256 rows for the policies, the rows themselves dealt evenly to the CUs.
-  if (cfg->tile < 0 && cfg->split_k <= 1 && cfg->C == ConvRowsCfg::CHANNELS && c->cfg.tile == CUSYNC_CONV_TILE_HALO_256x64x64 &&
-      !(cfg->fused && cfg->sync != CUSYNC_SYNC_STREAM)) {
+  if (cfg->tile < 0 && cfg->split_k <= 1 && cfg->C == ConvRowsCfg::CHANNELS && c->cfg.tile == CUSYNC_CONV_TILE_HALO_256x64x64 && ownKernels) {
     c->rows = rowsPerWorkgroup(cfg->N, cfg->H, cfg->W);
     c->splitK = 1;
   }
