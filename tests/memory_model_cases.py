@@ -5,7 +5,8 @@ The library's shortcuts around the plain release/acquire protocol (posts without
 went through, waits without a cache invalidation over whole-line tiles, a host-side hold-back instead of the
 wait kernel) may only change timing: the parent compares the digests of the processes with each other.
 
-usage: python memory_model_cases.py out.json"""
+usage: python memory_model_cases.py out.json [few]        few: the kernels for few tiles and few rows, which hand over by counts of
+their own or wait with one wavefront for all"""
 import hashlib
 import json
 import os
@@ -87,10 +88,29 @@ def main(path):
     for sync, tag in ((api.SYNC.ROW, "row"), (api.SYNC.TILE, "tile")):
         print("conv 56x56x64", tag, flush=True)
         conv_case(out, "conv_56x56x64_%s" % tag, 32, 56, 56, 64, 2, sync)
+    write(path, out)
+
+
+def main_few(path):
+    out = {}
+    # two halves of columns to a tile; halves whose units are cut into four runs; runs of rows in several tiles, tiles of several runs
+    for N, H, W, Cc in ((32, 14, 14, 256), (2, 7, 7, 512), (6, 56, 56, 64)):
+        for sync, tag in ((api.SYNC.ROW, "row"), (api.SYNC.TILE, "tile")):
+            print("conv", N, H, W, Cc, tag, flush=True)
+            conv_case(out, "conv_%dx%dx%dx%d_%s" % (N, H, W, Cc, tag), N, H, W, Cc, 3, sync)
+    # the output projection with its weights in registers, behind the few-row attention and behind the general one
+    for S in (16, 64):
+        for sync, tag in ((api.SYNC.ROW, "row"), (api.SYNC.TILE, "tile"), (api.SYNC.STRIDED, "strided")):
+            print("attention", S, tag, flush=True)
+            attention_case(out, "attention_s%d_%s" % (S, tag), S, 12288, 12, sync)
+    write(path, out)
+
+
+def write(path, out):
     with open(path, "w") as f:
         json.dump(out, f, indent=1, sort_keys=True)
     print("wrote", path, flush=True)
 
 
 if __name__ == "__main__":
-    main(sys.argv[1])
+    (main_few if sys.argv[2:] == ["few"] else main)(sys.argv[1])

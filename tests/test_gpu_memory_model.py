@@ -23,26 +23,39 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 SWITCHES = ("CUSYNC_FORCE_ACQUIRE", "CUSYNC_FORCE_RELEASE", "CUSYNC_WAIT_KERNEL")
 
 
-def run_child(tmp_path, name, env_extra):
+def run_child(tmp_path, name, env_extra, *group):
     env = {k: v for k, v in os.environ.items() if k not in SWITCHES}
     env.update(env_extra)
     out = tmp_path / (name + ".json")
-    print("child", name, env_extra, flush=True)
-    r = subprocess.run([sys.executable, "-u", os.path.join(HERE, "memory_model_cases.py"), str(out)], env=env,
+    print("child", name, env_extra, *group, flush=True)
+    r = subprocess.run([sys.executable, "-u", os.path.join(HERE, "memory_model_cases.py"), str(out), *group], env=env,
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=400, text=True)
     assert r.returncode == 0, "child %s failed:\n%s" % (name, r.stdout[-4000:])
     with open(out) as f:
         return json.load(f)
 
 
+SETTINGS = (("acquire", {"CUSYNC_FORCE_ACQUIRE": "1"}),
+            ("release", {"CUSYNC_FORCE_RELEASE": "1"}),
+            ("wait_kernel", {"CUSYNC_WAIT_KERNEL": "1"}),
+            ("plain_protocol", {"CUSYNC_FORCE_ACQUIRE": "1", "CUSYNC_FORCE_RELEASE": "1", "CUSYNC_WAIT_KERNEL": "1"}))
+
+
 def test_protocol_shortcuts_change_no_bit(tmp_path):
     base = run_child(tmp_path, "default", {})
     assert len(base) == 9
-    for name, env in (("acquire", {"CUSYNC_FORCE_ACQUIRE": "1"}),
-                      ("release", {"CUSYNC_FORCE_RELEASE": "1"}),
-                      ("wait_kernel", {"CUSYNC_WAIT_KERNEL": "1"}),
-                      ("plain_protocol", {"CUSYNC_FORCE_ACQUIRE": "1", "CUSYNC_FORCE_RELEASE": "1", "CUSYNC_WAIT_KERNEL": "1"})):
+    for name, env in SETTINGS:
         got = run_child(tmp_path, name, env)
+        assert got.keys() == base.keys()
+        for case in base:
+            assert got[case] == base[case], "%s differs under %s: %r vs %r" % (case, env, got[case], base[case])
+
+
+def test_protocol_shortcuts_change_no_bit_of_few_tiles_and_few_rows(tmp_path):
+    base = run_child(tmp_path, "default", {}, "few")
+    assert len(base) == 12
+    for name, env in SETTINGS:
+        got = run_child(tmp_path, name, env, "few")
         assert got.keys() == base.keys()
         for case in base:
             assert got[case] == base[case], "%s differs under %s: %r vs %r" % (case, env, got[case], base[case])
