@@ -26,6 +26,7 @@
 #include "conv3x3_solo_kernel.h"
 #include "conv3x3_rows_kernel.h"
 #include "split_choice.h"
+#include "occupancy_table.h"
 
 namespace {
 
@@ -36,7 +37,6 @@ struct ConvTile {
   uint32_t threads;
   size_t lds;
   void (*kernel)(GemmParams);
-  int residentPerCU;
   void (*chainKernel)(ConvChainParams);     // several layers in one launch; halo tiles only
   void (*splitKernel)(GemmParams);          // the same tile with its steps cut into runs (split_k > 1); halo tiles only
   uint32_t (*haloLds)(uint32_t W, uint32_t C);      // a launch's LDS for images of width W with C channels; halo tiles only
@@ -44,11 +44,11 @@ struct ConvTile {
 
 #define CUSYNC_CONV_TILE(BM, BN, BK, WM, WN, ST, OCC) \
   { BM, BN, BK, kThreads, (size_t)DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>::LDS_BYTES, \
-    gemmDmaKernel<DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>, kAConv>, -1, nullptr, nullptr, nullptr }
+    gemmDmaKernel<DmaCfg<BM, BN, BK, WM, WN, ST, OCC, true>, kAConv>, nullptr, nullptr, nullptr }
 #define CUSYNC_SOLO_TILE(CFG) \
-  { CFG::BM, 2 * CFG::BN, CFG::BK, CFG::THREADS, 0, convHaloSoloKernel<CFG, false>, -1, nullptr, convHaloSoloKernel<CFG, true>, CFG::ldsBytes }
+  { CFG::BM, 2 * CFG::BN, CFG::BK, CFG::THREADS, 0, convHaloSoloKernel<CFG, false>, nullptr, convHaloSoloKernel<CFG, true>, CFG::ldsBytes }
 #define CUSYNC_HALO_TILE(CFG) \
-  { CFG::BM, CFG::BN, CFG::BK, CFG::THREADS, 0, convHalo3x3Kernel<CFG>, -1, convHalo3x3ChainKernel<CFG>, convHalo3x3Kernel<CFG, true>, CFG::ldsBytes }
+  { CFG::BM, CFG::BN, CFG::BK, CFG::THREADS, 0, convHalo3x3Kernel<CFG>, convHalo3x3ChainKernel<CFG>, convHalo3x3Kernel<CFG, true>, CFG::ldsBytes }
 
 using HaloA = Halo3x3Cfg<256, 64, 4, 1, 4, 2>;     // 64 output channels per tile: four waves of 64 x 64 stacked
 using HaloB = Halo3x3Cfg<128, 128, 2, 2, 3, 2, 2>;    // 128 output channels per tile
@@ -101,40 +101,45 @@ ConvTile* convTileFor(int tile, uint32_t W, uint32_t C) {
 }
 
 int g_convNumCUs = 0;
-uint32_t g_haloLds[kConvKernels] = {};      // LDS size the cached occupancy of a halo kernel was computed for
+cusync::rt::OccupancyTable<kConvKernels, kMaxLds / 1024> g_convOccupancy;
+bool g_convLdsAllowed[kConvKernels] = {};
 
+// Whether all kernels of a tile may ask for the LDS they will (set once).
+bool allowConvLds(const ConvTile* ti) {
+  bool& allowed = g_convLdsAllowed[ti - g_convTiles];
+  if (allowed) return true;
+  const int most = ti->haloLds ? (int)kMaxLds : (int)ti->lds;
+  const void* kernels[3] = {reinterpret_cast<const void*>(ti->kernel), reinterpret_cast<const void*>(ti->chainKernel), reinterpret_cast<const void*>(ti->splitKernel)};
+  for (const void* k : kernels)
+    if (k && CUSYNC_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, most))) return false;
+  return allowed = true;
+}
+
+// Workgroups of a tile's launches, with `lds` bytes, that the device holds at once; 0 after an error.
 int residentConv(ConvTile* ti, size_t lds) {
   std::lock_guard<std::mutex> lock(g_convMutex);
-  const int idx = (int)(ti - g_convTiles);
-  const bool halo = ti->haloLds != nullptr;
-  if (ti->residentPerCU < 0 || (halo && g_haloLds[idx] != lds)) {
+  if (g_convNumCUs == 0) {
     int dev = 0;
     hipDeviceProp_t prop;
     if (CUSYNC_HIP(hipGetDevice(&dev)) || CUSYNC_HIP(hipGetDeviceProperties(&prop, dev))) return 0;
     g_convNumCUs = prop.multiProcessorCount;
-    if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ti->kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, halo ? (int)kMaxLds : (int)lds))) return 0;
-    int n = 0;
-    if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ti->kernel, (int)ti->threads, lds))) return 0;
+  }
+  if (!allowConvLds(ti)) return 0;
+  const int perCU = g_convOccupancy.perCU((int)(ti - g_convTiles), lds, [ti](size_t bytes) {
+    // the chain kernel is the same code in a loop, the split kernel the same with its steps in runs: the least of the three
+    int least = 0, n = 0;
+    if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&least, ti->kernel, (int)ti->threads, bytes))) return -1;
     if (ti->chainKernel) {
-      // the chain kernel is the same code in a loop: it gets the same LDS allowance and must fit as often
-      int m = 0;
-      if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ti->chainKernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds)) ||
-          CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, ti->chainKernel, (int)ti->threads, lds))) return 0;
-      n = std::min(n, m);
+      if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ti->chainKernel, (int)ti->threads, bytes))) return -1;
+      least = std::min(least, n);
     }
     if (ti->splitKernel) {
-      int m = 0;
-      if (CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ti->splitKernel),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds)) ||
-          CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, ti->splitKernel, (int)ti->threads, lds))) return 0;
-      n = std::min(n, m);
+      if (CUSYNC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ti->splitKernel, (int)ti->threads, bytes))) return -1;
+      least = std::min(least, n);
     }
-    ti->residentPerCU = n;
-    if (halo) g_haloLds[idx] = (uint32_t)lds;
-  }
-  return ti->residentPerCU * g_convNumCUs;
+    return least;
+  });
+  return std::max(0, perCU) * g_convNumCUs;
 }
 
 // The kernel of conv3x3_solo_kernel.h, where a tile's split_k workgroups can be its two halves of columns times one, two or four
@@ -318,8 +323,9 @@ cusync_error cusync_conv2d_run(const cusync_conv2d_args* a, void* stream) {
   cusync_error e = cusync_conv2d_can_implement(a);
   if (e != CUSYNC_SUCCESS) return e;
   const uint32_t tiles = a->stage.grid.x * a->stage.grid.y * a->stage.grid.z;
-  ConvTile* ti = soloTileFor(a->tile, a->split_k, tiles, a->W, a->C, a->stage.opts);
-  if (!ti || (a->max_workgroups > 0 && (uint32_t)a->max_workgroups < tiles)) ti = convTileFor(a->tile, a->W, a->C);
+  const bool capped = a->max_workgroups > 0 && (uint32_t)a->max_workgroups < tiles;
+  ConvTile* ti = capped ? nullptr : soloTileFor(a->tile, a->split_k, tiles, a->W, a->C, a->stage.opts);
+  if (!ti) ti = convTileFor(a->tile, a->W, a->C);
   const size_t lds = ti->haloLds ? ti->haloLds(a->W, a->C) : ti->lds;
   const int resident = residentConv(ti, lds);
   if (resident <= 0) { cusync::rt::setError("conv2d: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
