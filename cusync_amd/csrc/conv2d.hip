@@ -182,6 +182,9 @@ uint32_t rowsPerWorkgroup(uint32_t N, uint32_t H, uint32_t W) {
   return ConvRowsCfg::ldsBytes(rows, W) <= kMaxLds ? rows : 0;
 }
 
+// A launch's LDS for images of width W with C channels.
+size_t launchLds(const ConvTile* ti, uint32_t W, uint32_t C) { return ti->haloLds ? ti->haloLds(W, C) : ti->lds; }
+
 uint32_t outExtent(uint32_t in, uint32_t filter, uint32_t pad, uint32_t stride) { return (in + 2 * pad - filter) / stride + 1; }
 
 size_t partialBytes(const cusync_conv2d_args* a, const ConvTile* ti) {
@@ -189,8 +192,25 @@ size_t partialBytes(const cusync_conv2d_args* a, const ConvTile* ti) {
   return (size_t)g.z * g.y * g.x * ti->bm * ti->bn * sizeof(float);
 }
 
+// Where the workgroups of a tile hand over to one another: partial sums, and counters that are 0 between launches.
+struct ConvScratch {
+  void* partials;
+  size_t bytes;
+  void* counters;
+};
+
+bool isSolo(const ConvTile* ti) { return ti == &g_convTiles[kSolo128] || ti == &g_convTiles[kSolo64]; }
+
+// What a caller's workspace holds: [split_k][row tiles][column tiles][BM * BN] fp32 partial sums, then two counters per output
+// tile, as the GEMM's.
+ConvScratch workspaceOf(const cusync_conv2d_args* a, const ConvTile* ti) {
+  if (a->split_k <= 1) return {};
+  const size_t bytes = partialBytes(a, ti);
+  return {a->workspace, bytes, (char*)a->workspace + bytes};
+}
+
 // Kernel parameters of one convolution launched with `launched` workgroups.
-GemmParams convParams(const cusync_conv2d_args* a, const ConvTile* ti, uint32_t launched) {
+GemmParams convParams(const cusync_conv2d_args* a, const ConvTile* ti, uint32_t launched, const ConvScratch& scratch) {
   const cusync_stage_desc& s = a->stage;
   GemmParams p = {};
   p.stage.d = s;
@@ -210,15 +230,10 @@ GemmParams convParams(const cusync_conv2d_args* a, const ConvTile* ti, uint32_t 
   p.kPerSlice = (chunks + p.splitK - 1) / p.splitK * ti->bk;
   p.mPad = s.grid.y * ti->bm;
   p.waitRound = 1;
-  p.coopReduce = 0; p.partialBytes = 0;
-  p.partials = nullptr; p.arrivals = nullptr;
-  if (p.splitK > 1) {
-    // [split_k][row tiles][column tiles][BM * BN] fp32 partial sums, then two counters per output tile, as the GEMM's
-    const size_t bytes = partialBytes(a, ti);
-    p.partials = (float*)a->workspace;
-    p.arrivals = (uint32_t*)((char*)a->workspace + bytes);
-    p.partialBytes = (uint32_t)bytes;
-  }
+  p.coopReduce = 0;
+  p.partials = (float*)scratch.partials;
+  p.partialBytes = (uint32_t)scratch.bytes;
+  p.arrivals = (uint32_t*)scratch.counters;
   cusync::rt::timeline(&p.timeline, &p.timelineCap);
   // Producer tiles are whole 128-byte lines of the activation tensor when a pixel's channels are.
   p.stage.lineAligned = !cusync::rt::forceAcquire() && s.in.kind != CUSYNC_POLICY_NOSYNC && (uintptr_t)a->x % 128 == 0 &&
@@ -227,6 +242,20 @@ GemmParams convParams(const cusync_conv2d_args* a, const ConvTile* ti, uint32_t 
   p.stage.releaseAll = cusync::rt::forceRelease();
   p.stage.prepare(launched);
   return p;
+}
+
+// One launch; the arguments are checked.  `resident`: residentConv of the kernel and these bytes of LDS.
+cusync_error launchConv(const cusync_conv2d_args* a, ConvTile* ti, int resident, const ConvScratch& scratch, hipStream_t stream) {
+  if (resident <= 0) { cusync::rt::setError("conv2d: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
+  const uint32_t tiles = a->stage.grid.x * a->stage.grid.y * a->stage.grid.z;
+  uint32_t launched = std::min<uint32_t>(tiles, (uint32_t)resident);
+  if (a->max_workgroups > 0) launched = std::min<uint32_t>(launched, (uint32_t)a->max_workgroups);
+  GemmParams p = convParams(a, ti, launched, scratch);
+  const bool split = a->split_k > (isSolo(ti) ? 2 : 1);
+  hipLaunchKernelGGL(split ? ti->splitKernel : ti->kernel, dim3(launched), dim3(ti->threads), launchLds(ti, a->W, a->C), stream, p);
+  if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
+  cusync::rt::noteLaunch(a->stage, launched >= (uint32_t)resident);
+  return CUSYNC_SUCCESS;
 }
 
 }  // namespace
@@ -316,7 +345,7 @@ cusync_error cusync_conv2d_can_implement(const cusync_conv2d_args* a) {
 int cusync_conv2d_max_resident(int tile) {
   ConvTile* ti = convTileFor(tile, 56, 64);
   if (!ti) return 0;
-  return residentConv(ti, ti->haloLds ? ti->haloLds(56, 64) : ti->lds);     // the halo tiles: for 56 x 56 x 64 images
+  return residentConv(ti, launchLds(ti, 56, 64));     // the halo tiles: for 56 x 56 x 64 images
 }
 
 cusync_error cusync_conv2d_run(const cusync_conv2d_args* a, void* stream) {
@@ -326,18 +355,7 @@ cusync_error cusync_conv2d_run(const cusync_conv2d_args* a, void* stream) {
   const bool capped = a->max_workgroups > 0 && (uint32_t)a->max_workgroups < tiles;
   ConvTile* ti = capped ? nullptr : soloTileFor(a->tile, a->split_k, tiles, a->W, a->C, a->stage.opts);
   if (!ti) ti = convTileFor(a->tile, a->W, a->C);
-  const size_t lds = ti->haloLds ? ti->haloLds(a->W, a->C) : ti->lds;
-  const int resident = residentConv(ti, lds);
-  if (resident <= 0) { cusync::rt::setError("conv2d: kernel does not fit on a CU"); return CUSYNC_ERROR_DEVICE; }
-  uint32_t launched = std::min<uint32_t>(tiles, (uint32_t)resident);
-  if (a->max_workgroups > 0) launched = std::min<uint32_t>(launched, (uint32_t)a->max_workgroups);
-
-  GemmParams p = convParams(a, ti, launched);
-  const bool solo = ti == &g_convTiles[kSolo128] || ti == &g_convTiles[kSolo64];
-  hipLaunchKernelGGL(a->split_k > (solo ? 2 : 1) ? ti->splitKernel : ti->kernel, dim3(launched), dim3(ti->threads), lds, (hipStream_t)stream, p);
-  if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
-  cusync::rt::noteLaunch(a->stage, launched >= (uint32_t)resident);
-  return CUSYNC_SUCCESS;
+  return launchConv(a, ti, residentConv(ti, launchLds(ti, a->W, a->C)), workspaceOf(a, ti), (hipStream_t)stream);
 }
 
 }  // extern "C"
@@ -350,7 +368,10 @@ struct cusync_conv_chain {
   std::vector<cusync_stage_desc> st;
   std::vector<hipStream_t> stream;
   std::vector<hipEvent_t> done;      // behind the run's last launch on each stream (see rt::waitEnd)
-  std::vector<void*> ws;             // per layer: partial sums and counters of the runs a tile's steps are cut into
+  void* ws = nullptr;                // the layers' scratch: all counters, then all partial sums
+  size_t counterBytes = 0, partialBytes = 0;      // of a layer
+  ConvTile* kernel = nullptr;        // what a layer runs where each has a launch of its own and it is not by rows
+  int resident = 0;
   int splitK = 1;
   uint32_t rows = 0;                 // rows of the product per workgroup of convRowsKernel, 0: the tile's own kernel
   uint32_t timeoutsSeen = 0;         // sum of the stages' give-up counters when the last run returned
@@ -374,12 +395,17 @@ cusync_policy_desc noSyncDesc() {
   return p;
 }
 
+ConvScratch scratchOf(const cusync_conv_chain* c, uint32_t layer) {
+  char* ws = (char*)c->ws;
+  if (!ws) return {};
+  return {c->partialBytes ? ws + c->cfg.layers * c->counterBytes + layer * c->partialBytes : nullptr, c->partialBytes, ws + layer * c->counterBytes};
+}
+
 // One layer by rows (conv3x3_rows_kernel.h).  The arguments are checked.
-cusync_error runRows(const cusync_conv2d_args* a, uint32_t rows, void* counters, hipStream_t stream) {
+cusync_error runRows(const cusync_conv2d_args* a, uint32_t rows, const ConvScratch& scratch, hipStream_t stream) {
   const uint32_t launched = (a->N * a->H * a->W + rows - 1) / rows;
-  GemmParams p = convParams(a, convTile(a->tile), launched);
+  GemmParams p = convParams(a, convTile(a->tile), launched, scratch);
   p.kPerSlice = rows;
-  p.arrivals = (uint32_t*)counters;
   hipLaunchKernelGGL(rowsKernel(a->epilogue), dim3(launched), dim3(ConvRowsCfg::THREADS), ConvRowsCfg::ldsBytes(rows, a->W), stream, p);
   if (CUSYNC_HIP(hipGetLastError())) return CUSYNC_ERROR_DEVICE;
   cusync::rt::noteLaunch(a->stage, launched >= (uint32_t)rowsCUs());
@@ -389,7 +415,7 @@ cusync_error runRows(const cusync_conv2d_args* a, uint32_t rows, void* counters,
 void freeChain(cusync_conv_chain* c) {
   for (auto s : c->stream) (void)hipStreamSynchronize(s);
   for (auto& d : c->st) cusync_stage_free(&d);
-  for (auto w : c->ws) (void)hipFree(w);
+  if (c->ws) (void)hipFree(c->ws);
   for (auto e : c->done) (void)hipEventDestroy(e);
   for (auto s : c->stream) (void)hipStreamDestroy(s);
   delete c;
@@ -502,6 +528,23 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
       return nullptr;
   }
   if (cfg->opts >= 0) opts |= cfg->opts;
+  // (Asked for the same way as cusync_conv2d_run does; an error or a tile that does not fit shows there or in the checks of a run)
+  c->kernel = soloTileFor(c->cfg.tile, c->splitK, g.x * g.y * g.z, cfg->W, cfg->C, opts);
+  if (!c->kernel) c->kernel = convTileFor(c->cfg.tile, cfg->W, cfg->C);
+  c->resident = residentConv(c->kernel, launchLds(c->kernel, cfg->W, cfg->C));
+  // Counters, and what is added up through memory: nothing by rows and where two halves of columns share a tile, half a tile for each
+  // run of a half, a tile for each run.  Only the counters have to begin as 0.  In front of the stages: the copies that these make on the
+  // same stream are waited for, so the counters are 0 when a run begins on the chain's own streams.
+  if (c->splitK > 1 || c->rows) {
+    const size_t tiles = (size_t)g.x * g.y;
+    c->counterBytes = ((c->rows ? 1 : 2) * tiles * sizeof(uint32_t) + 127) / 128 * 128;
+    if (!c->rows && !(isSolo(c->kernel) && c->splitK == 2))
+      c->partialBytes = tiles * c->splitK * tm * (isSolo(c->kernel) ? tn / 2 : tn) * sizeof(float);
+    if (CUSYNC_HIP(hipMalloc(&c->ws, cfg->layers * (c->counterBytes + c->partialBytes))) || CUSYNC_HIP(hipMemset(c->ws, 0, cfg->layers * c->counterBytes))) {
+      freeChain(c);
+      return nullptr;
+    }
+  }
   c->st.resize(cfg->layers);
   for (uint32_t i = 0; i < cfg->layers; i++) memset(&c->st[i], 0, sizeof c->st[i]);
   for (uint32_t i = 0; i < cfg->layers; i++) {
@@ -529,18 +572,6 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
   c->st[0].flags |= CUSYNC_STAGE_STAMPS_START;
   for (uint32_t i = 0; i < cfg->layers; i++)
     if (!oneLaunch || i + 1 == cfg->layers) c->st[i].flags |= CUSYNC_STAGE_STAMPS_END;
-  if (c->splitK > 1 || c->rows) {
-    cusync_conv2d_args a;
-    memset(&a, 0, sizeof a);
-    a.N = cfg->N; a.H = cfg->H; a.W = cfg->W; a.C = cfg->C; a.K = cfg->C; a.R = a.S = 3; a.pad = 1; a.stride = 1;
-    a.tile = c->cfg.tile; a.split_k = c->splitK;
-    const size_t bytes = c->rows ? (size_t)g.x * g.y * sizeof(uint32_t) : cusync_conv2d_workspace_size(&a);
-    for (uint32_t i = 0; i < cfg->layers; i++) {
-      void* w = nullptr;
-      if (CUSYNC_HIP(hipMalloc(&w, bytes)) || CUSYNC_HIP(hipMemset(w, 0, bytes))) { if (w) (void)hipFree(w); freeChain(c); return nullptr; }
-      c->ws.push_back(w);
-    }
-  }
   return c;
 }
 
@@ -566,7 +597,7 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
     a.epilogue = (c->cfg.relu && i + 1 < n) ? CUSYNC_EPILOGUE_RELU : CUSYNC_EPILOGUE_NONE;
     a.tile = c->cfg.tile;
     a.split_k = c->splitK;
-    a.workspace = c->splitK > 1 ? c->ws[i] : nullptr;
+    a.workspace = c->splitK > 1 ? c->ws : nullptr;      // (for the checks)
     return a;
   };
   for (uint32_t i = 0; runs > 0 && i < n; i++) {      // before anything is launched
@@ -588,7 +619,7 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
       cp.layers = n;
       for (uint32_t i = 0; i < n; i++) {
         const cusync_conv2d_args a = layerArgs(i);
-        cp.layer[i] = convParams(&a, ti, launched);
+        cp.layer[i] = convParams(&a, ti, launched, {});
       }
       hipLaunchKernelGGL(ti->chainKernel, dim3(launched), dim3(ti->threads), lds, c->stream[0], cp);
       if (CUSYNC_HIP(hipGetLastError()) || CUSYNC_HIP(hipEventRecord(c->done[0], c->stream[0]))) return failed(CUSYNC_ERROR_DEVICE);
@@ -608,7 +639,8 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
       // where that layer's launch left workgroup slots free (392 tiles on 512 slots for the benchmark shapes), so
       // that the wait kernel's wave takes nothing from the producer; from this thread where the launch took them all.
       if (overlapped && i > 0 && (e = cusync_hold_back(&c->st[i - 1], s)) != CUSYNC_SUCCESS) return failed(e);
-      if ((e = c->rows ? runRows(&a, c->rows, c->ws[i], s) : cusync_conv2d_run(&a, s)) != CUSYNC_SUCCESS) return i ? failed(e) : e;
+      e = c->rows ? runRows(&a, c->rows, scratchOf(c, i), s) : launchConv(&a, c->kernel, c->resident, scratchOf(c, i), s);
+      if (e != CUSYNC_SUCCESS) return i ? failed(e) : e;
     }
     for (uint32_t i = 0; i < (overlapped ? n : 1); i++) if (CUSYNC_HIP(hipEventRecord(c->done[i], c->stream[i]))) return failed(CUSYNC_ERROR_DEVICE);
     for (uint32_t i = n; i-- > (overlapped ? 0 : n - 1);) {

@@ -69,3 +69,19 @@ def test_rounding_of_parts():
     for tile, parts in ((T128, 2), (T128, 4), (T64, 8)):
         x, w = uniform_f16((2, 14, 14, 256), 21), he_filters(256, 3, 3, 256, 22)
         assert_close(run_conv(x, w, tile, split_k=parts), orc.conv2d_nhwc(x, w), "y")
+
+
+def test_chain_allocates_what_it_adds_up():
+    # two halves of columns share a tile and add nothing up through memory: 16 layers of 20x14x14x256, 124 tiles of 64x128 each, had
+    # 130 MB of partial sums between them; 64 channels have a word per tile.  (What else a handle holds is far below this line.)
+    import torch
+    for shape, choice in (((20, 14, 14, 256), (T64, 2)), ((32, 56, 56, 64), (api.CONV_TILE.HALO_256x64x64, 1))):
+        Cc = shape[3]
+        dw = torch.zeros(Cc * 9 * Cc, dtype=torch.float16, device="cuda")
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        chain = api.ConvChain(*shape, [dw.data_ptr()] * 16, api.SYNC.STREAM)
+        taken = free - torch.cuda.mem_get_info()[0]
+        got = chain.tile(), chain.split()
+        chain.destroy()
+        assert got == choice and taken < 48 << 20, (shape, taken)
