@@ -377,25 +377,10 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   }
   if (cfg->opts >= 0) opts |= cfg->opts;
 
-  const cusync_dim3 grids[3] = {g1, g2, g3};
-  const cusync_policy_desc ins[3] = {noSync(), sync1, sync2}, outs[3] = {sync1, sync2, noSync()};
-  for (int i = 0; i < 3; i++) {
-    memset(&L->st[i], 0, sizeof L->st[i]);
-    L->st[i].grid = grids[i]; L->st[i].tileSize = {1, 1, 1}; L->st[i].iter = 1; L->st[i].opts = opts;
-    L->st[i].in = ins[i]; L->st[i].out = outs[i];
-    if (cusync_stage_create(&L->st[i], CUSYNC_ORDER_TRANSPOSE_XY) != CUSYNC_SUCCESS) { discardLayer(L); return nullptr; }
-  }
-  if (cfg->sync != CUSYNC_SYNC_STREAM &&
-      (cusync_set_producer_consumer_pair(&L->st[0], &L->st[1]) != CUSYNC_SUCCESS ||
-       cusync_set_producer_consumer_pair(&L->st[1], &L->st[2]) != CUSYNC_SUCCESS)) {
-    setError("attn layer: pairing the stages failed");
-    discardLayer(L);
-    return nullptr;
-  }
+  // ahead of the stages, which wait for what is cleared here (cusync_stage_alloc)
   for (int which = 0; which < 2; which++) {
     cusync_gemm_args a;
     memset(&a, 0, sizeof a);
-    a.stage = L->st[which == 0 ? 0 : 2];
     a.M = cfg->seq; a.N = which == 0 ? 3 * L->E : cfg->hidden; a.K = which == 0 ? cfg->hidden : L->E;
     a.tile = which == 0 ? L->tile1 : L->tile3;
     a.split_k = which == 0 ? L->split1 : L->split3;
@@ -411,6 +396,21 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
     a.seq = cfg->seq; a.heads = cfg->heads; a.cached_rows = cfg->cached_rows; a.kv_split_blocks = L->kvSplit;
     const size_t bytes = cusync_attention_workspace_size(&a);
     if (bytes && (CUSYNC_HIP(hipMalloc(&L->ws2, bytes)) || CUSYNC_HIP(hipMemset(L->ws2, 0, bytes)))) { discardLayer(L); return nullptr; }
+  }
+  const cusync_dim3 grids[3] = {g1, g2, g3};
+  const cusync_policy_desc ins[3] = {noSync(), sync1, sync2}, outs[3] = {sync1, sync2, noSync()};
+  for (int i = 0; i < 3; i++) {
+    memset(&L->st[i], 0, sizeof L->st[i]);
+    L->st[i].grid = grids[i]; L->st[i].tileSize = {1, 1, 1}; L->st[i].iter = 1; L->st[i].opts = opts;
+    L->st[i].in = ins[i]; L->st[i].out = outs[i];
+    if (cusync_stage_create(&L->st[i], CUSYNC_ORDER_TRANSPOSE_XY) != CUSYNC_SUCCESS) { discardLayer(L); return nullptr; }
+  }
+  if (cfg->sync != CUSYNC_SYNC_STREAM &&
+      (cusync_set_producer_consumer_pair(&L->st[0], &L->st[1]) != CUSYNC_SUCCESS ||
+       cusync_set_producer_consumer_pair(&L->st[1], &L->st[2]) != CUSYNC_SUCCESS)) {
+    setError("attn layer: pairing the stages failed");
+    discardLayer(L);
+    return nullptr;
   }
   for (int i = 0; i < 3; i++)
     if (CUSYNC_HIP(hipStreamCreateWithFlags(&L->stream[i], hipStreamNonBlocking))) { discardLayer(L); return nullptr; }

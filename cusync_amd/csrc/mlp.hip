@@ -486,6 +486,15 @@ cusync_mlp* cusync_mlp_create(const cusync_mlp_config* cfg, const void* w1, cons
 
   memset(&m->prod, 0, sizeof m->prod);
   memset(&m->cons, 0, sizeof m->cons);
+  // ahead of the stages, which wait for what is cleared here (cusync_stage_alloc)
+  for (int which = 0; which < 2; which++) {
+    cusync_gemm_args a = gemmArgs(m, which, nullptr, nullptr, nullptr);
+    const size_t bytes = cusync_gemm_workspace_size(&a);
+    if (bytes == 0) continue;
+    void* ws = nullptr;
+    if (CUSYNC_HIP(hipMalloc(&ws, bytes)) || CUSYNC_HIP(hipMemset(ws, 0, bytes))) { discard(m); return nullptr; }
+    (which == 0 ? m->ws1 : m->ws2) = ws;
+  }
   m->prod.grid = g1; m->prod.tileSize = {1, 1, 1}; m->prod.iter = 1; m->prod.opts = opts;
   m->prod.in = noSync(); m->prod.out = pol;
   m->cons.grid = g2; m->cons.tileSize = {1, 1, 1}; m->cons.iter = 1; m->cons.opts = opts;
@@ -514,14 +523,6 @@ cusync_mlp* cusync_mlp_create(const cusync_mlp_config* cfg, const void* w1, cons
       discard(m);
       return nullptr;
     }
-  }
-  for (int which = 0; which < 2; which++) {
-    cusync_gemm_args a = gemmArgs(m, which, nullptr, nullptr, nullptr);
-    const size_t bytes = cusync_gemm_workspace_size(&a);
-    if (bytes == 0) continue;
-    void* ws = nullptr;
-    if (CUSYNC_HIP(hipMalloc(&ws, bytes)) || CUSYNC_HIP(hipMemset(ws, 0, bytes))) { discard(m); return nullptr; }
-    (which == 0 ? m->ws1 : m->ws2) = ws;
   }
   // in one launch the second GEMM's end is the launch's
   m->prod.flags |= CUSYNC_STAGE_STAMPS_START | (m->cfg.one_launch ? 0 : CUSYNC_STAGE_STAMPS_END);

@@ -232,6 +232,10 @@ cusync_error cusync_stage_alloc(cusync_stage_desc* d, const cusync_dim3* host_ti
   d->spinTimeouts = (uint32_t*)shared;
   const bool producer = d->out.kind != CUSYNC_POLICY_NOSYNC;
   if (producer && !(d->opts & CUSYNC_OPT_AVOID_WAIT_KERNEL)) d->kernelExecuted = (uint32_t*)(counters + 3 * line);
+  if (producer) {
+    if (RT(hipMalloc((void**)&d->tileStatusWrite, sizeof(uint32_t) * n * CUSYNC_SEM_STRIDE))) return fail();
+    if (RT(hipMemset(d->tileStatusWrite, 0, sizeof(uint32_t) * n * CUSYNC_SEM_STRIDE))) return fail();
+  }
   bool identity = true;
   for (uint32_t i = 0; i < n && identity; i++) {
     const cusync_dim3& t = host_tile_order[i];
@@ -239,11 +243,10 @@ cusync_error cusync_stage_alloc(cusync_stage_desc* d, const cusync_dim3* host_ti
   }
   d->flags = identity ? CUSYNC_STAGE_IDENTITY_ORDER : 0;
   if (RT(hipMalloc((void**)&d->tileOrder, sizeof(cusync_dim3) * n))) return fail();
+  // Last: hipMemset of device memory returns before it is done, and the stage's kernels go to streams that are not ordered behind
+  // the one it is on.  This copy is on that stream and is waited for, so all that was cleared ahead of it is 0 from here on, the
+  // handles' workspaces included.
   if (RT(hipMemcpy(d->tileOrder, host_tile_order, sizeof(cusync_dim3) * n, hipMemcpyHostToDevice))) return fail();
-  if (producer) {
-    if (RT(hipMalloc((void**)&d->tileStatusWrite, sizeof(uint32_t) * n * CUSYNC_SEM_STRIDE))) return fail();
-    if (RT(hipMemset(d->tileStatusWrite, 0, sizeof(uint32_t) * n * CUSYNC_SEM_STRIDE))) return fail();
-  }
   return CUSYNC_SUCCESS;
 }
 
