@@ -310,8 +310,8 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   // 2048 328 / 299; 64 heads, 512 rows behind 64: 194 / 217 and 203 / 210).
   const uint32_t kvBlocks = (cfg->cached_rows + cfg->seq + kBKV - 1) / kBKV;
   uint32_t perSplit = kvBlocks >= 8 ? (kvBlocks + 1) / 2 : 0u;
+  if (residentAttention(kShallow) <= 0) { discardLayer(L); return nullptr; }      // reads the device's CU count
   if (cfg->cached_rows) {
-    if (residentAttention(kShallow) <= 0) { discardLayer(L); return nullptr; }      // reads the device's CU count
     const uint32_t rowTiles = (cfg->seq + kBQ - 1) / kBQ, most = std::max(1u, (uint32_t)g_attnNumCUs / (cfg->heads * rowTiles));
     perSplit = std::max((kvBlocks + most - 1) / most, rowTiles > 1 ? 8u : 1u);
     while (perSplit * perSplit < kvBlocks) perSplit++;
@@ -336,9 +336,10 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   const int givenOpts = cfg->opts >= 0 ? cfg->opts : 0;
   const cusync_dim3 g1 = cusync_gemm_grid(L->tile1, cfg->seq, 3 * L->E, L->split1);
   const cusync_dim3 g2 = cusync_attention_grid_split(cfg->seq, cfg->heads, cfg->cached_rows, L->kvSplit);
-  if (cfg->tile3 < 0 && !(givenOpts & CUSYNC_OPT_AVOID_WAIT_KERNEL) && cusync::gemm::weightsFitRegisters(cfg->seq, cfg->hidden, L->E)) {
-    L->resident3 = cusync::gemm::residentColumns(cfg->hidden, cfg->sync == CUSYNC_SYNC_STREAM ? 0 : g2.x * g2.y * g2.z);
+  if (cfg->tile3 < 0 && !(givenOpts & CUSYNC_OPT_AVOID_WAIT_KERNEL) && cusync::gemm::weightsFitRegisters(cfg->seq, cfg->hidden, L->E, (uint32_t)g_attnNumCUs)) {
+    L->resident3 = cusync::gemm::residentColumns(cfg->hidden, cfg->sync == CUSYNC_SYNC_STREAM ? 0 : g2.x * g2.y * g2.z, (uint32_t)g_attnNumCUs);
     L->split3 = 1;
+    if (!cusync::gemm::residentReady(L->resident3)) { discardLayer(L); return nullptr; }
   }
   const cusync_dim3 g3 = L->resident3 ? cusync::gemm::residentGrid(cfg->hidden, L->resident3) : cusync_gemm_grid(L->tile3, cfg->seq, cfg->hidden, L->split3);
 

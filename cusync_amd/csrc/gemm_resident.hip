@@ -7,6 +7,12 @@ namespace cusync {
 namespace gemm {
 
 template<class C>
+static bool ready() {
+  return !CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemmResidentKernel<C>), hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES));
+}
+bool residentReady(uint32_t columns) { return columns == 64 ? ready<ResidentCfg<64>>() : ready<ResidentCfg<128>>(); }
+
+template<class C>
 static cusync_error launchResident(const cusync_gemm_args* a, void* stream) {
   const cusync_stage_desc& s = a->stage;
   const bool waits = s.in.kind != CUSYNC_POLICY_NOSYNC;
@@ -16,8 +22,6 @@ static cusync_error launchResident(const cusync_gemm_args* a, void* stream) {
     rt::setError("gemm: not a problem for weights held in registers");
     return CUSYNC_ERROR_NOT_INITIALIZED;
   }
-  static const bool allowed = !CUSYNC_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemmResidentKernel<C>), hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES));
-  if (!allowed) return CUSYNC_ERROR_DEVICE;
   GemmParams p = {};
   p.stage.d = s;
   p.stage.lineAligned = waits && !rt::forceAcquire() && (uintptr_t)a->A % 128 == 0 && (a->lda * 2) % 128 == 0 &&

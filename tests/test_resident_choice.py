@@ -22,7 +22,7 @@ SRC = r"""
 #include "gemm_resident.h"
 int main(int argc, char** argv) {
   for (int i = 1; i + 2 < argc; i += 3)
-    std::printf("%d\n", (int)cusync::gemm::weightsFitRegisters((uint32_t)std::atoi(argv[i]), (uint32_t)std::atoi(argv[i + 1]), 128u * (uint32_t)std::atoi(argv[i + 2])));
+    std::printf("%d\n", (int)cusync::gemm::weightsFitRegisters((uint32_t)std::atoi(argv[i]), (uint32_t)std::atoi(argv[i + 1]), 128u * (uint32_t)std::atoi(argv[i + 2]), 256));
   return 0;
 }
 """
