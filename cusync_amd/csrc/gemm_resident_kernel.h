@@ -121,7 +121,6 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemmResidentKernel(GemmParams p
   const unsigned long long tl1 = p.timeline ? wall_clock64() : 0;
 
   const __amdgpu_buffer_rsrc_t rD = makeRsrc(p.D, p.M * p.ldd * 2);
-  const bool through = stage.storesThrough();
   for (uint32_t m0 = 0; m0 < p.M; m0 += C::ROWS) {
     if (m0 == 0) waitVmcnt<0>();
     else if (wave < C::STORING) waitVmcnt<1>();      // the store of the rows before is behind these rows' loads
@@ -175,8 +174,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemmResidentKernel(GemmParams p
 #pragma unroll
       for (int c = 0; c < 4; c++) o[c] = (half_t)sum[c];
       const int off = m0 + row < p.M && n0 + col < p.N ? (int)(((m0 + row) * p.ldd + n0 + col) * 2) : (int)kOutOfRange;
-      if (through) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, o), rD, off, 0, 16 /* sc1 */);
-      else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, o), rD, off, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, o), rD, off, 0, 16 /* sc1: the stage stamps its end */);
     }
     if (m0 + C::ROWS < p.M) __syncthreads();
   }
