@@ -99,6 +99,7 @@ struct cusync_attn_layer {
   int tile1, tile3;
   int split1, split3;              // k-slices of the two projections
   uint32_t resident3;              // the output projection holds its weights in registers (gemm_resident.h), this many columns a workgroup; 0: it does not
+  void* ws;                        // one allocation of the three workspaces
   void* ws1;
   void* ws3;                       // their split-K workspaces (null without slices)
   uint32_t kvSplit;                // key/value blocks per attention workgroup, 0 = no split
@@ -291,7 +292,7 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   if (cfg->tile1 < 0 && L->tile1 == CUSYNC_TILE_256x192x64 && (3 * L->E) % 384 == 0 &&
       cusync::gemm::wideInThreeSlices(3 * L->E / 384 * ((S + 255) / 256), cfg->hidden, cusync_gemm_max_resident(CUSYNC_TILE_256x384x32))) L->tile1 = CUSYNC_TILE_256x384x32;
   if (cfg->tile3 < 0 && S > 1024 && cfg->hidden % 384 == 0 && L->E % 64 == 0) L->tile3 = CUSYNC_TILE_256x384x32;
-  L->ws1 = L->ws3 = L->ws2 = nullptr;
+  L->ws = L->ws1 = L->ws3 = L->ws2 = nullptr;
   // Key ranges of 8 blocks (512 rows) or more are cut in two: under a causal mask the last row tiles walk the
   // longest ranges and the launch is as long as its longest workgroup.  Measured alone at 12 heads: 512 rows
   // 26.7 -> 25.3 us, 1024 rows 37.8 -> 30.8 us, 2048 rows 61 -> 50 us; finer cuts lose again (2048 rows in four:
@@ -379,25 +380,23 @@ cusync_attn_layer* cusync_attn_layer_create(const cusync_attn_layer_config* cfg,
   if (cfg->opts >= 0) opts |= cfg->opts;
 
   // ahead of the stages, which wait for what is cleared here (cusync_stage_alloc)
+  size_t bytes[3];
   for (int which = 0; which < 2; which++) {
     cusync_gemm_args a;
     memset(&a, 0, sizeof a);
     a.M = cfg->seq; a.N = which == 0 ? 3 * L->E : cfg->hidden; a.K = which == 0 ? cfg->hidden : L->E;
     a.tile = which == 0 ? L->tile1 : L->tile3;
     a.split_k = which == 0 ? L->split1 : L->split3;
-    const size_t bytes = cusync_gemm_workspace_size(&a);
-    if (bytes == 0) continue;
-    void* ws = nullptr;
-    if (CUSYNC_HIP(hipMalloc(&ws, bytes)) || CUSYNC_HIP(hipMemset(ws, 0, bytes))) { discardLayer(L); return nullptr; }
-    (which == 0 ? L->ws1 : L->ws3) = ws;
+    bytes[which] = cusync_gemm_workspace_size(&a);
   }
   {
     cusync_attention_args a;
     memset(&a, 0, sizeof a);
     a.seq = cfg->seq; a.heads = cfg->heads; a.cached_rows = cfg->cached_rows; a.kv_split_blocks = L->kvSplit;
-    const size_t bytes = cusync_attention_workspace_size(&a);
-    if (bytes && (CUSYNC_HIP(hipMalloc(&L->ws2, bytes)) || CUSYNC_HIP(hipMemset(L->ws2, 0, bytes)))) { discardLayer(L); return nullptr; }
+    bytes[2] = cusync_attention_workspace_size(&a);
   }
+  void** const parts[3] = {&L->ws1, &L->ws3, &L->ws2};
+  if (!cusync::rt::allocCleared(&L->ws, parts, bytes, 3)) { discardLayer(L); return nullptr; }
   const cusync_dim3 grids[3] = {g1, g2, g3};
   const cusync_policy_desc ins[3] = {noSync(), sync1, sync2}, outs[3] = {sync1, sync2, noSync()};
   for (int i = 0; i < 3; i++) {
@@ -430,9 +429,7 @@ void cusync_attn_layer_destroy(cusync_attn_layer* L) {
   for (int i = 0; i < 3; i++) cusync_stage_free(&L->st[i]);
   for (auto e : L->done) if (e) (void)hipEventDestroy(e);
   for (int i = 0; i < 3; i++) if (L->stream[i]) (void)hipStreamDestroy(L->stream[i]);
-  if (L->ws1) (void)hipFree(L->ws1);
-  if (L->ws3) (void)hipFree(L->ws3);
-  if (L->ws2) (void)hipFree(L->ws2);
+  if (L->ws) (void)hipFree(L->ws);
   delete L;
 }
 

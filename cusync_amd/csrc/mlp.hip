@@ -22,6 +22,7 @@ struct cusync_mlp {
   const void* w2;
   int tile1, tile2;
   int split1, split2;
+  void* ws;           // one allocation of the two workspaces
   void* ws1;
   void* ws2;
   uint32_t n1, k1, n2, k2;          // GEMM1 is [batch,k1]x[k1,n1], GEMM2 is [batch,k2]x[k2,n2]
@@ -440,7 +441,7 @@ cusync_mlp* cusync_mlp_create(const cusync_mlp_config* cfg, const void* w1, cons
   int opts = 0;
   const uint32_t tnOut = m->fused ? tn1 / 2 : tn1;      // width of a GEMM1 tile in columns of the intermediate
   m->split1 = ch.split1; m->split2 = ch.split2;
-  m->ws1 = m->ws2 = nullptr;
+  m->ws = m->ws1 = m->ws2 = nullptr;
   const cusync_dim3 g1 = cusync_gemm_grid(m->tile1, cfg->batch, m->n1, m->split1);
   const cusync_dim3 g2 = cusync_gemm_grid(m->tile2, cfg->batch, m->n2, m->split2);
   switch (sync) {
@@ -487,14 +488,10 @@ cusync_mlp* cusync_mlp_create(const cusync_mlp_config* cfg, const void* w1, cons
   memset(&m->prod, 0, sizeof m->prod);
   memset(&m->cons, 0, sizeof m->cons);
   // ahead of the stages, which wait for what is cleared here (cusync_stage_alloc)
-  for (int which = 0; which < 2; which++) {
-    cusync_gemm_args a = gemmArgs(m, which, nullptr, nullptr, nullptr);
-    const size_t bytes = cusync_gemm_workspace_size(&a);
-    if (bytes == 0) continue;
-    void* ws = nullptr;
-    if (CUSYNC_HIP(hipMalloc(&ws, bytes)) || CUSYNC_HIP(hipMemset(ws, 0, bytes))) { discard(m); return nullptr; }
-    (which == 0 ? m->ws1 : m->ws2) = ws;
-  }
+  const cusync_gemm_args gemms[2] = {gemmArgs(m, 0, nullptr, nullptr, nullptr), gemmArgs(m, 1, nullptr, nullptr, nullptr)};
+  const size_t wsBytes[2] = {cusync_gemm_workspace_size(&gemms[0]), cusync_gemm_workspace_size(&gemms[1])};
+  void** const wsParts[2] = {&m->ws1, &m->ws2};
+  if (!cusync::rt::allocCleared(&m->ws, wsParts, wsBytes, 2)) { discard(m); return nullptr; }
   m->prod.grid = g1; m->prod.tileSize = {1, 1, 1}; m->prod.iter = 1; m->prod.opts = opts;
   m->prod.in = noSync(); m->prod.out = pol;
   m->cons.grid = g2; m->cons.tileSize = {1, 1, 1}; m->cons.iter = 1; m->cons.opts = opts;
@@ -571,8 +568,7 @@ void cusync_mlp_destroy(cusync_mlp* m) {
   cusync_stage_free(&m->cons);
   cusync_stage_free(&m->mid);
   if (m->act) (void)hipFree(m->act);
-  if (m->ws1) (void)hipFree(m->ws1);
-  if (m->ws2) (void)hipFree(m->ws2);
+  if (m->ws) (void)hipFree(m->ws);
   if (m->w1p) (void)hipFree(m->w1p);
   if (m->w2p) (void)hipFree(m->w2p);
   for (auto e : m->done) if (e) (void)hipEventDestroy(e);

@@ -82,6 +82,22 @@ cusync_error checkSpinTimeouts(const cusync_stage_desc* const* stages, int count
   return CUSYNC_ERROR_DEVICE;
 }
 
+bool allocCleared(void** block, void** const* parts, const size_t* bytes, int count) {
+  const size_t line = 256;
+  size_t all = 0;
+  for (int i = 0; i < count; i++) all += (bytes[i] + line - 1) / line * line;
+  *block = nullptr;
+  for (int i = 0; i < count; i++) *parts[i] = nullptr;
+  if (all == 0) return true;
+  if (CUSYNC_HIP(hipMalloc(block, all)) || CUSYNC_HIP(hipMemset(*block, 0, all))) return false;
+  char* at = (char*)*block;
+  for (int i = 0; i < count; i++) {
+    if (bytes[i]) *parts[i] = at;
+    at += (bytes[i] + line - 1) / line * line;
+  }
+  return true;
+}
+
 static unsigned long long stampOf(const cusync_stage_desc& s, int which) {
   return __atomic_load_n(reinterpret_cast<const unsigned long long*>(s.spinTimeouts + CUSYNC_HOST_STAMP_OFFSET) + which, __ATOMIC_ACQUIRE);
 }
