@@ -175,10 +175,15 @@ int rowsCUs() {
 
 // Rows of the product per workgroup of convRowsKernel (conv3x3_rows_kernel.h) for a layer of 64 channels, a workgroup per CU: whole
 // sixteens, no fewer than four wavefronts have work for; 0 where its input tile and the filter do not fit the LDS.
-uint32_t rowsPerWorkgroup(uint32_t N, uint32_t H, uint32_t W) {
+// `overlapped`: the layers' launches go beside each other.  Where a workgroup for each CU comes out, which happens at whole multiples of
+// 4096 rows, a run is sixteen rows longer: a consumer finds no CU free otherwise and is held back by the host until all of its producer
+// has started, layer by layer (16x16 images under RowSync, us, 256 workgroups / this: 20 480 rows, two layers 29.9 / 24.3, four 57.1 / 42.4;
+// 32 768 rows, where the sixteen are a turn more of each wavefront, 29.8 / 25.7 and 57.6 / 44.8; 98 304 rows 32.2 / 32.5 and 61.1 / 57.5).
+uint32_t rowsPerWorkgroup(uint32_t N, uint32_t H, uint32_t W, bool overlapped) {
   const uint32_t M = N * H * W, cus = (uint32_t)rowsCUs();
   if (!cus) return 0;
-  const uint32_t rows = std::max<uint32_t>(ConvRowsCfg::WAVES * ConvRowsCfg::T, ((M + cus - 1) / cus + ConvRowsCfg::T - 1) / ConvRowsCfg::T * ConvRowsCfg::T);
+  uint32_t rows = std::max<uint32_t>(ConvRowsCfg::WAVES * ConvRowsCfg::T, ((M + cus - 1) / cus + ConvRowsCfg::T - 1) / ConvRowsCfg::T * ConvRowsCfg::T);
+  if (overlapped && (M + rows - 1) / rows >= cus && ConvRowsCfg::ldsBytes(rows + ConvRowsCfg::T, W) <= kMaxLds) rows += ConvRowsCfg::T;      // (the kernel itself is the same for every sync)
   return ConvRowsCfg::ldsBytes(rows, W) <= kMaxLds ? rows : 0;
 }
 
@@ -459,7 +464,7 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
                   : cfg->C % 128 == 0 ? CUSYNC_CONV_TILE_128x128x32 : CUSYNC_CONV_TILE_256x64x32;
   // 64 channels, the built-in choice: tiles of 256 rows for the policies, the rows themselves dealt evenly to the CUs.
   if (cfg->tile < 0 && cfg->split_k <= 1 && cfg->C == ConvRowsCfg::CHANNELS && c->cfg.tile == CUSYNC_CONV_TILE_HALO_256x64x64 && ownKernels) {
-    c->rows = rowsPerWorkgroup(cfg->N, cfg->H, cfg->W);
+    c->rows = rowsPerWorkgroup(cfg->N, cfg->H, cfg->W, cfg->sync != CUSYNC_SYNC_STREAM && cfg->layers > 1);
     c->splitK = 1;
   }
   uint32_t tm = 0, tn = 0;

@@ -74,3 +74,23 @@ def test_chain_of_64_channels_in_one_launch_or_with_a_tile_given():
         assert all(st.spin_timeouts == 0 for st in states)
         for i in range(2):
             assert_close(got[i], want[i], "y%d" % i)
+
+
+def test_overlapped_layers_leave_cus_free():
+    # 20480 rows are 256 runs of 80; a consumer that finds no CU free is held back until its producer has started everywhere
+    import torch
+    from test_gpu_conv_avoid_wait import launched
+    N, H, W = 5, 64, 64
+    print("conv rows, CUs left", flush=True)
+    rng = np.random.default_rng(3)
+    dx = to_dev(rng.integers(-2, 3, (N, H, W, 64)).astype(np.float16))
+    dws = [to_dev((rng.integers(-1, 2, (64, 3, 3, 64)) / 16).astype(np.float16)) for _ in range(2)]
+    outs = []
+    for sync, layers, workgroups in ((api.SYNC.STREAM, 1, 256), (api.SYNC.ROW, 2, 214), (api.SYNC.TILE, 2, 214)):
+        dys = [empty_dev((N, H, W, 64), fill=float("nan")) for _ in range(layers)]
+        torch.cuda.synchronize()
+        chain = api.ConvChain(N, H, W, 64, [w.data_ptr() for w in dws[:layers]], sync, relu=False)
+        assert launched(chain, dx, dys, layers) == [{workgroups}] * layers, sync
+        chain.destroy()
+        outs.append([to_host(y).view(np.uint16) for y in dys])
+    assert np.array_equal(outs[1][0], outs[0][0]) and np.array_equal(outs[2][0], outs[0][0]) and np.array_equal(outs[1][1], outs[2][1])
