@@ -76,9 +76,9 @@ uint32_t haloLds(int tile, uint32_t W, uint32_t C) { return g_convTiles[tile].ha
 constexpr uint32_t kMaxLds = 160 * 1024 - 1024;      // what one workgroup may ask for (the kernel has 8 bytes of static LDS)
 
 // The halo kernel needs 3x3, pad 1, stride 1, a power-of-two channel count of at least 64, and its tile plus
-// halo in LDS.
+// halo in LDS.  (Two lines of pixels first: of images wider than that the bytes of the halo can wrap around 32 bits.)
 bool haloEligible(int tile, uint32_t W, uint32_t C, uint32_t R, uint32_t S, uint32_t pad, uint32_t stride) {
-  return R == 3 && S == 3 && pad == 1 && stride == 1 && C >= 64 && (C & (C - 1)) == 0 && haloLds(tile, W, C) <= kMaxLds;
+  return R == 3 && S == 3 && pad == 1 && stride == 1 && C >= 64 && (C & (C - 1)) == 0 && (uint64_t)W * C * 4 <= kMaxLds && haloLds(tile, W, C) <= kMaxLds;
 }
 
 std::mutex g_convMutex;
