@@ -146,7 +146,8 @@ int residentConv(ConvTile* ti, size_t lds) {
 // runs and every one of the launch's `parts` has a workgroup from the start; null elsewhere (three runs, five, a cap, several
 // rounds: the tile's own kernel with its steps in runs).  Where both can run, this one is ahead at every size measured: pairs
 // under RowSync, us, runs -> this, 128x128 tile in two 1x14x14x256 45 -> 33, 32x14x14x256 47 -> 36, in four 8x14x14x256 39.2 -> 34.0;
-// 64x128 tile in two 32x7x7x512 49.6 -> 42.2, in four 16x7x7x512 40.3 -> 37.1, in eight 2x7x7x512 34.4 -> 30.4.
+// 64x128 tile in two 32x7x7x512 49.6 -> 42.2, in four 16x7x7x512 40.3 -> 37.1, in eight 2x7x7x512 34.4 -> 30.4; one convolution by
+// itself, 128x128 tile, 4x28x28x64 in two, four and eight 13.9 -> 9.4, 14.4 -> 11.4, 17.2 -> 12.2, and nowhere behind at 64 to 512 channels.
 // Not under AvoidWaitKernel (`opts`): its caller has seen to it that all stages fit on the device at once, by the tile and what
 // cusync_conv2d_max_resident says of it, and here a workgroup has a CU to itself.
 ConvTile* soloTileFor(int tile, int split, uint32_t parts, uint32_t W, uint32_t C, int opts) {
@@ -477,20 +478,20 @@ cusync_conv_chain* cusync_conv_chain_create(const cusync_conv_chain_config* cfg,
   }
   cusync_dim3 g = cusync_conv2d_grid(c->cfg.tile, cfg->N, cfg->H, cfg->W, cfg->C, 3, 3, 1, 1);
   if (g.x == 0 || g.y == 0) { setError("conv chain: empty shape"); delete c; return nullptr; }
-  // Layers whose tiles leave most of the device idle (14 x 14 x 256 at batch 32: 98 tiles; 7 x 7 x 512: 100) have the
-  // 9 * C / 64 steps of a tile cut into runs, a workgroup each, whose partial sums are put together as the GEMM's
-  // k-slices are: as many runs as stay resident together, of at least nine steps each (measured, pairs in us without
-  // runs -> with: 32x14x14x256 63 -> 54 in two; 32x7x7x512 82 -> 59 in two; 8x14x14x256 65 -> 50 in four;
+  // What is left for runs: a tile that the caller gives, AvoidWaitKernel, and layers whose halo fits beside the tile kernel's ring of filter
+  // stages but not beside the 64 KB of the kernel above (512 channels, images 15 and 16 wide).  Where their tiles leave most of the device
+  // idle the 9 * C / 64 steps of a tile are cut into runs, a workgroup each, whose partial sums are put together as the GEMM's
+  // k-slices are: as many runs as stay resident together, of at least nine steps each (pairs in us without runs -> with, all under
+  // AvoidWaitKernel or with the tile given: 32x14x14x256 63 -> 54 in two; 32x7x7x512 82 -> 59 in two; 8x14x14x256 65 -> 50 in four;
   // 1x7x7x512 82 -> 43 in eight; with shorter runs the exchange costs more than the idle CUs: 1x56x56x64 35 -> 50
-  // in nine runs of one step), and a number the 32-row pieces of a 128-row tile divide among, so that the runs
-  // share the adding up.
+  // in nine runs of one step), and at 128 rows a tile two or four of them.
   if (cfg->split_k > 0) c->splitK = cfg->split_k;
   else if (c->splitK == 0 && isHalo(c->cfg.tile) && !(c->cfg.fused && cfg->sync != CUSYNC_SYNC_STREAM)) {
     ConvTile* ti = convTileFor(c->cfg.tile, cfg->W, cfg->C);
     const int resident = residentConv(ti, ti->haloLds(cfg->W, cfg->C));
     const uint32_t tiles = g.x * g.y, steps = 9 * (cfg->C / 64);
     uint32_t s = resident > 0 && tiles * 2 <= (uint32_t)g_convNumCUs ? std::min<uint32_t>((uint32_t)resident / tiles, steps / 9) : 1u;
-    if (tm >= 128) s = s >= 4 ? 4 : s == 3 ? 2 : s;      // a 128-row tile's four pieces divide among two or four runs
+    if (tm >= 128) s = s >= 4 ? 4 : s == 3 ? 2 : s;
     while (s > 1 && (steps + s - 1) / s * (s - 1) >= steps) s--;      // no run without steps
     c->splitK = (int)std::max(1u, s);
   }
@@ -641,8 +642,8 @@ cusync_error cusync_conv_chain_run(cusync_conv_chain* c, const void* x, void* co
       const cusync_conv2d_args a = layerArgs(i);
       cusync_error e;
       // overlapped: layer i's stream is held back until layer i - 1 is on the device: by the reference's wait kernel
-      // where that layer's launch left workgroup slots free (392 tiles on 512 slots for the benchmark shapes), so
-      // that the wait kernel's wave takes nothing from the producer; from this thread where the launch took them all.
+      // where that layer's launch left workgroup slots free (32x56x56x64: 251 workgroups on 256 CUs), so that the wait
+      // kernel's wave takes nothing from the producer; from this thread where the launch took them all.
       if (overlapped && i > 0 && (e = cusync_hold_back(&c->st[i - 1], s)) != CUSYNC_SUCCESS) return failed(e);
       e = c->rows ? runRows(&a, c->rows, scratchOf(c, i), s) : launchConv(&a, c->kernel, c->resident, scratchOf(c, i), s);
       if (e != CUSYNC_SUCCESS) return i ? failed(e) : e;

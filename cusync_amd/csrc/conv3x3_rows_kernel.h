@@ -7,8 +7,11 @@
 // registers, and takes 16 rows at a time to all 64 columns: one LDS read for four MFMAs, and no barrier once the run's pixels
 // and halo have landed.  A tile is posted by the workgroup that finishes its last rows (a count of rows per tile).
 //
-// Pairs, us, 256x64 tiles -> this: 1x56x56x64 under RowSync 27.6 -> 18.4, 4x 27.9 -> 21.0, 16x 30.9 -> 26.3, 32x 38.2 -> 32.2 (a
-// layer alone 16 -> 11).  What bounds it at 32 images: seven times 72 MFMAs a wavefront take 7.9 us (5.1 us by themselves at the 1.95 GHz
+// Pairs, us, 256x64 tiles -> this: 1x56x56x64 under RowSync 27.6 -> 18.8, 4x 27.6 -> 21.3, 16x 31.2 -> 27.5, 32x 39.7 -> 34.3 (a
+// layer's kernel alone 16 -> 11).  Longer chains: four layers 1x 47.6 -> 30.2, 16x 53.1 -> 47.3, 32x 62.0 -> 58.6; sixteen 1x 176 -> 112, 16x 180 -> 171,
+// 32x 217 -> 218 (214 -> 218 on another machine; in stream order 279 -> 239): there the middle layers' workgroups, which count themselves
+// started only behind their own wait, hold back the layer after them.  (Counted ahead of the wait: 8 images, four layers 44.3 -> 40.5, 32 images 58.6 ->
+// 60.2.)  What bounds it at 32 images: seven times 72 MFMAs a wavefront take 7.9 us (5.1 us by themselves at the 1.95 GHz
 // the device runs them at; stores 0.7, the rest issue slots, one wavefront per SIMD having all the registers), loads before them 2.6.
 // 32 rows at a time (half the address arithmetic, but 13 tiles of 32 rows do not divide among four wavefronts): level there,
 // 19.4 at one image.

@@ -6,12 +6,12 @@
 // device have their steps cut into runs whose sums go through memory.  Here a wavefront takes whole units (64 channels of one
 // tap) by itself, every fourth one: BM x 64 outputs in its accumulators, a ring of its own for its units' filter rows, no
 // barrier between the halo's arrival and the end.  The four partial sums come together through LDS, a quarter of the tile per
-// wavefront.  A fragment read from LDS is used twice (filter) or TM times (halo): 6 reads per 8 MFMAs of the 128-row tile,
+// wavefront.  A fragment read from LDS is used twice (halo) or TM times (filter): 6 reads per 8 MFMAs of the 128-row tile,
 // where 64 x 64 per wavefront takes 8.
 //
-// Pairs, us, this kernel against tiles in runs: 32x14x14x256 under TileSync 48.9 -> 37.1, RowSync 47.2 -> 36.4 (a layer's loop 10.3
-// -> 8.2, start to first load 2.0 -> 0.3, exchange and store 4.5 -> 2.2); 8x14x14x256 39.2 -> 27.4; 32x7x7x512 49.6 -> 42.3; 8x28x28x128
-// 35.3 -> 24.5; 1x28x28x128 33.9 -> 21.9.  What bounds it at 32x14x14x256: MFMAs alone on as many CUs take 5.8 us a layer (1.95 GHz
+// Pairs, us, tiles in runs -> this kernel, under RowSync: 32x14x14x256 49.1 -> 37.3, under TileSync 49.5 -> 38.1 (a layer's loop 10.3
+// -> 8.2, start to first load 2.0 -> 0.3, exchange and store 4.5 -> 2.2); 8x14x14x256 39.4 -> 27.0; 32x7x7x512 51.3 -> 42.6; 8x28x28x128
+// 35.2 -> 24.7; 1x28x28x128 33.6 -> 22.0.  Chains of four: 32x14x14x256 85.3 -> 65.4, 1x14x14x256 67.7 -> 45.6, 32x7x7x512 89.9 -> 76.4.  What bounds it at 32x14x14x256: MFMAs alone on as many CUs take 5.8 us a layer (1.95 GHz
 // on such data), the loop 7.7 without its direct loads; at 512 channels the filter: 590 KB per workgroup at 53 bytes/ns.
 //
 // A workgroup has one tile and the launch a workgroup for each (soloTileFor): with a loop over tiles around it the compiler

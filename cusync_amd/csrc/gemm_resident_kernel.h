@@ -9,9 +9,10 @@
 // trips, 3 us for up to 16 rows, 1.7 us for each further 16, which bounds it.  K goes to the wavefronts the same way whatever the
 // columns, so results do not depend on them.
 //
-// The layer, 12 heads, hidden 12288, us, tiles in k-slices -> this: 16 rows behind 2048 under RowSync 60.8 -> 55.0, TileSync 58.6 ->
-// 53.3; 32 behind 2048 62.3 -> 58.3; 1 behind 64 53.0 -> 47.1; without a cache under RowSync 16 rows 53.7 -> 51.1, 64 64.9 -> 61.1,
-// 96 82.0 -> 77.7, 112 83.1 -> 79.9; in stream order 48 rows 67.8 -> 63.0, 80 rows 82.5 -> 79.2.
+// The layer, 12 heads, hidden 12288, us, tiles in k-slices -> this, each pass on other operands than the one before: behind 2000 rows
+// under RowSync 1 row 59.0 -> 52.3, 16 60.3 -> 54.4, 32 61.9 -> 57.6, 64 77.7 -> 73.4, 112 93.8 -> 92.5; TileSync 16 rows 58.2 -> 52.2; without a
+// cache under RowSync 16 rows 53.7 -> 51.0, 64 65.0 -> 60.9, 96 82.1 -> 76.8; in stream order, where nothing is read ahead and the gain is the k-slices'
+// exchange, 1 row 56.6 -> 53.1, 16 57.3 -> 54.9, 32 58.7 -> 57.7, 64 69.4 -> 66.0, 112 85.2 -> 85.1.  (Which projections: weightsFitRegisters.)
 //
 // A workgroup has a CU's LDS to itself although it would do with half: two to a CU, half the CUs read all the weights, and 16 rows
 // behind 2048 took 61.4 us.

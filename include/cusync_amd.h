@@ -380,7 +380,8 @@ typedef struct cusync_conv2d_args {
   int32_t max_workgroups;      /* 0 = as many as stay resident */
   int32_t split_k;             /* Conv2dProblemSize::split_k_slices (CV/resnet.cu:246, 689, 765): 0 or 1 = none; n (halo tiles):
                                   a tile is n workgroups', grid z = n: the R*S*C/64 steps in n runs, partial sums added in run
-                                  order, or (128x128 and 64x128 tiles, n = 2, 4, 8, all resident) n/2 runs of each half of the columns */
+                                  order, or (128x128 and 64x128 tiles, n = 2, 4, 8, all resident, no CUSYNC_OPT_AVOID_WAIT_KERNEL)
+                                  n/2 runs of each half of the columns */
   void *workspace;             /* split_k > 1: cusync_conv2d_workspace_size bytes, 16-byte aligned; its counters (the last
                                   2 * tiles words) zero before the first run, the kernel leaves them zero */
 } cusync_conv2d_args;
@@ -430,8 +431,11 @@ void cusync_conv_chain_destroy(cusync_conv_chain *chain);
 cusync_error cusync_conv_chain_run(cusync_conv_chain *chain, const void *x, void *const *ys, int runs,
                                    double *times_us, double *layer_us);
 const cusync_stage_desc *cusync_conv_chain_stage(const cusync_conv_chain *chain, uint32_t which);
+/* The tile of the stages' grids and policies, and the workgroups a tile is divided among (cusync_conv2d_args.split_k).  Left to the chain
+ * and without CUSYNC_OPT_AVOID_WAIT_KERNEL, layers of 64 channels take a kernel that deals runs of rows to the CUs: tile and grid are
+ * then those it posts by, and its launch has up to a workgroup per CU, each with a CU to itself, whatever their number. */
 int cusync_conv_chain_tile(const cusync_conv_chain *chain);
-int cusync_conv_chain_split(const cusync_conv_chain *chain);      /* runs per tile the chain runs with */
+int cusync_conv_chain_split(const cusync_conv_chain *chain);
 
 /* ------------------------------------------------------------------------- */
 /* Fused multi-head attention stage: O = softmax(mask(Q K^T * scale)) V per    */

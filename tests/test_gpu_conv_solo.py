@@ -64,6 +64,21 @@ def test_chain_choice(shape, choice):
             assert np.array_equal(outs[sync][i].view(np.uint16), src.view(np.uint16)), (sync, i)
 
 
+def test_chain_whose_halo_leaves_no_room_for_halves():
+    # 512 channels, 16 wide: the halo fits beside the 48 KB ring of the tile's own kernel and not beside 64 KB; its tiles take eight runs
+    print("conv chain in runs", flush=True)
+    outs = {}
+    for sync in (api.SYNC.STREAM, api.SYNC.ROW, api.SYNC.TILE):
+        x, ws, ys, states, tile, _ = run_chain(1, 16, 16, 512, 2, sync, runs=2)
+        assert (tile, run_chain.split) == (T64, 8)
+        assert all(st.spin_timeouts == 0 for st in states)
+        outs[sync] = ys
+    for i, src in enumerate((x, outs[api.SYNC.STREAM][0])):
+        assert_close(outs[api.SYNC.STREAM][i], orc.conv2d_nhwc(src, ws[i], epilogue=orc.EPI_RELU if i == 0 else orc.EPI_NONE), "y%d" % i)
+        for sync in (api.SYNC.ROW, api.SYNC.TILE):
+            assert np.array_equal(outs[sync][i].view(np.uint16), outs[api.SYNC.STREAM][i].view(np.uint16)), (sync, i)
+
+
 def test_rounding_of_parts():
     # random operands: the distance the other tiles' tests allow
     for tile, parts in ((T128, 2), (T128, 4), (T64, 8)):
